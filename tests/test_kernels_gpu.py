@@ -167,6 +167,36 @@ def test_linear_bf16(ops, algo, m, n, k):
     assert rel_l2(got_d, ref) < 4e-3
 
 
+# the tiles of 8 waves (12: 256 x 256, 13: 256 x 192, 14: 192 x 256, 15: 256 x 128): one k step, two, three and a long odd number
+# of them, a tile and one row more or less, an N that is no multiple of 8 or 4 (outputs element by element), a last K slice
+# that is shorter, more tiles than CUs
+@pytest.mark.parametrize("algo", [12, 13, 14, 15])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (255, 257, 64), (257, 190, 128), (192, 384, 192), (193, 129, 320), (300, 1001, 1088),
+                                   (513, 2304, 2048), (1000, 250, 4672), (2100, 9000, 192)])
+def test_linear_wide_tiles(ops, algo, m, n, k):
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=7), randn(n, k, dtype=torch.bfloat16, seed=8, scale=0.05)
+    into = torch.full((m * n + 1,), 7.0, dtype=torch.bfloat16, device=DEV)
+    half = n // 2 // 16 * 16
+    ops.force_linear = algo
+    try:
+        got_b = ops.linear(x, w, torch.bfloat16)
+        got_f = ops.linear(x, w, torch.float32, softcap=3.0)
+        got_d = ops.rows(ops.linear(x, w, torch.bfloat16, defer=True), torch.float32)
+        got_s = ops.linear_act(x, w, torch.float32, "silu", columns=n // 2 or 1)
+        ops.linear(x, w, torch.bfloat16, out=into[1:].view(m, n))                         # two bytes beyond an aligned address
+        got_g = ops.gated_linear(x, ops.pack_gate_up(w[:half - 3], w[half:2 * half - 3]), half - 3, "silu", torch.bfloat16) if half else None
+    finally:
+        ops.force_linear = 0
+    ref = x.cpu().double() @ w.cpu().double().T
+    assert rel_l2(got_b, ref) < 4e-3 and rel_l2(got_d, ref) < 4e-3
+    assert rel_l2(got_f, 3.0 * torch.tanh(ref / 3.0)) < 1e-5
+    split = n // 2 or 1
+    assert rel_l2(got_s, torch.cat([torch.nn.functional.silu(ref[:, :split]), ref[:, split:]], 1)) < 1e-5
+    assert torch.equal(into[1:].view(m, n), got_b) and float(into[0]) == 7.0
+    if half:
+        assert rel_l2(got_g, torch.nn.functional.silu(ref[:, :half - 3]) * ref[:, half:2 * half - 3]) < 4e-3
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (8, 2304, 2048), (70, 331, 88), (300, 77, 136)])
 def test_linear_with_a_bias(ops, dt, m, n, k):

@@ -55,3 +55,7 @@ int gemm_rows8_launch(const GemmArgs& a);
 bool gemm_mfma_supports(const GemmArgs& a);
 int gemm_mfma_splits(const GemmArgs& a);
 int gemm_mfma_launch(const GemmArgs& a);
+// bf16 on the matrix cores for many rows, blocks of 8 waves (K a multiple of 64): rows of X by rows of W a block, K in `splits`
+// slices of kps elements (left in the workspace when there are several)
+enum { TP_WIDE_256x256 = 0, TP_WIDE_256x192, TP_WIDE_192x256, TP_WIDE_256x128, TP_WIDE_SHAPES };
+int gemm_wide_launch(const GemmArgs& a, int shape, int splits, int kps);

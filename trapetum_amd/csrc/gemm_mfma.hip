@@ -316,7 +316,7 @@ gemm_mfma_direct_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, v
 }
 
 bool gemm_mfma_supports(const GemmArgs& a) {
-    if (a.algo == 8 || a.algo == 9) return a.in_dtype == TP_BF16 && a.K % BK == 0 && (long)(a.M > a.N ? a.M : a.N) * a.K * 2 < (1L << 32);
+    if (a.algo == 8 || a.algo == 9 || a.algo >= 12) return a.in_dtype == TP_BF16 && a.K % BK == 0 && (long)(a.M > a.N ? a.M : a.N) * a.K * 2 < (1L << 32);
     return a.in_dtype == TP_BF16 && a.K % 8 == 0;
 }
 
@@ -326,7 +326,7 @@ bool gemm_mfma_supports(const GemmArgs& a) {
 // instruction; two blocks fit a CU) for grids of at least four rounds of those 512 places (2B gate/up, register-staged:
 // 930 against 790 TFLOP/s at 8192 rows, 700 against 790 at 2048).
 struct Tile { int tm, tn, wm = 2; bool deep = false; };        // wm: waves along the rows of X (2 x 2 or 4 x 1)
-struct Plan { Tile tile; int splits; bool direct = false; };
+struct Plan { Tile tile; int splits; bool direct = false; int wide = -1; };       // wide: TP_WIDE_* of the kernel of 8 waves
 
 // K slices of a product of few rows, which is bound by reading W and wants every CU streaming.  From 17 rows on one
 // block a CU: more slices cost their consumer more than they gain (a 2B decode step of 64 sequences takes 3.52 ms
@@ -354,9 +354,35 @@ static double direct_step_us(long blocks) {
     return (double)(per_cu / 3) * 1.43 + (rest == 2 ? 1.17 : rest == 1 ? 1.0 : 0.0);
 }
 
+// The kernel of 8 waves runs a block a CU: rounds of 256 blocks, each a fixed part and a time per k step of 64, shorter while
+// the grid leaves CUs idle (clock and L2 are shared).  Fitted to 2B and 9B products at 1,716 to 8,192 rows, cold weights
+// (256 x 256: 174 us for 3 rounds of 36 steps, 1,310 for 14 of 56, 193 for 2 of 64, 680 for 2 of 224); within 8 per cent of
+// each of the 40 measured.  The loop of 128-row tiles is priced 1.17 times its model above, which is what it takes with cold
+// weights beside these.
+struct WideShape { int bm, bn; double fixed_us, step_us; };
+static const WideShape WIDE[TP_WIDE_SHAPES] = {{256, 256, 4.0, 1.52}, {256, 192, 6.0, 1.18}, {192, 256, 4.5, 1.13}, {256, 128, 2.5, 0.90}};
+
+static double wide_us(const WideShape& w, long blocks, double k_steps) {
+    const double part = blocks < 256 ? 0.75 + 0.25 * (double)blocks / 256 : 1.0;
+    return (double)tp_cdiv(blocks, 256) * (w.fixed_us + w.step_us * k_steps * part);
+}
+
+static Plan wide_plan(const GemmArgs& a, int shape, bool may_slice, double slice_us, double* cost) {
+    const WideShape& w = WIDE[shape];
+    Plan best{{4, 4}, 1, false, shape};
+    *cost = 1e30;
+    for (int s = 1; s <= (may_slice ? 4 : 1); s++) {
+        if (s > 1 && a.K / s < 512) break;
+        const double c = wide_us(w, (long)tp_cdiv(a.M, w.bm) * tp_cdiv(a.N, w.bn) * s, (double)tp_cdiv(tp_cdiv(a.K, s), BK)) + (s - 1) * slice_us;
+        if (c < *cost) { *cost = c; best.splits = s; }
+    }
+    return best;
+}
+
 // (tile, K slices) of a product of many rows: the cheapest by the model above (register-staged loop, for a K that is
 // no multiple of 64: the most blocks a CU gets x 0.64 us a step, fitted to the 2B down product at 2,048 rows), plus
-// what writing and reading a further float32 slice of Y costs.
+// what writing and reading a further float32 slice of Y costs.  The wide tiles of
+// gemm_wide.hip take part where they can run.
 static Plan mid_tile_plan(const GemmArgs& a, bool may_slice) {
     const double step_us = 0.64, slice_us = (double)a.M * a.N * 8 / 4.0e6;
     const bool direct = direct_ok(a) && a.algo != 7;
@@ -371,18 +397,27 @@ static Plan mid_tile_plan(const GemmArgs& a, bool may_slice) {
             // a grid of at most one block a CU is faster by the register-staged loop (0.85 us a step against 1.0:
             // 128 x 96 tiles at 512 rows, 2B shapes: qkv 30.7 against 35.5 us, down 102 against 119)
             const bool d = direct && tiles * s > 256;
-            const double per_step = d ? direct_step_us(tiles * s) : tiles * s <= 256 ? 0.85 : (double)tp_cdiv(tiles * s, 256) * step_us;
+            const double per_step = d ? 1.17 * direct_step_us(tiles * s) : tiles * s <= 256 ? 0.85 : (double)tp_cdiv(tiles * s, 256) * step_us;
             const double cost = per_step * k_steps * (tn == 3 ? 0.8 : 1.0) + (s - 1) * slice_us;
             if (cost < best_cost * 0.97) { best_cost = cost; best = {{4, tn}, s, d}; }   // a tie stays with the earlier, plainer plan
         }
+    }
+    for (int shape = 0; direct && shape < TP_WIDE_SHAPES; shape++) {
+        double cost;
+        const Plan p = wide_plan(a, shape, may_slice, slice_us, &cost);
+        if (cost < best_cost * 0.97) { best_cost = cost; best = p; }
     }
     return best;
 }
 
 static Plan plan_of(const GemmArgs& a) {
-    const bool may_slice = a.defer && a.epilogue == TP_EPI_NONE && (a.algo < 6 || a.algo == 11);
+    const bool may_slice = a.defer && a.epilogue == TP_EPI_NONE && (a.algo < 6 || a.algo == 11 || a.algo >= 12);
     if (a.algo == 10) return {{1, 2, 4, true}, 1};
     if (a.algo == 11) return {{2, 2, 2, true}, may_slice ? small_tile_splits(a, (long)tp_cdiv(a.M, 64) * tp_cdiv(a.N, 64)) : 1};
+    if (a.algo >= 12) {
+        double cost;
+        return wide_plan(a, a.algo - 12, may_slice, (double)a.M * a.N * 8 / 4.0e6, &cost);
+    }
     if (a.algo == 6) return {{4, 8}, 1};
     if (a.algo == 7) return {{4, a.epilogue == TP_EPI_GATED ? 4 : 3}, 1};
     if (a.algo == 8) return {{4, 4}, 1, true};
@@ -476,10 +511,12 @@ int gemm_mfma_launch(const GemmArgs& a) {
         TP_REQUIRE(a.workspace && a.workspace_bytes >= need, "tiled product: workspace of %zu bytes, %zu needed", a.workspace_bytes, need);
         const int kstep = t.tm <= 2 ? SMALL_KS : BK;
         const int kps = tp_cdiv(tp_cdiv(a.K, splits), kstep) * kstep;
+        if (plan.wide >= 0) return gemm_wide_launch(a, plan.wide, tp_cdiv(a.K, kps), kps);
         if (plan.direct) mfma_launch_direct<TP_EPI_NONE>(a, t, a.workspace, TP_F32, tp_cdiv(a.K, kps), kps);
         else mfma_launch_tile<TP_EPI_NONE>(a, t, a.workspace, TP_F32, tp_cdiv(a.K, kps), kps);
         return tp_check_launch("linear (tiled kernel, K slices)");
     }
+    if (plan.wide >= 0) return gemm_wide_launch(a, plan.wide, 1, a.K);
     if (plan.direct) {
         if (a.epilogue == TP_EPI_GATED) mfma_launch_direct<TP_EPI_GATED>(a, t, a.y, a.out_dtype, 1, a.K);
         else if (a.epilogue == TP_EPI_SOFTCAP) mfma_launch_direct<TP_EPI_SOFTCAP>(a, t, a.y, a.out_dtype, 1, a.K);
