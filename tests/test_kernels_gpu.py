@@ -224,6 +224,33 @@ def test_linear_f32(ops, m, n, k):
     assert torch.equal(alone[0], got[m - 1])
 
 
+# few rows (up to 32) and many, a row tile and one more or less, parts of K that end inside a block of 16 or are empty, a K of one
+# piece, K slices for the consumer, two tiles of W a block (from 16384 rows of W on), operands off their 16 bytes
+@pytest.mark.parametrize("m,n,k", [(1, 16, 4), (16, 17, 260), (17, 2304, 2048), (32, 33, 2300), (33, 129, 36), (64, 500, 1028), (309, 250, 4100),
+                                   (5, 16400, 68), (20, 16390, 84), (70, 200, 71)])
+def test_linear_f32_is_one_order(ops, m, n, k):
+    x, w = randn(m, k, seed=9), randn(n, k, seed=10, scale=0.05)
+    half = n // 2 // 16 * 16
+    ref = x.cpu().double() @ w.cpu().double().T
+    got = ops.linear(x, w, torch.float32)
+    assert rel_l2(got, ref) < 2e-6
+    assert rel_l2(ops.linear(x, w, torch.float32, softcap=3.0), 3.0 * torch.tanh(ref / 3.0)) < 2e-6
+    # the bits of an element are those of its row alone, of the product left in slices, and of a view that starts anywhere
+    row = m // 2
+    assert torch.equal(ops.linear(x[row:row + 1].contiguous(), w, torch.float32)[0], got[row])
+    assert torch.equal(ops.rows(ops.linear(x, w, torch.float32, defer=True), torch.float32), got)
+    off = torch.empty(m * k + 1, device=DEV)[1:].view(m, k)
+    off.copy_(x)
+    assert rel_l2(ops.linear(off, w, torch.float32), ref) < 2e-6
+    if half > 3:
+        packed = ops.pack_gate_up(w[:half - 3], w[half:2 * half - 3])
+        gated = ops.gated_linear(x, packed, half - 3, "silu", torch.float32, limit=2.0, up_shift=0.5)
+        g, u = ref[:, :half - 3].clamp(max=2.0), ref[:, half:2 * half - 3].clamp(-2.0, 2.0)
+        assert rel_l2(gated, torch.nn.functional.silu(g) * (u + 0.5)) < 5e-6
+        assert torch.equal(ops.gated_linear(x[row:row + 1].contiguous(), packed, half - 3, "silu", torch.float32, limit=2.0, up_shift=0.5)[0], gated[row])
+        assert rel_l2(ops.gated_linear(off, packed, half - 3, "silu", torch.float32, limit=2.0, up_shift=0.5), gated) < 5e-6
+
+
 @pytest.mark.parametrize("algo", [1, 2, 3, 4, 5, 6, 8, 10, 11])
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
 @pytest.mark.parametrize("m,inter,k", [(1, 16, 16), (4, 200, 88), (40, 320, 96), (9, 1000, 2304), (150, 72, 136),

@@ -1,8 +1,7 @@
 // Entry points of the matrix products and the plain tiled kernel.
 //
-// The plain kernel is the whole of the float32 path (no matrix-core mode, every output element summed
-// over k in index order whatever the batch is) and the fallback of the bf16 path for shapes the
-// matrix-core kernels refuse.  The reference's products are 4-bit codebook GEMVs
+// The plain kernel (every output element summed over k in index order whatever the batch is) is the fallback of both paths for
+// shapes that the matrix-core kernels refuse: a K that is no multiple of 4 (float32) or 8 (bf16), operands off their 16 bytes.  The reference's products are 4-bit codebook GEMVs
 // (runtime/cuda/codebook_gemv.cu:86-114); its only dense one is gemv_fp16_warp_k (cu:496-517).
 #include "gemm.h"
 
@@ -110,7 +109,7 @@ static int check_args(const GemmArgs& a) {
 
 // algo: 0 = choose, 1 = plain, 2 = skinny matrix-core, 3 = tiled matrix-core (6: with its wide tile, 7: with its 128 x 96 tile,
 // 8, 9: with its loop that loads straight into LDS, 128 x 128 and 128 x 96; 10, 11: its 64 x 32 and 64 x 64 tiles with two k
-// steps asked for ahead; 12 - 15: with the wide tiles of TP_WIDE_*), 4 = multiply-adds for one or two rows, 5 = matrix-core kernel for up to eight rows
+// steps asked for ahead; 12 - 15: with the wide tiles of TP_WIDE_*), 4 = multiply-adds for one or two rows, 5 = matrix-core kernel for up to eight rows.  (float32: 1, or chosen.)
 static int pick(const GemmArgs& a, int algo) {
     if (algo == 1) return 1;
     if (algo == 4) return gemv_supports(a) ? 4 : -4;
@@ -124,6 +123,7 @@ static int pick(const GemmArgs& a, int algo) {
     //   qkv     N 4096  K 2304      8 rows  8.0 /  7.1   32 rows 11.7 /  7.5   64 rows 13.5 /  8.5   (K slices)
     //   o       N 2304  K 2048      8 rows  5.2 /  5.5   32 rows  7.7 /  6.0   64 rows 13.3 /  6.7   (K slices)
     //   gate/up N 18432 K 2304      8 rows 26.9 / 24.2   32 rows 40.7 / 24.7   64 rows 48.5 / 26.5   (no slices: gated)
+    if (a.in_dtype == TP_F32) return gemm_f32_supports(a) ? 20 : 1;
     if (gemv_supports(a)) return 4;          // one or two rows: 2B gate/up 16.8 against 22.6 us on the skinny kernel
     // Three to eight rows: the kernel whose blocks read 8 rows of W in one go, where it was measured faster than the
     // choice below (microseconds from a replayed graph, cold weights, that choice / this kernel / a kernel that only reads):
@@ -180,6 +180,7 @@ extern "C" long tp_linear_workspace_bytes(int in_dtype, int out_dtype, int M, in
     if (p == 4) return (long)gemv_workspace(a);
     if (p == 5) return (long)gemm_rows8_workspace(a);
     if (p == 3) { const int s = gemm_mfma_splits(a); return s > 1 ? (long)s * M * N * 4 : 0; }
+    if (p == 20) { const int s = gemm_f32_splits(a); return s > 1 ? (long)s * M * N * 4 : 0; }
     if (p == 1 && epilogue == TP_EPI_GATED) return (long)M * N * 4;
     return 0;
 }
@@ -196,5 +197,6 @@ extern "C" int tp_linear(const void* x, const void* w, void* y, int in_dtype, in
     if (p == 4) return gemv_launch(a);
     if (p == 5) return gemm_rows8_launch(a);
     if (p == 3) return gemm_mfma_launch(a);
+    if (p == 20) return gemm_f32_launch(a);
     return gemm_simple_launch(a);
 }

@@ -1,0 +1,273 @@
+// float32 products on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands, products and sums), for few and many rows.
+//
+// Every output element is formed in one order whatever the batch is, so that a row alone gives the bits it gives among
+// others: K is cut into 16 parts of whole blocks of 16 k, a part is one chain of matrix instructions over its blocks (four
+// a block: instruction t takes the block's k = t, 4 + t, 8 + t, 12 + t), four neighbouring parts are added in order to a
+// group, and the four groups in order.  (Its error against 64 bits is smaller than that of one chain over K.)
+//
+// Few rows (a decode step) are bound by reading W.  A block owns 16 NT rows of W, a wave of it one part: six blocks of 16 k
+// of W and X are asked for together, so that a CU has 96 KB in flight, and the parts are added in LDS.
+// Many rows are bound by the matrix cores, 157 TFLOP/s in float32: a block of four waves owns 64 x 128 outputs (32 x 64 a
+// wave, 32 matrix instructions of 32 cycles for six 16-byte fragment reads), k steps of 32 straight from global memory into
+// one of two LDS buffers, three blocks a CU.  Where the outputs alone leave CUs idle and the consumer adds slices, the four
+// groups are four slices.
+#include "gemm.h"
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f3_f32x4;
+
+namespace {
+constexpr int PARTS = 16, GROUP = 4;
+constexpr int TM = 64, TN = 128;
+
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
+__device__ __forceinline__ float epilogue_f32(int epilogue, float o, float4 epi, int n) {
+    if (epilogue == TP_EPI_SILU) return (float)n < epi.z ? gate_act_exact(o, TP_ACT_SILU) : o;
+    return plain_epilogue(epilogue, o, epi, n);
+}
+}
+
+// NT, MT: tiles of 16 rows of W and of X.  Gated: NT = 2, the gate rows and the up rows of 16 units.
+template <int NT, int MT, bool GATED>
+__global__ void __launch_bounds__(1024)
+gemm_f32_few_k(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int part_blocks,
+               int epilogue, float4 epi, int units, int act) {
+    constexpr int AHEAD = NT * MT > 2 ? 4 : 6;             // blocks of 16 k asked for together (the wave's registers hold no more of four tiles)
+    __shared__ f3_f32x4 sums[PARTS][NT * MT][64];
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+    const int k_blocks = (K + 15) >> 4, from = part * part_blocks, to = min(k_blocks, from + part_blocks);
+    const float *wr[NT], *xr[MT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) wr[j] = W + (size_t)min(n0 + 16 * j + r, N - 1) * K;
+#pragma unroll
+    for (int i = 0; i < MT; i++) xr[i] = X + (size_t)min(m0 + 16 * i + r, M - 1) * K;
+    f3_f32x4 acc[NT][MT];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int b = from; b < to; b += AHEAD) {
+        f3_f32x4 w[AHEAD][NT], x[AHEAD][MT];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const int k = min(min(b + u, to - 1) * 16 + 4 * g, K - 4);       // past the end: elements that exist, zeroed or unused below
+#pragma unroll
+            for (int j = 0; j < NT; j++) w[u][j] = *reinterpret_cast<const f3_f32x4*>(wr[j] + k);
+#pragma unroll
+            for (int i = 0; i < MT; i++) x[u][i] = *reinterpret_cast<const f3_f32x4*>(xr[i] + k);
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            if (b + u >= to) break;
+            if ((b + u) * 16 + 16 > K) {                                     // the last, partial block
+                const bool in = (b + u) * 16 + 4 * g < K;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int j = 0; j < NT; j++) w[u][j][v] = in ? w[u][j][v] : 0.f;
+#pragma unroll
+                    for (int i = 0; i < MT; i++) x[u][i][v] = in ? x[u][i][v] : 0.f;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][j][t], x[u][i][t], acc[j][i], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) sums[part][j * MT + i][lane] = acc[j][i];
+    __syncthreads();
+    // element e of a tile: lane e / 4, register e % 4 of the accumulators: row of X lane % 16, row of W 4 (lane / 16) + register
+    auto total = [&](int tile, int e) {
+        float t = 0.f;
+#pragma unroll
+        for (int q = 0; q < PARTS / GROUP; q++) {
+            float s = 0.f;
+#pragma unroll
+            for (int p = 0; p < GROUP; p++) s += reinterpret_cast<const float*>(&sums[q * GROUP + p][tile][0])[e];
+            t += s;
+        }
+        return t;
+    };
+    for (int idx = threadIdx.x; idx < (GATED ? 1 : NT) * MT * 256; idx += 1024) {
+        const int tile = idx >> 8, e = idx & 255, l = e >> 2;
+        const int j = GATED ? 0 : tile / MT, i = GATED ? tile : tile % MT;
+        const int m = m0 + 16 * i + (l & 15), row = 16 * j + 4 * (l >> 4) + (e & 3);
+        if (m >= M) continue;
+        if (GATED) {
+            const int unit = (n0 >> 1) + row;
+            if (unit < units) Y[(size_t)m * units + unit] = gated_unit_exact(total(i, e), total(MT + i, e), act, epi.z, epi.w);
+        } else if (n0 + row < N) Y[(size_t)m * N + n0 + row] = epilogue_f32(epilogue, total(tile, e), epi, n0 + row);
+    }
+}
+
+template <bool GATED>
+__global__ void __launch_bounds__(256)
+gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int part_blocks,
+                int m_tiles, int epilogue, float4 epi, int units, int act) {
+    constexpr int BUF = (TM + TN) * 128;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * BUF];
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
+    const int m0 = (blockIdx.x % m_tiles) * TM, n0 = (blockIdx.x / m_tiles) * TN;
+    const bool sliced = gridDim.y > 1;
+    const int k_blocks = (K + 15) >> 4;
+    const int from = sliced ? blockIdx.y * GROUP * part_blocks : 0, to = sliced ? min(k_blocks, from + GROUP * part_blocks) : k_blocks;
+    const int steps = max(0, (to - from + 1) >> 1);
+    if (sliced) Y += (size_t)blockIdx.y * M * N;
+
+    // loads: 8 rows of 128 bytes an instruction, lane l's place (row l / 8, place l % 8) holds chunk place ^ row; rows past the
+    // edge of Y read the last row, chunks past the end of K its last one
+    const float* const xb = X + (size_t)m0 * K;
+    const float* const wb = W + (size_t)n0 * K;
+    const int chunk = (lane & 7) ^ (lane >> 3);
+    unsigned xo[2], wo[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) xo[i] = (unsigned)min(i * 32 + wave * 8 + (lane >> 3), M - 1 - m0) * (unsigned)K;
+#pragma unroll
+    for (int i = 0; i < 4; i++) wo[i] = (unsigned)min(i * 32 + wave * 8 + (lane >> 3), N - 1 - n0) * (unsigned)K;
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lds + wave * 1024;
+    auto fill = [&](int step) {
+        const unsigned k = (unsigned)min(from * 16 + step * 32 + chunk * 4, K - 4), to_ = lds0 + (step & 1) * BUF;
+        // (written as the instruction: told of it, the compiler waits for every such load before any LDS read)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"((xo[i] + k) * 4u), "s"(xb), "s"(to_ + i * 4096) : "memory");
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"((wo[i] + k) * 4u), "s"(wb), "s"(to_ + TM * 128 + i * 4096) : "memory");
+    };
+    f3_f32x4 acc[4][2], grp[4][2], tot[4][2];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) acc[j][i] = grp[j][i] = tot[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+    int part_end = from + part_blocks, parts = 0;
+    fill(0);
+    for (int step = 0; step < steps; step++) {
+        wait_loads();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();            // the step's tiles are there, and the other buffer has been read by everyone
+        asm volatile("" ::: "memory");
+        if (step + 1 < steps) fill(step + 1);
+        const unsigned char* const xs = lds + (step & 1) * BUF + (wm * 32 + r) * 128;
+        const unsigned char* const ws = lds + (step & 1) * BUF + TM * 128 + (wn * 64 + r) * 128;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int b = from + 2 * step + h;
+            if (b >= to) break;
+            const int at = ((4 * h + g) ^ (r & 7)) * 16;
+            f3_f32x4 w[4], x[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) x[i] = *reinterpret_cast<const f3_f32x4*>(xs + i * 2048 + at);
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = *reinterpret_cast<const f3_f32x4*>(ws + j * 2048 + at);
+            if (b * 16 + 16 > K) {               // the last, partial block
+                const bool in = b * 16 + 4 * g < K;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int i = 0; i < 2; i++) x[i][v] = in ? x[i][v] : 0.f;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) w[j][v] = in ? w[j][v] : 0.f;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][t], x[i][t], acc[j][i], 0, 0, 0);
+            if (b + 1 == part_end || b + 1 == to) {
+                parts++;
+                part_end += part_blocks;
+                const bool whole = parts % GROUP == 0 || b + 1 == to;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        grp[j][i] += acc[j][i];
+                        acc[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+                        if (whole) {
+                            tot[j][i] += grp[j][i];
+                            grp[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+                        }
+                    }
+            }
+        }
+    }
+    const int width = GATED ? units : N;
+    const bool wide = (width & 3) == 0 && ((uintptr_t)Y & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int m = m0 + wm * 32 + 16 * i + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 4; j += GATED ? 2 : 1) {
+            const int n = n0 + wn * 64 + 16 * j;
+            const int c = (GATED ? n >> 1 : n) + 4 * g;
+            f3_f32x4 o;
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                o[v] = GATED ? gated_unit_exact(tot[j][i][v], tot[j + 1 < 4 ? j + 1 : j][i][v], act, epi.z, epi.w) : epilogue_f32(epilogue, tot[j][i][v], epi, c + v);
+            if (c >= width) continue;
+            float* const to_ = Y + (size_t)m * width + c;
+            if (wide) *reinterpret_cast<f3_f32x4*>(to_) = o;
+            else {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (c + v < width) to_[v] = o[v];
+            }
+        }
+    }
+}
+
+// rows read in 16-byte pieces; a tile's rows within 32-bit offsets
+bool gemm_f32_supports(const GemmArgs& a) {
+    return a.in_dtype == TP_F32 && a.out_dtype == TP_F32 && a.K % 4 == 0 && a.K < (1 << 23) && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0;
+}
+
+// Up to 32 rows the kernel of few rows reads W once and its matrix instructions fit into that time; from 33 on the other
+// does the same work on whole tiles.
+static bool few(const GemmArgs& a) { return a.M <= 32; }
+
+int gemm_f32_splits(const GemmArgs& a) {
+    return !few(a) && a.defer && a.epilogue == TP_EPI_NONE && a.K >= 1024 && (long)tp_cdiv(a.M, TM) * tp_cdiv(a.N, TN) < 256 ? PARTS / GROUP : 1;
+}
+
+template <int NT, bool GATED>
+static void few_launch(const GemmArgs& a, int part_blocks, float4 epi) {
+    const int blocks = tp_cdiv(a.N, 16 * NT);
+    if (a.M <= 16) gemm_f32_few_k<NT, 1, GATED><<<blocks, 1024, 0, a.stream>>>((const float*)a.x, (const float*)a.w, (float*)a.y, a.M, a.N, a.K, part_blocks, a.epilogue, epi, a.units, a.act);
+    else gemm_f32_few_k<NT, 2, GATED><<<blocks, 1024, 0, a.stream>>>((const float*)a.x, (const float*)a.w, (float*)a.y, a.M, a.N, a.K, part_blocks, a.epilogue, epi, a.units, a.act);
+}
+
+int gemm_f32_launch(const GemmArgs& a) {
+    const int part_blocks = tp_cdiv(tp_cdiv(a.K, 16), PARTS);
+    const bool gated = a.epilogue == TP_EPI_GATED;
+    const float4 epi = gated ? make_float4(0.f, 0.f, a.limit, a.shift) : make_float4(a.cap, 0.f, (float)a.units, 0.f);
+    if (few(a)) {
+        // two tiles of W share the block's X where that leaves two blocks a CU
+        if (gated) few_launch<2, true>(a, part_blocks, epi);
+        else if (a.N >= 32 * 512) few_launch<2, false>(a, part_blocks, epi);
+        else few_launch<1, false>(a, part_blocks, epi);
+        return tp_check_launch("linear (float32, few rows)");
+    }
+    const int splits = gemm_f32_splits(a), m_tiles = tp_cdiv(a.M, TM);
+    const size_t need = (size_t)splits * a.M * a.N * sizeof(float);
+    TP_REQUIRE(splits == 1 || (a.workspace && a.workspace_bytes >= need), "float32 product: workspace of %zu bytes, %zu needed", a.workspace_bytes, need);
+    TP_REQUIRE((long)m_tiles * tp_cdiv(a.N, TN) < (1L << 31), "float32 product: too many tiles for one launch (M=%d N=%d)", a.M, a.N);
+    float* const y = (float*)(splits > 1 ? a.workspace : a.y);
+    const dim3 grid((unsigned)(m_tiles * tp_cdiv(a.N, TN)), splits);
+    if (gated) gemm_f32_many_k<true><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act);
+    else gemm_f32_many_k<false><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act);
+    return tp_check_launch("linear (float32)");
+}
