@@ -1,8 +1,13 @@
-// Plain attention kernel for any dtype, head size up to 1024 and any grouping: one wave per (row, query head),
-// keys visited one after the other in position order with a running softmax.
+// Plain attention kernel for any dtype, head size up to 1024 and any grouping: a block of eight waves per (row, query head).
 //
-// It is the float32 path's attention for prefill and decode alike (the same instruction sequence per key in
-// both, so a token's result does not depend on how the prompt was cut), and the bf16 path's fallback for
+// The keys that the query sees are cut, from the first on, into groups of up to four; wave w takes the groups w, w + 8, ..
+// with a running softmax of its own, and the eight states are joined in wave order at the end.  What bounds it is latency: a
+// group's key and value rows are fetched while the group before is worked on, the dot products of its keys are summed over the
+// wave together (seven exchanges instead of six a key), and eight waves have their chains in flight.  (One wave, a key after
+// the other, took 0.63 us a key: 132 us of a float32 decode step's layer at 200 keys and heads of 256, 11 us so.)
+//
+// It is the float32 path's attention for prefill and decode alike (the groups and their order depend on what the query
+// sees alone, so a token's result does not depend on how the prompt was cut), and the bf16 path's fallback for
 // shapes the matrix-core kernels refuse.  Formula and order as the reference's attn_k
 // (runtime/cuda/codebook_gemv.cu:240-270): score = dot * scale, cap * tanh(score / cap), softmax, weighted
 // sum of v, kv head = head / (heads / kv_heads); the scale is an argument (rsqrt(head_dim) there), and a
@@ -29,11 +34,16 @@ struct AttnSimpleArgs {
     int keep, pin;                                       // positions seen beside the window; rows of the cache in front of its ring
 };
 
-// NJ: elements of a head a lane holds (head sizes up to 64 NJ)
-template <typename T, int NJ>
-__global__ void __launch_bounds__(64)
+namespace {
+constexpr int WAVES = 8;
+}
+
+// NJ: elements of a head a lane holds (head sizes up to 64 NJ); KEYS: keys of a group (4, 2 or 1: what the registers hold)
+template <typename T, int NJ, int KEYS>
+__global__ void __launch_bounds__(64 * WAVES)
 attn_simple_k(AttnSimpleArgs a) {
-    const int h = blockIdx.y, r = blockIdx.x, lane = threadIdx.x;
+    __shared__ float part_o[WAVES][64 * NJ], part_m[WAVES], part_l[WAVES];
+    const int h = blockIdx.y, r = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = h / (a.H / a.KV);
     int seq, p, start = 0;                              // start: the first position that is a row of the step
     if (a.paged) { seq = r; p = a.new_len[r] - 1; start = p + 1; }
@@ -58,71 +68,114 @@ attn_simple_k(AttnSimpleArgs a) {
     // the keys in order: the kept ones before the window, then the window's; key i stands at position at(i)
     const int kept = min(a.keep, lo), n_keys = kept + p - lo + 1;
     auto at = [&](int i) { return i < kept ? i : lo + i - kept; };
-    // a key's row and value row are fetched while the two keys before it are worked on (the arithmetic per key, and
-    // its order, stay as they are: the loop would otherwise pay a trip to memory, or two through the page table, per key)
-    auto fetch = [&](int i, float (&kk)[NJ], float (&vv)[NJ]) {
-        const int t = min(at(i), p);                     // past the last key: a row that exists, never used
-        const T *kp, *vp;
-        if (t < start) {
-            const int row = a.rows_cap > 0 && t >= a.pin ? a.pin + (t - a.pin) % (a.rows_cap - a.pin) : t;
-            const int pg = a.table[(size_t)seq * a.table_w + row / a.page];
-            const size_t off = (((size_t)pg * a.KV + g) * a.page + row % a.page) * a.hd;
-            kp = (const T*)a.k_pool + off;
-            vp = (const T*)a.v_pool + off;
-        } else {
-            const size_t row = (size_t)(a.cu_rows[seq] + t - start);
-            kp = (const T*)a.k + row * a.k_stride + (size_t)g * a.hd;
-            vp = (const T*)a.v + row * a.v_stride + (size_t)g * a.hd;
+    auto fetch = [&](int first, float (&kk)[KEYS][NJ], float (&vv)[KEYS][NJ]) {
+#pragma unroll
+        for (int n = 0; n < KEYS; n++) {
+            const int t = min(at(first + n), p);             // past the last key: a row that exists, without weight
+            const T *kp, *vp;
+            if (t < start) {
+                const int row = a.rows_cap > 0 && t >= a.pin ? a.pin + (t - a.pin) % (a.rows_cap - a.pin) : t;
+                const int pg = a.table[(size_t)seq * a.table_w + row / a.page];
+                const size_t off = (((size_t)pg * a.KV + g) * a.page + row % a.page) * a.hd;
+                kp = (const T*)a.k_pool + off;
+                vp = (const T*)a.v_pool + off;
+            } else {
+                const size_t row = (size_t)(a.cu_rows[seq] + t - start);
+                kp = (const T*)a.k + row * a.k_stride + (size_t)g * a.hd;
+                vp = (const T*)a.v + row * a.v_stride + (size_t)g * a.hd;
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const int d = lane + 64 * j;
+                const int dc = d < a.hd ? d : 0;
+                const float kx = ld_f32(kp + dc), vx = ld_f32(vp + dc);
+                kk[n][j] = d < a.hd ? kx : 0.f;
+                vv[n][j] = d < a.hd ? vx : 0.f;
+            }
         }
+    };
+    auto use = [&](int first, const float (&kk)[KEYS][NJ], const float (&vv)[KEYS][NJ]) {
+        float part[KEYS];
+#pragma unroll
+        for (int n = 0; n < KEYS; n++) {
+            part[n] = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; j++) part[n] = fmaf(qv[j], kk[n][j], part[n]);
+        }
+        // the sums over the wave: a lane is left with that of key `mine`, lane % KEYS
+        const int mine = lane & (KEYS - 1);
+        float s = part[0];
+        if constexpr (KEYS == 4) {
+            const float s01 = ((lane & 1) ? part[1] : part[0]) + __shfl_xor((lane & 1) ? part[0] : part[1], 1, 64);
+            const float s23 = ((lane & 1) ? part[3] : part[2]) + __shfl_xor((lane & 1) ? part[2] : part[3], 1, 64);
+            s = ((lane & 2) ? s23 : s01) + __shfl_xor((lane & 2) ? s01 : s23, 2, 64);
+        } else if constexpr (KEYS == 2) {
+            s = ((lane & 1) ? part[1] : part[0]) + __shfl_xor((lane & 1) ? part[0] : part[1], 1, 64);
+        }
+#pragma unroll
+        for (int x = KEYS; x < 64; x <<= 1) s += __shfl_xor(s, x, 64);
+        s *= scale;
+        if (a.cap > 0.f) s = softcap_f(s, a.cap);
+        if (bias) s += bias[min(max(p - at(first + mine), 0), (int)a.by_position.reach)];
+        if (first + mine >= n_keys) s = -INFINITY;
+        float top = s;
+#pragma unroll
+        for (int x = 1; x < KEYS; x <<= 1) top = fmaxf(top, __shfl_xor(top, x, 64));
+        const float m_new = fmaxf(m, top);
+        const float alpha = expf(m - m_new), pr = first + mine < n_keys ? expf(s - m_new) : 0.f;
+        float sum = pr;
+#pragma unroll
+        for (int x = 1; x < KEYS; x <<= 1) sum += __shfl_xor(sum, x, 64);
+        l = l * alpha + sum;
+        float w[KEYS];
+#pragma unroll
+        for (int n = 0; n < KEYS; n++) w[n] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(pr), n));
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const int d = lane + 64 * j;
-            const int dc = d < a.hd ? d : 0;
-            const float kx = ld_f32(kp + dc), vx = ld_f32(vp + dc);
-            kk[j] = d < a.hd ? kx : 0.f;
-            vv[j] = d < a.hd ? vx : 0.f;
+            o[j] *= alpha;
+#pragma unroll
+            for (int n = 0; n < KEYS; n++) o[j] = fmaf(w[n], vv[n][j], o[j]);
         }
-    };
-    auto use = [&](int i, const float (&kk)[NJ], const float (&vv)[NJ]) {
-        float part = 0.f;
-#pragma unroll
-        for (int j = 0; j < NJ; j++) part = fmaf(qv[j], kk[j], part);
-        float s = wave_sum(part) * scale;
-        if (a.cap > 0.f) s = softcap_f(s, a.cap);
-        if (bias) s += bias[min(p - at(i), (int)a.by_position.reach)];
-        const float m_new = fmaxf(m, s);
-        const float alpha = expf(m - m_new), pr = expf(s - m_new);
-        l = l * alpha + pr;
-#pragma unroll
-        for (int j = 0; j < NJ; j++) o[j] = o[j] * alpha + pr * vv[j];
         m = m_new;
     };
-    float k0[NJ], v0[NJ], k1[NJ], v1[NJ], k2[NJ], v2[NJ];
-    fetch(0, k0, v0);
-    fetch(1, k1, v1);
-    for (int i = 0; i < n_keys; i += 3) {
-        fetch(i + 2, k2, v2);
-        use(i, k0, v0);
-        if (i + 1 >= n_keys) break;
-        fetch(i + 3, k0, v0);
-        use(i + 1, k1, v1);
-        if (i + 2 >= n_keys) break;
-        fetch(i + 4, k1, v1);
-        use(i + 2, k2, v2);
+    float k0[KEYS][NJ], v0[KEYS][NJ], k1[KEYS][NJ], v1[KEYS][NJ];
+    int i = wave * KEYS;
+    if (i < n_keys) {
+        fetch(i, k0, v0);
+        while (true) {
+            const int i1 = i + WAVES * KEYS;
+            if (i1 < n_keys) fetch(i1, k1, v1);
+            use(i, k0, v0);
+            if (i1 >= n_keys) break;
+            i = i1 + WAVES * KEYS;
+            if (i < n_keys) fetch(i, k0, v0);
+            use(i1, k1, v1);
+            if (i >= n_keys) break;
+        }
     }
-    if (a.sink) {
-        const float sk = a.sink[h], m_new = fmaxf(m, sk);
-        const float alpha = expf(m - m_new);
-        l = l * alpha + expf(sk - m_new);
 #pragma unroll
-        for (int j = 0; j < NJ; j++) o[j] *= alpha;
+    for (int j = 0; j < NJ; j++) part_o[wave][lane + 64 * j] = o[j];
+    if (lane == 0) { part_m[wave] = m; part_l[wave] = l; }
+    __syncthreads();
+    const int used = min(WAVES, (n_keys + KEYS - 1) / KEYS);       // waves that saw a key
+    float top = part_m[0];
+    for (int w = 1; w < used; w++) top = fmaxf(top, part_m[w]);
+    if (a.sink) top = fmaxf(top, a.sink[h]);
+    float f[WAVES], total = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        f[w] = w < used ? expf(part_m[w] - top) : 0.f;
+        if (w < used) total += part_l[w] * f[w];
     }
+    if (a.sink) total += expf(a.sink[h] - top);
     T* out = (T*)a.out + ((size_t)r * a.H + h) * a.hd;
-    const float inv = (a.by_position.gate ? head_gate(a.by_position, r, h) : 1.f) / l;
+    const float inv = (a.by_position.gate ? head_gate(a.by_position, r, h) : 1.f) / total;
+    for (int d = threadIdx.x; d < a.hd; d += 64 * WAVES) {
+        float t = 0.f;
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int d = lane + 64 * j;
-        if (d < a.hd) st_f32(out + d, o[j] * inv);
+        for (int w = 0; w < WAVES; w++)
+            if (w < used) t = fmaf(part_o[w][d], f[w], t);
+        st_f32(out + d, t * inv);
     }
 }
 
@@ -135,10 +188,10 @@ static int launch(const AttnSimpleArgs& a, int dtype, int M, hipStream_t s) {
     TP_REQUIRE(a.H <= 65535, "attention (plain kernel): %d heads exceed one launch (65535)", a.H);
     dim3 grid(M, a.H);
     if (dtype != TP_BF16 && dtype != TP_F32) return tp_fail("attention: unknown dtype %d", dtype);
-#define TP_ATTN_SIMPLE(NJ) do { if (dtype == TP_BF16) attn_simple_k<bf16_t, NJ><<<grid, 64, 0, s>>>(a); else attn_simple_k<float, NJ><<<grid, 64, 0, s>>>(a); } while (0)
-    if (a.hd <= 256) TP_ATTN_SIMPLE(4);
-    else if (a.hd <= 512) TP_ATTN_SIMPLE(8);
-    else TP_ATTN_SIMPLE(16);
+#define TP_ATTN_SIMPLE(NJ, KEYS) do { if (dtype == TP_BF16) attn_simple_k<bf16_t, NJ, KEYS><<<grid, 64 * WAVES, 0, s>>>(a); else attn_simple_k<float, NJ, KEYS><<<grid, 64 * WAVES, 0, s>>>(a); } while (0)
+    if (a.hd <= 256) TP_ATTN_SIMPLE(4, 4);
+    else if (a.hd <= 512) TP_ATTN_SIMPLE(8, 2);
+    else TP_ATTN_SIMPLE(16, 1);
 #undef TP_ATTN_SIMPLE
     return tp_check_launch("attention (plain kernel)");
 }
