@@ -769,6 +769,24 @@ def test_sample_follows_the_plain_sampler(ops, vocab, temperature, top_k, top_p)
     assert got[2] == vocab - 1
 
 
+@pytest.mark.parametrize("vocab", [32768, 50001])
+@pytest.mark.parametrize("top_k", [1, 300, 1024])
+def test_sample_in_turn_on_one_workspace(ops, vocab, top_k):
+    """What the candidate filter leaves behind is ready for the next call: rows with few candidates, with more than are sorted
+    at once, with more than a block or the list holds (the whole row is read then), one after the other."""
+    flat = torch.zeros(3, vocab)                             # every logit in one bin
+    flat[:, 7] = 5.0
+    crowd = randn(3, vocab, seed=91, scale=0.01).cpu()       # thousands of logits in the bins of the largest
+    steep = randn(3, vocab, seed=92, scale=4.0).cpu()
+    u = torch.tensor([0.1, 0.6, 0.95], dtype=torch.float32)
+    for z in (steep, flat, steep, crowd, flat, steep):
+        got = ops.sample(z.to(DEV), 0.9, top_k, 0.97, u.to(DEV)).cpu().tolist()
+        for b in range(3):
+            near = {int(ref_ops.sample(z[b:b + 1], 0.9, top_k, 0.97, torch.tensor([min(max(float(u[b]) + du, 0.0), 0.9999999)]))[0])
+                    for du in (-2e-6, 0.0, 2e-6)}            # float32 rounding at a boundary of the walk
+            assert got[b] in near, (b, got[b], near)
+
+
 def test_recent_push(ops):
     """A row's id goes to the place its cursor names, the cursor moves on and wraps at the ring's end."""
     ring = torch.full((3, 5), -1, dtype=torch.int32, device=DEV)
