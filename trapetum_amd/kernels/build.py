@@ -12,6 +12,7 @@ import shutil
 import subprocess
 import sys
 import tempfile
+import threading
 import time
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
@@ -36,7 +37,7 @@ def build_dir():
     d = os.path.join(CSRC, "_build")
     try:
         os.makedirs(d, exist_ok=True)
-        probe = os.path.join(d, f".w{os.getpid()}")
+        probe = os.path.join(d, f".w{os.getpid()}.{threading.get_ident()}")       # libraries are built by several threads
         with open(probe, "w"):
             pass
         os.remove(probe)
