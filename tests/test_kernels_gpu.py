@@ -167,6 +167,40 @@ def test_linear_bf16(ops, algo, m, n, k):
     assert rel_l2(got_d, ref) < 4e-3
 
 
+# the kernel that streams up to 64 rows through LDS: each of its blocks (32, 64 and 128 rows of W, up to 16, 32 and 64 of X), one
+# k step and fewer than it asks for ahead, an N that ends inside a block and is no multiple of 4 (outputs element by element),
+# K slices of which the last is shorter; it is what is chosen from two rows on where the consumer adds the slices
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (2, 77, 128), (3, 2304, 2048), (16, 1001, 320), (17, 8200, 64), (32, 4099, 640),
+                                   (33, 130, 1088), (64, 250, 4672), (48, 18432, 64), (9, 18432, 704), (64, 16500, 192), (40, 33000, 512)])
+def test_linear_up_to_64_rows(ops, m, n, k):
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=7), randn(n, k, dtype=torch.bfloat16, seed=8, scale=0.05)
+    into = torch.full((m * n + 1,), 7.0, dtype=torch.bfloat16, device=DEV)
+    half = n // 2 // 16 * 16
+    ops.force_linear = 16
+    try:
+        got_b = ops.linear(x, w, torch.bfloat16)
+        got_f = ops.linear(x, w, torch.float32, softcap=3.0)
+        deferred = ops.linear(x, w, torch.bfloat16, defer=True)
+        got_d = ops.rows(deferred, torch.float32)
+        got_s = ops.linear_act(x, w, torch.float32, "silu", columns=n // 2 or 1)
+        ops.linear(x, w, torch.bfloat16, out=into[1:].view(m, n))                         # two bytes beyond an aligned address
+        got_g = ops.gated_linear(x, ops.pack_gate_up(w[:half - 3], w[half:2 * half - 3]), half - 3, "silu", torch.bfloat16) if half else None
+        with pytest.raises(Exception, match="does not take"):
+            ops.linear(x[:, :k - 8].contiguous(), w[:, :k - 8].contiguous(), torch.bfloat16)
+    finally:
+        ops.force_linear = 0
+    if m > 1 and not isinstance(deferred, torch.Tensor):
+        assert torch.equal(ops.rows(ops.linear(x, w, torch.bfloat16, defer=True), torch.float32), got_d)
+    ref = x.cpu().double() @ w.cpu().double().T
+    assert rel_l2(got_b, ref) < 4e-3 and rel_l2(got_d, ref) < 4e-3
+    assert rel_l2(got_f, 3.0 * torch.tanh(ref / 3.0)) < 1e-5
+    cols = n // 2 or 1
+    assert rel_l2(got_s, torch.cat([torch.nn.functional.silu(ref[:, :cols]), ref[:, cols:]], 1)) < 1e-5
+    assert torch.equal(into[1:].view(m, n), got_b) and float(into[0]) == 7.0
+    if half:
+        assert rel_l2(got_g, torch.nn.functional.silu(ref[:, :half - 3]) * ref[:, half:2 * half - 3]) < 4e-3
+
+
 # the tiles of 8 waves (12: 256 x 256, 13: 256 x 192, 14: 192 x 256, 15: 256 x 128): one k step, two, three and a long odd number
 # of them, a tile and one row more or less, an N that is no multiple of 8 or 4 (outputs element by element), a last K slice
 # that is shorter, more tiles than CUs

@@ -63,3 +63,7 @@ int gemm_wide_launch(const GemmArgs& a, int shape, int splits, int kps);
 bool gemm_f32_supports(const GemmArgs& a);
 int gemm_f32_splits(const GemmArgs& a);
 int gemm_f32_launch(const GemmArgs& a);
+// bf16 on the matrix cores for up to 64 rows (K a multiple of 64): streams W once through LDS, several k steps in flight
+bool gemm_stream_supports(const GemmArgs& a);
+size_t gemm_stream_workspace(const GemmArgs& a);
+int gemm_stream_launch(const GemmArgs& a);

@@ -109,46 +109,44 @@ static int check_args(const GemmArgs& a) {
 
 // algo: 0 = choose, 1 = plain, 2 = skinny matrix-core, 3 = tiled matrix-core (6: with its wide tile, 7: with its 128 x 96 tile,
 // 8, 9: with its loop that loads straight into LDS, 128 x 128 and 128 x 96; 10, 11: its 64 x 32 and 64 x 64 tiles with two k
-// steps asked for ahead; 12 - 15: with the wide tiles of TP_WIDE_*), 4 = multiply-adds for one or two rows, 5 = matrix-core kernel for up to eight rows.  (float32: 1, or chosen.)
+// steps asked for ahead; 12 - 15: with the wide tiles of TP_WIDE_*), 16 = its own kernel for
+// up to 64 rows that streams W through LDS, 4 = multiply-adds for one or two rows, 5 = matrix-core kernel for up to eight rows.  (float32: 1, or chosen.)
 static int pick(const GemmArgs& a, int algo) {
     if (algo == 1) return 1;
     if (algo == 4) return gemv_supports(a) ? 4 : -4;
     if (algo == 5) return gemm_rows8_supports(a) ? 5 : -5;
+    if (algo == 16) return gemm_stream_supports(a) ? 16 : -16;
     if (algo == 2) return gemm_skinny_supports(a) ? 2 : -2;
     if (algo == 3 || (algo >= 6 && algo <= 15)) return gemm_mfma_supports(a) ? 3 : -3;
-    // Up to 64 rows both matrix-core kernels stream W once; which is faster was measured on MI355X at the 2B shapes
-    // (cold weights, microseconds, skinny / tiled with 64 x 64 tiles and k steps of 128):
-    //   logits  N 256000            8 rows 277 / 222
-    //   down    N 2304  K 9216      8 rows 15.8 / 11.3   32 rows 20.1 / 12.0   64 rows 26.3 / 13.5   (K slices left to the consumer)
-    //   qkv     N 4096  K 2304      8 rows  8.0 /  7.1   32 rows 11.7 /  7.5   64 rows 13.5 /  8.5   (K slices)
-    //   o       N 2304  K 2048      8 rows  5.2 /  5.5   32 rows  7.7 /  6.0   64 rows 13.3 /  6.7   (K slices)
-    //   gate/up N 18432 K 2304      8 rows 26.9 / 24.2   32 rows 40.7 / 24.7   64 rows 48.5 / 26.5   (no slices: gated)
     if (a.in_dtype == TP_F32) return gemm_f32_supports(a) ? 20 : 1;
+    // Two to 64 rows, K a multiple of 64: the kernel that streams W through LDS, wherever enough blocks of it read at once
+    // (its figures beside its plan).  With K slices for the consumer that is always (2 rows, against the multiply-adds: 9B down
+    // 27.6 / 23.8 us, qkv 15.3 / 12.8, 2B down 16.1 / 14.5); without, from 128 blocks of 64 rows of W on (8 rows, N 9216 K 2304:
+    // 13.2 / 11.8; 16 rows 21.4 / 13.0; but 8 rows, N 4096: 6.5 / 9.1).  A single row stays with the multiply-adds (2B down
+    // 14.4 / 14.3, gate/up 16.6 / 18.6), and products without slices with the multiply-adds for two rows (2B gate/up 17.5 / 18.7)
+    // and the 8-row kernel for three to seven where that reads K in one round, gates, or has the logits' many rows (2B gate/up
+    // 17.2 / 18.7 at 4 rows, 18.2 / 18.7 at 6; logits 189 / 199).
+    constexpr int ONE_ROUND_K = TP_R8_MAX_STEPS * 256, WIDE_N = 64 * 512, STREAM_N = 64 * 127;
+    const bool sliced = a.defer && a.epilogue == TP_EPI_NONE;
+    if (gemm_stream_supports(a) && a.M > 1) {
+        const bool rows8 = a.M < 8 && gemm_rows8_supports(a) && (a.epilogue == TP_EPI_GATED || a.K <= ONE_ROUND_K || a.N >= WIDE_N);
+        if ((sliced && gemm_stream_workspace(a)) || (a.N > STREAM_N && (a.M > 2 || !gemv_supports(a)) && !rows8)) return 16;
+    }
     if (gemv_supports(a)) return 4;          // one or two rows: 2B gate/up 16.8 against 22.6 us on the skinny kernel
-    // Three to eight rows: the kernel whose blocks read 8 rows of W in one go, where it was measured faster than the
-    // choice below (microseconds from a replayed graph, cold weights, that choice / this kernel / a kernel that only reads):
-    //   2B  gate/up 24.1 / 21.7 / 15.2   down 14.5 / 11.5 / 9.1   qkv 7.1 / 6.3 / 4.9   o 5.0 / 5.2 / 4.2   logits 209 / 253 / 204
-    //   9B  gate/up 43.2 / 45.6 / 36.1   down 22.0 / 24.5 / 18.6  qkv 13.5 / 15.1 / 12.1  o 10.0 / 9.2 / 7.6
-    //   27B gate/up 141 / 136 / 116      down 72.4 / 76.7 / 58.2  qkv 16.8 / 19.9 / 14.9  o 14.5 / 10.8 / 8.3   logits 407 / 462 / 414
-    // at 8 rows; at 3 and 4 rows, where the choice below is the skinny kernel, 2B logits 250 / 228, 9B gate/up 49.3 / 41.8,
-    // 27B gate/up 142 / 127, 27B qkv 16.9 / 19.4.  A slice of K beyond 2,304 takes the kernel a second round of loads.
-    // A decode step of 8 sequences at the 2B sizes: 2.30 -> 2.00 ms.
-    // The bounds below are what those measurements have in common, in the kernels' own terms:
+    // What is left: few rows of W, or K no multiple of 64.  Three to eight rows: the kernel whose blocks read 8 rows of W in one
+    // go, where it was measured faster than the choice below.  The bounds in the kernels' own terms:
     //   ONE_ROUND_K  the K a block of the 8-row kernel reads in one round of loads (TP_R8_MAX_STEPS steps of 64 k by four
     //                waves): beyond it the kernel loops, and a slice of K left to the consumer keeps it within one round;
     //   WIDE_N       from here on a product is the logits' kind: so many rows of W that the tiled kernel's 64 x 64 tiles
     //                fill every CU several times over (512 tiles = two a CU) and its larger k steps win;
-    //   LARGE_NK     elements of W from which the tiled kernel's streaming wins at 8 rows and more (the 27B matrices and
-    //                every gated product: 340 MB, 93 -> 74 us), measured between 21 M (2B down: the 8-row kernel wins)
-    //                and 42 M (2B gate/up: the tiled kernel wins);
+    //   LARGE_NK     elements of W from which the tiled kernel's streaming wins at 8 rows and more, measured between 21 M (the
+    //                8-row kernel wins) and 42 M (the tiled kernel wins);
     //   R8_SLICED_NK elements of W up to which the 8-row kernel, its K in slices for the consumer, beat the tiled kernel
-    //                in a whole step (all the 2B and 9B products but the 9B feed-forward; the 27B ones lose).
-    constexpr int ONE_ROUND_K = TP_R8_MAX_STEPS * 256, WIDE_N = 64 * 512;
+    //                in a whole step.
     constexpr long LARGE_NK = 24000000, R8_SLICED_NK = 32000000;
     if (a.M <= 8 && gemm_rows8_supports(a)) {
-        const long nk = (long)a.N * a.K;
-        if (a.defer && a.epilogue == TP_EPI_NONE) {
-            if (nk <= R8_SLICED_NK) return 5;     // (2B o alone is no faster, 5.0 / 5.2, but a step of 8 sequences is: 2.001 -> 1.988 ms)
+        if (sliced) {
+            if ((long)a.N * a.K <= R8_SLICED_NK) return 5;
         } else if (a.M < 8) {
             if (a.epilogue == TP_EPI_GATED || a.K <= ONE_ROUND_K || a.N >= WIDE_N) return 5;
         } else if (a.K <= ONE_ROUND_K && a.N < WIDE_N) {
@@ -156,13 +154,11 @@ static int pick(const GemmArgs& a, int algo) {
         }
     }
     if (gemm_mfma_supports(a)) {
-        const bool sliced = a.defer && a.epilogue == TP_EPI_NONE;
-        // (at 8 rows the tiled kernel's lead on qkv and down is lost again in their consumers, which then add 9 and 16
-        // slices instead of 2 and 4; a single sequence is faster on the skinny kernel throughout)
+        // (a single sequence is faster on the skinny kernel throughout)
         if (a.M >= 8 && (a.epilogue == TP_EPI_GATED || (long)a.N * a.K >= LARGE_NK)) return 3;
         if (a.M >= 8 && a.N >= WIDE_N) return 3;
         // from 9 rows on the tiled kernel wins every product of a layer against the skinny one (2B, 16 rows, cold
-        // weights: qkv 6.4 / 8.0 us, o 5.1 / 5.3, down 11.5 / 18.6; a step of 16 sequences 2.47 -> 2.32 ms)
+        // weights: qkv 6.4 / 8.0 us, o 5.1 / 5.3, down 11.5 / 18.6)
         if (a.M > 8 && (sliced || a.N >= 8192)) return 3;
     }
     if (gemm_skinny_supports(a)) return 2;
@@ -179,6 +175,7 @@ extern "C" long tp_linear_workspace_bytes(int in_dtype, int out_dtype, int M, in
     if (p == 2) return (long)gemm_skinny_workspace(a);
     if (p == 4) return (long)gemv_workspace(a);
     if (p == 5) return (long)gemm_rows8_workspace(a);
+    if (p == 16) return (long)gemm_stream_workspace(a);
     if (p == 3) { const int s = gemm_mfma_splits(a); return s > 1 ? (long)s * M * N * 4 : 0; }
     if (p == 20) { const int s = gemm_f32_splits(a); return s > 1 ? (long)s * M * N * 4 : 0; }
     if (p == 1 && epilogue == TP_EPI_GATED) return (long)M * N * 4;
@@ -197,6 +194,7 @@ extern "C" int tp_linear(const void* x, const void* w, void* y, int in_dtype, in
     if (p == 4) return gemv_launch(a);
     if (p == 5) return gemm_rows8_launch(a);
     if (p == 3) return gemm_mfma_launch(a);
+    if (p == 16) return gemm_stream_launch(a);
     if (p == 20) return gemm_f32_launch(a);
     return gemm_simple_launch(a);
 }
