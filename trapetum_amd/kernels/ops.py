@@ -1243,12 +1243,14 @@ class HipOps:
 
     @staticmethod
     def decode_splits(n, KV, hd, keys):
-        """Slices of the keys per (sequence, kv head) in a decode step: enough blocks to keep every CU streaming
-        (about 1536; 768 when the pairs alone are many), each with at least one round of 64 keys.  Measured on
-        MI355X from 1 to 64 sequences and 500 to 8000 keys this is within 7 % of the best count everywhere; more
-        slices cost little (a second launch adds them), fewer cost up to half."""
+        """Slices of the keys per (sequence, kv head) in a decode step, each with at least one round of 64 keys: two blocks
+        a CU in all, one where the pairs are few (the slices' sums then cost more than another block brings), and none
+        where the pairs alone are a block a CU.  Measured on MI355X (heads of 256, microseconds, three to six blocks a
+        CU / this): 1 x 8,000 keys 22.8 / 18.4, 1 x 4,000 of 8 kv heads 18.4 / 16.6, 4 of up to 7,000 29.3 / 24.5, 8 x 4,096
+        34.8 / 32.7, 16 x 2,000 32.6 / 32.0, 32 x 1,000 33.1 / 32.7, 64 x 500 30.8 / 31.0, 64 x 2,000 101.2 / 98.0, 64 of up to 80
+        keys 12.4 / 10.2."""
         pairs = n * KV
-        want = -(-(1536 if pairs < 192 else 768) // pairs)
+        want = (256 if pairs < 16 else 512) // pairs if pairs < 256 else 1
         return max(1, min(want, -(-keys // 64), 128))
 
     def _check_pools(self, what, dtype, n, KV, hd, new_len, table, k_pool, v_pool):
