@@ -167,6 +167,28 @@ def test_linear_bf16(ops, algo, m, n, k):
     assert rel_l2(got_d, ref) < 4e-3
 
 
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+@pytest.mark.parametrize("counts,H,KV", [([1, 5, 300, 1], 8, 4), ([290, 1, 2], 4, 2), ([1, 33, 1, 700, 1, 1, 40], 4, 1), ([1, 500], 16, 16)])
+def test_attention_of_uneven_sequences(ops, counts, H, KV, shape):
+    """Where a step's sequences differ much in length, its blocks go round the chip in another order: every sequence's rows
+    are what they are alone, bit for bit (a choice by size may give the short ones other blocks: to rounding)."""
+    hd, M = 256, sum(counts)
+    q = randn(M, H * hd, dtype=torch.bfloat16, seed=61)
+    k, v = randn(M, KV * hd, dtype=torch.bfloat16, seed=62), randn(M, KV * hd, dtype=torch.bfloat16, seed=63)
+
+    def attend(q, k, v, counts, shape):
+        cu = torch.tensor([sum(counts[:i]) for i in range(len(counts) + 1)], dtype=torch.int32, device=DEV)
+        return ops.attention_prefill(q, k, v, H, KV, hd, cu, max(counts), hd ** -0.5, 30.0, 0, torch.bfloat16, shape=shape)
+    got, at = attend(q, k, v, counts, shape), 0
+    for n in counts:
+        own = attend(q[at:at + n], k[at:at + n], v[at:at + n], [n], shape)
+        if shape:
+            assert torch.equal(got[at:at + n], own)
+        else:
+            assert rel_l2(got[at:at + n], own) < 4e-3
+        at += n
+
+
 # the kernel that streams up to 64 rows through LDS: each of its blocks (32, 64 and 128 rows of W, up to 16, 32 and 64 of X), one
 # k step and fewer than it asks for ahead, an N that ends inside a block and is no multiple of 4 (outputs element by element),
 # K slices of which the last is shorter; it is what is chosen from two rows on where the consumer adds the slices

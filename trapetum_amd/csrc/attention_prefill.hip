@@ -56,6 +56,7 @@ struct PrefillArgs {
     int page_shift, page_mask, rows_cap;
     int H, KV, ghb_shift, pt_shift;           // heads of a kv head a block takes: 1 << ghb_shift; its position tiles: 1 << pt_shift
     int n_streams, pos_blocks;                // (sequence, kv head, head group) triples; blocks of positions per stream
+    int turn;                                 // streams the next block of positions starts further on, so that a stream meets every XCD
     float scale, cap; int window;
     int chunk;                                // C > 0: the query at p sees keys from floor(p / C) C on only
     const float* head_scale;                  // [H] or null: a factor on every head's scores
@@ -138,7 +139,8 @@ attn_prefill_k(PrefillArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / CG, cg = wave % CG;
 
     // ---- which part of the step this block owns ---------------------------------------------------------------
-    const int stream = blockIdx.x % a.n_streams, rank = blockIdx.x / a.n_streams;
+    const int rank = blockIdx.x / a.n_streams;
+    const int stream = (blockIdx.x % a.n_streams + rank * a.turn) % a.n_streams;
     const int G = a.H / a.KV, HG = G >> a.ghb_shift;
     const int hg = stream % HG, kvh = (stream / HG) % a.KV, seq = stream / (HG * a.KV);
     const int PT = 1 << a.pt_shift, PB = 32 * PT;
@@ -561,21 +563,39 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
     // blocks are at most two a CU (at head sizes whose tiles let one 8-wave block fit a CU), 2 x 4: a quarter of the
     // rounds for the longest block.  Measured for 4x1 / 2x2 / 2x4: 2B sizes, 2,048 tokens 94 / 61 / 51 us, 4,096 tokens
     // 186 / 130 / 114, 8 x 512 tokens 34 / 27 / 36; 9B sizes, 2,048 tokens 100 / 72 / 69; 27B (heads of 128) 85 / 78 / 89.
+    // A step of uneven sequences launches more blocks than hold queries (a portion of a long prompt beside single tokens): the
+    // blocks that can hold any are bounded by its rows.  Where they are no more than the CUs, 2 x 4 is the choice from 512
+    // tokens on and wherever there may be a cache to walk (2x2 / 2x4: 866 rows at 6,135 beside three tokens 235 / 149 us, 600
+    // at 4,096 137 / 103, 2 x 512 at 2,048 79 / 63, 8 prompts of up to 700 31 / 26; 257 tokens 15.5 / 16.8).
     int cg = 4, kg = 1;
+    bool uneven = false;
     {
         int gs, pts;
+        auto longest = [&]() { return (long)tp_cdiv(max_count, 32 << pts) * n_seq * KV * (G >> gs); };
+        auto filled = [&]() {
+            const long rows = ((long)M / (32 << pts) + n_seq) * KV * (G >> gs);
+            return rows < longest() ? rows : longest();
+        };
         plan(4, gs, pts);
-        const long blocks4 = (long)tp_cdiv(max_count, 32 << pts) * n_seq * KV * (G >> gs);
+        const long blocks4 = filled();
         plan(2, gs, pts);
-        const long blocks2 = (long)tp_cdiv(max_count, 32 << pts) * n_seq * KV * (G >> gs);
-        if (shape == 0 && blocks4 < 4L * cus) shape = HD > 128 && blocks2 <= 2L * cus && max_count >= 1024 ? 2 : 3;
+        const bool alone = HD > 128 && filled() <= cus && (paged || max_count >= 512);
+        if (shape == 0 && blocks4 < 4L * cus) shape = alone || (HD > 128 && longest() <= 2L * cus && max_count >= 1024) ? 2 : 3;
         if (shape == 2) { cg = 2; kg = 4; }
         if (shape == 3) { cg = 2; kg = 2; }
+        plan(cg, gs, pts);
+        uneven = 2 * filled() < longest();
     }
     plan(cg, a.ghb_shift, a.pt_shift);
     a.n_streams = n_seq * KV * (G >> a.ghb_shift);
     a.pos_blocks = tp_cdiv(max_count, 32 << a.pt_shift);
     const long blocks = (long)a.n_streams * a.pos_blocks;
+    // Blocks go round the 8 XCDs, so that a stream's blocks, every n_streams-th, meet the same ones: good for its keys' way through
+    // an L2, and for the load where all streams are alike, but one long sequence among short ones then runs on a few
+    // XCDs.  There every block of positions starts so many streams further on that a sequence's streams move round as if
+    // they were alone (2,045 rows at 4,090 beside three tokens, 2x2: 364 -> 208 us; where all are alike it costs: 8 x 7,900
+    // tokens 2.10 -> 2.20 ms).
+    a.turn = uneven ? (a.n_streams - a.n_streams / n_seq) % 8 : 0;
     TP_REQUIRE(blocks < (1L << 31), "attention prefill: %ld blocks exceed one launch", blocks);
     hipStream_t s = (hipStream_t)stream;
     int rc;
