@@ -565,7 +565,7 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
     // 186 / 130 / 114, 8 x 512 tokens 34 / 27 / 36; 9B sizes, 2,048 tokens 100 / 72 / 69; 27B (heads of 128) 85 / 78 / 89.
     // A step of uneven sequences launches more blocks than hold queries (a portion of a long prompt beside single tokens): the
     // blocks that can hold any are bounded by its rows.  Where they are no more than the CUs, 2 x 4 is the choice from 512
-    // tokens on and wherever there may be a cache to walk (2x2 / 2x4: 866 rows at 6,135 beside three tokens 235 / 149 us, 600
+    // tokens on, cached positions before them or not (2x2 / 2x4: 866 rows at 6,135 beside three tokens 235 / 149 us, 600
     // at 4,096 137 / 103, 2 x 512 at 2,048 79 / 63, 8 prompts of up to 700 31 / 26; 257 tokens 15.5 / 16.8).
     int cg = 4, kg = 1;
     bool uneven = false;
@@ -579,7 +579,7 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
         plan(4, gs, pts);
         const long blocks4 = filled();
         plan(2, gs, pts);
-        const bool alone = HD > 128 && filled() <= cus && (paged || max_count >= 512);
+        const bool alone = HD > 128 && filled() <= cus && max_count >= 512;
         if (shape == 0 && blocks4 < 4L * cus) shape = alone || (HD > 128 && longest() <= 2L * cus && max_count >= 1024) ? 2 : 3;
         if (shape == 2) { cg = 2; kg = 4; }
         if (shape == 3) { cg = 2; kg = 2; }
