@@ -87,6 +87,17 @@ def test_deferred_product_into_add_rms_norm(ops, m, n, k):
     assert rel_l2(stream, ref_stream) < 1e-5 and rel_l2(got, ref) < 6e-3
 
 
+# shapes that the tiles of 128 rows and the kernels of few rows would cut in slices, and of which the faster plan makes one
+@pytest.mark.parametrize("m,n,k", [(1145, 2304, 2048), (1280, 2304, 2048), (2048, 2304, 2048), (2049, 2048, 2048), (1500, 4096, 2304), (1000, 4608, 2304),
+                                   (2500, 1536, 2304), (8, 9216, 2304), (16, 12288, 2304), (64, 9216, 2304), (512, 9216, 2304)])
+def test_deferred_product_of_one_slice_keeps_its_sums(ops, m, n, k):
+    """What the consumer of a deferred product adds up is float32 whether the plan makes one slice of it or several."""
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=76), randn(n, k, dtype=torch.bfloat16, seed=77, scale=0.05)
+    rows = ops.linear(x, w, torch.bfloat16, defer=True)
+    ref = x.cpu().double() @ w.cpu().double().T
+    assert rows.dtype == torch.float32 and rel_l2(ops.rows(rows, torch.float32), ref) < 1e-5
+
+
 def test_rows_wider_than_the_fused_kernel_takes_are_added_first(ops):
     """A product in K slices whose rows are wider than `add_rms_norm` keeps in registers (8192): the slices are added by
     a kernel of their own, in slice order, and the result is what the fused path gives for narrower rows."""

@@ -53,17 +53,18 @@ bool gemm_rows8_supports(const GemmArgs& a);
 size_t gemm_rows8_workspace(const GemmArgs& a);
 int gemm_rows8_launch(const GemmArgs& a);
 bool gemm_mfma_supports(const GemmArgs& a);
-int gemm_mfma_splits(const GemmArgs& a);
+int gemm_mfma_slices_left(const GemmArgs& a);          // slices in the workspace after a deferred product; 0: rows of Y
 int gemm_mfma_launch(const GemmArgs& a);
 // bf16 on the matrix cores for many rows, blocks of 8 waves (K a multiple of 64): rows of X by rows of W a block, K in `splits`
-// slices of kps elements (left in the workspace when there are several)
+// slices of kps elements; slices: left in the workspace as float32 for the consumer to add
 enum { TP_WIDE_256x256 = 0, TP_WIDE_256x192, TP_WIDE_192x256, TP_WIDE_256x128, TP_WIDE_SHAPES };
-int gemm_wide_launch(const GemmArgs& a, int shape, int splits, int kps);
+int gemm_wide_launch(const GemmArgs& a, int shape, bool slices, int splits, int kps);
 // float32 on the matrix cores (K a multiple of 4, operands on 16 bytes), any number of rows; one fixed summation order per element
 bool gemm_f32_supports(const GemmArgs& a);
 int gemm_f32_splits(const GemmArgs& a);
 int gemm_f32_launch(const GemmArgs& a);
 // bf16 on the matrix cores for up to 64 rows (K a multiple of 64): streams W once through LDS, several k steps in flight
 bool gemm_stream_supports(const GemmArgs& a);
-size_t gemm_stream_workspace(const GemmArgs& a);
+int gemm_stream_splits(const GemmArgs& a);
+int gemm_stream_slices_left(const GemmArgs& a);        // as gemm_mfma_slices_left
 int gemm_stream_launch(const GemmArgs& a);

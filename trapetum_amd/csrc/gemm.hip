@@ -130,7 +130,7 @@ static int pick(const GemmArgs& a, int algo) {
     const bool sliced = a.defer && a.epilogue == TP_EPI_NONE;
     if (gemm_stream_supports(a) && a.M > 1) {
         const bool rows8 = a.M < 8 && gemm_rows8_supports(a) && (a.epilogue == TP_EPI_GATED || a.K <= ONE_ROUND_K || a.N >= WIDE_N);
-        if ((sliced && gemm_stream_workspace(a)) || (a.N > STREAM_N && (a.M > 2 || !gemv_supports(a)) && !rows8)) return 16;
+        if ((sliced && gemm_stream_splits(a) > 1) || (a.N > STREAM_N && (a.M > 2 || !gemv_supports(a)) && !rows8)) return 16;
     }
     if (gemv_supports(a)) return 4;          // one or two rows: 2B gate/up 16.8 against 22.6 us on the skinny kernel
     // What is left: few rows of W, or K no multiple of 64.  Three to eight rows: the kernel whose blocks read 8 rows of W in one
@@ -166,8 +166,8 @@ static int pick(const GemmArgs& a, int algo) {
     return 1;
 }
 
-// bytes of workspace a product needs; with defer, a positive multiple of M * N * 4 above one slice means the
-// product comes back as that many K slices
+// bytes of workspace a product needs; with defer, a positive multiple of M * N * 4 means the product comes back as that
+// many float32 K slices (one of them, where its sums are not to be rounded), 0 that the call is to be made again without defer
 extern "C" long tp_linear_workspace_bytes(int in_dtype, int out_dtype, int M, int N, int K, int epilogue, int units,
                                           int defer, int algo) {
     GemmArgs a{nullptr, nullptr, nullptr, in_dtype, out_dtype, M, N, K, epilogue, 1.f, units, 0, INFINITY, 0.f, nullptr, 0, defer, algo, nullptr};
@@ -175,8 +175,8 @@ extern "C" long tp_linear_workspace_bytes(int in_dtype, int out_dtype, int M, in
     if (p == 2) return (long)gemm_skinny_workspace(a);
     if (p == 4) return (long)gemv_workspace(a);
     if (p == 5) return (long)gemm_rows8_workspace(a);
-    if (p == 16) return (long)gemm_stream_workspace(a);
-    if (p == 3) { const int s = gemm_mfma_splits(a); return s > 1 ? (long)s * M * N * 4 : 0; }
+    if (p == 16) return (long)gemm_stream_slices_left(a) * M * N * 4;
+    if (p == 3) return (long)gemm_mfma_slices_left(a) * M * N * 4;
     if (p == 20) { const int s = gemm_f32_splits(a); return s > 1 ? (long)s * M * N * 4 : 0; }
     if (p == 1 && epilogue == TP_EPI_GATED) return (long)M * N * 4;
     return 0;

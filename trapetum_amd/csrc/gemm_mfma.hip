@@ -326,7 +326,8 @@ bool gemm_mfma_supports(const GemmArgs& a) {
 // instruction; two blocks fit a CU) for grids of at least four rounds of those 512 places (2B gate/up, register-staged:
 // 930 against 790 TFLOP/s at 8192 rows, 700 against 790 at 2048).
 struct Tile { int tm, tn, wm = 2; bool deep = false; };        // wm: waves along the rows of X (2 x 2 or 4 x 1)
-struct Plan { Tile tile; int splits; bool direct = false; int wide = -1; };       // wide: TP_WIDE_* of the kernel of 8 waves
+// wide: TP_WIDE_* of the kernel of 8 waves; sums: a deferred product leaves its sums as float32 slices, one of them included
+struct Plan { Tile tile; int splits; bool direct = false; int wide = -1; bool sums = false; };
 
 // K slices of a product of few rows, which is bound by reading W and wants every CU streaming.  From 17 rows on one
 // block a CU: more slices cost their consumer more than they gain (a 2B decode step of 64 sequences takes 3.52 ms
@@ -383,11 +384,16 @@ static Plan wide_plan(const GemmArgs& a, int shape, bool may_slice, double slice
 // no multiple of 64: the most blocks a CU gets x 0.64 us a step, fitted to the 2B down product at 2,048 rows), plus
 // what writing and reading a further float32 slice of Y costs.  The wide tiles of
 // gemm_wide.hip take part where they can run.
+// Where these tiles alone would be cut in slices, the consumer gets float32 sums, and it gets them also where the faster plan
+// has one slice: no sum is rounded to bf16 that was not before there were wide tiles (W_o at 2,048 rows, N 2304, K 2048: error
+// against 64 bits 1.7e-3 rounded, 2.7e-7 so, 40.0 / 44.6 us with the norm that reads it).  The others stay bf16 rows (8,191
+// rows, N 3584, K 4096: 266 us with the norm, 289 as float32).
 static Plan mid_tile_plan(const GemmArgs& a, bool may_slice) {
     const double step_us = 0.64, slice_us = (double)a.M * a.N * 8 / 4.0e6;
     const bool direct = direct_ok(a) && a.algo != 7;
     Plan best{{4, 4}, 1, direct};
-    double best_cost = 1e30;
+    double best_cost = 1e30, alone_cost = 1e30;
+    int alone = 1;                                   // slices of the cheapest plan of these tiles by their own model
     for (int tn = 4; tn >= 3; tn--) {
         if (tn == 3 && a.epilogue == TP_EPI_GATED) continue;             // gate and up columns come in pairs of tiles
         const long tiles = (long)tp_cdiv(a.M, 128) * tp_cdiv(a.N, 32 * tn);
@@ -397,8 +403,10 @@ static Plan mid_tile_plan(const GemmArgs& a, bool may_slice) {
             // a grid of at most one block a CU is faster by the register-staged loop (0.85 us a step against 1.0:
             // 128 x 96 tiles at 512 rows, 2B shapes: qkv 30.7 against 35.5 us, down 102 against 119)
             const bool d = direct && tiles * s > 256;
-            const double per_step = d ? 1.17 * direct_step_us(tiles * s) : tiles * s <= 256 ? 0.85 : (double)tp_cdiv(tiles * s, 256) * step_us;
-            const double cost = per_step * k_steps * (tn == 3 ? 0.8 : 1.0) + (s - 1) * slice_us;
+            const double per_step = d ? direct_step_us(tiles * s) : tiles * s <= 256 ? 0.85 : (double)tp_cdiv(tiles * s, 256) * step_us;
+            const double steps_us = per_step * k_steps * (tn == 3 ? 0.8 : 1.0), own = steps_us + (s - 1) * slice_us;
+            const double cost = (d ? 1.17 * steps_us : steps_us) + (s - 1) * slice_us;
+            if (own < alone_cost * 0.97) { alone_cost = own; alone = s; }
             if (cost < best_cost * 0.97) { best_cost = cost; best = {{4, tn}, s, d}; }   // a tie stays with the earlier, plainer plan
         }
     }
@@ -407,6 +415,7 @@ static Plan mid_tile_plan(const GemmArgs& a, bool may_slice) {
         const Plan p = wide_plan(a, shape, may_slice, slice_us, &cost);
         if (cost < best_cost * 0.97) { best_cost = cost; best = p; }
     }
+    best.sums = alone > 1;
     return best;
 }
 
@@ -453,11 +462,12 @@ static Plan final_plan(const GemmArgs& a) {
         const int kps = tp_cdiv(tp_cdiv(a.K, p.splits), kstep) * kstep;
         p.splits = tp_cdiv(a.K, kps);
     }
+    p.sums = a.defer && (p.sums || p.splits > 1);
     return p;
 }
 
-// K slices for products whose tiles alone do not fill the chip and whose consumer adds the slices (defer)
-int gemm_mfma_splits(const GemmArgs& a) { return final_plan(a).splits; }
+// K slices for products whose tiles alone do not fill the chip and whose consumer adds the slices (defer); 0: none are left
+int gemm_mfma_slices_left(const GemmArgs& a) { const Plan p = final_plan(a); return p.sums ? p.splits : 0; }
 
 template <int EPI, int TM, int TN, int KS = BK, int WM = 2, bool DEEP = false>
 static void mfma_launch(const GemmArgs& a, void* y, int out_dtype, int splits, int kps) {
@@ -506,17 +516,17 @@ int gemm_mfma_launch(const GemmArgs& a) {
     const Plan plan = final_plan(a);
     const Tile t = plan.tile;
     const int splits = plan.splits;
-    if (splits > 1) {
+    if (plan.sums) {
         const size_t need = (size_t)splits * a.M * a.N * sizeof(float);
         TP_REQUIRE(a.workspace && a.workspace_bytes >= need, "tiled product: workspace of %zu bytes, %zu needed", a.workspace_bytes, need);
         const int kstep = t.tm <= 2 ? SMALL_KS : BK;
         const int kps = tp_cdiv(tp_cdiv(a.K, splits), kstep) * kstep;
-        if (plan.wide >= 0) return gemm_wide_launch(a, plan.wide, tp_cdiv(a.K, kps), kps);
+        if (plan.wide >= 0) return gemm_wide_launch(a, plan.wide, true, tp_cdiv(a.K, kps), kps);
         if (plan.direct) mfma_launch_direct<TP_EPI_NONE>(a, t, a.workspace, TP_F32, tp_cdiv(a.K, kps), kps);
         else mfma_launch_tile<TP_EPI_NONE>(a, t, a.workspace, TP_F32, tp_cdiv(a.K, kps), kps);
         return tp_check_launch("linear (tiled kernel, K slices)");
     }
-    if (plan.wide >= 0) return gemm_wide_launch(a, plan.wide, 1, a.K);
+    if (plan.wide >= 0) return gemm_wide_launch(a, plan.wide, false, 1, a.K);
     if (plan.direct) {
         if (a.epilogue == TP_EPI_GATED) mfma_launch_direct<TP_EPI_GATED>(a, t, a.y, a.out_dtype, 1, a.K);
         else if (a.epilogue == TP_EPI_SOFTCAP) mfma_launch_direct<TP_EPI_SOFTCAP>(a, t, a.y, a.out_dtype, 1, a.K);

@@ -237,9 +237,9 @@ static void wide_launch(const GemmArgs& a, void* y, int out_dtype, int splits, i
         (const bf16_t*)a.x, (const bf16_t*)a.w, y, a.M, a.N, a.K, m_tiles, out_dtype, epi_constants(a), a.units, kps, 4);
 }
 
-int gemm_wide_launch(const GemmArgs& a, int shape, int splits, int kps) {
-    void* y = splits > 1 ? a.workspace : a.y;
-    const int out_dtype = splits > 1 ? TP_F32 : a.out_dtype;
+int gemm_wide_launch(const GemmArgs& a, int shape, bool slices, int splits, int kps) {
+    void* y = slices ? a.workspace : a.y;
+    const int out_dtype = slices ? TP_F32 : a.out_dtype;
 #define TP_WIDE(EPI) do { \
         if (shape == TP_WIDE_256x256) wide_launch<EPI, 4, 2, 2, 2>(a, y, out_dtype, splits, kps); \
         else if (shape == TP_WIDE_256x192) wide_launch<EPI, 2, 3, 4, 2>(a, y, out_dtype, splits, kps); \

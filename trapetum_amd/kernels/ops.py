@@ -1082,7 +1082,7 @@ class HipOps:
             algo = 1                   # off the 16 bytes that the float32 matrix-core kernels read at once: the plain kernel
         nbytes = self.lib.tp_linear_workspace_bytes(_code(x.dtype), _code(out_dtype), m, n, k, epilogue, units,
                                                     1 if defer else 0, algo)
-        if defer and epilogue == EPI_NONE and nbytes and nbytes % (m * n * 4) == 0 and nbytes // (m * n * 4) > 1:
+        if defer and nbytes:           # of a product without an epilogue: all of the workspace is its slices, which may be one
             slices = torch.empty((nbytes // (m * n * 4), m, n), dtype=torch.float32, device=self.device)
             self._call(self.lib, "tp_linear", x.data_ptr(), w.data_ptr(), None, _code(x.dtype), _code(out_dtype),
                        m, n, k, epilogue, float(cap), units, act, float(limit), float(shift), slices.data_ptr(), nbytes, 1, algo, self._stream())
