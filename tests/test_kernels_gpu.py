@@ -737,6 +737,36 @@ def test_attention_decode_step(ops, splits, slices, H, KV, hd, lens, page, windo
         assert torch.equal(before[0], pools[0]) and torch.equal(before[1], pools[1])
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("H,KV,hd", [(2, 1, 64), (2, 2, 300), (1, 1, 520)])
+def test_plain_attention_with_hidden_groups_and_infinite_values(ops, dt, H, KV, hd):
+    """A bias of minus infinity hides whole groups of keys, a wave's first ones among them; a value of infinity at the query's
+    own position comes out as infinity in its element and nowhere else."""
+    n, reach = 131, 140
+    q, k = randn(n, H * hd, dtype=DT[dt], seed=80), randn(n, KV * hd, dtype=DT[dt], seed=81)
+    v = randn(n, KV * hd, dtype=DT[dt], seed=82)
+    bias = randn(H, reach + 1, seed=83).float()
+    bias[:, 60:87] = bias[:, 30:34] = bias[:, 97:127] = -math.inf
+    cu = torch.tensor([0, n], dtype=torch.int32)
+    args = (H, KV, hd, cu, n, hd ** -0.5, 20.0, 0)
+    more = dict(row_seq=torch.zeros(n, dtype=torch.int32), row_pos=torch.arange(n, dtype=torch.int32))
+    ref = ref_ops.attention_prefill(q.cpu(), k.cpu(), v.cpu(), *args, torch.float32, **more, by_position=ref_ops.ByPosition(bias=bias.cpu()))
+    dev = dict((name, t.to(DEV)) for name, t in more.items())
+    ops.force_plain_attention = True
+    try:
+        run = lambda v: ops.attention_prefill(q, k, v, H, KV, hd, cu.to(DEV), *args[4:], DT[dt], **dev, by_position=ops.ByPosition(bias=bias))
+        got = run(v)
+        v[100, 3] = math.inf
+        last = run(v)[100].float()
+    finally:
+        ops.force_plain_attention = False
+    assert rel_l2(got, ref) < (3e-6 if dt == "f32" else 8e-3)
+    of_head = [h * hd + 3 for h in range(H) if h // (H // KV) == 0]
+    assert all(float(last[c]) == math.inf for c in of_head)
+    rest = [c for c in range(H * hd) if c not in of_head]
+    assert torch.equal(last[rest], got[100].float()[rest])
+
+
 def test_attention_far_key_stands_out(ops):
     """One key among hundreds carries the answer: its score is made to dominate, so a kernel that drops
     or misplaces it (a chunk boundary, a page boundary) returns another value row."""

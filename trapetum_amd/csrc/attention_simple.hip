@@ -90,7 +90,7 @@ attn_simple_k(AttnSimpleArgs a) {
                 const int dc = d < a.hd ? d : 0;
                 const float kx = ld_f32(kp + dc), vx = ld_f32(vp + dc);
                 kk[n][j] = d < a.hd ? kx : 0.f;
-                vv[n][j] = d < a.hd ? vx : 0.f;
+                vv[n][j] = d < a.hd && first + n < n_keys ? vx : 0.f;      // (no weight times an infinite value)
             }
         }
     };
@@ -122,7 +122,8 @@ attn_simple_k(AttnSimpleArgs a) {
 #pragma unroll
         for (int x = 1; x < KEYS; x <<= 1) top = fmaxf(top, __shfl_xor(top, x, 64));
         const float m_new = fmaxf(m, top);
-        const float alpha = expf(m - m_new), pr = first + mine < n_keys ? expf(s - m_new) : 0.f;
+        // (a group whose scores are all -infinity, by a bias or an overflow, leaves the state as it is; a NaN goes through)
+        const float alpha = m == m_new ? 1.f : expf(m - m_new), pr = s == -INFINITY ? 0.f : expf(s - m_new);
         float sum = pr;
 #pragma unroll
         for (int x = 1; x < KEYS; x <<= 1) sum += __shfl_xor(sum, x, 64);
@@ -164,7 +165,7 @@ attn_simple_k(AttnSimpleArgs a) {
     float f[WAVES], total = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; w++) {
-        f[w] = w < used ? expf(part_m[w] - top) : 0.f;
+        f[w] = w < used && part_m[w] != -INFINITY ? expf(part_m[w] - top) : 0.f;
         if (w < used) total += part_l[w] * f[w];
     }
     if (a.sink) total += expf(a.sink[h] - top);
