@@ -19,7 +19,8 @@ namespace {
 constexpr int PARTS = 16, GROUP = 4;
 constexpr int TM = 64, TN = 128;
 
-__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+// until every load, and every LDS read (whose buffer is filled again behind the barrier), is done
+__device__ __forceinline__ void wait_all() { __builtin_amdgcn_s_waitcnt(0x0070); }
 
 __device__ __forceinline__ float epilogue_f32(int epilogue, float o, float4 epi, int n) {
     if (epilogue == TP_EPI_SILU) return (float)n < epi.z ? gate_act_exact(o, TP_ACT_SILU) : o;
@@ -153,7 +154,8 @@ gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float*
     int part_end = from + part_blocks, parts = 0;
     fill(0);
     for (int step = 0; step < steps; step++) {
-        wait_loads();
+        asm volatile("" ::: "memory");
+        wait_all();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();            // the step's tiles are there, and the other buffer has been read by everyone
         asm volatile("" ::: "memory");
