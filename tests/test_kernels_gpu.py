@@ -318,6 +318,22 @@ def test_linear_f32_is_one_order(ops, m, n, k):
         assert rel_l2(ops.gated_linear(off, packed, half - 3, "silu", torch.float32, limit=2.0, up_shift=0.5), gated) < 5e-6
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 16, 4), (17, 33, 260), (33, 129, 36), (70, 200, 2304), (309, 250, 1028)])
+def test_linear_f32_bits_do_not_depend_on_where_operands_lie(ops, m, n, k):
+    def off(t, by):
+        room = torch.empty(t.numel() + by, device=DEV)[by:].view(t.shape)
+        return room.copy_(t)
+    x, w = randn(m, k, seed=11), randn(n, k, seed=12, scale=0.05)
+    got = ops.linear(x, w, torch.float32)
+    half = n // 2 // 16 * 16
+    for i, j in ((1, 0), (0, 2), (3, 1)):
+        assert torch.equal(ops.linear(off(x, i), off(w, j), torch.float32), got)
+        assert torch.equal(ops.rows(ops.linear(off(x, i), off(w, j), torch.float32, defer=True), torch.float32), got)
+        if half:
+            packed = ops.pack_gate_up(w[:half], w[half:2 * half])
+            assert torch.equal(ops.gated_linear(off(x, i), off(packed, j), half, "silu", torch.float32), ops.gated_linear(x, packed, half, "silu", torch.float32))
+
+
 @pytest.mark.parametrize("algo", [1, 2, 3, 4, 5, 6, 8, 10, 11])
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
 @pytest.mark.parametrize("m,inter,k", [(1, 16, 16), (4, 200, 88), (40, 320, 96), (9, 1000, 2304), (150, 72, 136),

@@ -59,7 +59,7 @@ int gemm_mfma_launch(const GemmArgs& a);
 // slices of kps elements; slices: left in the workspace as float32 for the consumer to add
 enum { TP_WIDE_256x256 = 0, TP_WIDE_256x192, TP_WIDE_192x256, TP_WIDE_256x128, TP_WIDE_SHAPES };
 int gemm_wide_launch(const GemmArgs& a, int shape, bool slices, int splits, int kps);
-// float32 on the matrix cores (K a multiple of 4, operands on 16 bytes), any number of rows; one fixed summation order per element
+// float32 on the matrix cores (K a multiple of 4), any number of rows; one fixed summation order per element
 bool gemm_f32_supports(const GemmArgs& a);
 int gemm_f32_splits(const GemmArgs& a);
 int gemm_f32_launch(const GemmArgs& a);

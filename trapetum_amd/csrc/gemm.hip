@@ -1,7 +1,7 @@
 // Entry points of the matrix products and the plain tiled kernel.
 //
 // The plain kernel (every output element summed over k in index order whatever the batch is) is the fallback of both paths for
-// shapes that the matrix-core kernels refuse: a K that is no multiple of 4 (float32) or 8 (bf16), operands off their 16 bytes.  The reference's products are 4-bit codebook GEMVs
+// shapes that the matrix-core kernels refuse: a K that is no multiple of 4 (float32) or 8 (bf16).  The reference's products are 4-bit codebook GEMVs
 // (runtime/cuda/codebook_gemv.cu:86-114); its only dense one is gemv_fp16_warp_k (cu:496-517).
 #include "gemm.h"
 

@@ -14,6 +14,7 @@
 #include "gemm.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f3_f32x4;
+typedef f3_f32x4 f3_anywhere __attribute__((aligned(4)));        // (the same load: a global one needs no more)
 
 namespace {
 constexpr int PARTS = 16, GROUP = 4;
@@ -55,9 +56,9 @@ gemm_f32_few_k(const float* __restrict__ X, const float* __restrict__ W, float* 
         for (int u = 0; u < AHEAD; u++) {
             const int k = min(min(b + u, to - 1) * 16 + 4 * g, K - 4);       // past the end: elements that exist, zeroed or unused below
 #pragma unroll
-            for (int j = 0; j < NT; j++) w[u][j] = *reinterpret_cast<const f3_f32x4*>(wr[j] + k);
+            for (int j = 0; j < NT; j++) w[u][j] = *reinterpret_cast<const f3_anywhere*>(wr[j] + k);
 #pragma unroll
-            for (int i = 0; i < MT; i++) x[u][i] = *reinterpret_cast<const f3_f32x4*>(xr[i] + k);
+            for (int i = 0; i < MT; i++) x[u][i] = *reinterpret_cast<const f3_anywhere*>(xr[i] + k);
         }
 #pragma unroll
         for (int u = 0; u < AHEAD; u++) {
@@ -232,14 +233,13 @@ gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float*
     }
 }
 
-// rows read in 16-byte pieces; a tile's rows within 32-bit offsets
-bool gemm_f32_supports(const GemmArgs& a) {
-    return a.in_dtype == TP_F32 && a.out_dtype == TP_F32 && a.K % 4 == 0 && a.K < (1 << 23) && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0;
-}
+// rows read in pieces of four; a tile's rows within 32-bit offsets
+bool gemm_f32_supports(const GemmArgs& a) { return a.in_dtype == TP_F32 && a.out_dtype == TP_F32 && a.K % 4 == 0 && a.K < (1 << 23); }
 
 // Up to 32 rows the kernel of few rows reads W once and its matrix instructions fit into that time; from 33 on the other
-// does the same work on whole tiles.
-static bool few(const GemmArgs& a) { return a.M <= 32; }
+// does the same work on whole tiles.  Its loads into LDS want operands on 16 bytes: off them any number of rows goes to the
+// first, in tiles of 32, so that a product's bits do not depend on where its operands lie.
+static bool few(const GemmArgs& a) { return a.M <= 32 || (uintptr_t)a.x % 16 || (uintptr_t)a.w % 16; }
 
 int gemm_f32_splits(const GemmArgs& a) {
     return !few(a) && a.defer && a.epilogue == TP_EPI_NONE && a.K >= 1024 && (long)tp_cdiv(a.M, TM) * tp_cdiv(a.N, TN) < 256 ? PARTS / GROUP : 1;
@@ -247,7 +247,7 @@ int gemm_f32_splits(const GemmArgs& a) {
 
 template <int NT, bool GATED>
 static void few_launch(const GemmArgs& a, int part_blocks, float4 epi) {
-    const int blocks = tp_cdiv(a.N, 16 * NT);
+    const dim3 blocks(tp_cdiv(a.N, 16 * NT), tp_cdiv(a.M, a.M <= 16 ? 16 : 32));
     if (a.M <= 16) gemm_f32_few_k<NT, 1, GATED><<<blocks, 1024, 0, a.stream>>>((const float*)a.x, (const float*)a.w, (float*)a.y, a.M, a.N, a.K, part_blocks, a.epilogue, epi, a.units, a.act);
     else gemm_f32_few_k<NT, 2, GATED><<<blocks, 1024, 0, a.stream>>>((const float*)a.x, (const float*)a.w, (float*)a.y, a.M, a.N, a.K, part_blocks, a.epilogue, epi, a.units, a.act);
 }
@@ -257,6 +257,8 @@ int gemm_f32_launch(const GemmArgs& a) {
     const bool gated = a.epilogue == TP_EPI_GATED;
     const float4 epi = gated ? make_float4(0.f, 0.f, a.limit, a.shift) : make_float4(a.cap, 0.f, (float)a.units, 0.f);
     if (few(a)) {
+        TP_REQUIRE(a.y, "float32 product: K slices are left of operands on 16 bytes only");
+        TP_REQUIRE(tp_cdiv(a.M, 32) <= 65535, "float32 product: %d rows off 16 bytes exceed one launch", a.M);
         // two tiles of W share the block's X where that leaves two blocks a CU
         if (gated) few_launch<2, true>(a, part_blocks, epi);
         else if (a.N >= 32 * 512) few_launch<2, false>(a, part_blocks, epi);

@@ -1078,8 +1078,8 @@ class HipOps:
             raise KernelError(f"linear: rows have {k} columns, the matrix {w.shape[1]}")
         cols = units if epilogue == EPI_GATED else n
         algo = self.force_linear
-        if algo == 0 and x.dtype == torch.float32 and (x.data_ptr() | w.data_ptr()) % 16:
-            algo = 1                   # off the 16 bytes that the float32 matrix-core kernels read at once: the plain kernel
+        if x.dtype == torch.float32 and (x.data_ptr() | w.data_ptr()) % 16:
+            defer = False              # slices are left by the float32 kernel that reads 16 bytes into LDS at once
         nbytes = self.lib.tp_linear_workspace_bytes(_code(x.dtype), _code(out_dtype), m, n, k, epilogue, units,
                                                     1 if defer else 0, algo)
         if defer and nbytes:           # of a product without an epilogue: all of the workspace is its slices, which may be one
