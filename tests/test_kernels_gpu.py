@@ -753,6 +753,50 @@ def test_attention_decode_step(ops, splits, slices, H, KV, hd, lens, page, windo
         assert torch.equal(before[0], pools[0]) and torch.equal(before[1], pools[1])
 
 
+# launches of many rows that see few keys, which a wave a row works on: prompts that end inside a group of keys, at one and after
+# the eighth, decode steps, a window over a long prompt, chunks; and rows that see more keys than the caller's bound says
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("H,KV,hd", [(8, 2, 48), (8, 8, 100), (8, 4, 256), (8, 2, 300), (8, 4, 520)])
+def test_plain_attention_of_many_rows_with_few_keys(ops, dt, H, KV, hd):
+    lens = ([1, 2, 3, 4, 5, 8, 9, 31, 32, 33] * 40)[:400 if hd > 256 else 120]
+    M, seqs = sum(lens), len(lens)
+    q, k, v = (randn(M, heads * hd, dtype=DT[dt], seed=84 + i) for i, heads in enumerate((H, KV, KV)))
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    seq = torch.repeat_interleave(torch.arange(seqs, dtype=torch.int32), torch.tensor(lens))
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
+    bias, sink, temp = randn(H, 12, seed=87), randn(H, seed=88), (0.5 + torch.rand(H)).to(DEV)
+
+    def run(a, b, cu, seq, pos, most, **more):
+        return ops.attention_prefill(q[a:b], k[a:b], v[a:b], H, KV, hd, cu.to(DEV), most, hd ** -0.5, 20.0, more.pop("window", 0), DT[dt],
+                                     row_seq=seq.to(DEV), row_pos=pos.to(DEV), **more)
+    ops.force_plain_attention = True
+    try:
+        for more in ({}, dict(window=5), dict(window=6, keep=2, sink=sink), dict(chunk=7, head_scale=temp),
+                     dict(by_position=ops.ByPosition(temperature=(0.3, 4), bias=bias))):
+            got = run(0, M, cu, seq, pos, 33, **more)
+            for s in range(0, seqs, 13 if seqs > 13 else 1):      # a sequence alone: few rows, which blocks work on
+                a, b = int(cu[s]), int(cu[s + 1])
+                own = run(a, b, torch.tensor([0, b - a], dtype=torch.int32), torch.zeros(b - a, dtype=torch.int32), pos[a:b], 1000, **more)
+                assert torch.equal(got[a:b], own), (s, more)
+        one, whole = torch.tensor([0, M], dtype=torch.int32), (torch.zeros(M, dtype=torch.int32), torch.arange(M, dtype=torch.int32))
+        assert torch.equal(run(0, M, one, *whole, 1), run(0, M, one, *whole, 10 ** 6))      # a bound that is too small costs time alone
+        few = run(0, M, one, *whole, 10 ** 6, window=40)
+        for r in range(0, M, 97):
+            a = max(0, r - 39)
+            own = ops.attention_prefill(q[a:r + 1], k[a:r + 1], v[a:r + 1], H, KV, hd, torch.tensor([0, r + 1 - a], dtype=torch.int32, device=DEV), 1000,
+                                        hd ** -0.5, 20.0, 40, DT[dt], row_seq=torch.zeros(r + 1 - a, dtype=torch.int32, device=DEV),
+                                        row_pos=torch.arange(r + 1 - a, dtype=torch.int32, device=DEV))[-1]
+            assert torch.equal(few[r], own), r
+        n, page = 300, 16
+        pools = [randn(n, KV, page, hd, dtype=DT[dt], seed=90 + i) for i in range(2)]
+        held, table = torch.arange(n, dtype=torch.int32, device=DEV) % page + 1, torch.arange(n, dtype=torch.int32, device=DEV).view(n, 1)
+        step = lambda a, b, most: ops.attention_decode(q[a:b], H, KV, hd, held[a:b], table[a:b], *pools, 0, hd ** -0.5, 20.0, 0, DT[dt], max_keys=most)
+        together = step(0, n, page if hd <= 256 else 4)
+        assert all(torch.equal(together[r:r + 1], step(r, r + 1, 1000)) for r in range(0, n, 7))
+    finally:
+        ops.force_plain_attention = False
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("H,KV,hd", [(2, 1, 64), (2, 2, 300), (1, 1, 520)])
 def test_plain_attention_with_hidden_groups_and_infinite_values(ops, dt, H, KV, hd):

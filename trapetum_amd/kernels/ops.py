@@ -57,8 +57,8 @@ _CORE_SIGS = {
     "tp_time_mix_scan_workspace_floats": [_I, _I, _I, _I],
     "tp_matrix_memory_scan_workspace_floats": [_I, _I, _I, _I, _I],
     "tp_linear_workspace_bytes": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
-    "tp_attn_simple_prefill": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _P, _P],
-    "tp_attn_simple_decode": [_P, _L, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _P, _P],
+    "tp_attn_simple_prefill": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P],
+    "tp_attn_simple_decode": [_P, _L, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P],
     "tp_argmax": [_P, _I, _I, _P, _P, _P],
     "tp_argmax_workspace_bytes": [_I, _I],
     "tp_repetition_penalty": [_P, _I, _I, _P, _I, _F, _P],
@@ -1229,8 +1229,15 @@ class HipOps:
                    m, H, KV, hd, cu_rows.data_ptr(), row_seq.data_ptr(), row_pos.data_ptr(), ptr(new_len), ptr(table), table_w,
                    ptr(k_pool), ptr(v_pool), page, rows_cap, float(scale), float(softcap),
                    int(window), int(chunk), ptr(head_scale), ptr(sink), int(keep), int(pin) if cached is not None else 0, pos_ref,
-                   out.data_ptr(), self._stream())
+                   self._most_keys(max_count if cached is None else None, window, chunk, keep), out.data_ptr(), self._stream())
         return out
+
+    @staticmethod
+    def _most_keys(longest, window, chunk, keep):
+        """A bound on the keys that a query of the step sees, 0 where there is none: what the plain kernel's way of sharing
+        out its waves is chosen by (its results do not depend on it)."""
+        bounds = [int(b) for b in (longest, window + keep if window else 0, chunk) if b]
+        return min(bounds) if bounds else 0
 
     def _head_vectors(self, what, H, chunk, head_scale, sink):
         """Checks a chunk size and the vectors of one number per head; whether any of them is asked for."""
@@ -1305,7 +1312,8 @@ class HipOps:
         self._call(self.lib, "tp_attn_simple_decode", q.data_ptr(), qs, _code(q.dtype), n, H, KV, hd, new_len.data_ptr(),
                    table.data_ptr(), table.shape[1], k_pool.data_ptr(), v_pool.data_ptr(), k_pool.shape[2], rows_cap,
                    float(scale), float(softcap), int(window), int(chunk), head_scale.data_ptr() if head_scale is not None else None,
-                   sink.data_ptr() if sink is not None else None, int(keep), int(pin), pos_ref, out.data_ptr(), self._stream())
+                   sink.data_ptr() if sink is not None else None, int(keep), int(pin), pos_ref,
+                   self._most_keys(max_keys, window, chunk, keep), out.data_ptr(), self._stream())
         return out
 
     def fuses_decode_step(self, dtype, H, KV, hd, k_pool):
