@@ -827,6 +827,26 @@ def test_plain_attention_with_hidden_groups_and_infinite_values(ops, dt, H, KV, 
     assert torch.equal(last[rest], got[100].float()[rest])
 
 
+@pytest.mark.parametrize("H,KV,hd,n,long,others", [(8, 4, 256, 64, 5000, 37), (4, 2, 64, 96, 2500, 70), (16, 16, 128, 17, 3001, 5), (8, 4, 256, 64, 120, 90)])
+def test_attention_decode_of_one_long_sequence_among_short_ones(ops, H, KV, hd, n, long, others):
+    """The slices are counted for the longest sequence: every sequence's result is that of its own keys."""
+    page, lens = 64, [others - i % 3 for i in range(n)]
+    lens[n // 3] = long
+    pages = [-(-x // page) for x in lens]
+    pools = [randn(sum(pages), KV, page, hd, dtype=torch.bfloat16, seed=94 + i) for i in range(2)]
+    table = torch.zeros(n, max(pages), dtype=torch.int32)
+    for i, c in enumerate(pages):
+        table[i, :c] = torch.arange(sum(pages[:i]), sum(pages[:i]) + c)
+    q, held = randn(n, H * hd, dtype=torch.bfloat16, seed=96), torch.tensor(lens, dtype=torch.int32)
+    got = ops.attention_decode(q, H, KV, hd, held.to(DEV), table.to(DEV), *pools, 0, hd ** -0.5, 30.0, 0, torch.bfloat16, max_keys=long)
+    some = [0, n // 3, n - 1]
+    ref = ref_ops.attention_decode(q.cpu()[some], H, KV, hd, held[some], table[some], *[p.cpu() for p in pools], 0, hd ** -0.5, 30.0, 0, torch.float32)
+    assert (ops.decode_splits(n, KV, hd, long) > 1) == (long > 128)
+    assert all(rel_l2(got[s], ref[i]) < 8e-3 for i, s in enumerate(some))
+    alone = ops.attention_decode(q[:1], H, KV, hd, held[:1].to(DEV), table[:1].to(DEV), *pools, 0, hd ** -0.5, 30.0, 0, torch.bfloat16, max_keys=lens[0])
+    assert rel_l2(got[:1], alone) < 8e-3
+
+
 def test_attention_far_key_stands_out(ops):
     """One key among hundreds carries the answer: its score is made to dominate, so a kernel that drops
     or misplaces it (a chunk boundary, a page boundary) returns another value row."""

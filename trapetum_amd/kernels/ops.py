@@ -1250,15 +1250,23 @@ class HipOps:
 
     @staticmethod
     def decode_splits(n, KV, hd, keys):
-        """Slices of the keys per (sequence, kv head) in a decode step, each with at least one round of 64 keys: two blocks
-        a CU in all, one where the pairs are few (the slices' sums then cost more than another block brings), and none
-        where the pairs alone are a block a CU.  Measured on MI355X (heads of 256, microseconds, three to six blocks a
-        CU / this): 1 x 8,000 keys 22.8 / 18.4, 1 x 4,000 of 8 kv heads 18.4 / 16.6, 4 of up to 7,000 29.3 / 24.5, 8 x 4,096
-        34.8 / 32.7, 16 x 2,000 32.6 / 32.0, 32 x 1,000 33.1 / 32.7, 64 x 500 30.8 / 31.0, 64 x 2,000 101.2 / 98.0, 64 of up to 80
-        keys 12.4 / 10.2."""
+        """Slices of the keys per (sequence, kv head) in a decode step.  `keys` is the longest sequence, or a graph's bound on
+        it; the others may be short, and the step takes as long as its longest block walks (31 ns a key, heads of 256).  So
+        there are one to four blocks a CU in all, by the number of pairs, and more where a block would walk over 320 keys (up
+        to six a CU), 512 from 128 pairs on and 1,024 from 512 on, where a further slice of every pair costs more (1.8 ns); a
+        slice has at least one round of 64 keys, two from 128 pairs on.  MI355X, heads of 256, 4 kv heads unless said,
+        microseconds, [three to six blocks a CU / one to two / this]: one sequence of 8,000 beside 63 of 100 [157 / 248 / 50],
+        beside 31 [51 / 90 / 44], beside 15 [33.6 / 50.7 / 33.6]; 64 of 50 to 7,900 [229 / 301 / 233], of 20 to 1,000 [32.0 / 39.1 /
+        32.0], of 2,000 [98.8 / 100.2 / 99.7], of up to 80 under a bound of 1,024 [11.0 / 9.0 / 11.0]; 32 of 1,000 [29.6 / 29.1 / 29.5];
+        8 of 7,900 [48.4 / 46.9 / 46.8]; 4 of up to 7,000 [27.3 / 21.2 / 21.6]; 1 of 8,000 [17.9 / 16.0 / 15.8]; 16 of 2,000 on 16 kv
+        heads of 128 [45.4 / 59.9 / 45.8]."""
         pairs = n * KV
-        want = (256 if pairs < 16 else 512) // pairs if pairs < 256 else 1
-        return max(1, min(want, -(-keys // 64), 128))
+        blocks = 256 if pairs < 16 else 512 if pairs < 64 else 1024 if pairs < 192 else 768
+        if pairs < 128:
+            long, rounds = min(keys // 320, -(-1536 // pairs)), 1
+        else:
+            long, rounds = keys // (512 if pairs < 512 else 1024), 2
+        return max(1, min(max(-(-blocks // pairs), long), -(-keys // (64 * rounds)), 128))
 
     def _check_pools(self, what, dtype, n, KV, hd, new_len, table, k_pool, v_pool):
         if new_len.numel() != n or new_len.dtype != torch.int32:
