@@ -200,6 +200,39 @@ def test_attention_of_uneven_sequences(ops, counts, H, KV, shape):
         at += n
 
 
+# portions of long prompts beside single tokens over a paged cache, without and with a ring: one long sequence of four (a
+# sequence's streams cover half of the XCDs, all of them, twice that), among three, sixteen and nine, two among six, and steps whose
+# plain order already spreads them; the blocks are turned in each of the shapes
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+@pytest.mark.parametrize("counts,held,H,KV,hd", [([1, 1, 1, 700], (150, 611, 48, 900), 8, 4, 256), ([1, 1, 600, 1], (150, 611, 700, 48), 16, 8, 256),
+                                                 ([1, 530, 1, 1], (30, 100, 70, 333), 32, 16, 128), ([520, 1, 1], (640, 1, 77), 16, 8, 64),
+                                                 ([1] * 15 + [580], tuple(range(20, 36)), 8, 4, 128), ([1] * 8 + [640], (50,) * 9, 8, 1, 192),
+                                                 ([300, 1, 1, 350, 1, 1], (500, 9, 8, 130, 6, 5), 4, 2, 64)])
+@pytest.mark.parametrize("window,rows_cap", [(0, 0), (190, 256)])
+def test_attention_of_uneven_portions_over_a_cache(ops, counts, held, H, KV, hd, shape, window, rows_cap):
+    """Every sequence's rows are what they are alone, bit for bit (a choice of the shape by size may give others: to rounding)."""
+    n, page = len(counts), 64
+    new_len = torch.tensor([a + b for a, b in zip(counts, held)], dtype=torch.int32, device=DEV)
+    width = rows_cap // page if rows_cap else -(-int(new_len.max()) // page)
+    table = torch.randperm(n * width, generator=torch.Generator().manual_seed(5)).to(torch.int32).view(n, width).to(DEV)
+    pools = [randn(n * width, KV, page, hd, dtype=torch.bfloat16, seed=64 + i) for i in range(2)]
+    q, k, v = (randn(sum(counts), heads * hd, dtype=torch.bfloat16, seed=66 + i) for i, heads in enumerate((H, KV, KV)))
+
+    def attend(first, last):
+        a, b = sum(counts[:first]), sum(counts[:last])
+        cu = torch.tensor([sum(counts[first:i]) for i in range(first, last + 1)], dtype=torch.int32, device=DEV)
+        return ops.attention_prefill(q[a:b], k[a:b], v[a:b], H, KV, hd, cu, max(counts[first:last]), hd ** -0.5, 30.0, window, torch.bfloat16, shape=shape,
+                                     cached=(new_len[first:last], table[first:last], *pools, rows_cap))
+    got, at = attend(0, n), 0
+    for i, c in enumerate(counts):
+        own = attend(i, i + 1)
+        if shape:
+            assert torch.equal(got[at:at + c], own), i
+        else:
+            assert rel_l2(got[at:at + c], own) < 4e-3, i
+        at += c
+
+
 # the kernel that streams up to 64 rows through LDS: each of its blocks (32, 64 and 128 rows of W, up to 16, 32 and 64 of X), one
 # k step and fewer than it asks for ahead, an N that ends inside a block and is no multiple of 4 (outputs element by element),
 # K slices of which the last is shorter; it is what is chosen from two rows on where the consumer adds the slices

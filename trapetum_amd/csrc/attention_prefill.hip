@@ -564,9 +564,11 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
     // rounds for the longest block.  Measured for 4x1 / 2x2 / 2x4: 2B sizes, 2,048 tokens 94 / 61 / 51 us, 4,096 tokens
     // 186 / 130 / 114, 8 x 512 tokens 34 / 27 / 36; 9B sizes, 2,048 tokens 100 / 72 / 69; 27B (heads of 128) 85 / 78 / 89.
     // A step of uneven sequences launches more blocks than hold queries (a portion of a long prompt beside single tokens): the
-    // blocks that can hold any are bounded by its rows.  Where they are no more than the CUs, 2 x 4 is the choice from 512
-    // tokens on, cached positions before them or not (2x2 / 2x4: 866 rows at 6,135 beside three tokens 235 / 149 us, 600
-    // at 4,096 137 / 103, 2 x 512 at 2,048 79 / 63, 8 prompts of up to 700 31 / 26; 257 tokens 15.5 / 16.8).
+    // blocks that can hold any are bounded by its rows.  They are what counts, for heads of more than 128 where they are less than
+    // 0.45 of the launched ones (beyond, 4 x 1 keeps its lead: 9B sizes, four of 1,000 rows at 2,000 beside four tokens, 0.55:
+    // 258 / 288 us for 4x1 / 2x2; at 0.25, one of 4,000 beside four of 200, 206 / 181).  Where they are no more than the CUs, 2 x 4
+    // is the choice from 512 tokens on, cached positions before them or not (2x2 / 2x4: 866 rows at 6,135 beside three tokens
+    // 235 / 149 us, 600 at 4,096 137 / 103, 2 x 512 at 2,048 79 / 63, 8 prompts of up to 700 31 / 26; 257 tokens 15.5 / 16.8).
     int cg = 4, kg = 1;
     bool uneven = false;
     {
@@ -577,25 +579,31 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
             return rows < longest() ? rows : longest();
         };
         plan(4, gs, pts);
-        const long blocks4 = filled();
+        const long blocks4 = HD <= 128 || 20 * filled() < 9 * longest() ? filled() : longest();
         plan(2, gs, pts);
         const bool alone = HD > 128 && filled() <= cus && max_count >= 512;
         if (shape == 0 && blocks4 < 4L * cus) shape = alone || (HD > 128 && longest() <= 2L * cus && max_count >= 1024) ? 2 : 3;
         if (shape == 2) { cg = 2; kg = 4; }
         if (shape == 3) { cg = 2; kg = 2; }
         plan(cg, gs, pts);
-        uneven = 2 * filled() < longest();
+        uneven = 4 * filled() < 3 * longest();
     }
     plan(cg, a.ghb_shift, a.pt_shift);
     a.n_streams = n_seq * KV * (G >> a.ghb_shift);
     a.pos_blocks = tp_cdiv(max_count, 32 << a.pt_shift);
     const long blocks = (long)a.n_streams * a.pos_blocks;
-    // Blocks go round the 8 XCDs, so that a stream's blocks, every n_streams-th, meet the same ones: good for its keys' way through
-    // an L2, and for the load where all streams are alike, but one long sequence among short ones then runs on a few
-    // XCDs.  There every block of positions starts so many streams further on that a sequence's streams move round as if
-    // they were alone (2,045 rows at 4,090 beside three tokens, 2x2: 364 -> 208 us; where all are alike it costs: 8 x 7,900
-    // tokens 2.10 -> 2.20 ms).
-    a.turn = uneven ? (a.n_streams - a.n_streams / n_seq) % 8 : 0;
+    // Blocks go round the 8 XCDs, and those of an XCD round its 4 shader engines: 32 places.  A stream's blocks are every
+    // n_streams-th, so where that is a multiple of a power of two they meet a few places only.  That is good for its keys' way
+    // through an L2, and for the load where all streams are alike (with a turn 8 x 7,900 tokens take 2.20 ms instead of 2.10), but
+    // one long sequence among short ones then leaves most of the chip idle.  So where the sequences are uneven (less than three
+    // quarters of the blocks can hold queries) and a sequence's streams do not fill the gap, every block of positions starts so many
+    // streams further on that they move round the XCDs as if they were alone or, if they cover the XCDs as it is, round the
+    // engines.  Microseconds, without / with: 2,045 rows at 4,090 beside three tokens 2B 364 / 208, 9B 614 / 304, 27B 452 / 345; 866
+    // at 6,135 9B 454 / 147; prompts of 700, 333, 64 and 1,025 9B 62 / 43; 2,000 beside 900 27B 98 / 82; four of 1,000 at 2,000
+    // beside four tokens, which are spread as they lie, 9B 258 / 270.
+    const int others = a.n_streams - a.n_streams / n_seq;
+    const int apart = a.n_streams & -a.n_streams;          // a stream's blocks meet every `apart`-th of 32 places by themselves
+    a.turn = !uneven || (apart < 32 ? apart : 32) <= a.n_streams / n_seq ? 0 : others % 8 ? others % 8 : others % 32;
     TP_REQUIRE(blocks < (1L << 31), "attention prefill: %ld blocks exceed one launch", blocks);
     hipStream_t s = (hipStream_t)stream;
     int rc;
