@@ -341,7 +341,7 @@ def test_linear_f32_is_one_order(ops, m, n, k):
     assert torch.equal(ops.rows(ops.linear(x, w, torch.float32, defer=True), torch.float32), got)
     off = torch.empty(m * k + 1, device=DEV)[1:].view(m, k)
     off.copy_(x)
-    assert rel_l2(ops.linear(off, w, torch.float32), ref) < 2e-6
+    assert torch.equal(ops.linear(off, w, torch.float32), got)
     if half > 3:
         packed = ops.pack_gate_up(w[:half - 3], w[half:2 * half - 3])
         gated = ops.gated_linear(x, packed, half - 3, "silu", torch.float32, limit=2.0, up_shift=0.5)
@@ -365,6 +365,15 @@ def test_linear_f32_bits_do_not_depend_on_where_operands_lie(ops, m, n, k):
         if half:
             packed = ops.pack_gate_up(w[:half], w[half:2 * half])
             assert torch.equal(ops.gated_linear(off(x, i), off(packed, j), half, "silu", torch.float32), ops.gated_linear(x, packed, half, "silu", torch.float32))
+
+
+def test_linear_f32_off_16_bytes_takes_more_rows_than_a_launch(ops):
+    m, n, k = 65535 * 32 + 21, 5, 4
+    x, w = torch.empty(m * k + 1, device=DEV)[1:].view(m, k).normal_(), randn(n, k, seed=12)
+    got = ops.linear(x, w, torch.float32)
+    some = [0, 31, 65535 * 32 - 1, 65535 * 32, m - 1]
+    assert torch.equal(got, ops.linear(x.clone(), w, torch.float32))
+    assert rel_l2(got[some], x[some].cpu().double() @ w.cpu().double().T) < 2e-6
 
 
 @pytest.mark.parametrize("algo", [1, 2, 3, 4, 5, 6, 8, 10, 11])

@@ -258,11 +258,17 @@ int gemm_f32_launch(const GemmArgs& a) {
     const float4 epi = gated ? make_float4(0.f, 0.f, a.limit, a.shift) : make_float4(a.cap, 0.f, (float)a.units, 0.f);
     if (few(a)) {
         TP_REQUIRE(a.y, "float32 product: K slices are left of operands on 16 bytes only");
-        TP_REQUIRE(tp_cdiv(a.M, 32) <= 65535, "float32 product: %d rows off 16 bytes exceed one launch", a.M);
-        // two tiles of W share the block's X where that leaves two blocks a CU
-        if (gated) few_launch<2, true>(a, part_blocks, epi);
-        else if (a.N >= 32 * 512) few_launch<2, false>(a, part_blocks, epi);
-        else few_launch<1, false>(a, part_blocks, epi);
+        constexpr long MOST = 65535L * 32;                 // rows that one launch takes
+        for (long m = 0; m < a.M; m += MOST) {
+            GemmArgs rows = a;
+            rows.M = (int)(a.M - m < MOST ? a.M - m : MOST);
+            rows.x = (const float*)a.x + (size_t)m * a.K;
+            rows.y = (float*)a.y + (size_t)m * (gated ? a.units : a.N);
+            // two tiles of W share the block's X where that leaves two blocks a CU
+            if (gated) few_launch<2, true>(rows, part_blocks, epi);
+            else if (a.N >= 32 * 512) few_launch<2, false>(rows, part_blocks, epi);
+            else few_launch<1, false>(rows, part_blocks, epi);
+        }
         return tp_check_launch("linear (float32, few rows)");
     }
     const int splits = gemm_f32_splits(a), m_tiles = tp_cdiv(a.M, TM);
