@@ -1,7 +1,7 @@
 // bf16 product for up to 64 rows (a decode step of many sequences): bound by reading W once, fp32 accumulation.
 //
 // A block owns BN = 32, 64 or 128 rows of W and all rows of X (MB = 16, 32 or 64 of them), and walks K in steps of 64.  W and X
-// come straight from global memory into LDS, S steps deep, so a CU has 40 to 100 KB of loads in flight without a register spent
+// come straight from global memory into LDS, S steps deep, so a CU has 72 to 128 KB of loads in flight without a register spent
 // on them (the register-staged 64 x 64 tiles of gemm_mfma.hip hold one step each and wait for it; the 8-row kernel of
 // gemm_rows8.hip holds eight loads a wave).  One barrier a step: behind it the step's tiles have arrived, and the place of the step
 // before, which everyone has read, takes the tiles S - 1 steps on.  Waves of up to MB rows of X by 32 rows of W
@@ -165,6 +165,12 @@ static StreamPlan stream_plan(const GemmArgs& a) {
 }
 
 int gemm_stream_splits(const GemmArgs& a) { return stream_plan(a).splits; }
+// rows of W a block of this kernel owns in a product (0: it is not one of its products)
+extern "C" int tp_linear_stream_rows(int M, int N, int K, int epilogue, int defer) {
+    GemmArgs a{};
+    a.in_dtype = TP_BF16; a.M = M; a.N = N; a.K = K; a.epilogue = epilogue; a.defer = defer;
+    return gemm_stream_supports(a) ? stream_plan(a).rows : 0;
+}
 // One slice is left as float32, too, where the choice of kernel is the library's: a product of so many rows of W that it has
 // one slice here had several by the kernels before it, and its sums stay float32 (N 9216, K 2304, 64 rows: error against 64
 // bits 1.7e-3 rounded to bf16, 2.9e-7 so).

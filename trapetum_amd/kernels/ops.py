@@ -56,6 +56,7 @@ _CORE_SIGS = {
     "tp_linear_scan_workspace_bytes": [_I, _I, _I, _I, _I],
     "tp_time_mix_scan_workspace_floats": [_I, _I, _I, _I],
     "tp_matrix_memory_scan_workspace_floats": [_I, _I, _I, _I, _I],
+    "tp_linear_stream_rows": [_I, _I, _I, _I, _I],
     "tp_linear_workspace_bytes": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
     "tp_attn_simple_prefill": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P],
     "tp_attn_simple_decode": [_P, _L, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P],
