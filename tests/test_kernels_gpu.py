@@ -98,6 +98,23 @@ def test_deferred_product_of_one_slice_keeps_its_sums(ops, m, n, k):
     assert rows.dtype == torch.float32 and rel_l2(ops.rows(rows, torch.float32), ref) < 1e-5
 
 
+# small matrices at few rows: both sides of where the kernel that streams W takes over from the 8-row kernel (and, at two rows, from
+# the multiply-adds, algo 4, where those cut K)
+@pytest.mark.parametrize("m,n,k,algo", [(2, 128, 1024, 5), (2, 1024, 2560, 5), (2, 1024, 2624, 4), (2, 1000, 20032, 4), (2, 1025, 7744, 4), (2, 1025, 7808, 16),
+                                        (3, 1024, 9216, 5), (3, 1024, 9280, 16), (8, 2048, 2048, 5), (8, 2049, 2048, 16), (5, 4096, 1024, 5), (9, 1024, 2304, 16)])
+def test_deferred_product_of_a_small_matrix(ops, m, n, k, algo):
+    """Few blocks of 64 rows of W are slower there than a wave for every 2 or 8 of them; the sums stay float32 slices."""
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=78), randn(n, k, dtype=torch.bfloat16, seed=79, scale=0.05)
+    got = ops.linear(x, w, torch.bfloat16, defer=True)
+    ops.force_linear = algo
+    try:
+        own = ops.linear(x, w, torch.bfloat16, defer=True)
+    finally:
+        ops.force_linear = 0
+    assert got.dtype == torch.float32 and got.slices.shape == own.slices.shape and torch.equal(got.slices, own.slices)
+    assert rel_l2(ops.rows(got, torch.float32), x.cpu().double() @ w.cpu().double().T) < 1e-5
+
+
 def test_rows_wider_than_the_fused_kernel_takes_are_added_first(ops):
     """A product in K slices whose rows are wider than `add_rms_norm` keeps in registers (8192): the slices are added by
     a kernel of their own, in slice order, and the result is what the fused path gives for narrower rows."""
@@ -235,7 +252,7 @@ def test_attention_of_uneven_portions_over_a_cache(ops, counts, held, H, KV, hd,
 
 # the kernel that streams up to 64 rows through LDS: each of its blocks (32, 64 and 128 rows of W, up to 16, 32 and 64 of X), one
 # k step and fewer than it asks for ahead, an N that ends inside a block and is no multiple of 4 (outputs element by element),
-# K slices of which the last is shorter; it is what is chosen from two rows on where the consumer adds the slices
+# K slices of which the last is shorter; it is what is chosen from two rows on where the consumer adds the slices of a large matrix
 @pytest.mark.parametrize("m,n,k", [(1, 8, 64), (2, 77, 128), (3, 2304, 2048), (16, 1001, 320), (17, 8200, 64), (32, 4099, 640),
                                    (33, 130, 1088), (64, 250, 4672), (48, 18432, 64), (9, 18432, 704), (64, 16500, 192), (40, 33000, 512),
                                    (33, 24609, 192), (64, 24610, 64), (40, 32701, 512), (50, 57344, 128)])

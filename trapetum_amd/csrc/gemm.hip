@@ -120,17 +120,31 @@ static int pick(const GemmArgs& a, int algo) {
     if (algo == 3 || (algo >= 6 && algo <= 15)) return gemm_mfma_supports(a) ? 3 : -3;
     if (a.in_dtype == TP_F32) return gemm_f32_supports(a) ? 20 : 1;
     // Two to 64 rows, K a multiple of 64: the kernel that streams W through LDS, wherever enough blocks of it read at once
-    // (its figures beside its plan).  With K slices for the consumer that is always (2 rows, against the multiply-adds: 9B down
-    // 27.6 / 23.8 us, qkv 15.3 / 12.8, 2B down 16.1 / 14.5); without, from 128 blocks of 64 rows of W on (8 rows, N 9216 K 2304:
-    // 13.2 / 11.8; 16 rows 21.4 / 13.0; but 8 rows, N 4096: 6.5 / 9.1).  A single row stays with the multiply-adds (2B down
+    // (its figures beside its plan).  With K slices for the consumer that is nearly always (2 rows, against the multiply-adds: 9B
+    // down 27.6 / 23.8 us, qkv 15.3 / 12.8, 2B down 16.1 / 14.5).  Up to eight rows of a small matrix are the exception: its blocks
+    // of 64 rows and slices of 512 k are too few to fetch it, and the kernels that start a wave every 2 or 8 rows of W are faster,
+    // up to FEW_N rows of W at any K but the longest, beyond up to SMALL_NK elements (with the norm that adds the slices, stream /
+    // 8-row kernel at 3 rows: N 256 K 2304 7.5 / 6.0 us, N 1024 K 4608 12.7 / 11.1, N 1536 K 2048 8.0 / 7.5; N 2304 K 2048 8.3 / 8.3,
+    // N 1024 K 14336 18.1 / 23.2, N 2304 K 4608 11.5 / 12.0).  Two rows stay with the multiply-adds where those cut K as well,
+    // up to SMALL_TWO_NK elements (N 384 K 9216 10.3 / 8.2, N 2048 K 3072 9.5 / 9.1, N 2560 K 3584 11.0 / 11.0); where they would
+    // not, their one slice would be rounded to bf16, and the 8-row kernel takes the same time.
+    // Without slices this kernel is the choice from 128 blocks of 64 rows of W on (8 rows, N 9216 K 2304: 13.2 / 11.8; 16 rows 21.4 / 13.0; but 8 rows, N 4096: 6.5 / 9.1).  A single row stays with the multiply-adds (2B down
     // 14.4 / 14.3, gate/up 16.6 / 18.6), and products without slices with the multiply-adds for two rows (2B gate/up 17.5 / 18.7)
     // and the 8-row kernel for three to seven where that reads K in one round, gates, or has the logits' many rows (2B gate/up
     // 17.2 / 18.7 at 4 rows, 18.2 / 18.7 at 6; logits 189 / 199).
     constexpr int ONE_ROUND_K = TP_R8_MAX_STEPS * 256, WIDE_N = 64 * 512, STREAM_N = 64 * 127;
+    constexpr int FEW_N = 1024, FEW_N_K = 9216;
+    constexpr long SMALL_NK = 1L << 22, SMALL_TWO_NK = 8000000;
     const bool sliced = a.defer && a.epilogue == TP_EPI_NONE;
     if (gemm_stream_supports(a) && a.M > 1) {
         const bool rows8 = a.M < 8 && gemm_rows8_supports(a) && (a.epilogue == TP_EPI_GATED || a.K <= ONE_ROUND_K || a.N >= WIDE_N);
-        if ((sliced && gemm_stream_splits(a) > 1) || (a.N > STREAM_N && (a.M > 2 || !gemv_supports(a)) && !rows8)) return 16;
+        const bool slices = sliced && gemm_stream_splits(a) > 1;
+        if (slices && a.M <= 8) {
+            const long elements = (long)a.N * a.K;
+            if (gemv_supports(a) && gemv_workspace(a) && (a.N <= FEW_N || elements <= SMALL_TWO_NK)) return 4;
+            if (gemm_rows8_supports(a) && ((a.N <= FEW_N && a.K <= FEW_N_K) || elements <= SMALL_NK)) return 5;
+        }
+        if (slices || (a.N > STREAM_N && (a.M > 2 || !gemv_supports(a)) && !rows8)) return 16;
     }
     if (gemv_supports(a)) return 4;          // one or two rows: 2B gate/up 16.8 against 22.6 us on the skinny kernel
     // What is left: few rows of W, or K no multiple of 64.  Three to eight rows: the kernel whose blocks read 8 rows of W in one
