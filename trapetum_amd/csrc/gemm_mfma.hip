@@ -331,8 +331,9 @@ struct Plan { Tile tile; int splits; bool direct = false; int wide = -1; bool su
 
 // K slices of a product of few rows, which is bound by reading W and wants every CU streaming.  From 17 rows on one
 // block a CU: more slices cost their consumer more than they gain (a 2B decode step of 64 sequences takes 3.52 ms
-// with 640 blocks, 3.34 with 256, 3.54 with 128).  Up to 16 rows the slices are small and the large matrices that
-// come here want more blocks (a 27B step of 8 sequences: 13.6 ms with 640 blocks, 14.5 with 256).
+// with 640 blocks, 3.34 with 256, 3.54 with 128).  Up to 16 rows the slices are small and large matrices want more blocks (a 27B
+// step of 8 sequences: 13.6 ms with 640 blocks, 14.5 with 256).  Those steps were measured while all their products came here; now
+// gemm_stream.hip takes the ones of up to 64 rows with a K that is a multiple of 64, and the rule serves the other K and 65 to 256 rows.
 static int small_tile_splits(const GemmArgs& a, long blocks) {
     if (blocks >= 512 || a.K < 512) return 1;
     int s = (int)tp_cdiv(a.M > 16 ? 256 : 640, blocks);
@@ -431,7 +432,9 @@ static Plan plan_of(const GemmArgs& a) {
     if (a.algo == 7) return {{4, a.epilogue == TP_EPI_GATED ? 4 : 3}, 1};
     if (a.algo == 8) return {{4, 4}, 1, true};
     if (a.algo == 9) return {{4, a.epilogue == TP_EPI_GATED ? 4 : 3}, 1, true};
-    // the logits of 64 rows: 250 us with 128 x 128, 275 with 64 x 64; up to 256 rows of a narrow product: 128 x 128
+    // Up to 64 rows what comes here has a K that is no multiple of 64 or, without slices, fewer than 8,129 rows of W (the rest is
+    // gemm_stream.hip's); where a figure below is of a larger matrix, it was taken before that and speaks for the other K.
+    // The logits of 64 rows: 250 us with 128 x 128, 275 with 64 x 64; up to 256 rows of a narrow product: 128 x 128
     // tiles would leave most CUs idle (down at 128 rows: 44 us on 72 blocks, against 15 us at 64 rows on 576 blocks
     // of 64 x 64; at 512 rows 128 x 128 wins again)
     if ((a.M <= 64 && !(a.M > 32 && a.N >= 32768)) || (a.M <= 256 && (long)tp_cdiv(a.M, 128) * tp_cdiv(a.N, 128) < 256)) {
@@ -443,7 +446,8 @@ static Plan plan_of(const GemmArgs& a) {
         // (never sliced) and of the slices of 17 rows and more (2B gate/up at 16 rows 27.6 -> 23.0 us, 27B at 8 rows
         // 141 -> 126, 9B qkv at 32 rows 21.1 -> 18.1); slices of a few steps (up to 16 rows) and 64 rows do not.
         // A gated product with about a block a CU in these tiles gains more from 64 x 32 tiles, twice the blocks with
-        // the same bytes in flight each (2B gate/up at 8 to 24 rows: 27.7 -> 22.5 us; the 9B and 27B shapes do not).
+        // the same bytes in flight each (N 18432 K 2312 at 8 / 32 rows: 28.4 -> 25.5, 30.3 -> 28.4 us; N 4608 K 2304 18.2 -> 15.4;
+        // N 28672 K 2312 at 32 rows 36.1, and 40.7 with them).
         if (a.M <= 32 && (a.epilogue == TP_EPI_GATED || (may_slice && a.M > 16))) t.deep = true;
         if (a.M <= 32 && a.epilogue == TP_EPI_GATED && tiles <= 320) t = {1, 2, 4, true};
         return {t, may_slice ? small_tile_splits(a, tiles) : 1};

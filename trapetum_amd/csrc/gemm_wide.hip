@@ -5,7 +5,7 @@
 // kilobyte into LDS (about 20 cycles each in the path), 192 KB of fragment reads and a barrier.  Measured on an 8,192^3
 // product, cycles a step: matrix instructions alone 2,140, with fragment reads 2,220, with loads bunched in half of the step
 // 2,780, spread over all of it 2,450.  The clock is a second bound: under this load the chip's power holds it at 1.7 - 1.9 GHz
-// (2.4 without), so no bf16 product of random numbers got beyond 1.65 PFLOP/s here, matrix instructions alone included.
+// (2.4 without), so on random numbers the matrix instructions alone reach 1.65 to 1.70 PFLOP/s here.
 // Hence the layout:
 // * Eight waves, two a SIMD, in WM x 8/WM, each MT x NT tiles of v_mfma_f32_32x32x16_bf16 with W as the A operand: a lane ends
 //   up with four neighbours of a row of Y, and with gate and up column of a unit in one accumulator.  Fragments of the next
@@ -18,12 +18,14 @@
 // * Outputs leave through LDS in whole 16-byte pieces of rows.  As the accumulators lie (8 bytes of 32 rows a store) the stores
 //   alone took 13,000 cycles of a 256 x 256 tile, a tenth of a product with K = 2,304.
 // Two groups of four waves that take turns at the matrix cores (a barrier a phase) reached 1,230 TFLOP/s where this loop reaches
-// 1,290 (9B gate/up at 8,192 rows); four waves of 128 x 128 with one a SIMD 1,170; k steps of 32 in five places 1,170.
+// 1,305 (9B gate/up at 8,191 rows); four waves of 128 x 128 with one a SIMD 1,170; k steps of 32 in five places 1,170.
 //
 // Microseconds, cold weights, gemm_mfma.hip / here / the vendor library's plain product (measured beside, never called):
 //   2B   2,048 rows: gate/up 180 / 154 / -    qkv 50 / 38 / 41    o 35 / 27 / 26    down (K slices, with their sum) 115 / 102 / -
 //   9B   8,191 rows: gate/up 1,455 / 1,290 / -    qkv 433 / 368 / 315    o 233 / 192 / 165    down 875 / 670 / 665
 //   2B logits, 1,716 rows, float32: 2,130 / 1,880 / -
+// The library is 1.17 times faster at 9B qkv and o, and only a little of that is known: the fixed part of a tile (its first loads, its
+// outputs) is 4 of the 92 us of each of qkv's four rounds, and o's second round fills 192 of the 256 CUs.
 #include "gemm.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 wd_bf16x8;
