@@ -1253,21 +1253,28 @@ class HipOps:
     def decode_splits(n, KV, hd, keys):
         """Slices of the keys per (sequence, kv head) in a decode step.  `keys` is the longest sequence, or a graph's bound on
         it; the others may be short, and the step takes as long as its longest block walks (31 ns a key, heads of 256).  So
-        there are one to four blocks a CU in all, by the number of pairs, and more where a block would walk over 320 keys (up
-        to six a CU), 512 from 128 pairs on and 1,024 from 512 on, where a further slice of every pair costs more (1.8 ns); a
-        slice has at least one round of 64 keys, two from 128 pairs on.  MI355X, heads of 256, 4 kv heads unless said,
+        there are one to four blocks a CU in all, by the number of pairs, and more where a block would walk over 512 keys (up
+        to six a CU), 320 from 64 pairs on, 512 from 128 on and 1,024 from 512 on, where a further slice of every pair costs more
+        (1.8 ns); a slice has at least one round of 64 keys, two from 128 pairs on.  Below 128 pairs more than eight slices are a
+        multiple of eight, as long as each has 128 keys: other numbers measured slower, for a reason that is not known (8 of 7,900,
+        16 / 24 / 25 / 32 slices: 51.6 / 55.5 / 59.8 / 54.6 us cold, one of 8,000 beside 7 of 100 31.2 / 33.0 / 38.2 / 33.9, one of 1,900
+        beside 14 of 100, 9 / 16 slices, 18.2 / 14.0; 12 of 3,000 under a bound of 4,096 lose, 16 slices for 10 2 us a layer).  MI355X, heads of 256, 4 kv heads unless said,
         microseconds, [three to six blocks a CU / one to two / this]: one sequence of 8,000 beside 63 of 100 [157 / 248 / 50],
         beside 31 [51 / 90 / 44], beside 15 [33.6 / 50.7 / 33.6]; 64 of 50 to 7,900 [229 / 301 / 233], of 20 to 1,000 [32.0 / 39.1 /
         32.0], of 2,000 [98.8 / 100.2 / 99.7], of up to 80 under a bound of 1,024 [11.0 / 9.0 / 11.0]; 32 of 1,000 [29.6 / 29.1 / 29.5];
-        8 of 7,900 [48.4 / 46.9 / 46.8]; 4 of up to 7,000 [27.3 / 21.2 / 21.6]; 1 of 8,000 [17.9 / 16.0 / 15.8]; 16 of 2,000 on 16 kv
+        8 of 7,900 [48.4 / 46.9 / 46.9]; 4 of up to 7,000 [27.3 / 21.2 / 21.6]; 1 of 8,000 [17.9 / 16.0 / 15.8]; 16 of 2,000 on 16 kv
         heads of 128 [45.4 / 59.9 / 45.8]."""
         pairs = n * KV
         blocks = 256 if pairs < 16 else 512 if pairs < 64 else 1024 if pairs < 192 else 768
         if pairs < 128:
-            long, rounds = min(keys // 320, -(-1536 // pairs)), 1
+            long, rounds = min(keys // (512 if pairs < 64 else 320), -(-1536 // pairs)), 1
         else:
             long, rounds = keys // (512 if pairs < 512 else 1024), 2
-        return max(1, min(max(-(-blocks // pairs), long), -(-keys // (64 * rounds)), 128))
+        slices = max(-(-blocks // pairs), long)
+        whole = -(-slices // 8) * 8
+        if pairs < 128 and slices > 8 and whole * 128 <= keys:
+            slices = whole
+        return max(1, min(slices, -(-keys // (64 * rounds)), 128))
 
     def _check_pools(self, what, dtype, n, KV, hd, new_len, table, k_pool, v_pool):
         if new_len.numel() != n or new_len.dtype != torch.int32:
