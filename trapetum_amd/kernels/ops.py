@@ -1258,7 +1258,7 @@ class HipOps:
         (1.8 ns); a slice has at least one round of 64 keys, two from 128 pairs on.  Below 128 pairs more than eight slices are a
         multiple of eight, as long as each has 128 keys: other numbers measured slower, for a reason that is not known (8 of 7,900,
         16 / 24 / 25 / 32 slices: 51.6 / 55.5 / 59.8 / 54.6 us cold, one of 8,000 beside 7 of 100 31.2 / 33.0 / 38.2 / 33.9, one of 1,900
-        beside 14 of 100, 9 / 16 slices, 18.2 / 14.0; 12 of 3,000 under a bound of 4,096 lose, 16 slices for 10 2 us a layer).  MI355X, heads of 256, 4 kv heads unless said,
+        beside 14 of 100, 9 / 16 slices, 18.2 / 14.0; 12 of 3,000 under a bound of 4,096 lose, 16 slices for 10: 3 us a layer).  MI355X, heads of 256, 4 kv heads unless said,
         microseconds, [three to six blocks a CU / one to two / this]: one sequence of 8,000 beside 63 of 100 [157 / 248 / 50],
         beside 31 [51 / 90 / 44], beside 15 [33.6 / 50.7 / 33.6]; 64 of 50 to 7,900 [229 / 301 / 233], of 20 to 1,000 [32.0 / 39.1 /
         32.0], of 2,000 [98.8 / 100.2 / 99.7], of up to 80 under a bound of 1,024 [11.0 / 9.0 / 11.0]; 32 of 1,000 [29.6 / 29.1 / 29.5];
