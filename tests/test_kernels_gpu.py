@@ -396,6 +396,26 @@ def test_linear_f32_bits_do_not_depend_on_where_operands_lie(ops, m, n, k):
             assert torch.equal(ops.gated_linear(off(x, i), off(packed, j), half, "silu", torch.float32), ops.gated_linear(x, packed, half, "silu", torch.float32))
 
 
+# up to 32 rows on 16 bytes: rings that wrap and rings with fewer steps than places, a step that ends in the next part, empty waves,
+# W's last tile and a gated tile's second half, slices for the consumer, two tiles of W a block; the order is that of operands off 16
+# bytes, whose kernel holds no ring
+@pytest.mark.parametrize("m,n,k", [(1, 7, 4), (3, 96, 9216), (4, 2304, 2048), (15, 100, 1028), (16, 64, 3620), (17, 48, 2304), (31, 16402, 260), (32, 130, 1500),
+                                   (2, 8208, 1100)])
+def test_linear_f32_ring(ops, m, n, k):
+    def off(t):
+        return torch.empty(t.numel() + 1, device=DEV)[1:].view(t.shape).copy_(t)
+    x, w = randn(m, k, seed=13), randn(n, k, seed=14, scale=0.05)
+    got = ops.linear(x, w, torch.float32)
+    assert rel_l2(got, x.cpu().double() @ w.cpu().double().T) < 2e-6
+    assert torch.equal(ops.linear(off(x), w, torch.float32), got)
+    assert torch.equal(ops.rows(ops.linear(x, w, torch.float32, defer=True), torch.float32), got)
+    half = n // 2 // 16 * 16
+    if half:
+        packed = ops.pack_gate_up(w[:half - 5], w[half:2 * half - 5])
+        gated = ops.gated_linear(x, packed, half - 5, "gelu_tanh", torch.float32)
+        assert torch.equal(ops.gated_linear(off(x), packed, half - 5, "gelu_tanh", torch.float32), gated)
+
+
 def test_linear_f32_off_16_bytes_takes_more_rows_than_a_launch(ops):
     m, n, k = 65535 * 32 + 21, 5, 4
     x, w = torch.empty(m * k + 1, device=DEV)[1:].view(m, k).normal_(), randn(n, k, seed=12)

@@ -5,8 +5,15 @@
 // a block: instruction t takes the block's k = t, 4 + t, 8 + t, 12 + t), four neighbouring parts are added in order to a
 // group, and the four groups in order.  (Its error against 64 bits is smaller than that of one chain over K.)
 //
-// Few rows (a decode step) are bound by reading W.  A block owns 16 NT rows of W, a wave of it one part: six blocks of 16 k
-// of W and X are asked for together, so that a CU has 96 KB in flight, and the parts are added in LDS.
+// Up to 32 rows (a decode step) are bound by reading W.  A block of four waves owns 16 rows of W; a wave takes a group (or, where
+// the groups are left to the consumer as slices, a part) and streams W and X through a ring of its own in LDS, three steps of
+// 32 k deep, so that three blocks a CU keep 72 KB of W in flight and no wave waits for another before the sums.  Microseconds at
+// 3 rows, cold weights, blocks of 16 waves that each asked for six blocks of 16 k in registers (one block a CU, so that its start
+// and end were nobody's work) / here: 2B gate/up 53.2 / 35-37 (4.6-4.9 TB/s), down 29.3 / 20.4, o 10.7 / 6.9, qkv 11.8 / 10.3,
+// logits 575 / 395 (6.0 TB/s); at 20 rows 74 / 48, 46 / 27, -, 18.7 / 13.9, 783 / 498.  Rings of four to eight steps and fewer
+// blocks a CU are slower (gate/up 38-44, qkv 10.9-11.8).
+// Operands off 16 bytes, which loads into LDS do not take, keep those blocks of 16 waves for any number of rows: a wave one part,
+// six blocks of 16 k of W and X asked for together, the parts added in LDS.
 // Many rows are bound by the matrix cores, 157 TFLOP/s in float32: a block of four waves owns 64 x 128 outputs (32 x 64 a
 // wave, 32 matrix instructions of 32 cycles for six 16-byte fragment reads), k steps of 32 straight from global memory into
 // one of two LDS buffers, three blocks a CU.  Where the outputs alone leave CUs idle and the consumer adds slices, the four
@@ -22,6 +29,9 @@ constexpr int TM = 64, TN = 128;
 
 // until every load, and every LDS read (whose buffer is filled again behind the barrier), is done
 __device__ __forceinline__ void wait_all() { __builtin_amdgcn_s_waitcnt(0x0070); }
+// until all but the N youngest loads are done; until every LDS read is done
+template <int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14)); }
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
 
 __device__ __forceinline__ float epilogue_f32(int epilogue, float o, float4 epi, int n) {
     if (epilogue == TP_EPI_SILU) return (float)n < epi.z ? gate_act_exact(o, TP_ACT_SILU) : o;
@@ -108,6 +118,156 @@ gemm_f32_few_k(const float* __restrict__ X, const float* __restrict__ W, float* 
             const int unit = (n0 >> 1) + row;
             if (unit < units) Y[(size_t)m * units + unit] = gated_unit_exact(total(i, e), total(MT + i, e), act, epi.z, epi.w);
         } else if (n0 + row < N) Y[(size_t)m * N + n0 + row] = epilogue_f32(epilogue, total(tile, e), epi, n0 + row);
+    }
+}
+
+// Up to 32 rows of operands on 16 bytes.  A wave walks PPW neighbouring parts of K of 16 NT rows of W and 16 MT of X through a
+// ring of D steps of 32 k in LDS that it alone fills and reads, so that no wave waits for another before the end: whole lines of
+// 128 bytes straight from global memory, a step read into registers and its place asked for again before its products.
+// PPW = 4: the four waves' groups are added in LDS; PPW = 1: a block holds one group, its four parts are added in LDS, and
+// the groups (blockIdx.y) are the consumer's slices.
+// Gated: NT = 1, eight gate rows and the eight up rows of the same units.
+template <int NT, int MT, bool GATED, int PPW, int D>
+__global__ void __launch_bounds__(256)
+gemm_f32_ring_k(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int part_blocks,
+                int epilogue, float4 epi, int units, int act) {
+    static_assert(!GATED || NT == 1, "a tile of 16 rows holds gate and up rows of eight units");
+    constexpr int STEP = (NT + MT) * 2048, L = (NT + MT) * 2, OUT = NT * MT;
+    static_assert(D >= 2 && (D - 1) * L < 64 && OUT <= 4 && D * STEP >= OUT * 1024, "ring");
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * D * STEP];
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = GATED ? (blockIdx.x >> 1) * 32 : blockIdx.x * 16 * NT;         // the first row of W; gated: of the 32 that the tile's 16 are among
+    const int k_blocks = (K + 15) >> 4, part = blockIdx.y * GROUP + wave * PPW;
+    const int from = part * part_blocks, to = min(k_blocks, from + PPW * part_blocks), steps = max(0, (to - from + 1) >> 1);
+
+    // loads: 8 rows of 128 bytes an instruction; the place p of row `row` holds chunk p ^ (row / 2), so that the 16 rows of a
+    // fragment read lie on all banks; rows past the edge of Y read the last row, chunks past the end of K its last one
+    const float* const wb = W + (size_t)n0 * K;
+    unsigned wo[NT][2], xo[MT][2];
+    int chunk[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int row = h * 8 + (lane >> 3);
+        chunk[h] = ((lane & 7) ^ (row >> 1)) * 4;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const int at = GATED ? (blockIdx.x & 1) * 8 + (row & 7) + (row >> 3) * 16 : 16 * j + row;
+            wo[j][h] = (unsigned)min(at, N - 1 - n0) * (unsigned)K;
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++) xo[i][h] = (unsigned)min(16 * i + row, M - 1) * (unsigned)K;
+    }
+    unsigned char* const ring = lds + wave * D * STEP;
+    const unsigned ring0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)ring;
+    auto fill = [&](int step, unsigned place) {
+        // (written as the instruction: told of it, the compiler waits for every such load before any LDS read)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const unsigned k = (unsigned)min((from + 2 * step) * 16 + chunk[h], K - 4);
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"((wo[j][h] + k) * 4u), "s"(wb), "s"(ring0 + place + j * 2048 + h * 1024) : "memory");
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"((xo[i][h] + k) * 4u), "s"(X), "s"(ring0 + place + (NT + i) * 2048 + h * 1024) : "memory");
+        }
+    };
+    f3_f32x4 acc[NT][MT], grp[NT][MT];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[j][i] = grp[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+    int part_end = from + part_blocks;
+#pragma unroll
+    for (int t = 0; t < D; t++)
+        if (t < steps) fill(t, t * STEP);
+    unsigned place = 0;
+    for (int step = 0; step < steps; step++) {
+        const int left = steps - 1 - step;                     // steps asked for behind this one, D - 1 at most
+        asm volatile("" ::: "memory");
+        if (left >= D - 1) wait_loads<(D - 1) * L>();
+        else if (left >= D / 2) wait_loads<(D / 2) * L>();
+        else wait_loads<0>();
+        asm volatile("" ::: "memory");
+        f3_f32x4 w[2][NT], x[2][MT];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const unsigned char* const at = ring + place + r * 128 + ((4 * h + g) ^ (r >> 1)) * 16;
+#pragma unroll
+            for (int j = 0; j < NT; j++) w[h][j] = *reinterpret_cast<const f3_f32x4*>(at + j * 2048);
+#pragma unroll
+            for (int i = 0; i < MT; i++) x[h][i] = *reinterpret_cast<const f3_f32x4*>(at + (NT + i) * 2048);
+        }
+        asm volatile("" ::: "memory");
+        wait_lds();                                            // the step is in registers: its place may be filled again
+        asm volatile("" ::: "memory");
+        if (left >= D) fill(step + D, place);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int b = from + 2 * step + h;
+            if (b >= to) break;
+            if (b * 16 + 16 > K) {                             // the last, partial block
+                const bool in = b * 16 + 4 * g < K;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int j = 0; j < NT; j++) w[h][j][v] = in ? w[h][j][v] : 0.f;
+#pragma unroll
+                    for (int i = 0; i < MT; i++) x[h][i][v] = in ? x[h][i][v] : 0.f;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][j][t], x[h][i][t], acc[j][i], 0, 0, 0);
+            if (PPW > 1 && (b + 1 == part_end || b + 1 == to)) {
+                part_end += part_blocks;
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++) {
+                        grp[j][i] += acc[j][i];
+                        acc[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+        }
+        place = place + STEP == D * STEP ? 0 : place + STEP;
+    }
+    // the waves' sums, each in its own ring, which it has read to the end
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) *reinterpret_cast<f3_f32x4*>(ring + (j * MT + i) * 1024 + lane * 16) = PPW > 1 ? grp[j][i] : acc[j][i];
+    __syncthreads();
+    if (wave >= OUT) return;
+    auto total = [&](int l) {
+        f3_f32x4 t = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 4; q++) t += *reinterpret_cast<const f3_f32x4*>(lds + q * D * STEP + wave * 1024 + l * 16);
+        return t;
+    };
+    const int j = wave / MT, i = wave % MT, m = 16 * i + r, width = GATED ? units : N;
+    const int c = GATED ? (n0 >> 1) + (blockIdx.x & 1) * 8 + 4 * g : n0 + 16 * j + 4 * g;
+    if (m >= M || c >= width || (GATED && g >= 2)) return;
+    f3_f32x4 o = total(lane);
+    if (GATED) {
+        const f3_f32x4 up = total(lane + 32);
+#pragma unroll
+        for (int v = 0; v < 4; v++) o[v] = gated_unit_exact(o[v], up[v], act, epi.z, epi.w);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; v++) o[v] = epilogue_f32(epilogue, o[v], epi, c + v);
+    }
+    float* const y = Y + (size_t)blockIdx.y * M * N + (size_t)m * width + c;
+    if ((width & 3) == 0 && ((uintptr_t)Y & 15) == 0) *reinterpret_cast<f3_f32x4*>(y) = o;
+    else {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (c + v < width) y[v] = o[v];
     }
 }
 
@@ -236,13 +396,18 @@ gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float*
 // rows read in pieces of four; a tile's rows within 32-bit offsets
 bool gemm_f32_supports(const GemmArgs& a) { return a.in_dtype == TP_F32 && a.out_dtype == TP_F32 && a.K % 4 == 0 && a.K < (1 << 23); }
 
-// Up to 32 rows the kernel of few rows reads W once and its matrix instructions fit into that time; from 33 on the other
-// does the same work on whole tiles.  Its loads into LDS want operands on 16 bytes: off them any number of rows goes to the
-// first, in tiles of 32, so that a product's bits do not depend on where its operands lie.
-static bool few(const GemmArgs& a) { return a.M <= 32 || (uintptr_t)a.x % 16 || (uintptr_t)a.w % 16; }
+// Up to 32 rows the ring kernel reads W once and its matrix instructions fit into that time; from 33 on whole tiles do the same
+// work.  Loads into LDS want operands on 16 bytes: off them any number of rows goes to the blocks of 16 waves, in tiles of 32, so
+// that a product's bits do not depend on where its operands lie.
+static bool aligned(const GemmArgs& a) { return (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0; }
+static bool few(const GemmArgs& a) { return a.M <= 32 || !aligned(a); }
 
+// Slices for the consumer: the four groups, where the outputs alone leave CUs idle (up to 32 rows: fewer than two blocks a CU,
+// three rows, N 2304: K 2048 9.1 us as one, 7.0 as slices, K 9216 30.0 and 20.4).
 int gemm_f32_splits(const GemmArgs& a) {
-    return !few(a) && a.defer && a.epilogue == TP_EPI_NONE && a.K >= 1024 && (long)tp_cdiv(a.M, TM) * tp_cdiv(a.N, TN) < 256 ? PARTS / GROUP : 1;
+    if (!a.defer || a.epilogue != TP_EPI_NONE || a.K < 1024) return 1;
+    if (a.M <= 32) return aligned(a) && tp_cdiv(a.N, 16) < 512 ? PARTS / GROUP : 1;
+    return !few(a) && (long)tp_cdiv(a.M, TM) * tp_cdiv(a.N, TN) < 256 ? PARTS / GROUP : 1;
 }
 
 template <int NT, bool GATED>
@@ -252,11 +417,33 @@ static void few_launch(const GemmArgs& a, int part_blocks, float4 epi) {
     else gemm_f32_few_k<NT, 2, GATED><<<blocks, 1024, 0, a.stream>>>((const float*)a.x, (const float*)a.w, (float*)a.y, a.M, a.N, a.K, part_blocks, a.epilogue, epi, a.units, a.act);
 }
 
+template <int NT, int MT, bool GATED, int PPW, int D>
+static void ring_launch(const GemmArgs& a, float* y, int part_blocks, float4 epi) {
+    gemm_f32_ring_k<NT, MT, GATED, PPW, D><<<dim3(tp_cdiv(a.N, 16 * NT), PPW == 1 ? PARTS / GROUP : 1), 256, 0, a.stream>>>(
+        (const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, a.epilogue, epi, a.units, a.act);
+}
+
 int gemm_f32_launch(const GemmArgs& a) {
-    const int part_blocks = tp_cdiv(tp_cdiv(a.K, 16), PARTS);
+    const int part_blocks = tp_cdiv(tp_cdiv(a.K, 16), PARTS), splits = gemm_f32_splits(a);
     const bool gated = a.epilogue == TP_EPI_GATED;
     const float4 epi = gated ? make_float4(0.f, 0.f, a.limit, a.shift) : make_float4(a.cap, 0.f, (float)a.units, 0.f);
-    if (few(a)) {
+    const size_t need = (size_t)splits * a.M * a.N * sizeof(float);
+    TP_REQUIRE(splits == 1 || (a.workspace && a.workspace_bytes >= need), "float32 product: workspace of %zu bytes, %zu needed", a.workspace_bytes, need);
+    float* const y = (float*)(splits > 1 ? a.workspace : a.y);
+    if (a.M <= 32 && aligned(a)) {
+        // depths: three blocks a CU (48 KB of LDS each, two where two tiles of each are held)
+        if (a.M <= 16) {
+            if (gated) ring_launch<1, 1, true, 4, 3>(a, y, part_blocks, epi);
+            else if (splits > 1) ring_launch<1, 1, false, 1, 3>(a, y, part_blocks, epi);
+            else ring_launch<1, 1, false, 4, 3>(a, y, part_blocks, epi);
+        } else if (gated) ring_launch<1, 2, true, 4, 2>(a, y, part_blocks, epi);
+        else if (splits > 1) ring_launch<1, 2, false, 1, 2>(a, y, part_blocks, epi);
+        // two tiles of W share X's where that leaves two blocks a CU (20 rows, N 256000 K 2304: 540 us with one, 498; N 4096: 13.9, 18.8)
+        else if (a.N >= 32 * 512) ring_launch<2, 2, false, 4, 2>(a, y, part_blocks, epi);
+        else ring_launch<1, 2, false, 4, 2>(a, y, part_blocks, epi);
+        return tp_check_launch("linear (float32, up to 32 rows)");
+    }
+    if (few(a)) {                                              // off 16 bytes
         TP_REQUIRE(a.y, "float32 product: K slices are left of operands on 16 bytes only");
         constexpr long MOST = 65535L * 32;                 // rows that one launch takes
         for (long m = 0; m < a.M; m += MOST) {
@@ -271,11 +458,8 @@ int gemm_f32_launch(const GemmArgs& a) {
         }
         return tp_check_launch("linear (float32, few rows)");
     }
-    const int splits = gemm_f32_splits(a), m_tiles = tp_cdiv(a.M, TM);
-    const size_t need = (size_t)splits * a.M * a.N * sizeof(float);
-    TP_REQUIRE(splits == 1 || (a.workspace && a.workspace_bytes >= need), "float32 product: workspace of %zu bytes, %zu needed", a.workspace_bytes, need);
+    const int m_tiles = tp_cdiv(a.M, TM);
     TP_REQUIRE((long)m_tiles * tp_cdiv(a.N, TN) < (1L << 31), "float32 product: too many tiles for one launch (M=%d N=%d)", a.M, a.N);
-    float* const y = (float*)(splits > 1 ? a.workspace : a.y);
     const dim3 grid((unsigned)(m_tiles * tp_cdiv(a.N, TN)), splits);
     if (gated) gemm_f32_many_k<true><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act);
     else gemm_f32_many_k<false><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act);
