@@ -15,9 +15,11 @@
 // Operands off 16 bytes, which loads into LDS do not take, keep those blocks of 16 waves for any number of rows: a wave one part,
 // six blocks of 16 k of W and X asked for together, the parts added in LDS.
 // Many rows are bound by the matrix cores, 157 TFLOP/s in float32: a block of four waves owns 64 x 128 outputs (32 x 64 a
-// wave, 32 matrix instructions of 32 cycles for six 16-byte fragment reads), k steps of 32 straight from global memory into
-// one of two LDS buffers, three blocks a CU.  Where the outputs alone leave CUs idle and the consumer adds slices, the four
-// groups are four slices.
+// wave, 32 matrix instructions of 32 cycles for six 16-byte fragment reads), or fewer columns where that leaves the fullest CU
+// less, k steps of 32 straight from global memory into one of two LDS buffers, three blocks a CU.  Where the outputs alone leave
+// CUs idle and the consumer adds slices, the four groups are four slices.  Microseconds, cold weights, before (accumulators moved
+// between register files every 16 k, which also kept the third block out; 128 columns always) / here: 2B at 309 rows gate/up
+// 286 / 246, qkv 113 / 73, o 46 / 34, down 172 / 126; at 2,048 rows 1,569 / 1,329 (131 TFLOP/s), 355 / 310, 251 / 158, 1,067 / 654.
 #include "gemm.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f3_f32x4;
@@ -25,7 +27,7 @@ typedef f3_f32x4 f3_anywhere __attribute__((aligned(4)));        // (the same lo
 
 namespace {
 constexpr int PARTS = 16, GROUP = 4;
-constexpr int TM = 64, TN = 128;
+constexpr int TM = 64, TN = 128;                 // of many rows: the outputs a block owns, at most
 
 // until every load, and every LDS read (whose buffer is filled again behind the barrier), is done
 __device__ __forceinline__ void wait_all() { __builtin_amdgcn_s_waitcnt(0x0070); }
@@ -271,11 +273,13 @@ gemm_f32_ring_k(const float* __restrict__ X, const float* __restrict__ W, float*
     }
 }
 
-template <bool GATED>
-__global__ void __launch_bounds__(256)
+// NJ: tiles of 16 rows of W a wave holds (32 rows of X by 16 NJ of W); gated: an even number, gate rows and up rows in turn.
+template <bool GATED, int NJ>
+__global__ void __launch_bounds__(256, 3)
 gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int part_blocks,
                 int m_tiles, int epilogue, float4 epi, int units, int act) {
-    constexpr int BUF = (TM + TN) * 128;
+    static_assert(!GATED || NJ % 2 == 0, "gate and up rows of a unit lie in two tiles of one wave");
+    constexpr int TN = 32 * NJ, BUF = (TM + TN) * 128;
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * BUF];
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
@@ -283,89 +287,92 @@ gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float*
     const bool sliced = gridDim.y > 1;
     const int k_blocks = (K + 15) >> 4;
     const int from = sliced ? blockIdx.y * GROUP * part_blocks : 0, to = sliced ? min(k_blocks, from + GROUP * part_blocks) : k_blocks;
-    const int steps = max(0, (to - from + 1) >> 1);
     if (sliced) Y += (size_t)blockIdx.y * M * N;
 
-    // loads: 8 rows of 128 bytes an instruction, lane l's place (row l / 8, place l % 8) holds chunk place ^ row; rows past the
-    // edge of Y read the last row, chunks past the end of K its last one
+    // loads: 8 rows of 128 bytes an instruction, lane l's place (row l / 8, place l % 8) holds chunk place ^ (row / 2) of the 16
+    // rows that a fragment read takes; rows past the edge of Y read the last row, chunks past the end of K its last one
     const float* const xb = X + (size_t)m0 * K;
     const float* const wb = W + (size_t)n0 * K;
-    const int chunk = (lane & 7) ^ (lane >> 3);
-    unsigned xo[2], wo[4];
+    const int chunk = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));
+    unsigned xo[2], wo[NJ];
 #pragma unroll
     for (int i = 0; i < 2; i++) xo[i] = (unsigned)min(i * 32 + wave * 8 + (lane >> 3), M - 1 - m0) * (unsigned)K;
 #pragma unroll
-    for (int i = 0; i < 4; i++) wo[i] = (unsigned)min(i * 32 + wave * 8 + (lane >> 3), N - 1 - n0) * (unsigned)K;
+    for (int i = 0; i < NJ; i++) wo[i] = (unsigned)min(i * 32 + wave * 8 + (lane >> 3), N - 1 - n0) * (unsigned)K;
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lds + wave * 1024;
-    auto fill = [&](int step) {
-        const unsigned k = (unsigned)min(from * 16 + step * 32 + chunk * 4, K - 4), to_ = lds0 + (step & 1) * BUF;
+    auto fill = [&](int b, unsigned buf) {
+        const unsigned k = (unsigned)min(b * 16 + chunk * 4, K - 4), to_ = lds0 + buf;
         // (written as the instruction: told of it, the compiler waits for every such load before any LDS read)
 #pragma unroll
         for (int i = 0; i < 2; i++)
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"((xo[i] + k) * 4u), "s"(xb), "s"(to_ + i * 4096) : "memory");
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < NJ; i++)
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"((wo[i] + k) * 4u), "s"(wb), "s"(to_ + TM * 128 + i * 4096) : "memory");
     };
-    f3_f32x4 acc[4][2], grp[4][2], tot[4][2];
+    f3_f32x4 acc[NJ][2], grp[NJ][2], tot[NJ][2];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
-        for (int i = 0; i < 2; i++) acc[j][i] = grp[j][i] = tot[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
-    int part_end = from + part_blocks, parts = 0;
-    fill(0);
-    for (int step = 0; step < steps; step++) {
-        asm volatile("" ::: "memory");
-        wait_all();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();            // the step's tiles are there, and the other buffer has been read by everyone
-        asm volatile("" ::: "memory");
-        if (step + 1 < steps) fill(step + 1);
-        const unsigned char* const xs = lds + (step & 1) * BUF + (wm * 32 + r) * 128;
-        const unsigned char* const ws = lds + (step & 1) * BUF + TM * 128 + (wn * 64 + r) * 128;
+        for (int i = 0; i < 2; i++) grp[j][i] = tot[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+    unsigned buf = 0;
+    if (from < to) fill(from, 0);
+    // One loop body, entered a part at a time: with the parts' ends as branches inside a loop over steps the compiler moved all
+    // accumulators between register files every 16 k, and kept a third block from the CU.
+    int b = from;
+    for (int parts = 1; b < to; parts++) {
+        const int part_end = min(to, b + part_blocks);
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int b = from + 2 * step + h;
-            if (b >= to) break;
-            const int at = ((4 * h + g) ^ (r & 7)) * 16;
-            f3_f32x4 w[4], x[2];
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int i = 0; i < 2; i++) x[i] = *reinterpret_cast<const f3_f32x4*>(xs + i * 2048 + at);
+            for (int i = 0; i < 2; i++) acc[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+        for (; b < part_end; b++) {
+            const int h = (b - from) & 1;            // a step of 32 k holds two blocks
+            if (h == 0) {
+                asm volatile("" ::: "memory");
+                wait_all();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();        // the step's tiles are there, and the other buffer has been read by everyone
+                asm volatile("" ::: "memory");
+                if (b + 2 < to) fill(b + 2, BUF - buf);
+            }
+            const unsigned at = ((4 * h + g) ^ (r >> 1)) * 16;
+            const unsigned char* const xs = lds + buf + (wm * 32 + r) * 128 + at;
+            const unsigned char* const ws = lds + buf + TM * 128 + (wn * 16 * NJ + r) * 128 + at;
+            f3_f32x4 w[NJ], x[2];
 #pragma unroll
-            for (int j = 0; j < 4; j++) w[j] = *reinterpret_cast<const f3_f32x4*>(ws + j * 2048 + at);
-            if (b * 16 + 16 > K) {               // the last, partial block
+            for (int i = 0; i < 2; i++) x[i] = *reinterpret_cast<const f3_f32x4*>(xs + i * 2048);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) w[j] = *reinterpret_cast<const f3_f32x4*>(ws + j * 2048);
+            if (b * 16 + 16 > K) {                   // the last, partial block
                 const bool in = b * 16 + 4 * g < K;
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
 #pragma unroll
                     for (int i = 0; i < 2; i++) x[i][v] = in ? x[i][v] : 0.f;
 #pragma unroll
-                    for (int j = 0; j < 4; j++) w[j][v] = in ? w[j][v] : 0.f;
+                    for (int j = 0; j < NJ; j++) w[j][v] = in ? w[j][v] : 0.f;
                 }
             }
 #pragma unroll
             for (int t = 0; t < 4; t++)
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+                for (int j = 0; j < NJ; j++)
 #pragma unroll
                     for (int i = 0; i < 2; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][t], x[i][t], acc[j][i], 0, 0, 0);
-            if (b + 1 == part_end || b + 1 == to) {
-                parts++;
-                part_end += part_blocks;
-                const bool whole = parts % GROUP == 0 || b + 1 == to;
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-#pragma unroll
-                    for (int i = 0; i < 2; i++) {
-                        grp[j][i] += acc[j][i];
-                        acc[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
-                        if (whole) {
-                            tot[j][i] += grp[j][i];
-                            grp[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
-                        }
-                    }
-            }
+            if (h) buf = BUF - buf;
         }
+        const bool whole = parts % GROUP == 0 || b >= to;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                grp[j][i] += acc[j][i];
+                if (whole) {
+                    tot[j][i] += grp[j][i];
+                    grp[j][i] = (f3_f32x4){0.f, 0.f, 0.f, 0.f};
+                }
+            }
     }
     const int width = GATED ? units : N;
     const bool wide = (width & 3) == 0 && ((uintptr_t)Y & 15) == 0;
@@ -374,13 +381,13 @@ gemm_f32_many_k(const float* __restrict__ X, const float* __restrict__ W, float*
         const int m = m0 + wm * 32 + 16 * i + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; j += GATED ? 2 : 1) {
-            const int n = n0 + wn * 64 + 16 * j;
+        for (int j = 0; j < NJ; j += GATED ? 2 : 1) {
+            const int n = n0 + wn * 16 * NJ + 16 * j;
             const int c = (GATED ? n >> 1 : n) + 4 * g;
             f3_f32x4 o;
 #pragma unroll
             for (int v = 0; v < 4; v++)
-                o[v] = GATED ? gated_unit_exact(tot[j][i][v], tot[j + 1 < 4 ? j + 1 : j][i][v], act, epi.z, epi.w) : epilogue_f32(epilogue, tot[j][i][v], epi, c + v);
+                o[v] = GATED ? gated_unit_exact(tot[j][i][v], tot[j + 1 < NJ ? j + 1 : j][i][v], act, epi.z, epi.w) : epilogue_f32(epilogue, tot[j][i][v], epi, c + v);
             if (c >= width) continue;
             float* const to_ = Y + (size_t)m * width + c;
             if (wide) *reinterpret_cast<f3_f32x4*>(to_) = o;
@@ -460,8 +467,15 @@ int gemm_f32_launch(const GemmArgs& a) {
     }
     const int m_tiles = tp_cdiv(a.M, TM);
     TP_REQUIRE((long)m_tiles * tp_cdiv(a.N, TN) < (1L << 31), "float32 product: too many tiles for one launch (M=%d N=%d)", a.M, a.N);
-    const dim3 grid((unsigned)(m_tiles * tp_cdiv(a.N, TN)), splits);
-    if (gated) gemm_f32_many_k<true><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act);
-    else gemm_f32_many_k<false><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act);
+    // The matrix cores of the CU with the most outputs decide: 128 rows of W a block, or 96 (gated: 64) where the fullest CU gets
+    // less by it.  Blocks of 128 tie.
+    const int narrow = gated ? 2 : 3;
+    auto most = [&](int nj) { return (long)tp_cdiv((long)m_tiles * tp_cdiv(a.N, 32 * nj) * splits, 256) * nj; };
+    const int nj = most(narrow) < most(4) ? narrow : 4;
+    const dim3 grid((unsigned)(m_tiles * tp_cdiv(a.N, 32 * nj)), splits);
+#define TP_MANY(GATED, NJ) gemm_f32_many_k<GATED, NJ><<<grid, 256, 0, a.stream>>>((const float*)a.x, (const float*)a.w, y, a.M, a.N, a.K, part_blocks, m_tiles, a.epilogue, epi, a.units, a.act)
+    if (gated) { if (nj == 4) TP_MANY(true, 4); else TP_MANY(true, 2); }
+    else { if (nj == 4) TP_MANY(false, 4); else TP_MANY(false, 3); }
+#undef TP_MANY
     return tp_check_launch("linear (float32)");
 }
