@@ -251,6 +251,25 @@ def test_matrix_memory_scan_in_chunks(rt, heads, dk, dv, i_bias, chunk):
         assert torch.equal(g[[4, 6, 8]].cpu(), w[[4, 6, 8]])
 
 
+# operands that are views of wider rows, on whole pieces and off them; keys and values that are no whole tiles, blocks of one wave to four
+@pytest.mark.parametrize("lead", [0, 8, 3])
+@pytest.mark.parametrize("heads,dk,dv", [(2, 128, 256), (1, 4, 4), (2, 68, 132), (1, 256, 48), (2, 17, 250)])
+def test_matrix_memory_in_chunks_of_views(rt, heads, dk, dv, lead):
+    from . import ref_ops
+    lens, slots = (65, 13, 1, 128), torch.tensor([2, 0, 4, 1], dtype=torch.int32)
+    cu, M = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32), sum(lens)
+    wide = acts(rt, rnd(M, lead + heads * (2 * dk + dv), seed=80, scale=0.5))[0]
+    q, k, v = torch.split(wide[:, lead:], [heads * dk, heads * dk, heads * dv], dim=1)
+    gates = torch.cat([rnd(M, heads, seed=81, scale=2.0), rnd(M, heads, seed=82, scale=2.0) + 1.0], dim=1).contiguous()
+    states = [rnd(5, heads, dk, dv, seed=83, scale=0.3), rnd(5, heads, dk, seed=84, scale=0.3), rnd(5, heads, seed=85)]
+    want_states, got_states = [t.double() for t in states], [t.to(rt.device) for t in states]
+    want = ref_ops.matrix_memory_scan(q.cpu(), k.cpu(), v.cpu(), gates, 8.0, dk ** -0.5, *want_states, slots, cu, max(lens), heads, dk, dv)
+    got = rt.ops.matrix_memory_scan(q, k, v, gates.to(rt.device), 8.0, dk ** -0.5, *got_states, slots.to(rt.device), cu.to(rt.device), max(lens), heads, dk, dv)
+    assert rel_l2(got, want) < 6e-5                      # the denominator's bound, as above
+    for g, w in zip(got_states, want_states):
+        assert rel_l2(g, w) < 1e-5
+
+
 @pytest.mark.parametrize("cut", ["whole", "pieces", "one by one"])
 def test_matrix_memory_keeps_its_first_tokens(rt, cut):
     """Forget gates of sigmoid(8) and small input gates after the first tokens: the memory is what the first tokens wrote,

@@ -709,7 +709,7 @@ class HipOps:
     SCAN_CHUNK_FROM = 96         # rows of the longest sequence from which a scan runs in chunks
 
     def scan_chunks(self, max_count):
-        """(rows of a chunk, chunks that cover the longest sequence) for the two scans of a matrix state; (0, 0): every
+        """(rows of a chunk, chunks that cover the longest sequence) for the time-mixing scan; (0, 0): every
         sequence in one piece, row after row.  Chunks of 32 rows give a prompt of a few thousand tokens as many waves
         as the chip has places for; longer ones take longer chunks, so that the states between them stay small."""
         n = int(max_count)
@@ -718,6 +718,9 @@ class HipOps:
         chunk = 32 if n <= 8192 else 64 if n <= 32768 else 128
         return chunk, -(-n // chunk)
 
+    MEMORY_CHUNK = 64              # rows of a chunk of the matrix memory, at most (the kernel library's)
+    MEMORY_CHUNKS_FROM = 12        # rows of the longest sequence from which it runs in chunks (where the two ways meet)
+
     def matrix_memory_scan(self, q, k, v, gates, cap, q_scale, memory, normalizer, maximum, slot_ids, cu_rows, max_count, heads, dk, dv,
                            chunk=None):
         """gates float32 [M, 2 heads]: the input gates' sums, then the forget gates'.  i = cap tanh(. / cap),
@@ -725,7 +728,8 @@ class HipOps:
         o = S^T q' / (max(|n . q'|, e^(-m')) + 1e-6) with q' = q q_scale, row after row of every sequence from the states
         memory [slots, heads, dk, dv], normalizer [slots, heads, dk] and maximum [slots, heads] (float32), which are left
         updated.  q, k [M, heads dk] and v [M, heads dv] may be views of wider rows.  Returns float32 [M, heads dv].
-        chunk: as in `time_mix_scan`."""
+        chunk: rows of a chunk (MEMORY_CHUNK at most; 0: whole sequences; None: by max_count, which no sequence's rows may
+        exceed)."""
         self._dev(q, k, v, gates, memory, normalizer, maximum, slot_ids, cu_rows)
         m = q.shape[0]
         qs, ks, vs = self._rows(q, "matrix_memory_scan q"), self._rows(k, "matrix_memory_scan k"), self._rows(v, "matrix_memory_scan v")
@@ -744,7 +748,10 @@ class HipOps:
             raise KernelError("matrix_memory_scan: the gates' cap must be positive")
         n_seq = self._geometry("matrix_memory_scan", m, slot_ids, cu_rows)
         y = torch.empty((m, heads * dv), dtype=torch.float32, device=self.device)
-        chunk, n_chunks = self.scan_chunks(max_count) if chunk is None else (int(chunk), -(-int(max_count) // int(chunk)) if chunk else 0)
+        if chunk is None:
+            chunk = self.MEMORY_CHUNK if int(max_count) >= self.MEMORY_CHUNKS_FROM else 0
+        chunk = min(int(chunk), self.MEMORY_CHUNK)
+        n_chunks = -(-int(max_count) // chunk) if chunk else 0
         ws = None
         if chunk:
             ws = torch.empty(self.lib.tp_matrix_memory_scan_workspace_floats(n_seq, n_chunks, heads, dk, dv), dtype=torch.float32, device=self.device)
