@@ -270,6 +270,30 @@ def test_matrix_memory_in_chunks_of_views(rt, heads, dk, dv, lead):
         assert rel_l2(g, w) < 1e-5
 
 
+# one row a sequence: blocks of 256 and 1,024 threads, one to sixteen rows a thread, sizes that whole sequences' kernels keep
+@pytest.mark.parametrize("heads,dk,dv", [(2, 128, 256), (3, 64, 64), (1, 256, 256), (2, 3, 4), (1, 255, 16), (2, 64, 128), (1, 72, 70)])
+def test_scans_of_one_row(rt, heads, dk, dv):
+    from . import ref_ops
+    n, slots = 3, torch.tensor([4, 0, 2], dtype=torch.int32)
+    cu = torch.arange(n + 1, dtype=torch.int32)
+    qd, kd, vd = (acts(rt, rnd(n, heads * d, seed=90 + i, scale=0.5))[0] for i, d in enumerate((dk, dk, dv)))
+    gates = rnd(n, 2 * heads, seed=93, scale=2.0)
+    states = [rnd(5, heads, dk, dv, seed=94, scale=0.3), rnd(5, heads, dk, seed=95, scale=0.3), rnd(5, heads, seed=96)]
+    want_states, got_states = [t.double() for t in states], [t.to(rt.device) for t in states]
+    want = ref_ops.matrix_memory_scan(qd.cpu(), kd.cpu(), vd.cpu(), gates, 8.0, dk ** -0.5, *want_states, slots, cu, 1, heads, dk, dv)
+    got = rt.ops.matrix_memory_scan(qd, kd, vd, gates.to(rt.device), 8.0, dk ** -0.5, *got_states, slots.to(rt.device), cu.to(rt.device), 1, heads, dk, dv)
+    assert rel_l2(got, want) < 6e-5                      # the denominator's bound, as above
+    for g, w, s in zip(got_states, want_states, states):
+        assert rel_l2(g, w) < 1e-6 and torch.equal(g[[1, 3]].cpu(), s[[1, 3]])
+    d, inner = dv, heads * dv
+    rd, kd, vd = (acts(rt, rnd(n, inner, seed=100 + i, scale=0.5))[0] for i in range(3))
+    rate, w0, bonus, state = rnd(n, inner, seed=103) - 1.0, rnd(inner, seed=104, scale=0.5), rnd(heads, d, seed=105, scale=0.5), rnd(5, heads, d, d, seed=106, scale=0.3)
+    want_state, got_state = state.double(), state.to(rt.device)
+    want = ref_ops.time_mix_scan(rd.cpu(), kd.cpu(), vd.cpu(), rate, w0, bonus, want_state, slots, cu, 1, heads, d)
+    got = rt.ops.time_mix_scan(rd, kd, vd, rate.to(rt.device), w0.to(rt.device), bonus.to(rt.device), got_state, slots.to(rt.device), cu.to(rt.device), 1, heads, d)
+    assert rel_l2(got, want) < 2e-6 and rel_l2(got_state, want_state) < 1e-6 and torch.equal(got_state[[1, 3]].cpu(), state[[1, 3]])
+
+
 @pytest.mark.parametrize("cut", ["whole", "pieces", "one by one"])
 def test_matrix_memory_keeps_its_first_tokens(rt, cut):
     """Forget gates of sigmoid(8) and small input gates after the first tokens: the memory is what the first tokens wrote,

@@ -3,7 +3,8 @@
 //   o = S^T q / (max(|n . q|, e^(-m')) + 1e-6), i and f capped by a tanh.
 // S [dk, dv], n [dk] and m of a (sequence, head) are states, float32 like gates and sums.
 //
-// Two ways to the same rows:
+// Three ways to the same rows:
+// * a step of one row a sequence: matrix_memory_step_k;
 // * up to CHUNK_FROM rows: matrix_memory_scan_k, row after row, a lane keeping rows of one column of S in registers;
 // * more: chunks of up to 64 rows side by side, as products on the float32 matrix instructions (float32 operands and sums; the
 //   queries, keys and values are exact in them).  With b_t the sum of the log forget gates of a chunk's rows up to t, a_s = i_s - b_s
@@ -30,6 +31,72 @@ struct MatrixMemoryArgs {
 };
 
 __device__ __forceinline__ float log_sigmoid_f(float z) { return -(log1pf(expf(-fabsf(z))) + fmaxf(-z, 0.f)); }
+
+// ---- one row a sequence --------------------------------------------------------------------------------------------------------
+// A block for each (sequence, head).  What bounds it is one CU's trip to memory for dk dv floats and their way back: 131 KB at keys of
+// 128 and values of 256.  (The kernel of whole sequences, which reads columns in four waves' parts and prepares for rows that do
+// not come, took 29.4 us for 4 sequences of 9 heads; 8.0 here.)  R: rows of S a thread holds.
+template <typename T, int R>
+__global__ void __launch_bounds__(1024)
+matrix_memory_step_k(MatrixMemoryArgs a) {
+    __shared__ __attribute__((aligned(16))) float parts[16][256];
+    __shared__ float sq[256], sk[256], dots[4];
+    const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv, H = a.H;
+    const int t = a.cu_rows[seq];
+    if (a.cu_rows[seq + 1] <= t) return;
+    const size_t slot = (size_t)a.slot_ids[seq];
+    const int Q = dv >> 2, c4 = tid & (Q - 1), first = tid / Q, RG = blockDim.x / Q;
+    float* const st = a.memory + (slot * H + h) * dk * dv + 4 * c4;
+    float4 S[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) S[i] = *reinterpret_cast<const float4*>(st + (size_t)min(first + RG * i, dk - 1) * dv);
+    float* const sn = a.normalizer + (slot * H + h) * dk;
+    const int row = min(tid, dk - 1);
+    const float q = ld_f32((const T*)a.q + (size_t)t * a.q_stride + (size_t)h * dk + row) * a.q_scale;
+    const float k = ld_f32((const T*)a.k + (size_t)t * a.k_stride + (size_t)h * dk + row);
+    const float n = sn[row], m = a.maximum[slot * H + h];
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = ld_f32((const T*)a.v + (size_t)t * a.v_stride + (size_t)h * dv + 4 * c4 + e);
+    const float gi = a.gates[(size_t)t * 2 * H + h], gf = a.gates[(size_t)t * 2 * H + H + h];
+    const float li = a.cap * tanhf(gi / a.cap), lf = log_sigmoid_f(a.cap * tanhf(gf / a.cap));
+    const float m_new = fmaxf(lf + m, li), keep = expf(lf + m - m_new), take = expf(li - m_new);
+    if (wave < 4) {
+        const float n_new = __builtin_fmaf(keep, n, take * k), dot = wave_sum(tid < dk ? n_new * q : 0.f);
+        if (tid < dk) { sq[tid] = q; sk[tid] = k; sn[tid] = n_new; }
+        if (lane == 0) dots[wave] = dot;
+    }
+    lds_barrier();
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] *= take;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int r = first + RG * i;
+        if (r < dk) {
+            const float kr = sk[r], qr = sq[r];
+            S[i].x = __builtin_fmaf(keep, S[i].x, kr * v[0]);
+            S[i].y = __builtin_fmaf(keep, S[i].y, kr * v[1]);
+            S[i].z = __builtin_fmaf(keep, S[i].z, kr * v[2]);
+            S[i].w = __builtin_fmaf(keep, S[i].w, kr * v[3]);
+            o.x = __builtin_fmaf(qr, S[i].x, o.x);
+            o.y = __builtin_fmaf(qr, S[i].y, o.y);
+            o.z = __builtin_fmaf(qr, S[i].z, o.z);
+            o.w = __builtin_fmaf(qr, S[i].w, o.w);
+            *reinterpret_cast<float4*>(st + (size_t)r * dv) = S[i];
+        }
+    }
+    step_parts(o, Q, lane, &parts[wave][4 * c4]);
+    lds_barrier();                                       // everyone has worked with m, too
+    if (tid == 0) a.maximum[slot * H + h] = m_new;
+    if (tid < dv) {
+        float sum = 0.f, dot = 0.f;
+        for (int w = 0; w < (int)blockDim.x >> 6; w++) sum += parts[w][tid];
+#pragma unroll
+        for (int w = 0; w < 4; w++) dot += dots[w];
+        a.y[((size_t)t * H + h) * dv + tid] = sum / (fmaxf(fabsf(dot), expf(-m_new)) + 1e-6f);
+    }
+}
 
 // ---- row after row ---------------------------------------------------------------------------------------------------------------
 // One block for a (sequence, head), a group of waves for every 64 value columns: every wave carries n and m along (they are the
@@ -542,12 +609,12 @@ static void chunks_launch(const MatrixMemoryArgs& a, int n_seq, bool vec, hipStr
     }
 }
 
-// chunk 0: whole sequences; otherwise chunks of up to 64 rows.
+// chunk 0: whole sequences, in pieces of one row where no sequence has more (one_row_each); otherwise chunks of up to 64 rows.
 // memory [slots, H, dk, dv], normalizer [slots, H, dk], maximum [slots, H], gates [M, 2 H] (input sums, then forget sums), all float32
 extern "C" int tp_matrix_memory_scan(const void* q, long q_stride, const void* k, long k_stride, const void* v, long v_stride, int dtype,
                                      const float* gates, float cap, float q_scale, float* memory, float* normalizer, float* maximum,
                                      const int* slot_ids, const int* cu_rows, float* y, int n_seq, int H, int dk, int dv,
-                                     int chunk, int n_chunks, float* workspace, void* stream) {
+                                     int chunk, int n_chunks, float* workspace, int one_row_each, void* stream) {
     TP_REQUIRE(n_seq > 0 && H > 0 && dk > 0 && dv > 0, "matrix_memory_scan: empty shape sequences=%d heads=%d key=%d value=%d", n_seq, H, dk, dv);
     TP_REQUIRE(dk <= 256, "matrix_memory_scan: keys of %d elements exceed the 256 a lane keeps", dk);
     TP_REQUIRE(dv <= 256, "matrix_memory_scan: values of %d elements exceed the 256 columns of a block", dv);
@@ -571,6 +638,14 @@ extern "C" int tp_matrix_memory_scan(const void* q, long q_stride, const void* k
         return tp_check_launch("matrix_memory_scan (chunks)");
     }
     const dim3 grid(n_seq, H);
+    const int step_threads = one_row_each && (uintptr_t)memory % 16 == 0 ? tp_step_threads(dk, dv) : 0;
+    if (step_threads) {
+        const int rows = tp_cdiv((long)dk * dv, 4 * step_threads);
+#define TP_STEP(R) do { if (dtype == TP_BF16) matrix_memory_step_k<bf16_t, R><<<grid, step_threads, 0, s>>>(a); else matrix_memory_step_k<float, R><<<grid, step_threads, 0, s>>>(a); } while (0)
+        if (rows <= 2) TP_STEP(2); else if (rows <= 4) TP_STEP(4); else if (rows <= 8) TP_STEP(8); else TP_STEP(16);
+#undef TP_STEP
+        return tp_check_launch("matrix_memory_scan (one row)");
+    }
     const int threads = 64 * tp_cdiv(dv, 64);            // times the waves a group of columns is split over
 #define TP_LAUNCH(DK) do { if (dtype == TP_BF16) matrix_memory_scan_k<bf16_t, DK><<<grid, threads * TP_MM_SPLIT(DK), 0, s>>>(a); else matrix_memory_scan_k<float, DK><<<grid, threads * TP_MM_SPLIT(DK), 0, s>>>(a); } while (0)
     TP_SCAN_SIZES(TP_LAUNCH, dk);

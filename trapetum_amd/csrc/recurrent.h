@@ -22,3 +22,29 @@ __device__ __forceinline__ void load_rows(float (&dst)[NR], const T* p, int rows
 #define TP_SCAN_SIZES(LAUNCH, rows) do { \
     if ((rows) <= 16) LAUNCH(16); else if ((rows) <= 32) LAUNCH(32); else if ((rows) <= 64) LAUNCH(64); \
     else if ((rows) <= 128) LAUNCH(128); else LAUNCH(256); } while (0)
+
+// ---- a step of one row for each sequence: its state read and written once, by whole rows.  A thread holds four columns of every
+// blockDim / (columns / 4)-th row, all of its loads asked for at once; what each row needs (its q, k, decay) reaches the threads
+// through LDS while they travel, and the row parts of an output meet there once.
+// threads for a state of rows x columns floats (0: sizes that it does not take): a thread holds at most 16 rows
+static inline int tp_step_threads(int rows, int cols) {
+    if (cols < 4 || cols > 256 || (cols & (cols - 1)) || rows > 256) return 0;
+    return (long)rows * cols > 4096 ? 1024 : 256;
+}
+// the barrier of a block whose loads from memory go on: it waits for LDS alone
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// four columns' sums of a thread, added over the wave's lanes of the same columns (Q column groups in turn), into the wave's part
+__device__ __forceinline__ void step_parts(float4 o, int Q, int lane, float* part) {
+    for (int x = Q; x < 64; x <<= 1) {
+        o.x += __shfl_xor(o.x, x, 64);
+        o.y += __shfl_xor(o.y, x, 64);
+        o.z += __shfl_xor(o.z, x, 64);
+        o.w += __shfl_xor(o.w, x, 64);
+    }
+    if (lane < Q) *reinterpret_cast<float4*>(part) = o;
+}

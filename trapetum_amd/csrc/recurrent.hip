@@ -353,6 +353,62 @@ time_mix_scan_k(TimeMixArgs a) {
         for (int n = 0; n < NR; n++) if (lane + 64 * n < d) a.ws_decay[((size_t)blockIdx.x * a.H + h) * d + lane + 64 * n] = expf(fall[n]);
 }
 
+// One row a sequence (recurrent.h).  A block for each (sequence, head); R: rows of S a thread holds.  (4 sequences, 36 heads of 64: 13.9 us
+// by the kernel of whole sequences, which reads columns and prepares for rows that do not come; 5.0 here.)
+template <typename T, int R>
+__global__ void __launch_bounds__(1024)
+time_mix_step_k(TimeMixArgs a) {
+    __shared__ __attribute__((aligned(16))) float parts[16][256];
+    __shared__ float sr[256], sk[256], sw[256], dots[4];
+    const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, d = a.d, HD = a.H * d;
+    const int t = a.cu_rows[seq];
+    if (a.cu_rows[seq + 1] <= t) return;
+    const int Q = d >> 2, c4 = tid & (Q - 1), first = tid / Q, RG = blockDim.x / Q;
+    float* const st = a.state + ((size_t)a.slot_ids[seq] * a.H + h) * d * d + 4 * c4;
+    float4 S[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) S[i] = *reinterpret_cast<const float4*>(st + (size_t)min(first + RG * i, d - 1) * d);
+    const int row = h * d + min(tid, d - 1);
+    const float r = ld_f32((const T*)a.r + (size_t)t * a.r_stride + row), k = ld_f32((const T*)a.k + (size_t)t * a.k_stride + row);
+    const float u = a.bonus[row], w = expf(-expf(a.log_rate[(size_t)t * HD + row] + a.w0[row]));
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = ld_f32((const T*)a.v + (size_t)t * a.v_stride + (size_t)h * d + 4 * c4 + e);
+    if (wave < 4) {
+        const float dot = wave_sum(tid < d ? (r * u) * k : 0.f);         // the row's bonus: sum_i r_i u_i k_i
+        if (tid < d) { sr[tid] = r; sk[tid] = k; sw[tid] = w; }
+        if (lane == 0) dots[wave] = dot;
+    }
+    lds_barrier();
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int at = first + RG * i;
+        if (at < d) {
+            const float rr = sr[at], kr = sk[at], wr = sw[at];
+            o.x = __builtin_fmaf(rr, S[i].x, o.x);
+            o.y = __builtin_fmaf(rr, S[i].y, o.y);
+            o.z = __builtin_fmaf(rr, S[i].z, o.z);
+            o.w = __builtin_fmaf(rr, S[i].w, o.w);
+            S[i].x = __builtin_fmaf(wr, S[i].x, kr * v[0]);
+            S[i].y = __builtin_fmaf(wr, S[i].y, kr * v[1]);
+            S[i].z = __builtin_fmaf(wr, S[i].z, kr * v[2]);
+            S[i].w = __builtin_fmaf(wr, S[i].w, kr * v[3]);
+            *reinterpret_cast<float4*>(st + (size_t)at * d) = S[i];
+        }
+    }
+    step_parts(o, Q, lane, &parts[wave][4 * c4]);
+    lds_barrier();
+    if (tid < d) {
+        float bonus = 0.f;
+#pragma unroll
+        for (int x = 0; x < 4; x++) bonus += dots[x];
+        float sum = bonus * ld_f32((const T*)a.v + (size_t)t * a.v_stride + (size_t)h * d + tid);
+        for (int x = 0; x < (int)blockDim.x >> 6; x++) sum += parts[x][tid];
+        a.y[(size_t)t * HD + (size_t)h * d + tid] = sum;
+    }
+}
+
 // Chunk after chunk of a sequence: the state a chunk starts from takes the place of what the chunk adds, and the next
 // one is  decay * state + what it adds.  grid (sequences, heads, blocks of 256 elements of the state); the loads of
 // eight chunks are in flight together.
@@ -402,11 +458,12 @@ extern "C" long tp_time_mix_scan_workspace_floats(int n_seq, int n_chunks, int H
 }
 
 // state [slots, H, d, d] float32 (key row, value column); log_rate float32 [M, H d] contiguous; y float32 [M, H d].
-// chunk > 0: sequences run in chunks of that many rows, n_chunks covering the longest; workspace: floats as above
+// chunk > 0: sequences run in chunks of that many rows, n_chunks covering the longest; workspace: floats as above.  one_row_each:
+// no sequence has more than one row
 extern "C" int tp_time_mix_scan(const void* r, long r_stride, const void* k, long k_stride, const void* v, long v_stride, int dtype,
                                 const float* log_rate, const float* w0, const float* bonus, float* state, const int* slot_ids,
                                 const int* cu_rows, float* y, int n_seq, int H, int d, int chunk, int n_chunks, float* workspace,
-                                void* stream) {
+                                int one_row_each, void* stream) {
     TP_REQUIRE(n_seq > 0 && H > 0 && d > 0, "time_mix_scan: empty shape sequences=%d heads=%d size=%d", n_seq, H, d);
     TP_REQUIRE(d <= 256, "time_mix_scan: heads of %d channels exceed the 256 a lane keeps", d);
     TP_REQUIRE(H <= 65535, "time_mix_scan: %d heads exceed one launch", H);
@@ -419,6 +476,15 @@ extern "C" int tp_time_mix_scan(const void* r, long r_stride, const void* k, lon
     dim3 grid(n_seq, H, tp_cdiv(d, 64)), chunk_grid(n_seq * (chunk > 0 ? n_chunks : 1), H, tp_cdiv(d, 64)), carry_grid(n_seq, H, tp_cdiv(d * d, 256));
     hipStream_t s = (hipStream_t)stream;
     if (dtype != TP_BF16 && dtype != TP_F32) return tp_fail("time_mix_scan: unknown dtype %d", dtype);
+    const int step_threads = one_row_each && chunk == 0 && (uintptr_t)state % 16 == 0 ? tp_step_threads(d, d) : 0;
+    if (step_threads) {
+        const dim3 heads(n_seq, H);
+        const int rows = tp_cdiv((long)d * d, 4 * step_threads);
+#define TP_STEP(R) do { if (dtype == TP_BF16) time_mix_step_k<bf16_t, R><<<heads, step_threads, 0, s>>>(a); else time_mix_step_k<float, R><<<heads, step_threads, 0, s>>>(a); } while (0)
+        if (rows <= 4) TP_STEP(4); else TP_STEP(16);
+#undef TP_STEP
+        return tp_check_launch("time_mix_scan (one row)");
+    }
 #define TP_LAUNCH(DK) TP_SCAN_MODES(time_mix_scan_k, (time_mix_carry_k<<<carry_grid, 256, 0, s>>>(state, slot_ids, cu_rows, workspace, ws_decay, H, d, chunk, n_chunks)), DK, grid, chunk_grid, 64 * TP_SCAN_SPLIT(DK))
     TP_SCAN_SIZES(TP_LAUNCH, d);
 #undef TP_LAUNCH

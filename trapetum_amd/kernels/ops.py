@@ -48,8 +48,8 @@ _CORE_SIGS = {
     "tp_unary_tanh": [_P, _I, _L, _P],
     "tp_weighted_sum": [_P, _F, _P, _F, _I, _P, _L, _P],
     "tp_head_norm_gate": [_P, _P, _P, _L, _I, _F, _P, _I, _I, _I, _I, _I, _P],
-    "tp_time_mix_scan": [_P, _L, _P, _L, _P, _L, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P],
-    "tp_matrix_memory_scan": [_P, _L, _P, _L, _P, _L, _I, _P, _F, _F, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P],
+    "tp_time_mix_scan": [_P, _L, _P, _L, _P, _L, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P],
+    "tp_matrix_memory_scan": [_P, _L, _P, _L, _P, _L, _I, _P, _F, _F, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P],
     "tp_delta_scan": [_P, _L, _P, _L, _P, _L, _P, _P, _L, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P, _L, _P],
     "tp_delta_scan_workspace_bytes": [_I, _I, _I, _I, _I],
     "tp_linear_scan": [_P, _L, _P, _L, _P, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P],
@@ -703,7 +703,7 @@ class HipOps:
             ws = torch.empty(self.lib.tp_time_mix_scan_workspace_floats(n_seq, n_chunks, heads, dim), dtype=torch.float32, device=self.device)
         self._call(self.lib, "tp_time_mix_scan", r.data_ptr(), rs, k.data_ptr(), ks, v.data_ptr(), vs, _code(r.dtype), log_rate.data_ptr(),
                    w0.data_ptr(), bonus.data_ptr(), state.data_ptr(), slot_ids.data_ptr(), cu_rows.data_ptr(), y.data_ptr(), n_seq, heads, dim,
-                   chunk, n_chunks, ws.data_ptr() if ws is not None else None, self._stream())
+                   chunk, n_chunks, ws.data_ptr() if ws is not None else None, 1 if int(max_count) == 1 else 0, self._stream())
         return y
 
     SCAN_CHUNK_FROM = 96         # rows of the longest sequence from which a scan runs in chunks
@@ -758,7 +758,7 @@ class HipOps:
         self._call(self.lib, "tp_matrix_memory_scan", q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, _code(q.dtype), gates.data_ptr(),
                    float(cap), float(q_scale), memory.data_ptr(), normalizer.data_ptr(), maximum.data_ptr(), slot_ids.data_ptr(),
                    cu_rows.data_ptr(), y.data_ptr(), n_seq, heads, dk, dv, chunk, n_chunks, ws.data_ptr() if ws is not None else None,
-                   self._stream())
+                   1 if int(max_count) == 1 else 0, self._stream())
         return y
 
     DELTA_CHUNK = 64               # tokens of a chunk (the kernel library's)
