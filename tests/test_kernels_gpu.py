@@ -250,6 +250,38 @@ def test_attention_of_uneven_portions_over_a_cache(ops, counts, held, H, KV, hd,
         at += c
 
 
+# one long sequence first, last and between short ones, so that only the blocks that hold a query are launched: two sequences and as many
+# as are packed, more blocks of a sequence than lanes look at once (64, and a cache of many times that before them), a last block of
+# one row, a sequence without rows, windows; without a cache and over one
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+@pytest.mark.parametrize("counts,held,H,KV,hd,window", [([1, 1, 1, 2113], (150, 611, 48, 700), 4, 2, 64, 0), ([2600, 3], (0, 0), 4, 2, 64, 0), ([1] * 11 + [641] + [1] * 12, (77,) * 24, 4, 2, 64, 0),
+                                                        ([33, 0, 1500, 7, 64], (0, 0, 0, 0, 0), 2, 2, 256, 0), ([1, 700, 1, 1], (3000, 5000, 40, 3), 4, 1, 256, 400),
+                                                        ([5, 1025, 5, 5, 5], (4, 4000, 300, 20, 1), 8, 4, 128, 0)])
+def test_attention_launches_the_blocks_that_hold_queries(ops, counts, held, H, KV, hd, window, shape):
+    """Every sequence's rows are what they are alone, bit for bit (a choice of the shape by size may give others: to rounding)."""
+    n, page = len(counts), 64
+    new_len = torch.tensor([a + b for a, b in zip(counts, held)], dtype=torch.int32, device=DEV)
+    width = -(-int(new_len.max()) // page)
+    table = torch.randperm(n * width, generator=torch.Generator().manual_seed(6)).to(torch.int32).view(n, width).to(DEV)
+    pools = [randn(n * width, KV, page, hd, dtype=torch.bfloat16, seed=70 + i) for i in range(2)]
+    q, k, v = (randn(sum(counts), heads * hd, dtype=torch.bfloat16, seed=72 + i) for i, heads in enumerate((H, KV, KV)))
+
+    def attend(first, last):
+        a, b = sum(counts[:first]), sum(counts[:last])
+        cu = torch.tensor([sum(counts[first:i]) for i in range(first, last + 1)], dtype=torch.int32, device=DEV)
+        return ops.attention_prefill(q[a:b], k[a:b], v[a:b], H, KV, hd, cu, max(counts[first:last]), hd ** -0.5, 30.0, window, torch.bfloat16, shape=shape,
+                                     cached=(new_len[first:last], table[first:last], *pools, 0) if any(held) else None)
+    got, at = attend(0, n), 0
+    for i, c in enumerate(counts):
+        if c:
+            own = attend(i, i + 1)
+            if shape:
+                assert torch.equal(got[at:at + c], own), i
+            else:
+                assert rel_l2(got[at:at + c], own) < 4e-3, i      # two shapes' sums, rounded to bfloat16, as above
+        at += c
+
+
 # the kernel that streams up to 64 rows through LDS: each of its blocks (32, 64 and 128 rows of W, up to 16, 32 and 64 of X), one
 # k step and fewer than it asks for ahead, an N that ends inside a block and is no multiple of 4 (outputs element by element),
 # K slices of which the last is shorter; it is what is chosen from two rows on where the consumer adds the slices of a large matrix

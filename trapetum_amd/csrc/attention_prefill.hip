@@ -57,6 +57,7 @@ struct PrefillArgs {
     int H, KV, ghb_shift, pt_shift;           // heads of a kv head a block takes: 1 << ghb_shift; its position tiles: 1 << pt_shift
     int n_streams, pos_blocks;                // (sequence, kv head, head group) triples; blocks of positions per stream
     int turn;                                 // streams the next block of positions starts further on, so that a stream meets every XCD
+    int packed;                               // sequences (up to 64: a lane each) whose blocks are launched without those that hold no query; 0: all alike
     float scale, cap; int window;
     int chunk;                                // C > 0: the query at p sees keys from floor(p / C) C on only
     const float* head_scale;                  // [H] or null: a factor on every head's scores
@@ -117,6 +118,41 @@ __device__ __forceinline__ bf16_t bf16_bits(float f) {
 }
 union PFrag { uint4 u; pf_bf16x8 v; pf_s16x4 h[2]; };
 
+// The j-th block of positions in a launch of n sequences (up to 64), blocks of 1 << shift rows, those of late positions first (counted
+// with the cached ones before the step's rows, new_len or null: they see the most keys), of one position in the sequences'
+// order.  False: there is none.  A lane holds a sequence's first block and the one behind its last, in blocks of positions;
+// from(x), how many blocks stand at x or behind, is asked by 64 lanes for 64 places at once.
+__device__ __forceinline__ bool packed_block(const int* cu_rows, const int* new_len, int n, int shift, int j, int lane, int& seq, int& q0) {
+    const int at = min(lane, n - 1), rows = cu_rows[at + 1] - cu_rows[at];
+    const int count = lane < n ? (rows + (1 << shift) - 1) >> shift : 0, begin = new_len ? (new_len[at] - rows) >> shift : 0, end = begin + count;
+    auto from = [&](int x) {
+        int sum = 0;
+        for (int s = 0; s < n; s++) sum += max(__builtin_amdgcn_readlane(end, s) - max(__builtin_amdgcn_readlane(begin, s), x), 0);
+        return sum;
+    };
+    int b = 0, range = 0, behind = 0;                            // from(b) > j >= from(b + range), if there is such a block
+    for (int s = 0; s < n; s++) range = max(range, __builtin_amdgcn_readlane(end, s));
+    while (true) {
+        const int step = (range + 63) >> 6, f = from(b + lane * step);
+        const unsigned long long more = __ballot(f > j);
+        if (!more) return false;
+        const int l = 63 - __builtin_clzll(more);
+        b += l * step;
+        range = min(step, range - l * step);
+        if (step == 1) {
+            behind = l < 63 ? __builtin_amdgcn_readlane(f, l + 1) : __builtin_amdgcn_readfirstlane(from(b + 1));
+            break;
+        }
+    }
+    const int r = j - behind;
+    const bool mine = begin <= b && b < end;
+    const unsigned long long have = __ballot(mine), it = __ballot(mine && __popcll(have & ((1ull << lane) - 1)) == r);
+    seq = __ffsll((long long)it) - 1;
+    if (seq < 0) return false;
+    q0 = (b - __builtin_amdgcn_readlane(begin, seq)) << shift;
+    return true;
+}
+
 template <int CG, int KG> struct PrefillShape {
     static constexpr int THREADS = 64 * CG * KG;
     static constexpr size_t TILES = (size_t)2 * KG * TILE_BYTES + (size_t)CG * QL * 1024;      // K and V tiles, query fragments
@@ -139,13 +175,21 @@ attn_prefill_k(PrefillArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / CG, cg = wave % CG;
 
     // ---- which part of the step this block owns ---------------------------------------------------------------
-    const int rank = blockIdx.x / a.n_streams;
-    const int stream = (blockIdx.x % a.n_streams + rank * a.turn) % a.n_streams;
-    const int G = a.H / a.KV, HG = G >> a.ghb_shift;
-    const int hg = stream % HG, kvh = (stream / HG) % a.KV, seq = stream / (HG * a.KV);
-    const int PT = 1 << a.pt_shift, PB = 32 * PT;
+    const int G = a.H / a.KV, HG = G >> a.ghb_shift, PT = 1 << a.pt_shift, PB = 32 * PT;
+    int hg, kvh, seq, q0;                                        // late positions see the most keys: they start first
+    if (a.packed) {
+        const int sub = blockIdx.x % (HG * a.KV);
+        hg = sub % HG;
+        kvh = sub / HG;
+        if (!packed_block(a.cu_rows, PAGED ? a.new_len : nullptr, a.packed, 5 + a.pt_shift, blockIdx.x / (HG * a.KV), lane, seq, q0)) return;
+    } else {
+        const int rank = blockIdx.x / a.n_streams, stream = (blockIdx.x % a.n_streams + rank * a.turn) % a.n_streams;
+        hg = stream % HG;
+        kvh = (stream / HG) % a.KV;
+        seq = stream / (HG * a.KV);
+        q0 = (a.pos_blocks - 1 - rank) * PB;
+    }
     const int row0 = a.cu_rows[seq], Tq = a.cu_rows[seq + 1] - row0;
-    const int q0 = (a.pos_blocks - 1 - rank) * PB;               // late positions see the most keys: they start first
     if (q0 >= Tq) return;
     const int start = PAGED ? a.new_len[seq] - Tq : 0, L = start + Tq;
     const int h = kvh * G + (hg << a.ghb_shift) + (cg >> a.pt_shift);
@@ -569,6 +613,15 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
     // 258 / 288 us for 4x1 / 2x2; at 0.25, one of 4,000 beside four of 200, 206 / 181).  Where they are no more than the CUs, 2 x 4
     // is the choice from 512 tokens on, cached positions before them or not (2x2 / 2x4: 866 rows at 6,135 beside three tokens
     // 235 / 149 us, 600 at 4,096 137 / 103, 2 x 512 at 2,048 79 / 63, 8 prompts of up to 700 31 / 26; 257 tokens 15.5 / 16.8).
+    // Where less than half of the launched blocks could hold a query, and the sequences are few, those that hold none are not launched:
+    // a block finds its sequence and its place by itself (packed_block), and the ones that see the most keys come first.  Launched
+    // between empty ones, the blocks of a long sequence met on some CUs and left others idle, and the last of them began when the
+    // first had ended.  Microseconds, 2B, every block launched / packed: 2,048 rows beside three tokens 71 / 54, at 2,048 cached
+    // 139 / 96, at 4,096 207 / 139 (alone: 50, 97, 139); 1,000 at 3,000 beside three 142 / 90; 3,000 beside two 93 / 72; prompts of
+    // 512, 77, 1,300 and 260 44 / 36; 9B, 2,048 at 2,048 beside three 172 / 148.  The search costs 0.3 to 0.5 us with 5 to 8
+    // sequences (prompts of 333, 97, 1,021, 5 and 260: 29.9 / 30.6), 1 with 16, 4 with 61; and where half of the blocks hold queries
+    // nothing is gained (9B, four of 1,000 rows at 2,000 beside four tokens: 203 / 212).
+    auto packs = [&](long held, long all) { return n_seq <= 24 && 2 * held < all; };
     int cg = 4, kg = 1;
     bool uneven = false;
     {
@@ -582,16 +635,18 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
         const long blocks4 = HD <= 128 || 20 * filled() < 9 * longest() ? filled() : longest();
         plan(2, gs, pts);
         const bool alone = HD > 128 && filled() <= cus && max_count >= 512;
-        if (shape == 0 && blocks4 < 4L * cus) shape = alone || (HD > 128 && longest() <= 2L * cus && max_count >= 1024) ? 2 : 3;
+        const long launched = packs(filled(), longest()) ? filled() : longest();
+        if (shape == 0 && blocks4 < 4L * cus) shape = alone || (HD > 128 && launched <= 2L * cus && max_count >= 1024) ? 2 : 3;
         if (shape == 2) { cg = 2; kg = 4; }
         if (shape == 3) { cg = 2; kg = 2; }
         plan(cg, gs, pts);
-        uneven = 4 * filled() < 3 * longest();
+        uneven = 4 * filled() < 3 * longest();                 // (of the shape that is chosen)
+        a.packed = packs(filled(), longest()) ? n_seq : 0;
     }
     plan(cg, a.ghb_shift, a.pt_shift);
     a.n_streams = n_seq * KV * (G >> a.ghb_shift);
     a.pos_blocks = tp_cdiv(max_count, 32 << a.pt_shift);
-    const long blocks = (long)a.n_streams * a.pos_blocks;
+    const long blocks = a.packed ? ((long)M / (32 << a.pt_shift) + n_seq) * KV * (G >> a.ghb_shift) : (long)a.n_streams * a.pos_blocks;
     // Blocks go round the 8 XCDs, and those of an XCD round its 4 shader engines: 32 places.  A stream's blocks are every
     // n_streams-th, so where that is a multiple of a power of two they meet a few places only.  That is good for its keys' way
     // through an L2, and for the load where all streams are alike (with a turn 8 x 7,900 tokens take 2.20 ms instead of 2.10), but
