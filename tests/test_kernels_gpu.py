@@ -328,6 +328,17 @@ def test_linear_up_to_64_rows_takes_blocks_of_each_height(ops):
     assert rows(32, 32701, 512, EPI_NONE, 0) == 64 and rows(65, 32701, 512, EPI_NONE, 0) == 0
 
 
+# blocks of 96 rows of W: the fewest and the most of them, a last one of one row or of rows that no unit has, as many k steps as the ring
+# holds and one more, rows of X in each of its two heights
+@pytest.mark.parametrize("m,n,k", [(2, 16450, 256), (32, 20449, 320), (33, 16417, 256), (64, 24576, 704), (9, 18432, 1088), (50, 16418, 640)])
+def test_linear_blocks_of_96_rows(ops, m, n, k):
+    from trapetum_amd.kernels.ops import EPI_GATED, EPI_NONE
+    half = n // 2 // 16 * 16
+    assert ops.lib.tp_linear_stream_rows(m, n, k, EPI_NONE, 0) == 96 and ops.lib.tp_linear_stream_rows(m, 2 * half, k, EPI_GATED, 0) == 96
+    assert ops.lib.tp_linear_stream_rows(m, n, 192, EPI_NONE, 0) == 32
+    test_linear_up_to_64_rows(ops, m, n, k)
+
+
 # the tiles of 8 waves (12: 256 x 256, 13: 256 x 192, 14: 192 x 256, 15: 256 x 128): one k step, two, three and a long odd number
 # of them, a tile and one row more or less, an N that is no multiple of 8 or 4 (outputs element by element), a last K slice
 # that is shorter, more tiles than CUs

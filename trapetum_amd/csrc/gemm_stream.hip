@@ -1,10 +1,10 @@
 // bf16 product for up to 64 rows (a decode step of many sequences): bound by reading W once, fp32 accumulation.
 //
-// A block owns BN = 32, 64 or 128 rows of W and all rows of X (MB = 16, 32 or 64 of them), and walks K in steps of 64.  W and X
+// A block owns BN = 32, 64, 96 or 128 rows of W and all rows of X (MB = 16, 32 or 64 of them), and walks K in steps of 64.  W and X
 // come straight from global memory into LDS, S steps deep, so a CU has 72 to 128 KB of loads in flight without a register spent
 // on them (the register-staged 64 x 64 tiles of gemm_mfma.hip hold one step each and wait for it; the 8-row kernel of
 // gemm_rows8.hip holds eight loads a wave).  One barrier a step: behind it the step's tiles have arrived, and the place of the step
-// before, which everyone has read, takes the tiles S - 1 steps on.  Waves of up to MB rows of X by 32 rows of W
+// before, which everyone has read, takes the tiles S - 1 steps on.  Waves of up to MB rows of X by 32 rows of W (a block of 96: by all)
 // (v_mfma_f32_16x16x32_bf16 with W as the A operand: a lane ends up with four neighbours of a row of Y, and with gate and up column
 // of a unit in two accumulators).  The 16-byte chunks of an LDS row (128 bytes) lie at chunk ^ (row % 8), the swizzle applied on
 // the global side of the load.
@@ -12,7 +12,7 @@
 // Measured on MI355X, cold weights, replayed graph, microseconds, before (the kernels named above) / here; down and o include
 // the norm that adds their slices:
 //             8 rows                                                    64 rows
-//   2B        gate/up 19.3 / 18.7  down 16.0 / 14.8  qkv 6.3 / 5.7       gate/up 26.6 / 25.2  down 20.6 / 16.8  qkv 8.5 / 6.5
+//   2B        gate/up 19.3 / 18.2  down 16.0 / 14.8  qkv 6.3 / 5.7       gate/up 26.6 / 21.6  down 20.6 / 16.8  qkv 8.5 / 6.5
 //             o 8.9 / 8.4    logits 209 / 202                            o 12.4 / 9.9   logits 258 / 243
 //   9B        gate/up 40.3 / 38.0  down 27.5 / 24.0  qkv 14.4 / 12.4     gate/up 44.0 / 39.7  down 37.3 / 28.8  qkv 19.5 / 14.2
 //             o 15.0 / 12.1                                              o 16.4 / 13.8
@@ -29,11 +29,11 @@ union StFrag { uint4 u; st_bf16x8 v; };
 template <int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14)); }
 }
 
-template <int EPI, int MB, int BN, int WAVES, int S>
+template <int EPI, int MB, int BN, int WAVES, int S, int WN = BN / 32>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_stream_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K,
               int out_dtype, float4 epi, int units, int k_per_split) {
-    constexpr int WN = BN / 32, WM = WAVES / WN, ROWS = 8 * WAVES, LX = MB / ROWS, LW = BN / ROWS, L = LX + LW, STAGE = (MB + BN) * 128, TM = MB / 16 / WM;
+    constexpr int WM = WAVES / WN, ROWS = 8 * WAVES, LX = MB / ROWS, LW = BN / ROWS, L = LX + LW, STAGE = (MB + BN) * 128, TM = MB / 16 / WM, TN = BN / 16 / WN;
     static_assert(TM >= 1 && LX >= 1 && LW >= 1 && (S - 2) * L < 64, "tile");
     __shared__ __attribute__((aligned(16))) unsigned char lds[S * STAGE];
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -64,9 +64,11 @@ gemm_stream_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* 
 #pragma unroll
         for (int i = 0; i < LX; i++) load(X + k, xo[i], stage + i * ROWS * 128);
     };
-    st_f32x4 acc[TM][2];
+    st_f32x4 acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < TM; i++) acc[i][0] = acc[i][1] = (st_f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (st_f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < S - 1; t++)
         if (t < steps) fill(t, t * STAGE);
@@ -79,13 +81,13 @@ gemm_stream_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* 
         asm volatile("" ::: "memory");
         if (step + S - 1 < steps) fill(step + S - 1, free_);
         const unsigned char* const xs = lds + cur + (wm * 16 * TM + r) * 128;
-        const unsigned char* const ws = lds + cur + (MB + wn * 32 + r) * 128;
-        StFrag a[2][TM], b[2][2];
+        const unsigned char* const ws = lds + cur + (MB + wn * 16 * TN + r) * 128;
+        StFrag a[2][TM], b[2][TN];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             const int at = ((4 * s + g) ^ (r & 7)) * 16;
 #pragma unroll
-            for (int j = 0; j < 2; j++) b[s][j].u = *reinterpret_cast<const uint4*>(ws + j * 2048 + at);
+            for (int j = 0; j < TN; j++) b[s][j].u = *reinterpret_cast<const uint4*>(ws + j * 2048 + at);
 #pragma unroll
             for (int i = 0; i < TM; i++) a[s][i].u = *reinterpret_cast<const uint4*>(xs + i * 2048 + at);
         }
@@ -94,7 +96,7 @@ gemm_stream_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* 
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j].v, a[s][i].v, acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j].v, a[s][i].v, acc[i][j], 0, 0, 0);
         free_ = cur;
         cur = cur + STAGE == S * STAGE ? 0 : cur + STAGE;
     }
@@ -105,12 +107,12 @@ gemm_stream_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* 
         const int m = wm * 16 * TM + i * 16 + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < (EPI == TP_EPI_GATED ? 1 : 2); j++) {
-            const int col = (EPI == TP_EPI_GATED ? (n0 + wn * 32) >> 1 : n0 + wn * 32 + j * 16) + g * 4;
+        for (int j = 0; j < TN; j += EPI == TP_EPI_GATED ? 2 : 1) {
+            const int at_n = n0 + (wn * TN + j) * 16, col = (EPI == TP_EPI_GATED ? at_n >> 1 : at_n) + g * 4;
             float o[4];
 #pragma unroll
             for (int v = 0; v < 4; v++)
-                o[v] = EPI == TP_EPI_GATED ? gated_unit_fast(acc[i][0][v], acc[i][1][v], epi) : plain_epilogue(EPI, acc[i][j][v], epi, col + v);
+                o[v] = EPI == TP_EPI_GATED ? gated_unit_fast(acc[i][j][v], acc[i][j + 1 < TN ? j + 1 : j][v], epi) : plain_epilogue(EPI, acc[i][j][v], epi, col + v);
             if (col >= width) continue;
             const size_t at = (size_t)m * width + col;
             if (wide) {
@@ -144,7 +146,11 @@ struct StreamPlan { int rows, splits, kps; };   // rows of W a block owns, K sli
 // busiest CU fewer rows and all blocks run at once, three a CU (2B gate/up, 288 blocks of 64 rows or 576 of 32: 21.5 / 18.7 us; 9B,
 // 448 or 896, beyond three a CU: 38.0 / 47.1).  128 rows a block from 33 rows of X on, where X's tile costs what W's costs, if
 // the busiest CU gets no more rows by it (64 rows of X, logits 262 / 243 us, 9B gate/up 45.6 / 39.7) - but not where rows of W
-// lie a multiple of 8 KB apart, when 128 of them meet in the same memory channels (N 32768, K 4096: 58.0 / 65.1).
+// lie a multiple of 8 KB apart, when 128 of them meet in the same memory channels (N 32768, K 4096: 58.0 / 65.1).  Where 32 rows a block
+// would be three blocks on the fullest CU, one block of 96 gives it the same rows of W and reads X once instead of three times:
+// always from 33 rows of X on (32 / 96 rows of W a block, K 2304, 64 rows: N 16512 24.6 / 20.3 us, 17408 26.1 / 22.7, 18432 25.5 / 21.6, 24576 29.0 / 24.5; K 4096,
+// N 16896 42.3 / 36.8), below where the CUs have two and a half on average at most (8 rows: N 18432 19.4 / 18.8, 24576 22.6 / 22.9;
+// 32 rows, N 18432 20.8 / 19.6).  Its ring is four steps deep, and shorter K keeps the blocks of 32: three and five are slower (8 rows 21.5 and 18.9, 64 rows 22.0 and 22.3).
 static StreamPlan stream_plan(const GemmArgs& a) {
     constexpr int CUS = 256, MAX_SPLITS = 16;
     const int blocks = tp_cdiv(a.N, 64), narrow = tp_cdiv(a.N, 32), wide = tp_cdiv(a.N, 128);
@@ -158,7 +164,8 @@ static StreamPlan stream_plan(const GemmArgs& a) {
     p.kps = tp_cdiv(tp_cdiv(a.K, p.splits), BK) * BK;
     p.splits = tp_cdiv(a.K, p.kps);
     if (p.splits == 1) {
-        if (narrow <= 3 * CUS && tp_cdiv(narrow, CUS) < 2 * tp_cdiv(blocks, CUS)) p.rows = 32;
+        if (a.K >= 4 * BK && narrow > 2 * CUS && tp_cdiv(a.N, 96) <= CUS && (a.M > 32 || 2 * narrow <= 5 * CUS)) p.rows = 96;
+        else if (narrow <= 3 * CUS && tp_cdiv(narrow, CUS) < 2 * tp_cdiv(blocks, CUS)) p.rows = 32;
         else if (a.M > 32 && blocks > CUS && a.K % 4096 && 2 * tp_cdiv(wide, CUS) <= tp_cdiv(blocks, CUS)) p.rows = 128;
     }
     return p;
@@ -179,16 +186,19 @@ int gemm_stream_slices_left(const GemmArgs& a) {
     return a.defer && (s > 1 || a.algo == 0) ? s : 0;
 }
 
-template <int EPI, int MB, int BN, int WAVES, int S>
+template <int EPI, int MB, int BN, int WAVES, int S, int WN = BN / 32>
 static void stream_tile(const GemmArgs& a, void* y, int out_dtype, const StreamPlan& p) {
-    gemm_stream_k<EPI, MB, BN, WAVES, S><<<dim3((unsigned)tp_cdiv(a.N, BN), p.splits), 64 * WAVES, 0, a.stream>>>(
+    gemm_stream_k<EPI, MB, BN, WAVES, S, WN><<<dim3((unsigned)tp_cdiv(a.N, BN), p.splits), 64 * WAVES, 0, a.stream>>>(
         (const bf16_t*)a.x, (const bf16_t*)a.w, y, a.M, a.N, a.K, out_dtype, epi_constants(a), a.units, p.kps);
 }
 
-// depths: two blocks a CU (72 to 80 KB of LDS each) but three for 32 rows of W (48 KB)
+// depths: two blocks a CU (72 to 80 KB of LDS each) but three for 32 rows of W (48 KB); blocks of 96 rows are one a CU by their number
 template <int EPI>
 static void stream_launch(const GemmArgs& a, void* y, int out_dtype, const StreamPlan& p) {
-    if (p.rows == 32) {
+    if (p.rows == 96) {
+        if (a.M <= 32) stream_tile<EPI, 32, 96, 2, 4, 1>(a, y, out_dtype, p);
+        else stream_tile<EPI, 64, 96, 4, 4, 1>(a, y, out_dtype, p);
+    } else if (p.rows == 32) {
         if (a.M <= 16) stream_tile<EPI, 16, 32, 1, 8>(a, y, out_dtype, p);
         else if (a.M <= 32) stream_tile<EPI, 32, 32, 1, 6>(a, y, out_dtype, p);
         else stream_tile<EPI, 64, 32, 1, 4>(a, y, out_dtype, p);
