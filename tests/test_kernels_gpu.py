@@ -396,6 +396,26 @@ def test_linear_f32(ops, m, n, k):
     assert torch.equal(alone[0], got[m - 1])
 
 
+# one launch: a matrix alone and as many as it takes, matrices of one row, of less than a block and of less than all of its last, with and
+# without a bias, both output types, one and two groups of 8 rows a block; beside it, what goes product after product (9 rows, a K
+# beyond one round, K no multiple of 8, more matrices)
+@pytest.mark.parametrize("m,k,ns", [(1, 8, (1,)), (4, 2304, (2304, 2304, 2304, 2304, 144)), (8, 256, (7, 8, 9, 33, 1, 16, 15, 500)), (3, 1160, (2056, 2048, 20)),
+                                    (5, 776, (4097,)), (9, 256, (40, 8)), (2, 2560, (24, 40)), (4, 20, (9, 3)), (8, 64, (8,) * 9)])
+def test_linear_group(ops, m, k, ns):
+    parts = []
+    for i, n in enumerate(ns):
+        x, w = randn(m, k, dtype=torch.bfloat16, seed=20 + i), randn(n, k, dtype=torch.bfloat16, seed=40 + i, scale=0.05)
+        parts.append((x, w, torch.float32 if i % 3 == 1 else torch.bfloat16, randn(n, seed=60 + i) if i % 2 else None))
+    for got, (x, w, dtype, bias) in zip(ops.linear_group(parts), parts):
+        ref = x.cpu().double() @ w.cpu().double().T + (bias.cpu().double() if bias is not None else 0.0)
+        assert got.dtype == dtype and rel_l2(got, ref) < (1e-5 if dtype == torch.float32 else 4e-3)
+    with pytest.raises(Exception, match="linear_group"):
+        ops.linear_group(parts + [(parts[0][0], parts[0][1][:, :-1].contiguous(), torch.bfloat16, None)])
+    if m <= 8 and k % 8 == 0 and k <= 2304:
+        with pytest.raises(Exception, match="bias"):
+            ops.linear_group([(parts[0][0], parts[0][1], torch.bfloat16, torch.zeros(ns[0] + 1, device=DEV))])
+
+
 # few rows (up to 32) and many, a row tile and one more or less, parts of K that end inside a block of 16 or are empty, a K of one
 # piece, K slices for the consumer, two tiles of W a block (from 16384 rows of W on), operands off their 16 bytes
 @pytest.mark.parametrize("m,n,k", [(1, 16, 4), (16, 17, 260), (17, 2304, 2048), (32, 33, 2300), (33, 129, 36), (64, 500, 1028), (309, 250, 4100),

@@ -6,6 +6,8 @@
 enum { TP_EPI_NONE = 0, TP_EPI_SOFTCAP = 1, TP_EPI_GATED = 2, TP_EPI_RELU2 = 3, TP_EPI_SILU = 4 };
 // steps of 64 k a wave of the 8-row kernel has in flight at once: four waves a block read a K of 2,304 in one round of loads
 #define TP_R8_MAX_STEPS 9
+// products that one launch of that kernel takes (tp_linear_group)
+#define TP_LINEAR_GROUP 8
 
 struct GemmArgs {
     const void* x; const void* w; void* y;

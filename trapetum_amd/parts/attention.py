@@ -60,7 +60,7 @@ product rides with the projections' as further columns.  All three are applied i
 from ..cache.store import TokenSpec
 from ..models.spec import TensorSpec
 from ..registry import build_part, register_part
-from .base import Mixer
+from .base import Mixer, products
 
 
 class Attention(Mixer):
@@ -370,7 +370,7 @@ class Attention(Mixer):
         if self.taps:
             qkv = self._convolved(ctx, x, w_in)
         else:
-            qkv = ops.linear(x, w_in, ctx.dtype, bias=bias) if bias is not None else ops.linear(x, w_in, ctx.dtype)
+            qkv = products(ops, [(x, w_in, ctx.dtype, bias)])[0] if bias is not None else ops.linear(x, w_in, ctx.dtype)
         if owns_cache:
             q, k, v = qkv[:, :Q], qkv[:, Q:Q + KVD], qkv[:, Q + KVD:Q + 2 * KVD]
         else:

@@ -36,6 +36,15 @@ step (`forward`).  Interfaces:
 """
 
 
+def products(ops, parts):
+    """[x @ w^T (+ bias) for x, w, out_dtype, bias in parts], inputs of one shape: in one launch where the kernels can (a kernel
+    library need not have the entry)."""
+    group = getattr(ops, "linear_group", None)
+    if group is not None:
+        return group(parts)
+    return [ops.linear(x, w, out_dtype, bias=bias) for x, w, out_dtype, bias in parts]
+
+
 class Part:
     def tensor_specs(self):
         """{local tensor name: TensorSpec}."""

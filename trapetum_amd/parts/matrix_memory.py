@@ -15,7 +15,7 @@ activation dtype.  A sequence keeps S, n and m between steps, float32 states by 
 from ..cache.store import StateSpec
 from ..models.spec import TensorSpec
 from ..registry import register_part
-from .base import Mixer
+from .base import Mixer, products
 
 
 class MatrixMemory(Mixer):
@@ -62,8 +62,8 @@ class MatrixMemory(Mixer):
         import torch
         ops, H = ctx.ops, self.num_heads
         qk, vv = H * self.key_dim, H * self.value_dim
-        u = ops.linear(x, self.w_in, ctx.dtype)                                                   # [M, q | k | v | g]
-        gates = ops.linear(x, self.w_gates, torch.float32, bias=self.b_gates)                     # [M, i | f] before the caps
+        u, gates = products(ops, [(x, self.w_in, ctx.dtype, None),                                # [M, q | k | v | g]
+                                  (x, self.w_gates, torch.float32, self.b_gates)])                # [M, i | f] before the caps
         y = ops.matrix_memory_scan(u[:, :qk], u[:, qk:2 * qk], u[:, 2 * qk:2 * qk + vv], gates, self.gate_cap, self.key_dim ** -0.5,
                                    self.state(ctx, "memory"), self.state(ctx, "normalizer"), self.state(ctx, "maximum"),
                                    ctx.slot_ids, ctx.cu_rows, ctx.max_count, H, self.key_dim, self.value_dim)

@@ -17,7 +17,7 @@ there is nothing per token.
 from ..cache.store import StateSpec
 from ..models.spec import TensorSpec
 from ..registry import register_part
-from .base import Mixer
+from .base import Mixer, products
 
 BRANCHES = ("r", "k", "v", "g", "w")
 
@@ -69,8 +69,8 @@ class TimeMix(Mixer):
         ops, w = ctx.ops, self.w
         mixes = ops.shift_mix(x, self.mu, self.state(ctx, "shift"), ctx.slot_ids, ctx.cu_rows, ctx.row_seq,
                               one_row_each=ctx.mode == "decode")                                  # [5, M, D]
-        r, k, v, g = (ops.linear(mixes[i], w[s], ctx.dtype) for i, s in enumerate(("r", "k", "v", "g")))
-        low = ops.unary_(ops.linear(mixes[4], w["w1"], ctx.dtype), "tanh")
+        r, k, v, g, low = products(ops, [(mixes[i], w[s], ctx.dtype, None) for i, s in enumerate(("r", "k", "v", "g", "w1"))])
+        low = ops.unary_(low, "tanh")
         log_rate = ops.linear(low, w["w2"], torch.float32)                                        # w0 is added in the scan
         y = ops.time_mix_scan(r, k, v, log_rate, self.w0, self.bonus, self.state(ctx, "memory"), ctx.slot_ids, ctx.cu_rows,
                               ctx.max_count, self.num_heads, self.head_dim)
