@@ -1118,6 +1118,30 @@ def test_sample_in_turn_on_one_workspace(ops, vocab, top_k):
             assert got[b] in near, (b, got[b], near)
 
 
+# numbers that come with the launch and numbers on the device; candidates of one wave, of two, of all sixteen, of more than the block
+# sorts at once (few different logits: a bin of many, and ties that the smaller id wins), the whole vocabulary
+@pytest.mark.parametrize("rows", [1, 5, 64])
+@pytest.mark.parametrize("vocab,top_k,levels", [(300, 40, 0), (40000, 1, 0), (40000, 100, 0), (256000, 256, 0), (33000, 1024, 0), (50000, 700, 37), (40000, 0, 0), (90, 90, 5)])
+def test_sample_takes_its_numbers_from_host_and_device(ops, rows, vocab, top_k, levels):
+    from .plain import gemma2_plain as plain
+    z = randn(rows, vocab, seed=80, scale=2.0)
+    if levels:
+        z = torch.round(z * (levels / 12.0)) * (12.0 / levels)
+    top_p = 0.9 if top_k else 1.0
+    u = torch.rand(rows, generator=torch.Generator().manual_seed(81))
+    device = ops.sample(z, 0.8, top_k, top_p, u.to(DEV))
+    assert torch.equal(ops.sample(z, 0.8, top_k, top_p, u.tolist()), device)
+    zc = z.cpu()
+    if top_k:                                                # (the whole vocabulary: 40,000 sums in another order may end on a neighbour)
+        some = range(0, rows, 13)
+        agree = sum(plain.sample(zc[i], 0.8, top_p, top_k, float(u[i])) == int(device[i]) for i in some)
+        assert agree >= len(some) - 1                        # a draw at a boundary of the cumulative sums may fall on either side
+    with pytest.raises(Exception, match="uniform"):
+        ops.sample(z, 0.8, top_k, top_p, u.tolist() + [0.5])
+    with pytest.raises(Exception, match="at most"):
+        ops.sample(z[:1].expand(65, -1).contiguous(), 0.8, top_k, top_p, [0.5] * 65)
+
+
 def test_recent_push(ops):
     """A row's id goes to the place its cursor names, the cursor moves on and wraps at the ring's end."""
     ring = torch.full((3, 5), -1, dtype=torch.int32, device=DEV)

@@ -206,6 +206,13 @@ extern "C" int tp_recent_push(const int* tokens, int* recent, int* cursor, int B
 // r = u * kept mass; falls back to the first candidate.  One block per row: a radix select over the value
 // bits finds the k-th largest logit, an id select breaks ties at that value, the at most 1024 candidates are
 // sorted in LDS, and the first wave does the short scans (sums in candidate order within a lane, then over the lanes). ---
+// a barrier that waits for LDS alone: stores on their way to memory hold nobody up
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 __device__ __forceinline__ uint32_t value_key(float f) {           // larger float -> larger key; NaN lowest
     uint32_t u = __float_as_uint(f);
     if ((u & 0x7fffffffu) > 0x7f800000u) return 0u;
@@ -258,37 +265,67 @@ __device__ __forceinline__ void pick_bucket(const unsigned* hist, bool from_top,
     rem_out = (unsigned)__shfl((int)r, L, 64);
 }
 
+// The value of lane ^ STRIDE, by data-parallel moves (a shuffle through LDS takes three times as long).
+template <int STRIDE>
+__device__ __forceinline__ uint32_t across(uint32_t v, int lane) {
+    if constexpr (STRIDE == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);            // quads 1 0 3 2
+    else if constexpr (STRIDE == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);       // quads 2 3 0 1
+    else if constexpr (STRIDE == 4) {                                                                             // rows of 16 turned by 4 and by 12
+        const uint32_t back = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xf, 0xf, true), ahead = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x12c, 0xf, 0xf, true);
+        return lane & 4 ? back : ahead;
+    } else if constexpr (STRIDE == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);    // turned by 8
+    else if constexpr (STRIDE == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return lane & 16 ? r[0] : r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return lane & 32 ? r[0] : r[1];
+    }
+}
+template <int STRIDE>
+__device__ __forceinline__ void sort_step(uint32_t& key, int& id, int tid, int size) {
+    const uint32_t ok = across<STRIDE>(key, tid), oi = across<STRIDE>((uint32_t)id, tid);
+    const bool before = key > ok || (key == ok && id < (int)oi);               // this thread's element belongs before the other
+    const bool wants_first = ((tid & STRIDE) == 0) == ((tid & size) == 0);
+    if (before != wants_first) { key = ok; id = (int)oi; }
+}
+
 // Sorts the block's elements, one a thread (key, id), by (key descending, id ascending), over the first `n` threads (a power of
-// two up to 1024): a bitonic network whose exchanges within a wave are shuffles, so that only the strides of 64 and more
-// meet in LDS (10 of 55 rounds at 1,024 elements, 6 of 45 at 512).
+// two from 64 to 1024): a bitonic network whose exchanges within a wave stay in registers, so that only the strides of 64 and more
+// meet in LDS (10 of 55 rounds at 1,024 elements, 6 of 45 at 512).  Waves beyond n keep their elements.
 __device__ __forceinline__ void block_sort(uint32_t& key, int& id, int n, uint32_t* lkey, int* lid) {
     const int tid = threadIdx.x;
-    for (int size = 2; size <= n; size <<= 1)
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            uint32_t ok;
-            int oi;
-            if (stride >= 64) {
-                __syncthreads();
-                lkey[tid] = key;
-                lid[tid] = id;
-                __syncthreads();
-                ok = lkey[tid ^ stride];
-                oi = lid[tid ^ stride];
-            } else {
-                ok = (uint32_t)__shfl_xor((int)key, stride, 64);
-                oi = __shfl_xor(id, stride, 64);
-            }
-            const bool before = key > ok || (key == ok && id < oi);           // this thread's element belongs before the other
-            const bool wants_first = ((tid & stride) == 0) == ((tid & size) == 0);
+    for (int size = 2; size <= n; size <<= 1) {
+        for (int stride = size >> 1; stride >= 64; stride >>= 1) {
+            lds_barrier();
+            lkey[tid] = key;
+            lid[tid] = id;
+            lds_barrier();
+            const uint32_t ok = lkey[tid ^ stride];
+            const int oi = lid[tid ^ stride];
+            const bool before = key > ok || (key == ok && id < oi), wants_first = ((tid & stride) == 0) == ((tid & size) == 0);
             if (before != wants_first) { key = ok; id = oi; }
         }
+        if (size > 32) sort_step<32>(key, id, tid, size);
+        if (size > 16) sort_step<16>(key, id, tid, size);
+        if (size > 8) sort_step<8>(key, id, tid, size);
+        if (size > 4) sort_step<4>(key, id, tid, size);
+        if (size > 2) sort_step<2>(key, id, tid, size);
+        sort_step<1>(key, id, tid, size);
+    }
 }
+
+// The rows' uniform numbers: an array on the device, or (null) up to TP_HOST_UNIFORMS of them that came with the launch, which saves a
+// caller who draws them on the host a copy and the wait for it.
+#define TP_HOST_UNIFORMS 64
+struct Draws { const float* at; float v[TP_HOST_UNIFORMS]; };
+__device__ __forceinline__ float draw_of(const Draws& d, int row) { return d.at ? d.at[row] : d.v[row]; }
 
 // With a candidate list (cand_count non-null): row b's candidates are cand_val/cand_id[b * cand_cap ..], a superset
 // of its top_k if their number fits cand_cap; the kernel then works on the list, else on the whole row.
 __global__ void __launch_bounds__(1024)
 sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p,
-         const float* __restrict__ uniforms, int* __restrict__ out,
+         Draws draws, int* __restrict__ out,
          unsigned* __restrict__ cand_count, const float* __restrict__ cand_val, const int* __restrict__ cand_id,
          int cand_cap, unsigned* __restrict__ row_hist, int row_bins) {
     __shared__ unsigned hist[256];
@@ -301,21 +338,24 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
     const int tid = threadIdx.x;
     const int k = top_k < V ? top_k : V;                       // of the whole row, whichever source is read
     const int* ids = nullptr;                                  // candidate -> token id; null: the index is the id
+    uint32_t mkey = 0u;                                        // this thread's candidate; empty entries (key 0, id max) sink
+    int mid = 0x7fffffff, sorted = 1024;
     if (cand_count) {
+        // (the list's first 1024 entries are asked for with its length: places that exist, used where the list reaches)
+        const float first = cand_val[(size_t)blockIdx.x * cand_cap + tid];
+        const int first_id = cand_id[(size_t)blockIdx.x * cand_cap + tid];
         const unsigned listed = cand_count[blockIdx.x];
         if (listed <= (unsigned)cand_cap && listed >= (unsigned)k) {
             V = (int)listed;
             z = cand_val + (size_t)blockIdx.x * cand_cap;
             ids = cand_id + (size_t)blockIdx.x * cand_cap;
         }
-        for (int i = tid; i < row_bins; i += 1024) row_hist[(size_t)blockIdx.x * row_bins + i] = 0u;
-        __syncthreads();                                       // everyone has read the count
+        if (ids && V <= 1024 && tid < V) { mkey = value_key(first); mid = first_id; }
+        lds_barrier();                                         // everyone has worked with the count
         if (tid == 0) cand_count[blockIdx.x] = 0u;
+        for (int i = tid; i < row_bins; i += 1024) row_hist[(size_t)blockIdx.x * row_bins + i] = 0u;
     }
-    uint32_t mkey = 0u;                                        // this thread's candidate; empty entries (key 0, id max) sink
-    int mid = 0x7fffffff, sorted = 1024;
     if (ids && V <= 1024) {
-        if (tid < V) { mkey = value_key(z[tid]); mid = ids[tid]; }
         sorted = 64;
         while (sorted < V) sorted <<= 1;
     } else {
@@ -394,15 +434,15 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
     }
     // 4. in order; the first k are the candidates
     block_sort(mkey, mid, sorted, ckey, cid);
-    __syncthreads();
+    lds_barrier();
     ckey[tid] = mkey;
     cid[tid] = mid;
-    __syncthreads();
+    lds_barrier();
     // 5. probabilities, the nucleus and the draw: the first wave, each lane 16 consecutive candidates; sums run over a
     // lane's candidates in order, then over the lanes in order
     const float mx = key_value(ckey[0]);
     prob[tid] = tid < k ? expf((key_value(mkey) - mx) / temperature) : 0.f;
-    __syncthreads();
+    lds_barrier();
     if (tid < 64) {
         const int j0 = tid * 16;
         float p[16], c[16];
@@ -431,7 +471,7 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
         for (int j = 0; j < 16; j++)
             if (j0 + j == keep - 1) last = c[j];
         const float kept = __shfl(last, (keep - 1) >> 4, 64);
-        const float r = uniforms[blockIdx.x] * kept;
+        const float r = draw_of(draws, blockIdx.x) * kept;
         // the walk: the first candidate whose cumulative mass exceeds r; none (rounding at the end): the first candidate
         int hit = keep;
 #pragma unroll
@@ -448,7 +488,7 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
 // row; thread t owns a contiguous range of ids, so sums run over ids in order within a thread, then over the threads
 // in order. ----------------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024)
-sample_full_k(const float* __restrict__ logits, int V, float temperature, const float* __restrict__ uniforms,
+sample_full_k(const float* __restrict__ logits, int V, float temperature, Draws draws,
               int* __restrict__ out) {
     __shared__ float part[1024];
     __shared__ float s_total;
@@ -478,7 +518,7 @@ sample_full_k(const float* __restrict__ logits, int V, float temperature, const 
         if (tid == 63) s_total = incl;
     }
     __syncthreads();
-    const float r = uniforms[blockIdx.x] * s_total;
+    const float r = draw_of(draws, blockIdx.x) * s_total;
     const float before = part[tid];
     // the first thread whose range reaches past r walks it; rounding may leave r past every range: the last one
     if (tid == 0) s_winner = (V - 1) / chunk;
@@ -505,7 +545,8 @@ sample_full_k(const float* __restrict__ logits, int V, float temperature, const 
 // Three launches: the histogram, the candidates (every block finds the bin from its row's histogram by itself), the sampler,
 // which also puts the histogram and the count back to zero.  A block asks for all of its logits together.
 // (8 rows of 256,000, top_k 256, microseconds: histogram 5.9, candidates 10.2; 8.7, 10.6 and 5.5 for the bin in a launch of its own while a thread
-// asked for its 32 logits one after the other.)
+// asked for its 32 logits one after the other.  Sampler 10.1; 12.8 with the exchanges of its sort as shuffles through LDS, the candidates
+// asked for once their number was known, and a barrier that waited for the zeros of the histogram.)
 constexpr int FILTER_BINS = 4096;
 constexpr int FILTER_PER = 16, FILTER_PART = 256 * FILTER_PER;       // logits per thread and block
 constexpr int FILTER_FROM = 32768;                                   // smaller vocabularies: the sampler alone
@@ -600,8 +641,8 @@ extern "C" long tp_sample_workspace_bytes(int B, int V) {
     return (long)B * (FILTER_BINS * 4 + 4 + (long)CAND_CAP * 8);
 }
 
-extern "C" int tp_sample(const float* logits, int B, int V, float temperature, int top_k, float top_p,
-                         const float* uniforms, int* out, void* workspace, void* stream) {
+static int sample_launch(const float* logits, int B, int V, float temperature, int top_k, float top_p, const Draws& draws, int* out,
+                         void* workspace, void* stream) {
     TP_REQUIRE(B > 0 && V > 0, "sample: empty shape B=%d V=%d", B, V);
     TP_REQUIRE(temperature > 0.f, "sample: temperature %g must be positive (0 means argmax)", temperature);
     TP_REQUIRE(top_k >= 0 && top_k <= 1024, "sample: top_k %d must lie in 0..1024 (0: the whole vocabulary)", top_k);
@@ -610,11 +651,11 @@ extern "C" int tp_sample(const float* logits, int B, int V, float temperature, i
     TP_REQUIRE(B <= 65535, "sample: %d rows exceed one launch", B);
     hipStream_t s = (hipStream_t)stream;
     if (top_k == 0) {
-        sample_full_k<<<B, 1024, 0, s>>>(logits, V, temperature, uniforms, out);
+        sample_full_k<<<B, 1024, 0, s>>>(logits, V, temperature, draws, out);
         return tp_check_launch("sample (whole vocabulary)");
     }
     if (!workspace || tp_sample_workspace_bytes(B, V) == 0) {
-        sample_k<<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, uniforms, out, nullptr, nullptr, nullptr, 0, nullptr, 0);
+        sample_k<<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, draws, out, nullptr, nullptr, nullptr, 0, nullptr, 0);
         return tp_check_launch("sample");
     }
     unsigned* hist = (unsigned*)workspace;
@@ -626,6 +667,24 @@ extern "C" int tp_sample(const float* logits, int B, int V, float temperature, i
     if (int rc = tp_check_launch("sample (histogram)")) return rc;
     filter_collect_k<<<grid, 256, 0, s>>>(logits, V, hist, top_k < V ? top_k : V, count, cand_val, cand_id, CAND_CAP);
     if (int rc = tp_check_launch("sample (candidates)")) return rc;
-    sample_k<<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, uniforms, out, count, cand_val, cand_id, CAND_CAP, hist, FILTER_BINS);
+    sample_k<<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, draws, out, count, cand_val, cand_id, CAND_CAP, hist, FILTER_BINS);
     return tp_check_launch("sample");
+}
+
+// uniforms: a float32 number per row, on the device
+extern "C" int tp_sample(const float* logits, int B, int V, float temperature, int top_k, float top_p,
+                         const float* uniforms, int* out, void* workspace, void* stream) {
+    TP_REQUIRE(uniforms, "sample: no uniform numbers");
+    Draws draws{};
+    draws.at = uniforms;
+    return sample_launch(logits, B, V, temperature, top_k, top_p, draws, out, workspace, stream);
+}
+
+// the same with the numbers in host memory, read before the call returns
+extern "C" int tp_sample_host_uniforms(const float* logits, int B, int V, float temperature, int top_k, float top_p,
+                                       const float* uniforms, int* out, void* workspace, void* stream) {
+    TP_REQUIRE(uniforms && B <= TP_HOST_UNIFORMS, "sample: uniform numbers for %d rows (at most %d come from the host)", B, TP_HOST_UNIFORMS);
+    Draws draws{};
+    for (int i = 0; i < B; i++) draws.v[i] = uniforms[i];
+    return sample_launch(logits, B, V, temperature, top_k, top_p, draws, out, workspace, stream);
 }

@@ -67,6 +67,7 @@ _CORE_SIGS = {
     "tp_recent_push": [_P, _P, _P, _I, _I, _P],
     "tp_add_bias": [_P, _I, _P, _I, _I, _P],
     "tp_sample": [_P, _I, _I, _F, _I, _F, _P, _P, _P, _P],
+    "tp_sample_host_uniforms": [_P, _I, _I, _F, _I, _F, _P, _P, _P, _P],
     "tp_sample_workspace_bytes": [_I, _I],
     "tp_probe_stream": [_P, _L, _P, _I, _P],
     "tp_probe_mfma": [_I, _I, _I, _P, _P, _P],
@@ -1455,12 +1456,23 @@ class HipOps:
         self._call(self.lib, "tp_recent_push", tokens.data_ptr(), recent.data_ptr(), cursor.data_ptr(), n, recent.shape[1],
                    self._stream())
 
+    HOST_UNIFORMS = 64             # rows whose uniform numbers `sample` takes as a sequence of floats (the kernel library's)
+
     def sample(self, logits, temperature, top_k, top_p, uniforms, out=None):
-        self._dev(logits, uniforms)
+        """A token per row, int32 (into `out` if given).  uniforms: float32 [rows] on the device, or for up to HOST_UNIFORMS rows a
+        list of floats, which goes along with the launch."""
+        host = isinstance(uniforms, list)
+        self._dev(logits, *(() if host else (uniforms,)))
         if logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_contiguous():
             raise KernelError("sample: logits must be contiguous float32 [rows, vocab]")
-        if uniforms.dtype != torch.float32 or uniforms.numel() != logits.shape[0] or not uniforms.is_contiguous():
-            raise KernelError("sample: one float32 uniform number per row")
+        if host:
+            if len(uniforms) != logits.shape[0] or len(uniforms) > self.HOST_UNIFORMS:
+                raise KernelError(f"sample: one uniform number per row, of at most {self.HOST_UNIFORMS} rows")
+            entry, draws = "tp_sample_host_uniforms", (_F * len(uniforms))(*uniforms)
+        else:
+            if uniforms.dtype != torch.float32 or uniforms.numel() != logits.shape[0] or not uniforms.is_contiguous():
+                raise KernelError("sample: one float32 uniform number per row")
+            entry, draws = "tp_sample", uniforms.data_ptr()
         if out is None:
             out = torch.empty(logits.shape[0], dtype=torch.int32, device=self.device)
         else:
@@ -1473,8 +1485,8 @@ class HipOps:
             nbytes = self.lib.tp_sample_workspace_bytes(shape[0], shape[1])
             self._sample_ws[shape] = torch.zeros(nbytes, dtype=torch.uint8, device=self.device) if nbytes else None
         ws = self._sample_ws[shape]
-        self._call(self.lib, "tp_sample", logits.data_ptr(), shape[0], shape[1], float(temperature),
-                   int(top_k), float(top_p), uniforms.data_ptr(), out.data_ptr(), ws.data_ptr() if ws is not None else None,
+        self._call(self.lib, entry, logits.data_ptr(), shape[0], shape[1], float(temperature),
+                   int(top_k), float(top_p), draws, out.data_ptr(), ws.data_ptr() if ws is not None else None,
                    self._stream())
         return out
 

@@ -114,8 +114,9 @@ class Sampler:
             ops.apply_repetition_penalty(logits, self.rt.upload_i32(recent), p.repetition_penalty)
         if p.temperature <= 0:
             return ops.argmax(logits)
-        u = np.asarray([r.next_uniform() for r in requests], dtype=np.float32)
-        uniforms = self.rt.upload_i32(u.view(np.int32)).view(torch.float32)
+        uniforms = [r.next_uniform() for r in requests]
+        if len(uniforms) > getattr(ops, "HOST_UNIFORMS", 0):              # more than go along with the launch (or kernels that take none)
+            uniforms = self.rt.upload_i32(np.asarray(uniforms, dtype=np.float32).view(np.int32)).view(torch.float32)
         return ops.sample(logits, p.temperature, p.top_k, p.top_p, uniforms)
 
     @staticmethod
