@@ -118,10 +118,11 @@ gemm_wide_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __
     const int steps = (k_end - k_begin) / BK;
 
     // ---- loads: one instruction of a wave brings 8 rows of 128 bytes straight into LDS; lane l's place is (row l / 8, place
-    // l % 8), and the chunk that belongs there is place ^ row.  Rows past the edge of Y read the last row (their products are
-    // not stored).
+    // l % 8), and the chunk that belongs there is place ^ (row / 2) % 8: the 16 rows of 128 bytes that a fragment read takes at a time
+    // then lie on all banks (place ^ row % 8 has two on each: 9B at 8,191 rows, gate/up 1,358 / 1,345 us, down 730 / 721).  Rows past
+    // the edge of Y read the last row (their products are not stored).
     unsigned xo[LX], wo[LW];
-    const unsigned chunk = (unsigned)((lane & 7) ^ (lane >> 3)) * 16u;
+    const unsigned chunk = (unsigned)((lane & 7) ^ ((wave & 1) * 4 + (lane >> 4))) * 16u;
 #pragma unroll
     for (int i = 0; i < LX; i++) xo[i] = (unsigned)min(m0 + i * 64 + wave * 8 + (lane >> 3), M - 1) * (unsigned)K * 2u + chunk;
 #pragma unroll
@@ -136,7 +137,7 @@ gemm_wide_k(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __
     // ---- fragments: row l % 32 of 32 rows, k chunk 2 s + l / 32 of the step; in the order they are used
     int at[KSUB];
 #pragma unroll
-    for (int s = 0; s < KSUB; s++) at[s] = l32 * 128 + (((2 * s + hi) ^ (l32 & 7)) << 4);
+    for (int s = 0; s < KSUB; s++) at[s] = l32 * 128 + (((2 * s + hi) ^ ((l32 >> 1) & 7)) << 4);
     WdFrag fa[2][MT], fb[2][NT];
     auto read = [&](unsigned px, unsigned pw, int s, int i) {
         const bool w = i == 0 || (i >= 2 && i <= NT);
