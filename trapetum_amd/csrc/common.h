@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <type_traits>
 
 typedef uint16_t bf16_t;   // raw bfloat16 bits
 
@@ -35,39 +36,46 @@ __device__ __forceinline__ void st_f32(float* p, float v) { *p = v; }
 __device__ __forceinline__ void st_f32(bf16_t* p, float v) { *p = f32_to_bf16(v); }
 
 // ---- device: reductions over a wave of 64 and over a block -------------------------------------
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// Butterflies over the lanes, 32 apart first, 1 apart last, in every lane the same: halves and rows of 16 by the swapping lane
+// moves, then within a row by moves that turn it (once lanes 8 apart agree, 4 on is as good as 4 across).  Six shuffles through
+// LDS, each a wait of some hundred cycles, gave the same bits; with them, a division by `groups` ahead of the loads and loops over
+// the block's waves, the two norms of a layer cost a decode step 1.7 us more (2B, chats of 8: 67.7 / 66.2 ms for 32 tokens, of one 55.5 / 53.3).
+template <typename OP>
+__device__ __forceinline__ float wave_butterfly(float v, OP op) {
+    auto turned = [&](auto dpp) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(dpp)::value, 0xf, 0xf, true)); };
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    v = op(v, turned(std::integral_constant<int, 0x128>()));        // row turned by 8
+    v = op(v, turned(std::integral_constant<int, 0x124>()));        // by 4
+    v = op(v, turned(std::integral_constant<int, 0x4e>()));         // quads 2 3 0 1
+    return op(v, turned(std::integral_constant<int, 0xb1>()));      // quads 1 0 3 2
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return wave_butterfly(v, [](float a, float b) { return a + b; }); }
+__device__ __forceinline__ float wave_max(float v) { return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); }); }
 
-// Sum over a block of up to 1024 threads; every thread gets the result.  `red` holds 16 floats of LDS.
-// The order of additions depends only on the block size, never on timing.
+// Sum over a block of up to 1024 threads (THREADS of them, where that is known); every thread gets the result.  `red` holds 16
+// floats of LDS.  The order of additions depends only on the block size, never on timing.
+template <int THREADS = 0>
+__device__ __forceinline__ float block_sum_once(float v, float* red) {     // `red` has not been used by the block before
+    v = wave_sum(v);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    float t = 0.f;
+    if constexpr (THREADS > 0) {
+#pragma unroll
+        for (int i = 0; i < (THREADS + 63) / 64; i++) t += red[i];
+    } else {
+        for (int i = 0; i < (int)((blockDim.x + 63) >> 6); i++) t += red[i];
+    }
+    return t;
+}
+template <int THREADS = 0>
 __device__ __forceinline__ float block_sum(float v, float* red) {
-    v = wave_sum(v);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = (blockDim.x + 63) >> 6;
     __syncthreads();                       // red may still be read from an earlier call
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < nw; i++) t += red[i];
-    return t;
-}
-
-// The same where `red` has not been used by the block before (a call's own 16 floats): one barrier less.
-__device__ __forceinline__ float block_sum_once(float v, float* red) {
-    v = wave_sum(v);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = (blockDim.x + 63) >> 6;
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < nw; i++) t += red[i];
-    return t;
+    return block_sum_once<THREADS>(v, red);
 }
 
 // ---- device: functions of the model ---------------------------------------------------------------

@@ -34,12 +34,16 @@ extern "C" int tp_embed_rows(const int* tokens, const void* table, int dtype, fl
 // times as many, part g of a row taking the g-th stretch of the gain: a block's row is blockIdx.x, its stretch
 // blockIdx.x % groups, and D is the part's length.
 // x_stride: elements from one row of x to the next (a view of wider rows; the output is contiguous).
+// (no division ahead of the loads where there is one part)
+__device__ __forceinline__ int part_of(int groups) { return groups > 1 ? (int)(blockIdx.x % (unsigned)groups) : 0; }
+__device__ __forceinline__ int row_of(int groups) { return groups > 1 ? (int)(blockIdx.x / (unsigned)groups) : (int)blockIdx.x; }
+
 template <typename TI, typename TO>
 __global__ void rms_norm_k(const TI* __restrict__ x, long x_stride, const float* __restrict__ gain, float eps,
                            TO* __restrict__ out, int D, int groups) {
     __shared__ float red[16];
-    gain += (size_t)(blockIdx.x % groups) * D;
-    const TI* xr = x + (size_t)(blockIdx.x / groups) * x_stride + (size_t)(blockIdx.x % groups) * D;
+    gain += (size_t)part_of(groups) * D;
+    const TI* xr = x + (size_t)row_of(groups) * x_stride + (size_t)part_of(groups) * D;
     TO* orow = out + (size_t)blockIdx.x * D;
     float ss = 0.f;
     for (int i = threadIdx.x; i < D; i += blockDim.x) { float v = ld_f32(xr + i); ss += v * v; }
@@ -53,8 +57,8 @@ template <typename TI, typename TO, int EPT, int NTH>
 __global__ void __launch_bounds__(NTH)
 rms_norm_reg_k(const TI* __restrict__ x, long x_stride, const float* __restrict__ gain, float eps, TO* __restrict__ out, int D, int groups) {
     __shared__ float red[16];
-    gain += (size_t)(blockIdx.x % groups) * D;
-    const TI* xr = x + (size_t)(blockIdx.x / groups) * x_stride + (size_t)(blockIdx.x % groups) * D;
+    gain += (size_t)part_of(groups) * D;
+    const TI* xr = x + (size_t)row_of(groups) * x_stride + (size_t)part_of(groups) * D;
     TO* orow = out + (size_t)blockIdx.x * D;
     float v[EPT], gn[EPT];
     float ss = 0.f;
@@ -66,7 +70,7 @@ rms_norm_reg_k(const TI* __restrict__ x, long x_stride, const float* __restrict_
     }
 #pragma unroll
     for (int j = 0; j < EPT; j++) ss += v[j] * v[j];
-    ss = block_sum(ss, red);
+    ss = block_sum<NTH>(ss, red);
     const float scale = rsqrtf(ss / (float)D + eps);
 #pragma unroll
     for (int j = 0; j < EPT; j++) {
@@ -108,8 +112,8 @@ __global__ void add_rms_norm_k(float* __restrict__ stream, const T* __restrict__
                                const float* __restrict__ gain_next, float eps_next,
                                T* __restrict__ out, int D, int groups) {
     __shared__ float red[16];
-    if (gain_post) gain_post += (size_t)(blockIdx.x % groups) * D;
-    if (gain_next) gain_next += (size_t)(blockIdx.x % groups) * D;
+    if (gain_post) gain_post += (size_t)part_of(groups) * D;
+    if (gain_next) gain_next += (size_t)part_of(groups) * D;
     float* sr = stream + (size_t)blockIdx.x * D;
     const T* ar = rows + (size_t)blockIdx.x * D;
     float scale_a = 1.f;
@@ -142,8 +146,8 @@ add_rms_norm_reg_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
                    const float* __restrict__ gain_post, float eps_post,
                    const float* __restrict__ gain_next, float eps_next, T* __restrict__ out, int D, int groups) {
     __shared__ float red[16];
-    if (gain_post) gain_post += (size_t)(blockIdx.x % groups) * D;
-    if (gain_next) gain_next += (size_t)(blockIdx.x % groups) * D;
+    if (gain_post) gain_post += (size_t)part_of(groups) * D;
+    if (gain_next) gain_next += (size_t)part_of(groups) * D;
     float* sr = stream + (size_t)blockIdx.x * D;
     const TR* ar = rows + (size_t)blockIdx.x * D;
     float a[EPT], v[EPT], gp[EPT], gn[EPT];
@@ -175,7 +179,7 @@ add_rms_norm_reg_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
         float ss = 0.f;
 #pragma unroll
         for (int j = 0; j < EPT; j++) ss += a[j] * a[j];
-        ss = block_sum(ss, red);
+        ss = block_sum<NTH>(ss, red);
         scale_a = rsqrtf(ss / (float)D + eps_post);
     }
     float ss2 = 0.f;
@@ -188,7 +192,7 @@ add_rms_norm_reg_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
         if (i < D) { sr[i] = v[j]; ss2 += v[j] * v[j]; }
     }
     if (!gain_next) return;
-    ss2 = block_sum(ss2, red);
+    ss2 = block_sum<NTH>(ss2, red);
     const float scale_s = rsqrtf(ss2 / (float)D + eps_next);
     T* orow = out + (size_t)blockIdx.x * D;
 #pragma unroll
@@ -225,8 +229,8 @@ add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
                    const float* __restrict__ gain_post, float eps_post,
                    const float* __restrict__ gain_next, float eps_next, T* __restrict__ out, int D, int groups) {
     __shared__ float red[16], red_next[16];             // one for each of the two sums: no barrier between their uses
-    if (gain_post) gain_post += (size_t)(blockIdx.x % groups) * D;
-    if (gain_next) gain_next += (size_t)(blockIdx.x % groups) * D;
+    if (gain_post) gain_post += (size_t)part_of(groups) * D;
+    if (gain_next) gain_next += (size_t)part_of(groups) * D;
     float* sr = stream + (size_t)blockIdx.x * D;
     const TR* ar = rows + (size_t)blockIdx.x * D;
     float a[CPT][4], v[CPT][4], gp[CPT][4], gn[CPT][4];
@@ -270,7 +274,7 @@ add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
         for (int j = 0; j < CPT; j++)
 #pragma unroll
             for (int e = 0; e < 4; e++) ss += a[j][e] * a[j][e];
-        ss = block_sum_once(ss, red);
+        ss = block_sum_once<NTH>(ss, red);
         scale_a = rsqrtf(ss / (float)D + eps_post);
     }
     float ss2 = 0.f;
@@ -287,7 +291,7 @@ add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
         if (i < D) st4(sr + i, v[j]);
     }
     if (!gain_next) return;
-    ss2 = block_sum_once(ss2, red_next);
+    ss2 = block_sum_once<NTH>(ss2, red_next);
     const float scale_s = rsqrtf(ss2 / (float)D + eps_next);
     T* orow = out + (size_t)blockIdx.x * D;
 #pragma unroll
@@ -469,7 +473,7 @@ join_rms_norm_k(JoinArgs x) {
         }
     }
     if (!x.gain) return;
-    ss = block_sum_once(ss, red);
+    ss = block_sum_once<NTH>(ss, red);
     const float scale = rsqrtf(ss / (float)D + x.eps);
     T* orow = (T*)x.out + row;
 #pragma unroll

@@ -138,7 +138,7 @@ long_norm_gate_k(const float* __restrict__ y, const float* __restrict__ gain, co
         gq[j] = *reinterpret_cast<const G4*>(gr + dc);
         if (d < hs) ss += a[j].x * a[j].x + a[j].y * a[j].y + a[j].z * a[j].z + a[j].w * a[j].w;
     }
-    const float inv = rsqrtf(block_sum_once(ss, red) / (float)hs + eps);
+    const float inv = rsqrtf(block_sum_once<256>(ss, red) / (float)hs + eps);
 #pragma unroll
     for (int j = 0; j < Q; j++) {
         const int d = (tid + 256 * j) * 4;
