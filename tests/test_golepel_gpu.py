@@ -9,6 +9,7 @@ from trapetum_amd.engine.runtime import Runtime
 from trapetum_amd.registry import build_part
 
 from . import golepel_tiny as gt
+from . import ref_ops
 from .plain import golepel_plain as plain
 from .tiny import random_tokens, rel_l2
 
@@ -143,6 +144,34 @@ def test_latent_attention_part(rt, H, dn, dr, dv, R, rot):
     assert at == n
     assert rel_l2(torch.cat(got), want) < tol
     assert rel_l2(torch.cat(got2), want2) < tol
+
+
+@pytest.mark.parametrize("m,H,dn,dr,R,rot,tailed", [
+    (1, 1, 3, 0, 9, 0, False), (7, 2, 5, 6, 33, 4, True), (5, 16, 8, 64, 192, 64, True),      # a head a thread: no turning part, pairs and elements that pass
+    (3, 2, 8, 520, 1025, 24, False),                 # more elements than threads in a head, a latent longer than a thread keeps
+    (300, 31, 2, 48, 1100, 48, True), (300, 30, 2, 96, 40, 32, False)])                       # four heads a thread, with remainders
+def test_latent_prepare(rt, m, H, dn, dr, R, rot, tailed):
+    """Each element is at most three roundings in float32 and one to the activations' type away."""
+    ops, row = rt.ops, dr + R
+    proj, _ = acts(rt, rnd(m, H * (dr + dn) + (0 if tailed else row), seed=1))
+    tail = acts(rt, rnd(m, row + 5, seed=2))[0][:, :row] if tailed else None
+    gain, inv_freq = rnd(R, seed=3).to(DEV), (rnd(rot // 2, seed=4).abs() * 0.1).to(DEV) if rot else None
+    seq = torch.tensor([i % 2 for i in range(m)], dtype=torch.int32, device=DEV)
+    pos = torch.tensor([3 + i // 2 for i in range(m)], dtype=torch.int32, device=DEV)
+    new_len = torch.tensor([3 + (m + 1) // 2, 3 + m // 2], dtype=torch.int32, device=DEV)
+    for cap in (0, 32):
+        table = torch.arange(2 * 20, dtype=torch.int32, device=DEV).flip(0).reshape(2, 20)
+        pool = torch.zeros((40, 1, 16, row), dtype=rt.dtype, device=DEV)
+        want_pool = pool.clone()
+        args = (proj, H, dn, dr, R, gain, 1e-5, inv_freq, rot, seq, pos, new_len, table)
+        q, mine = ops.latent_prepare(*args, pool, cap, own=True, out_dtype=rt.dtype, tail=tail)
+        want_q, want_mine = ref_ops.latent_prepare(*args, want_pool, cap, own=True, tail=tail)
+        atol = 1e-5 if rt.dtype == torch.float32 else 2 ** -7
+        for got, want in ((q.view(m, H, row)[..., :dr], want_q.view(m, H, row)[..., :dr]), (mine, want_mine), (pool, want_pool)):
+            assert bool(((got.double() - want.double()).abs() <= atol * want.double().abs().clamp(min=1.0)).all()), cap
+    if not tailed:
+        q2, none = ops.latent_prepare(proj[:, :H * (dr + dn)], *args[1:5], None, *args[6:], pool, 0, own=False, out_dtype=rt.dtype)
+        assert none is None and torch.equal(q2.view(m, H, row)[..., :dr], q.view(m, H, row)[..., :dr])
 
 
 def test_latent_attention_long_context(rt):

@@ -8,65 +8,102 @@
 // proj row: H heads of [dr rotated | dn unrotated] query elements, then (own) [dr key part | R latent].
 // q row: H heads of [dr | R]; this kernel fills the first dr of each (the rest is a product's output).
 // The first `rot` of the dr elements turn in pairs (f, f + rot / 2) by pos * inv_freq[f]; the others pass.
-// grid (rows); dynamic LDS: rot floats (cosines, sines).
-template <typename T>
+// grid (rows, [the latent] + heads by HPT * at_once).  All of it is waiting: the position, then what is read, then what is
+// stored.  So a row is shared out: one block for the latent's norm, the others for the heads (the key part counts as one more),
+// each thread keeping its pair f (its angle is its own, no table and no barrier) for HPT heads whose elements are asked for
+// before the angle is worked out.  A block for the whole row, its angles in a table in LDS, took (bf16; 16 heads, 64 turning,
+// latent of 192: rows 8 / 128 / 1300 / 4096) 5.2 / 5.3 / 8.0 / 17.8 us, this 2.9 / 3.1 / 7.6 / 17.3; with 128 heads and a latent
+// of 512 15.5 / 16.0 / 36.9 / 81.3 us, this 3.1 / 4.1 / 18.7 / 52.0.
+template <typename T, int HPT>
 __global__ void __launch_bounds__(256)
 latent_prepare_k(const T* __restrict__ proj, long proj_stride, int H, int dn, int dr, int R,
                  const float* __restrict__ gain, float eps, const float* __restrict__ inv_freq, int rot,
                  const int* __restrict__ row_seq, const int* __restrict__ row_pos, const int* __restrict__ new_len,
                  const int* __restrict__ table, int table_w, T* __restrict__ pool, int page, int rows_cap,
-                 T* __restrict__ q, T* __restrict__ mine, int own, const T* __restrict__ tail_rows, long tail_stride) {
-    extern __shared__ float cs[];                        // [rot / 2] cosines, [rot / 2] sines
-    __shared__ float red[16];
-    const int r = blockIdx.x, pos = row_pos[r], half = rot / 2, row = dr + R;
-    for (int f = threadIdx.x; f < half; f += blockDim.x) {
-        const float ang = (float)pos * inv_freq[f];
-        cs[f] = cosf(ang);
-        cs[half + f] = sinf(ang);
-    }
-    __syncthreads();
+                 T* __restrict__ q, T* __restrict__ mine, int own, const T* __restrict__ tail_rows, long tail_stride,
+                 int per_head, int at_once) {
+    __shared__ float red[4];
+    const int r = blockIdx.x, pos = row_pos[r], half = rot / 2, row = dr + R, tid = threadIdx.x;
     const T* pr = proj + (size_t)r * proj_stride;
-    T* qr = q + (size_t)r * H * row;
-    for (int item = threadIdx.x; item < H * dr; item += blockDim.x) {
-        const int h = item / dr, e = item - h * dr;
-        const T* src = pr + (size_t)h * (dr + dn);
-        float y;
-        if (e < half) y = ld_f32(src + e) * cs[e] - ld_f32(src + e + half) * cs[half + e];
-        else if (e < rot) y = ld_f32(src + e) * cs[e - half] + ld_f32(src + e - half) * cs[e];
-        else y = ld_f32(src + e);
-        st_f32(qr + (size_t)h * row + e, y);
-    }
-    if (!own) return;
     const T* tail = tail_rows ? tail_rows + (size_t)r * tail_stride : pr + (size_t)H * (dr + dn);     // a product of its own, or the row's end
+    const int h_block = ((int)blockIdx.y - own) * at_once * HPT;          // below 0: the latent
+    T* mr = nullptr;
     T* dst = nullptr;                                    // the row's place in the cache
-    if (table) {
-        const int seq = row_seq[r];
-        int at = pos;
-        bool keep = true;
-        if (rows_cap > 0) {
-            keep = pos + rows_cap >= new_len[seq];       // else a later row of this step takes the same ring row
-            at = pos % rows_cap;
+    if (own && (h_block < 0 || h_block + at_once * HPT > H)) {
+        mr = mine + (size_t)r * row;
+        if (table) {
+            const int seq = row_seq[r];
+            int at = pos;
+            bool keep = true;
+            if (rows_cap > 0) {
+                keep = pos + rows_cap >= new_len[seq];   // else a later row of this step takes the same ring row
+                at = pos % rows_cap;
+            }
+            const int pg = keep && at / page < table_w ? table[(size_t)seq * table_w + at / page] : -1;     // a table too narrow for the position caches nothing
+            if (pg >= 0) dst = pool + ((size_t)pg * page + at % page) * row;
         }
-        const int pg = keep && at / page < table_w ? table[(size_t)seq * table_w + at / page] : -1;     // a table too narrow for the position caches nothing
-        if (pg >= 0) dst = pool + ((size_t)pg * page + at % page) * row;
     }
-    T* mr = mine + (size_t)r * row;
-    for (int e = threadIdx.x; e < dr; e += blockDim.x) {
-        float y;
-        if (e < half) y = ld_f32(tail + e) * cs[e] - ld_f32(tail + e + half) * cs[half + e];
-        else if (e < rot) y = ld_f32(tail + e) * cs[e - half] + ld_f32(tail + e - half) * cs[e];
-        else y = ld_f32(tail + e);
-        st_f32(mr + e, y);
-        if (dst) st_f32(dst + e, y);
+    if (h_block < 0) {
+        constexpr int NR = 4;                            // elements a thread keeps; a longer latent is read again
+        float v[NR], w[NR], ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            const int e = tid + i * 256;
+            v[i] = e < R ? ld_f32(tail + dr + e) : 0.f;
+            w[i] = e < R ? gain[e] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < NR; i++) ss += v[i] * v[i];
+        for (int e = tid + NR * 256; e < R; e += 256) { const float x = ld_f32(tail + dr + e); ss += x * x; }
+        ss = block_sum_once<256>(ss, red);
+        const float scale = rsqrtf(ss / (float)R + eps);
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            const int e = tid + i * 256;
+            if (e >= R) continue;
+            const float y = (v[i] * scale) * w[i];
+            st_f32(mr + dr + e, y);
+            if (dst) st_f32(dst + dr + e, y);
+        }
+        for (int e = tid + NR * 256; e < R; e += 256) {
+            const float y = (ld_f32(tail + dr + e) * scale) * gain[e];
+            st_f32(mr + dr + e, y);
+            if (dst) st_f32(dst + dr + e, y);
+        }
+        return;
     }
-    float ss = 0.f;
-    for (int e = threadIdx.x; e < R; e += blockDim.x) { const float v = ld_f32(tail + dr + e); ss += v * v; }
-    ss = block_sum(ss, red);
-    const float scale = rsqrtf(ss / (float)R + eps);
-    for (int e = threadIdx.x; e < R; e += blockDim.x) {
-        const float y = (ld_f32(tail + dr + e) * scale) * gain[e];
-        st_f32(mr + dr + e, y);
-        if (dst) st_f32(dst + dr + e, y);
+    const int heads = H + own;
+    const int h0 = h_block + tid / per_head;             // per_head: threads a head takes (its pairs and its elements that pass, at most 256)
+    if (h0 >= h_block + at_once) return;
+    for (int f = tid % per_head; f < dr - half; f += per_head) {
+        const int lo = f < half ? f : f + half, hi = f + half;            // a pair, or twice an element that passes
+        float a[HPT], b[HPT];
+#pragma unroll
+        for (int i = 0; i < HPT; i++) {
+            const int h = min(h0 + i * at_once, heads - 1);
+            const T* src = h < H ? pr + (size_t)h * (dr + dn) : tail;
+            a[i] = ld_f32(src + lo);
+            b[i] = ld_f32(src + hi);
+        }
+        float co = 1.f, si = 0.f;
+        if (f < half) {
+            const float ang = (float)pos * inv_freq[f];
+            co = cosf(ang);
+            si = sinf(ang);
+        }
+#pragma unroll
+        for (int i = 0; i < HPT; i++) {
+            const int h = h0 + i * at_once;
+            if (h >= heads) continue;
+            const float x = f < half ? a[i] * co - b[i] * si : a[i], y = f < half ? b[i] * co + a[i] * si : b[i];
+            T* o = h < H ? q + ((size_t)r * H + h) * row : mr;
+            st_f32(o + lo, x);
+            if (f < half) st_f32(o + hi, y);
+            if (h == H && dst) {
+                st_f32(dst + lo, x);
+                if (f < half) st_f32(dst + hi, y);
+            }
+        }
     }
 }
 
@@ -85,16 +122,24 @@ extern "C" int tp_latent_prepare(const void* proj, long proj_stride, int dtype, 
     TP_REQUIRE(!table || (pool && page > 0 && table_w > 0), "latent_prepare: a page table without a cache pool");
     if (!table) { page = 1; rows_cap = 0; }
     TP_REQUIRE(rows_cap >= 0 && (rows_cap == 0 || rows_cap % page == 0), "latent_prepare: ring of %d rows is no multiple of the page size %d", rows_cap, page);
-    TP_REQUIRE(rot * sizeof(float) <= 32768, "latent_prepare: %d turning elements exceed the kernel's table", rot);
+    TP_REQUIRE(rot * sizeof(float) <= 32768, "latent_prepare: %d turning elements are more than a head may have", rot);
     hipStream_t s = (hipStream_t)stream;
-    const size_t lds = (size_t)rot * sizeof(float);
-    if (dtype == TP_BF16)
-        latent_prepare_k<bf16_t><<<M, 256, lds, s>>>((const bf16_t*)proj, proj_stride, H, dn, dr, R, gain, eps, inv_freq, rot, row_seq, row_pos,
-            new_len, table, table_w, (bf16_t*)pool, page, rows_cap, (bf16_t*)q, (bf16_t*)mine, own, (const bf16_t*)tail, tail_stride);
-    else if (dtype == TP_F32)
-        latent_prepare_k<float><<<M, 256, lds, s>>>((const float*)proj, proj_stride, H, dn, dr, R, gain, eps, inv_freq, rot, row_seq, row_pos,
-            new_len, table, table_w, (float*)pool, page, rows_cap, (float*)q, (float*)mine, own, (const float*)tail, tail_stride);
+    const int items = dr - rot / 2, per_head = items > 256 ? 256 : items > 0 ? items : 1, at_once = 256 / per_head, heads = items ? H + !!own : 0;
+    // Four heads a thread once that many still fill the chip: one angle then serves four heads.  Below, more blocks with one
+    // head a thread end sooner.  One / four heads a thread, 16 heads:
+    // 8 rows 3.1 / 3.7 us, 256 rows 3.5 / 3.7, 512 rows 4.7 / 4.6, 4096 rows 21.6 / 17.3; 128 heads: 32 rows 3.2 / 3.4, 64 rows
+    // 3.7 / 3.6, 4096 rows 74.3 / 51.5.
+    const bool many = (long)M * heads > 8192;
+    const int per_block = at_once * (many ? 4 : 1), blocks = !!own + tp_cdiv(heads, per_block);
+    if (blocks == 0) return 0;                           // nothing turns and nothing is cached
+    TP_REQUIRE(blocks <= 65535, "latent_prepare: %d heads exceed one launch", H);
+    dim3 grid(M, blocks);
+#define TP_LATENT_PREPARE(T, HPT) latent_prepare_k<T, HPT><<<grid, 256, 0, s>>>((const T*)proj, proj_stride, H, dn, dr, R, gain, eps, inv_freq, rot, row_seq, row_pos, \
+        new_len, table, table_w, (T*)pool, page, rows_cap, (T*)q, (T*)mine, !!own, (const T*)tail, tail_stride, per_head, at_once)
+    if (dtype == TP_BF16) { if (many) TP_LATENT_PREPARE(bf16_t, 4); else TP_LATENT_PREPARE(bf16_t, 1); }
+    else if (dtype == TP_F32) { if (many) TP_LATENT_PREPARE(float, 4); else TP_LATENT_PREPARE(float, 1); }
     else return tp_fail("latent_prepare: unknown dtype %d", dtype);
+#undef TP_LATENT_PREPARE
     return tp_check_launch("latent_prepare");
 }
 
