@@ -409,6 +409,9 @@ def test_linear_group(ops, m, k, ns):
     for got, (x, w, dtype, bias) in zip(ops.linear_group(parts), parts):
         ref = x.cpu().double() @ w.cpu().double().T + (bias.cpu().double() if bias is not None else 0.0)
         assert got.dtype == dtype and rel_l2(got, ref) < (1e-5 if dtype == torch.float32 else 4e-3)
+    turned = range(0, len(ns), 2)                        # through tanh: the bits of the rounded products' own tanh
+    for i, (got, plain) in enumerate(zip(ops.linear_group(parts, tanh=turned), ops.linear_group(parts))):
+        assert torch.equal(got, ops.unary_(plain, "tanh") if i in turned else plain)
     with pytest.raises(Exception, match="linear_group"):
         ops.linear_group(parts + [(parts[0][0], parts[0][1][:, :-1].contiguous(), torch.bfloat16, None)])
     if m <= 8 and k % 8 == 0 and k <= 2304:

@@ -223,6 +223,7 @@ int gemm_rows8_launch(const GemmArgs& a) {
 struct Rows8Group {
     const bf16_t* x[TP_LINEAR_GROUP]; const bf16_t* w[TP_LINEAR_GROUP]; void* y[TP_LINEAR_GROUP]; const float* bias[TP_LINEAR_GROUP];
     int n[TP_LINEAR_GROUP], f32[TP_LINEAR_GROUP], first[TP_LINEAR_GROUP];       // rows of W; a float32 output; its first block
+    unsigned tanh;                                                              // bit p: product p, rounded, goes through tanh and is rounded again
 };
 
 template <int NG, int NS>
@@ -233,9 +234,10 @@ gemm_rows8_group_k(Rows8Group g, int parts, int M, int K) {
     void* Y = g.y[0];
     const float* bias = g.bias[0];
     int N = g.n[0], f32 = g.f32[0], first = 0;
+    unsigned bit = 1;
 #pragma unroll
     for (int p = 1; p < TP_LINEAR_GROUP; p++)
-        if (p < parts && (int)blockIdx.x >= g.first[p]) { X = g.x[p]; W = g.w[p]; Y = g.y[p]; bias = g.bias[p]; N = g.n[p]; f32 = g.f32[p]; first = g.first[p]; }
+        if (p < parts && (int)blockIdx.x >= g.first[p]) { X = g.x[p]; W = g.w[p]; Y = g.y[p]; bias = g.bias[p]; N = g.n[p]; f32 = g.f32[p]; first = g.first[p]; bit = 1u << p; }
     const int row0 = (blockIdx.x - first) * NG * 8;
     const bf16_t* wrow[NG];
 #pragma unroll
@@ -247,19 +249,22 @@ gemm_rows8_group_k(Rows8Group g, int parts, int M, int K) {
     for (int t = 0; t < NG; t++) {
         const int n = row0 + 8 * t + wr;
         if (n >= N) continue;
-        const float o = bias ? v[t] + bias[n] : v[t];
+        float o = bias ? v[t] + bias[n] : v[t];
+        if (g.tanh & bit) o = tanhf(f32 ? o : bf16_to_f32(f32_to_bf16(o)));
         if (f32) ((float*)Y)[(size_t)m * N + n] = o;
         else ((bf16_t*)Y)[(size_t)m * N + n] = f32_to_bf16(o);
     }
 }
 
 // y[p] [M, n[p]] = x[p] [M, K] . w[p] [n[p], K]^T (+ bias[p]), `parts` of them (up to TP_LINEAR_GROUP), bf16 rows and matrices, up to 8 rows,
-// a K that a block reads in one round.
+// a K that a block reads in one round.  Bit p of `tanh`: y[p] is tanh of the rounded product, as a launch of its own would leave it
+// (that launch took 4.5 us of a decode step's time mix).
 extern "C" int tp_linear_group(const void* const* x, const void* const* w, void* const* y, const float* const* bias, const int* n, const int* out_dtype,
-                               int parts, int M, int K, void* stream) {
+                               int tanh, int parts, int M, int K, void* stream) {
     TP_REQUIRE(parts > 0 && parts <= TP_LINEAR_GROUP, "linear group: %d products (at most %d)", parts, TP_LINEAR_GROUP);
     TP_REQUIRE(M > 0 && M <= 8 && K > 0 && K % 8 == 0 && K <= R8_MAX_STEPS * 256, "linear group: needs at most 8 rows and a K that is a multiple of 8 up to %d (M=%d K=%d)", R8_MAX_STEPS * 256, M, K);
     Rows8Group g{};
+    g.tanh = (unsigned)tanh;
     long tiles = 0;
     for (int p = 0; p < parts; p++) {
         TP_REQUIRE(x[p] && w[p] && y[p] && n[p] > 0 && (out_dtype[p] == TP_BF16 || out_dtype[p] == TP_F32), "linear group: product %d is empty or of an unknown output dtype", p);

@@ -57,7 +57,7 @@ _CORE_SIGS = {
     "tp_time_mix_scan_workspace_floats": [_I, _I, _I, _I],
     "tp_matrix_memory_scan_workspace_floats": [_I, _I, _I, _I, _I],
     "tp_linear_stream_rows": [_I, _I, _I, _I, _I],
-    "tp_linear_group": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "tp_linear_group": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "tp_linear_workspace_bytes": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
     "tp_attn_simple_prefill": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P],
     "tp_attn_simple_decode": [_P, _L, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _I, _I, _F, _F, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P],
@@ -1141,16 +1141,18 @@ class HipOps:
 
     GROUP_ROWS, GROUP_K, GROUP_PARTS = 8, 2304, 8        # what one launch of `linear_group` takes (the kernel library's)
 
-    def linear_group(self, parts):
+    def linear_group(self, parts, tanh=()):
         """Several products [x @ w^T (+ bias) for x, w, out_dtype, bias in parts] of inputs of one shape; bias: float32 [rows of w] or
-        None.  A few bf16 rows go in one launch, the bias added to the float32 sums; others one after the other (`linear`)."""
+        None.  A few bf16 rows go in one launch, the bias added to the float32 sums; others one after the other (`linear`).
+        tanh: indices of the products that go through tanh, once rounded."""
         m, k = parts[0][0].shape
         if any(x.dim() != 2 or tuple(x.shape) != (m, k) or w.dim() != 2 or w.shape[1] != k for x, w, _, _ in parts):
             raise KernelError("linear_group: rows of one shape and matrices of as many columns")
         one = (m <= self.GROUP_ROWS and k <= self.GROUP_K and k % 8 == 0 and len(parts) <= self.GROUP_PARTS and not self.force_linear and
                all(x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0 for x, w, _, _ in parts))
         if not one:
-            return [self.linear(x, w, out_dtype, bias=bias) for x, w, out_dtype, bias in parts]
+            out = [self.linear(x, w, out_dtype, bias=bias) for x, w, out_dtype, bias in parts]
+            return [self.unary_(y, "tanh") if i in tanh else y for i, y in enumerate(out)]
         for x, w, _, bias in parts:
             self._dev(x, w, bias)
             if bias is not None and (bias.dtype != torch.float32 or bias.numel() != w.shape[0] or not bias.is_contiguous()):
@@ -1160,7 +1162,7 @@ class HipOps:
         pointers = lambda values: (_P * n)(*values)
         self._call(self.lib, "tp_linear_group", pointers(p[0].data_ptr() for p in parts), pointers(p[1].data_ptr() for p in parts),
                    pointers(t.data_ptr() for t in out), pointers(p[3].data_ptr() if p[3] is not None else None for p in parts),
-                   (_I * n)(*(p[1].shape[0] for p in parts)), (_I * n)(*(_code(p[2]) for p in parts)), n, m, k, self._stream())
+                   (_I * n)(*(p[1].shape[0] for p in parts)), (_I * n)(*(_code(p[2]) for p in parts)), sum(1 << i for i in set(tanh)), n, m, k, self._stream())
         return out
 
     def gated_linear(self, x, w_packed, inter, activation, out_dtype, limit=None, up_shift=0.0):

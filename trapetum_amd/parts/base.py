@@ -36,13 +36,14 @@ step (`forward`).  Interfaces:
 """
 
 
-def products(ops, parts):
-    """[x @ w^T (+ bias) for x, w, out_dtype, bias in parts], inputs of one shape: in one launch where the kernels can (a kernel
-    library need not have the entry)."""
+def products(ops, parts, tanh=()):
+    """[x @ w^T (+ bias) for x, w, out_dtype, bias in parts], inputs of one shape, those with an index in `tanh` through tanh: in one
+    launch where the kernels can (a kernel library need not have the entry)."""
     group = getattr(ops, "linear_group", None)
     if group is not None:
-        return group(parts)
-    return [ops.linear(x, w, out_dtype, bias=bias) for x, w, out_dtype, bias in parts]
+        return group(parts, tanh)
+    out = [ops.linear(x, w, out_dtype, bias=bias) for x, w, out_dtype, bias in parts]
+    return [ops.unary_(y, "tanh") if i in tanh else y for i, y in enumerate(out)]
 
 
 class Part:

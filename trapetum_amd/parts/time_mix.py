@@ -69,8 +69,7 @@ class TimeMix(Mixer):
         ops, w = ctx.ops, self.w
         mixes = ops.shift_mix(x, self.mu, self.state(ctx, "shift"), ctx.slot_ids, ctx.cu_rows, ctx.row_seq,
                               one_row_each=ctx.mode == "decode")                                  # [5, M, D]
-        r, k, v, g, low = products(ops, [(mixes[i], w[s], ctx.dtype, None) for i, s in enumerate(("r", "k", "v", "g", "w1"))])
-        low = ops.unary_(low, "tanh")
+        r, k, v, g, low = products(ops, [(mixes[i], w[s], ctx.dtype, None) for i, s in enumerate(("r", "k", "v", "g", "w1"))], tanh=(4,))
         log_rate = ops.linear(low, w["w2"], torch.float32)                                        # w0 is added in the scan
         y = ops.time_mix_scan(r, k, v, log_rate, self.w0, self.bonus, self.state(ctx, "memory"), ctx.slot_ids, ctx.cu_rows,
                               ctx.max_count, self.num_heads, self.head_dim)
