@@ -16,8 +16,9 @@
 //   chunks is a chain of a few hundred multiply-adds and reads a row, took 690 us for prompts of 700, 333, 64 and 1,025 rows, nine
 //   heads, keys of 128 and values of 256; 125 so (43 + 24 + 58).  The two meet at about 12 rows a sequence (4 sequences of 8 rows
 //   31 us row by row, 34 in chunks; of 16 48 and 35; one of 64 149 and 53).
-// Error against 64 bits, prompts of 12 to 1,300 rows, row after row / in chunks: outputs 1.2e-7 to 8.3e-7 / 1.3e-7 to 1.1e-6 (the
-// denominator is a small difference now and then), states 3.2e-8 to 2.2e-7 / 4.3e-8 to 2.1e-7.
+// Error against 64 bits in chunks over that row after row, geometric means over twenty prompts of 12 to 699 rows and gates of three
+// spreads: outputs 0.94 (the median row's 0.81), matrix 0.98, normalizer 0.97; outputs 1.3e-7 to 1.1e-6 (the denominator is a small
+// difference now and then), states 3.5e-8 to 2.8e-7.
 #include "recurrent.h"
 
 struct MatrixMemoryArgs {
@@ -288,8 +289,9 @@ __device__ __forceinline__ void store_quad(float* row, int c, int n, mm_f32x4 x)
         for (int e = 0; e < 4; e++) if (c + e < n) row[c + e] = x[e];
     }
 }
-// (Every sum over more than 16 terms is taken in pieces of 16 from zero: a chain over a whole head, let alone with the rows behind it,
-// loses more than the four waves' parts of the kernel of whole sequences do.)
+// (Every sum over more than 16 terms of one size is taken in pieces of 16 from zero: a chain over a whole head, let alone with the rows
+// behind it, loses more than the four waves' parts of the kernel of whole sequences do.  Rows go in as they follow one another, 4 u + g of
+// 16, and into a state in one chain: where gates forget, the last are the largest, and every sum after them is rounded at their size.)
 __device__ __forceinline__ mm_f32x4 mm_mfma(float a, float b, mm_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // e^x to float32's last place: the library's function of x rounded, corrected by what was rounded off
@@ -350,7 +352,7 @@ mm_chunk_k(MatrixMemoryArgs a) {
     auto fetch = [&](int kb, int to) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            const size_t t = (size_t)begin + min(16 * kb + 4 * g + u, n - 1);
+            const size_t t = (size_t)begin + min(16 * kb + 4 * u + g, n - 1);
             kq[to][u] = quad<VEC>(kh + t * a.k_stride, i0 + 4 * r, dk);
             vq[to][u] = quad<VEC>(vh + t * a.v_stride, j0 + 4 * r, dv);
         }
@@ -362,18 +364,15 @@ mm_chunk_k(MatrixMemoryArgs a) {
         if (kb + 1 < blocks) fetch(kb + 1, (kb + 1) & 1);
         float w[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) w[u] = weights[wave][16 * kb + 4 * g + u];
+        for (int u = 0; u < 4; u++) w[u] = weights[wave][16 * kb + 4 * u + g];
 #pragma unroll
         for (int y = 0; y < 4; y++) {
-            mm_f32x4 p[4] = {};
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const float kw = kq[kb & 1][u][y] * w[u];
 #pragma unroll
-                for (int x = 0; x < 4; x++) p[x] = mm_mfma(vq[kb & 1][u][x], kw, p[x]);
+                for (int x = 0; x < 4; x++) acc[x][y] = mm_mfma(vq[kb & 1][u][x], kw, acc[x][y]);
             }
-#pragma unroll
-            for (int x = 0; x < 4; x++) acc[x][y] += p[x];
         }
     }
     float* const ws = a.ws_state + ((size_t)blockIdx.x * H + h) * ((size_t)dk * dv + dk);
@@ -564,11 +563,13 @@ mm_outputs_k(MatrixMemoryArgs a) {
         if (kb >= tiles) break;
         mm_f32x4 v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = quad<VEC>(vh + (size_t)(begin + min(16 * kb + 4 * g + u, n - 1)) * a.v_stride, j0 + 4 * r, dv);
+        for (int u = 0; u < 4; u++) v[u] = quad<VEC>(vh + (size_t)(begin + min(16 * kb + 4 * u + g, n - 1)) * a.v_stride, j0 + 4 * r, dv);
 #pragma unroll
         for (int tt = kb; tt < 4; tt++) {
             if (tt >= tiles) break;
-            const mm_f32x4 w = *reinterpret_cast<const mm_f32x4*>(&P[16 * tt + r][16 * kb + 4 * g]);
+            float w[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) w[u] = P[16 * tt + r][16 * kb + 4 * u + g];
             mm_f32x4 p[4] = {};
 #pragma unroll
             for (int u = 0; u < 4; u++)
