@@ -294,6 +294,31 @@ def test_scans_of_one_row(rt, heads, dk, dv):
     assert rel_l2(got, want) < 2e-6 and rel_l2(got_state, want_state) < 1e-6 and torch.equal(got_state[[1, 3]].cpu(), state[[1, 3]])
 
 
+# sequences without rows, before the first row, between rows and behind the last: row after row, in chunks, of one row each
+@pytest.mark.parametrize("lens,chunk", [((0, 5, 0, 9, 0), 0), ((0, 33, 0, 130, 0), 32), ((0, 1, 0, 1, 0), 0), ((0, 1, 0, 1, 0), None)])
+@pytest.mark.parametrize("heads,dk,dv", [(2, 20, 36), (1, 128, 64)])
+def test_scans_leave_a_sequence_without_rows_alone(rt, heads, dk, dv, lens, chunk):
+    from . import ref_ops
+    slots, M, most = torch.tensor([3, 0, 5, 2, 1], dtype=torch.int32), sum(lens), max(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    q, k, v = (acts(rt, rnd(M, heads * d, seed=110 + i, scale=0.5))[0] for i, d in enumerate((dk, dk, dv)))
+    gates = rnd(M, 2 * heads, seed=113, scale=2.0)
+    states = [rnd(6, heads, dk, dv, seed=114, scale=0.3), rnd(6, heads, dk, seed=115, scale=0.3), rnd(6, heads, seed=116)]
+    want_states, got_states = [t.double() for t in states], [t.to(rt.device) for t in states]
+    want = ref_ops.matrix_memory_scan(q.cpu(), k.cpu(), v.cpu(), gates, 8.0, dk ** -0.5, *want_states, slots, cu, most, heads, dk, dv)
+    got = rt.ops.matrix_memory_scan(q, k, v, gates.to(rt.device), 8.0, dk ** -0.5, *got_states, slots.to(rt.device), cu.to(rt.device), most, heads, dk, dv, chunk=chunk)
+    assert rel_l2(got, want) < 6e-5                      # the denominator's bound, as above
+    for g, w, s in zip(got_states, want_states, states):
+        assert rel_l2(g, w) < 1e-5 and torch.equal(g[[1, 3, 4, 5]].cpu(), s[[1, 3, 4, 5]])
+    d, inner = dv, heads * dv
+    r, k, v = (acts(rt, rnd(M, inner, seed=120 + i, scale=0.5))[0] for i in range(3))
+    rate, w0, bonus, state = rnd(M, inner, seed=123) - 1.0, rnd(inner, seed=124, scale=0.5), rnd(heads, d, seed=125, scale=0.5), rnd(6, heads, d, d, seed=126, scale=0.3)
+    want_state, got_state = state.double(), state.to(rt.device)
+    want = ref_ops.time_mix_scan(r.cpu(), k.cpu(), v.cpu(), rate, w0, bonus, want_state, slots, cu, most, heads, d)
+    got = rt.ops.time_mix_scan(r, k, v, rate.to(rt.device), w0.to(rt.device), bonus.to(rt.device), got_state, slots.to(rt.device), cu.to(rt.device), most, heads, d, chunk=chunk)
+    assert rel_l2(got, want) < 5e-6 and rel_l2(got_state, want_state) < 5e-6 and torch.equal(got_state[[1, 3, 4, 5]].cpu(), state[[1, 3, 4, 5]])
+
+
 @pytest.mark.parametrize("cut", ["whole", "pieces", "one by one"])
 def test_matrix_memory_keeps_its_first_tokens(rt, cut):
     """Forget gates of sigmoid(8) and small input gates after the first tokens: the memory is what the first tokens wrote,

@@ -115,6 +115,7 @@ matrix_memory_scan_k(MatrixMemoryArgs a) {
     const int dk = a.dk, dv = a.dv, H = a.H;
     const bool col = j < dv;
     const int begin = a.cu_rows[seq], end = a.cu_rows[seq + 1];
+    if (begin >= end) return;                               // no rows: what `fetch` would read past the end may lie before the first row
     const size_t slot = (size_t)a.slot_ids[seq];
     float* st = a.memory + (slot * H + h) * dk * dv;
     float* sn = a.normalizer + (slot * H + h) * dk;

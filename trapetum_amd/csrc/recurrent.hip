@@ -211,9 +211,9 @@ time_mix_scan_k(TimeMixArgs a) {
     const bool col = j < d;
     int begin = a.cu_rows[seq], end = a.cu_rows[seq + 1];
     bool last = true;
+    if (MODE != TP_SCAN_WHOLE) begin += (blockIdx.x % a.n_chunks) * a.chunk;
+    if (begin >= end) return;                               // no rows: what `fetch` would read past the end may lie before the first row
     if (MODE != TP_SCAN_WHOLE) {
-        begin += (blockIdx.x % a.n_chunks) * a.chunk;
-        if (begin >= end) return;
         last = begin + a.chunk >= end;
         if (MODE == TP_SCAN_LOCAL && last) return;           // nothing comes after it
         end = min(end, begin + a.chunk);
