@@ -466,6 +466,8 @@ def shift_mix(x, mu, state, slot_ids, cu_rows, row_seq, one_row_each=False, out_
     before = torch.empty_like(xf)
     for i in range(len(cu_rows) - 1):
         a, b, slot = int(cu_rows[i]), int(cu_rows[i + 1]), int(slot_ids[i])
+        if a == b:
+            continue
         before[a] = state[slot]
         before[a + 1:b] = xf[a:b - 1]
         state[slot] = xf[b - 1]

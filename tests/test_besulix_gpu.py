@@ -319,6 +319,20 @@ def test_scans_leave_a_sequence_without_rows_alone(rt, heads, dk, dv, lens, chun
     assert rel_l2(got, want) < 5e-6 and rel_l2(got_state, want_state) < 5e-6 and torch.equal(got_state[[1, 3, 4, 5]].cpu(), state[[1, 3, 4, 5]])
 
 
+@pytest.mark.parametrize("lens", [(0, 3, 0, 1, 0), (0, 0, 70)])
+def test_shift_mix_leaves_a_sequence_without_rows_alone(rt, lens):
+    from . import ref_ops
+    n, d, M = len(lens), 300, sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    row_seq, slots = torch.repeat_interleave(torch.arange(n, dtype=torch.int32), torch.tensor(lens)), torch.arange(n, dtype=torch.int32).flip(0)
+    x, mu, state = acts(rt, rnd(M, d, seed=130))[0], rnd(2, d, seed=131), rnd(n + 1, d, seed=132)
+    want_state, got_state = state.clone(), state.to(rt.device)
+    want = ref_ops.shift_mix(x.cpu(), mu, want_state, slots, cu, row_seq)
+    got = rt.ops.shift_mix(x, mu.to(rt.device), got_state, slots.to(rt.device), cu.to(rt.device), row_seq.to(rt.device))
+    assert torch.equal(got_state.cpu(), want_state)
+    assert rel_l2(got, want) < (1e-6 if rt.dtype == torch.float32 else 4e-3)
+
+
 @pytest.mark.parametrize("cut", ["whole", "pieces", "one by one"])
 def test_matrix_memory_keeps_its_first_tokens(rt, cut):
     """Forget gates of sigmoid(8) and small input gates after the first tokens: the memory is what the first tokens wrote,

@@ -39,7 +39,7 @@ template <typename T>
 __global__ void __launch_bounds__(256)
 shift_save_k(const T* __restrict__ x, float* __restrict__ state, const int* __restrict__ slot_ids, const int* __restrict__ cu_rows, int D) {
     const int seq = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
-    if (c >= D) return;
+    if (c >= D || cu_rows[seq + 1] <= cu_rows[seq]) return;     // without rows of its own it keeps the last one it had
     state[(size_t)slot_ids[seq] * D + c] = ld_f32(x + (size_t)(cu_rows[seq + 1] - 1) * D + c);
 }
 
