@@ -319,6 +319,34 @@ def test_scans_leave_a_sequence_without_rows_alone(rt, heads, dk, dv, lens, chun
     assert rel_l2(got, want) < 5e-6 and rel_l2(got_state, want_state) < 5e-6 and torch.equal(got_state[[1, 3, 4, 5]].cpu(), state[[1, 3, 4, 5]])
 
 
+# infinities and NaN in single values, keys and states: in the middle of a tile of rows, in a chunk's and a sequence's last row, in the last
+# of keys that end inside of a block; with whole pieces and element by element
+@pytest.mark.parametrize("chunk", [64, 40, 0])
+@pytest.mark.parametrize("dk,dv", [(64, 128), (36, 68), (23, 70)])
+def test_matrix_memory_rows_before_an_infinity_do_not_see_it(rt, dk, dv, chunk):
+    from . import ref_ops
+    inf, heads, lens, slots = float("inf"), 2, (75, 130, 21), torch.tensor([2, 0, 1], dtype=torch.int32)
+    cu, M = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32), sum(lens)
+    q, k, v = (acts(rt, rnd(M, heads * d, seed=140 + i, scale=0.5))[0] for i, d in enumerate((dk, dk, dv)))
+    gates = torch.cat([rnd(M, heads, seed=143), rnd(M, heads, seed=144) + 1.0], dim=1).contiguous()
+    states = [rnd(3, heads, dk, dv, seed=145, scale=0.3), rnd(3, heads, dk, seed=146, scale=0.3), rnd(3, heads, seed=147)]
+    for row, column, x in ((23, 5, inf), (74, dv + 9, -inf), (75 + 63, 1, float("nan")), (75 + 100, 64, inf), (75 + 129, 2 * dv - 1, inf), (75 + 130 + 20, 0, -inf)):
+        v[row, column] = x
+    k[75 + 130 + 7, 3] = inf
+    states[0][1, 1, dk - 1, 2] = inf
+    want_states, got_states = [t.double() for t in states], [t.to(rt.device) for t in states]
+    want = ref_ops.matrix_memory_scan(q.cpu(), k.cpu(), v.cpu(), gates, 8.0, dk ** -0.5, *want_states, slots, cu, max(lens), heads, dk, dv)
+    got = rt.ops.matrix_memory_scan(q, k, v, gates.to(rt.device), 8.0, dk ** -0.5, *got_states, slots.to(rt.device), cu.to(rt.device), max(lens), heads, dk, dv, chunk=chunk)
+    assert bool(torch.isfinite(want[:23]).all()) and not bool(torch.isfinite(want).all())
+    ok, got = torch.isfinite(want), got.cpu()            # (of an output that sees one, infinity or NaN: S^T q adds both signs, (k . q) v is one)
+    assert torch.equal(torch.isfinite(got), ok) and rel_l2(got[ok], want[ok]) < 6e-5
+    for g, w in zip(got_states, want_states):
+        g, w = g.cpu(), w.float()
+        ok = torch.isfinite(w)
+        assert torch.equal(torch.isnan(g), torch.isnan(w)) and torch.equal(g[torch.isinf(w)], w[torch.isinf(w)]) and torch.equal(torch.isfinite(g), ok)
+        assert rel_l2(g[ok], w[ok]) < 1e-5
+
+
 @pytest.mark.parametrize("lens", [(0, 3, 0, 1, 0), (0, 0, 70)])
 def test_shift_mix_leaves_a_sequence_without_rows_alone(rt, lens):
     from . import ref_ops

@@ -366,6 +366,11 @@ mm_chunk_k(MatrixMemoryArgs a) {
         float w[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) w[u] = weights[wave][16 * kb + 4 * u + g];
+        if (16 * kb + 16 > n) {                          // rows past the chunk's end are its last again: no infinity of it may meet their weight of 0
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (16 * kb + 4 * u + g >= n) kq[kb & 1][u] = vq[kb & 1][u] = (mm_f32x4){0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int y = 0; y < 4; y++) {
 #pragma unroll
@@ -537,6 +542,10 @@ mm_outputs_k(MatrixMemoryArgs a) {
     fetch(0, sq, qq);
     for (int kb = 0; kb < blocks; kb++) {
         if (kb + 1 < blocks) fetch(kb + 1, sn, qn);
+        if (16 * kb + 16 > dk) {                         // keys past the end are the last again, as above
+#pragma unroll
+            for (int u = 0; u < 4; u++) if (16 * kb + 4 * g + u >= dk) sq[u] = (mm_f32x4){0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int tt = 0; tt < 4; tt++) {
             if (tt >= tiles) break;
@@ -565,9 +574,33 @@ mm_outputs_k(MatrixMemoryArgs a) {
         mm_f32x4 v[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) v[u] = quad<VEC>(vh + (size_t)(begin + min(16 * kb + 4 * u + g, n - 1)) * a.v_stride, j0 + 4 * r, dv);
+        // The tile's own rows t do not see the rows behind them: a weight of 0 keeps finite values out, but no infinity and no NaN.
+        // Where a value is none, the tile is summed row after row without what is not seen.
+        float none = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) none = __builtin_fmaf(v[u][x], 0.f, none);
+        const bool finite = !__any(none != 0.f);
+        if (!finite) {
+            const int t = 16 * kb + r;
+            mm_f32x4 p[4] = {};
+            for (int s = 16 * kb; s < min(16 * kb + 16, n); s++) {
+                const float w = P[t][s];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const mm_f32x4 value = quad<VEC>(vh + (size_t)(begin + s) * a.v_stride, j0 + 16 * g + 4 * e, dv);
+#pragma unroll
+                    for (int x = 0; x < 4; x++) p[x][e] = s <= t ? __builtin_fmaf(value[x], w, p[x][e]) : p[x][e];
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < 4; x++) acc[x][kb] += p[x];
+        }
 #pragma unroll
         for (int tt = kb; tt < 4; tt++) {
             if (tt >= tiles) break;
+            if (tt == kb && !finite) continue;
             float w[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) w[u] = P[16 * tt + r][16 * kb + 4 * u + g];
