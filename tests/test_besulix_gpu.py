@@ -319,6 +319,33 @@ def test_scans_leave_a_sequence_without_rows_alone(rt, heads, dk, dv, lens, chun
     assert rel_l2(got, want) < 5e-6 and rel_l2(got_state, want_state) < 5e-6 and torch.equal(got_state[[1, 3, 4, 5]].cpu(), state[[1, 3, 4, 5]])
 
 
+# more sequences than a block looks at together, long ones first, last and between single rows, some without rows, one exactly a chunk long
+@pytest.mark.parametrize("lens", [[1] * 70 + [200, 0, 64] + [1] * 62 + [33], [130] + [1] * 64, [1] * 63 + [100], [12, 64, 128, 129, 63, 0, 65]])
+@pytest.mark.parametrize("chunk", [None, 24])
+def test_matrix_memory_chunks_find_their_sequences(rt, lens, chunk):
+    """The rows and states of every sequence, and no more workspace than the step's rows fill and a chunk for each sequence."""
+    from . import ref_ops
+    n, heads, dk, dv = len(lens), 2, 16, 32
+    cu, M = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32), sum(lens)
+    slots = torch.randperm(n + 1, generator=torch.Generator().manual_seed(150))[:n].to(torch.int32)
+    q, k, v = (acts(rt, rnd(M, heads * d, seed=151 + i, scale=0.5))[0] for i, d in enumerate((dk, dk, dv)))
+    gates = torch.cat([rnd(M, heads, seed=154, scale=2.0), rnd(M, heads, seed=155, scale=2.0) + 1.0], dim=1).contiguous()
+    states = [rnd(n + 1, heads, dk, dv, seed=156, scale=0.3), rnd(n + 1, heads, dk, seed=157, scale=0.3), rnd(n + 1, heads, seed=158)]
+    want_states, got_states = [t.double() for t in states], [t.to(rt.device) for t in states]
+    want = ref_ops.matrix_memory_scan(q.cpu(), k.cpu(), v.cpu(), gates, 8.0, dk ** -0.5, *want_states, slots, cu, max(lens), heads, dk, dv)
+    args = (q, k, v, gates.to(rt.device), 8.0, dk ** -0.5, *got_states, slots.to(rt.device), cu.to(rt.device), max(lens), heads, dk, dv)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    got = rt.ops.matrix_memory_scan(*args, chunk=chunk)
+    floats = M * heads * dv + (M // (chunk or 64) + n) * heads * (dk * dv + dk + 8) + n
+    assert torch.cuda.max_memory_allocated() - before <= 4 * floats + 2048       # (two allocations, each rounded up to 512 bytes)
+    assert rel_l2(got, want) < 6e-5                      # the denominator's bound, as above
+    for g, w, s in zip(got_states, want_states, states):
+        assert rel_l2(g, w) < 1e-5
+        for i, c in enumerate(lens):
+            assert c or torch.equal(g[slots[i]].cpu(), s[slots[i]]), i
+
+
 # infinities and NaN in single values, keys and states: in the middle of a tile of rows, in a chunk's and a sequence's last row, in the last
 # of keys that end inside of a block; with whole pieces and element by element
 @pytest.mark.parametrize("chunk", [64, 40, 0])

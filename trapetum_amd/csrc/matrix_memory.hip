@@ -5,7 +5,7 @@
 //
 // Three ways to the same rows:
 // * a step of one row a sequence: matrix_memory_step_k;
-// * up to CHUNK_FROM rows: matrix_memory_scan_k, row after row, a lane keeping rows of one column of S in registers;
+// * up to 11 rows of the longest sequence: matrix_memory_scan_k, row after row, a lane keeping rows of one column of S in registers;
 // * more: chunks of up to 64 rows side by side, as products on the float32 matrix instructions (float32 operands and sums; the
 //   queries, keys and values are exact in them).  With b_t the sum of the log forget gates of a chunk's rows up to t, a_s = i_s - b_s
 //   and m0 the maximum that the chunk starts from, M_t = max(m0, a_0 .. a_t) gives m_t = b_t + M_t, and
@@ -24,11 +24,12 @@
 struct MatrixMemoryArgs {
     const void* q; long q_stride; const void* k; long k_stride; const void* v; long v_stride;
     const float* gates; float cap, q_scale; float* memory; float* normalizer; float* maximum;
-    const int* slot_ids; const int* cu_rows; float* y; int H, dk, dv;
-    // chunks of `chunk` rows, n_chunks covering the longest sequence.  ws_state [sequences n_chunks, H, dk dv + dk]: a chunk's matrix,
-    // then its normalizer, both in units of e^(its maximum); ws_aux [sequences n_chunks, H, 8]: the maximum of a chunk run from
-    // nothing, the sum of its log forget gates, the maximum it starts from, the maximum it leaves, what the sum was rounded by
-    int chunk, n_chunks; float* ws_state; float* ws_aux;
+    const int* slot_ids; const int* cu_rows; float* y; int n_seq, H, dk, dv;
+    // chunks of `chunk` rows, each in a place of its own (chunk_at).  ws_state [places, H, dk dv + dk]: a chunk's matrix,
+    // then its normalizer, both in units of e^(its maximum); ws_aux [places, H, 8]: the maximum of a chunk run from
+    // nothing, the sum of its log forget gates, the maximum it starts from, the maximum it leaves, what the sum was rounded by, and as
+    // whole numbers its sequence, first row and rows (0: no chunk).  ws_first [n_seq]: a sequence's first place
+    int chunk, places; float* ws_state; float* ws_aux; int* ws_first;
 };
 
 __device__ __forceinline__ float log_sigmoid_f(float z) { return -(log1pf(expf(-fabsf(z))) + fmaxf(-z, 0.f)); }
@@ -301,6 +302,34 @@ __device__ __forceinline__ float exp_of(double x) {
     return e > 0.f ? __builtin_fmaf(e, (float)(x - (double)hi), e) : e;
 }
 
+// The chunks lie in places one after the other, those of sequence 0 first, so that a launch has as many blocks as the step's rows fill and
+// those of the sequences' last chunks, whatever the longest sequence has.  (With as many for every sequence as the longest needs, 2,048
+// rows beside 63 single ones took 2.4 GB of workspace and 1,437 us, nearly all for chunks without rows; 0.13 GB and 289 us here.)
+// The chunk at a place: its sequence, its number there, first row and rows.  False: there is none.  A lane counts a sequence's chunks,
+// 64 sequences at a time.
+__device__ __forceinline__ bool chunk_at(const MatrixMemoryArgs& a, int place, int lane, int& seq, int& number, int& begin, int& n) {
+    for (int s0 = 0; s0 < a.n_seq; s0 += 64) {
+        const int at = min(s0 + lane, a.n_seq - 1), row = a.cu_rows[at], rows = s0 + lane < a.n_seq ? a.cu_rows[at + 1] - row : 0;
+        const int mine = (int)((unsigned)(rows + a.chunk - 1) / (unsigned)a.chunk);
+        int up_to = mine;                                // the chunks up to and with the lane's sequence
+        for (int o = 1; o < min(64, a.n_seq - s0); o <<= 1) {
+            const int x = __shfl_up(up_to, o, 64);
+            if (lane >= o) up_to += x;
+        }
+        const unsigned long long behind = __ballot(place < up_to);
+        if (behind) {
+            const int l = __ffsll((long long)behind) - 1;
+            seq = s0 + l;
+            number = place - (lane_value(up_to, l) - lane_value(mine, l));
+            begin = lane_value(row, l) + number * a.chunk;
+            n = min(lane_value(rows, l) - number * a.chunk, a.chunk);
+            return true;
+        }
+        place -= lane_value(up_to, 63);
+    }
+    return false;
+}
+
 // A lane's row of a chunk of n rows: b, the sum of the log forget gates up to it, and a, its log input gate less b (-infinity past the
 // chunk's end, where b stands still).
 __device__ __forceinline__ void chunk_gates(const MatrixMemoryArgs& g, int begin, int n, int h, int lane, double& a, double& b) {
@@ -316,7 +345,7 @@ __device__ __forceinline__ void chunk_gates(const MatrixMemoryArgs& g, int begin
 }
 }
 
-// What a chunk adds to the state, sum over its rows s of e^(a_s - M) k_s v_s^T with M about the largest a.  grid (sequences n_chunks, heads,
+// What a chunk adds to the state, sum over its rows s of e^(a_s - M) k_s v_s^T with M about the largest a.  grid (places, heads,
 // groups of 64 keys), a wave for every 64 values.  v is the A operand and the weighted k the B operand; a lane's four neighbours
 // of a row of k or v belong to four tiles (element 4 r + tile of 64), so a lane ends up with four neighbours of a row of S.
 template <typename T, bool VEC>
@@ -324,9 +353,14 @@ __global__ void __launch_bounds__(256)
 mm_chunk_k(MatrixMemoryArgs a) {
     __shared__ float weights[4][CHUNK];
     const int h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, H = a.H, dk = a.dk, dv = a.dv;
-    const int seq = blockIdx.x / a.n_chunks, begin = a.cu_rows[seq] + (blockIdx.x % a.n_chunks) * a.chunk;
-    const int n = min(a.cu_rows[seq + 1] - begin, a.chunk);
-    if (n <= 0) return;
+    float* const aux = a.ws_aux + ((size_t)blockIdx.x * H + h) * AUX;
+    int seq = 0, number, begin = 0, n = 0;
+    const bool any = chunk_at(a, blockIdx.x, lane, seq, number, begin, n);
+    if (blockIdx.z == 0 && threadIdx.x == 0) {
+        aux[5] = __int_as_float(seq); aux[6] = __int_as_float(begin); aux[7] = __int_as_float(n);
+        if (any && number == 0 && h == 0) a.ws_first[seq] = blockIdx.x;
+    }
+    if (!any) return;
     double al, bl;
     chunk_gates(a, begin, n, h, lane, al, bl);
     double top = al;
@@ -335,7 +369,6 @@ mm_chunk_k(MatrixMemoryArgs a) {
     const double all = __shfl(bl, 63, 64);
     const float m = (float)(all + top);                  // the units of what is left are e^m as it is stored
     weights[wave][lane] = lane < n ? (float)exp(al - ((double)m - all)) : 0.f;
-    float* const aux = a.ws_aux + ((size_t)blockIdx.x * H + h) * AUX;
     if (blockIdx.z == 0 && threadIdx.x == 0) { aux[0] = m; aux[1] = (float)all; aux[4] = (float)(all - (double)(float)all); }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -413,7 +446,7 @@ mm_carry_k(MatrixMemoryArgs a) {
     float* const home = e < dk * dv ? a.memory + (slot * H + h) * dk * dv + e : a.normalizer + (slot * H + h) * dk + e - dk * dv;
     Piece x = *reinterpret_cast<const Piece*>(home);
     float m = a.maximum[slot * H + h];
-    const size_t g0 = (size_t)seq * a.n_chunks;
+    const size_t g0 = (size_t)a.ws_first[seq];
     for (int c0 = 0; c0 < n; c0 += 8) {
         Piece L[8];
         float M[8];
@@ -442,7 +475,7 @@ mm_carry_k(MatrixMemoryArgs a) {
     *reinterpret_cast<Piece*>(home) = x;
 }
 
-// A chunk's outputs from the state that it starts from.  grid (sequences n_chunks, heads), a wave for every 64 values.  The chunk's
+// A chunk's outputs from the state that it starts from.  grid (places, heads), a wave for every 64 values.  The chunk's
 // weighted scores P[t, s] (k as the A operand, q as B) go to LDS, 16 rows t a wave; then every wave forms S0^T q and, its columns
 // scaled, adds v^T P for its values, tiles of 16 rows t and 64 values whose A operand is four neighbours of a row of S0 or v.
 template <typename T, bool VEC>
@@ -453,11 +486,10 @@ mm_outputs_k(MatrixMemoryArgs a) {
     __shared__ double as[4][CHUNK], tops[4][CHUNK];
     __shared__ float scales[4][CHUNK], floors[4][CHUNK], dens[CHUNK];
     const int h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, H = a.H, dk = a.dk, dv = a.dv;
-    const int seq = blockIdx.x / a.n_chunks, begin = a.cu_rows[seq] + (blockIdx.x % a.n_chunks) * a.chunk;
-    const int n = min(a.cu_rows[seq + 1] - begin, a.chunk);
+    const float* const aux = a.ws_aux + ((size_t)blockIdx.x * H + h) * AUX;
+    const int seq = __float_as_int(aux[5]), begin = __float_as_int(aux[6]), n = __float_as_int(aux[7]);
     if (n <= 0) return;
     const float* const ws = a.ws_state + ((size_t)blockIdx.x * H + h) * ((size_t)dk * dv + dk);
-    const float* const aux = a.ws_aux + ((size_t)blockIdx.x * H + h) * AUX;
     const T* const qh = (const T*)a.q + (size_t)h * dk;
     const T* const kh = (const T*)a.k + (size_t)h * dk;
     const T* const vh = (const T*)a.v + (size_t)h * dv;
@@ -625,51 +657,53 @@ mm_outputs_k(MatrixMemoryArgs a) {
     }
 }
 
-extern "C" long tp_matrix_memory_scan_workspace_floats(int n_seq, int n_chunks, int H, int dk, int dv) {
-    return (long)n_seq * n_chunks * H * ((long)dk * dv + dk + AUX);
+extern "C" long tp_matrix_memory_scan_workspace_floats(int n_seq, int places, int H, int dk, int dv) {
+    return (long)places * H * ((long)dk * dv + dk + AUX) + n_seq;
 }
 
 template <typename T>
-static void chunks_launch(const MatrixMemoryArgs& a, int n_seq, bool vec, hipStream_t s) {
+static void chunks_launch(const MatrixMemoryArgs& a, bool vec, hipStream_t s) {
     const int threads = 64 * tp_cdiv(a.dv, 64), per = a.dk * a.dv + a.dk;
-    const dim3 chunks(n_seq * a.n_chunks, a.H), groups(n_seq * a.n_chunks, a.H, tp_cdiv(a.dk, 64));
+    const dim3 chunks(a.places, a.H), groups(a.places, a.H, tp_cdiv(a.dk, 64));
     if (vec) {
         mm_chunk_k<T, true><<<groups, threads, 0, s>>>(a);
-        mm_carry_k<4><<<dim3(n_seq, a.H, tp_cdiv(per, 1024)), 256, 0, s>>>(a);
+        mm_carry_k<4><<<dim3(a.n_seq, a.H, tp_cdiv(per, 1024)), 256, 0, s>>>(a);
         mm_outputs_k<T, true><<<chunks, threads, 0, s>>>(a);
     } else {
         mm_chunk_k<T, false><<<groups, threads, 0, s>>>(a);
-        mm_carry_k<1><<<dim3(n_seq, a.H, tp_cdiv(per, 256)), 256, 0, s>>>(a);
+        mm_carry_k<1><<<dim3(a.n_seq, a.H, tp_cdiv(per, 256)), 256, 0, s>>>(a);
         mm_outputs_k<T, false><<<chunks, threads, 0, s>>>(a);
     }
 }
 
-// chunk 0: whole sequences, in pieces of one row where no sequence has more (one_row_each); otherwise chunks of up to 64 rows.
+// chunk 0: whole sequences, in pieces of one row where no sequence has more (one_row_each); otherwise chunks of up to 64 rows, `places`
+// of them in all sequences or more.
 // memory [slots, H, dk, dv], normalizer [slots, H, dk], maximum [slots, H], gates [M, 2 H] (input sums, then forget sums), all float32
 extern "C" int tp_matrix_memory_scan(const void* q, long q_stride, const void* k, long k_stride, const void* v, long v_stride, int dtype,
                                      const float* gates, float cap, float q_scale, float* memory, float* normalizer, float* maximum,
                                      const int* slot_ids, const int* cu_rows, float* y, int n_seq, int H, int dk, int dv,
-                                     int chunk, int n_chunks, float* workspace, int one_row_each, void* stream) {
+                                     int chunk, int places, float* workspace, int one_row_each, void* stream) {
     TP_REQUIRE(n_seq > 0 && H > 0 && dk > 0 && dv > 0, "matrix_memory_scan: empty shape sequences=%d heads=%d key=%d value=%d", n_seq, H, dk, dv);
     TP_REQUIRE(dk <= 256, "matrix_memory_scan: keys of %d elements exceed the 256 a lane keeps", dk);
     TP_REQUIRE(dv <= 256, "matrix_memory_scan: values of %d elements exceed the 256 columns of a block", dv);
     TP_REQUIRE(H <= 65535, "matrix_memory_scan: %d heads exceed one launch", H);
     TP_REQUIRE(cap > 0.f, "matrix_memory_scan: the gates' cap must be positive");
     TP_REQUIRE(q && k && v && gates && memory && normalizer && maximum && slot_ids && cu_rows && y, "matrix_memory_scan: null operand");
-    TP_REQUIRE(chunk == 0 || (chunk > 0 && chunk <= CHUNK && n_chunks > 0 && workspace && (long)n_seq * n_chunks <= 0x7fffffffL),
-               "matrix_memory_scan: %d chunks of %d rows (at most %d) need a workspace", n_chunks, chunk, CHUNK);
+    TP_REQUIRE(chunk == 0 || (chunk > 0 && chunk <= CHUNK && places > 0 && workspace),
+               "matrix_memory_scan: %d chunks of %d rows (at most %d) need a workspace", places, chunk, CHUNK);
     TP_REQUIRE(dtype == TP_BF16 || dtype == TP_F32, "matrix_memory_scan: unknown dtype %d", dtype);
     hipStream_t s = (hipStream_t)stream;
-    float* ws_aux = workspace ? workspace + (size_t)n_seq * n_chunks * H * ((size_t)dk * dv + dk) : nullptr;
-    const MatrixMemoryArgs a{q, q_stride, k, k_stride, v, v_stride, gates, cap, q_scale, memory, normalizer, maximum, slot_ids, cu_rows, y, H, dk, dv,
-                             chunk, n_chunks, workspace, ws_aux};
+    float* ws_aux = workspace ? workspace + (size_t)places * H * ((size_t)dk * dv + dk) : nullptr;
+    int* ws_first = workspace ? (int*)(ws_aux + (size_t)places * H * AUX) : nullptr;
+    const MatrixMemoryArgs a{q, q_stride, k, k_stride, v, v_stride, gates, cap, q_scale, memory, normalizer, maximum, slot_ids, cu_rows, y, n_seq, H, dk, dv,
+                             chunk, places, workspace, ws_aux, ws_first};
     const size_t piece = dtype == TP_BF16 ? 8 : 16;
     if (chunk > 0) {
         const bool vec = dk % 4 == 0 && dv % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
                          ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % piece == 0 &&
                          ((uintptr_t)memory | (uintptr_t)normalizer | (uintptr_t)workspace | (uintptr_t)y) % 16 == 0;
-        if (dtype == TP_BF16) chunks_launch<bf16_t>(a, n_seq, vec, s);
-        else chunks_launch<float>(a, n_seq, vec, s);
+        if (dtype == TP_BF16) chunks_launch<bf16_t>(a, vec, s);
+        else chunks_launch<float>(a, vec, s);
         return tp_check_launch("matrix_memory_scan (chunks)");
     }
     const dim3 grid(n_seq, H);

@@ -4,9 +4,8 @@
 
 #define TP_SCAN_AHEAD 4          // tokens whose loads are issued together
 
-__device__ __forceinline__ float lane_value(float x, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-}
+__device__ __forceinline__ int lane_value(int x, int lane) { return __builtin_amdgcn_readlane(x, lane); }
+__device__ __forceinline__ float lane_value(float x, int lane) { return __int_as_float(lane_value(__float_as_int(x), lane)); }
 
 // DK: key rows a lane keeps of its column (the head's key size rounded up to 16, 32 or a multiple of 64); NR registers
 // hold a per-row vector, row (lane + 64 n) in register n.
