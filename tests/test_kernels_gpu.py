@@ -397,10 +397,11 @@ def test_linear_f32(ops, m, n, k):
 
 
 # one launch: a matrix alone and as many as it takes, matrices of one row, of less than a block and of less than all of its last, with and
-# without a bias, both output types, one and two groups of 8 rows a block; beside it, what goes product after product (9 rows, a K
-# beyond one round, K no multiple of 8, more matrices)
+# without a bias, both output types, one and two groups of 8 rows a block, a K of one round, of two and of four, the last of them short;
+# beside it, what goes product after product (9 rows, a single product whose K is beyond one round, a K beyond all, K no multiple of 8, more matrices)
 @pytest.mark.parametrize("m,k,ns", [(1, 8, (1,)), (4, 2304, (2304, 2304, 2304, 2304, 144)), (8, 256, (7, 8, 9, 33, 1, 16, 15, 500)), (3, 1160, (2056, 2048, 20)),
-                                    (5, 776, (4097,)), (9, 256, (40, 8)), (2, 2560, (24, 40)), (4, 20, (9, 3)), (8, 64, (8,) * 9)])
+                                    (5, 776, (4097,)), (9, 256, (40, 8)), (2, 2560, (24, 40)), (4, 20, (9, 3)), (8, 64, (8,) * 9),
+                                    (1, 2312, (2312, 20)), (8, 4104, (2056, 2048, 9)), (7, 9216, (33, 16)), (3, 9224, (24, 8)), (4, 2568, (40,))])
 def test_linear_group(ops, m, k, ns):
     parts = []
     for i, n in enumerate(ns):

@@ -256,13 +256,13 @@ gemm_rows8_group_k(Rows8Group g, int parts, int M, int K) {
     }
 }
 
-// y[p] [M, n[p]] = x[p] [M, K] . w[p] [n[p], K]^T (+ bias[p]), `parts` of them (up to TP_LINEAR_GROUP), bf16 rows and matrices, up to 8 rows,
-// a K that a block reads in one round.  Bit p of `tanh`: y[p] is tanh of the rounded product, as a launch of its own would leave it
+// y[p] [M, n[p]] = x[p] [M, K] . w[p] [n[p], K]^T (+ bias[p]), `parts` of them (up to TP_LINEAR_GROUP), bf16 rows and matrices, up to 8 rows.
+// Bit p of `tanh`: y[p] is tanh of the rounded product, as a launch of its own would leave it
 // (that launch took 4.5 us of a decode step's time mix).
 extern "C" int tp_linear_group(const void* const* x, const void* const* w, void* const* y, const float* const* bias, const int* n, const int* out_dtype,
                                int tanh, int parts, int M, int K, void* stream) {
     TP_REQUIRE(parts > 0 && parts <= TP_LINEAR_GROUP, "linear group: %d products (at most %d)", parts, TP_LINEAR_GROUP);
-    TP_REQUIRE(M > 0 && M <= 8 && K > 0 && K % 8 == 0 && K <= R8_MAX_STEPS * 256, "linear group: needs at most 8 rows and a K that is a multiple of 8 up to %d (M=%d K=%d)", R8_MAX_STEPS * 256, M, K);
+    TP_REQUIRE(M > 0 && M <= 8 && K > 0 && K % 8 == 0, "linear group: needs at most 8 rows and a K that is a multiple of 8 (M=%d K=%d)", M, K);
     Rows8Group g{};
     g.tanh = (unsigned)tanh;
     long tiles = 0;
@@ -282,7 +282,7 @@ extern "C" int tp_linear_group(const void* const* x, const void* const* w, void*
     hipStream_t s = (hipStream_t)stream;
 #define TP_GROUP(NS) do { if (ng == 2) gemm_rows8_group_k<2, NS><<<(unsigned)blocks, 256, 0, s>>>(g, parts, M, K); \
                           else gemm_rows8_group_k<1, NS><<<(unsigned)blocks, 256, 0, s>>>(g, parts, M, K); } while (0)
-    const int steps = tp_cdiv(K, 256);
+    const int all = tp_cdiv(K, 256), steps = tp_cdiv(all, tp_cdiv(all, R8_MAX_STEPS));      // rounds of equal length
     if (steps <= 1) TP_GROUP(1); else if (steps <= 3) TP_GROUP(3); else if (steps <= 5) TP_GROUP(5); else if (steps <= 7) TP_GROUP(7); else TP_GROUP(R8_MAX_STEPS);
 #undef TP_GROUP
     return tp_check_launch("linear group");

@@ -1141,16 +1141,24 @@ class HipOps:
             return self._linear(x, w, out_dtype, EPI_SOFTCAP, softcap, 0)
         return self._linear(x, w, out_dtype, EPI_NONE, 0.0, 0, defer=defer)
 
-    GROUP_ROWS, GROUP_K, GROUP_PARTS = 8, 2304, 8        # what one launch of `linear_group` takes (the kernel library's)
+    GROUP_ROWS, GROUP_PARTS = 8, 8                       # what one launch of `linear_group` takes (the kernel library's)
+    # Columns up to which it does: a single product's while a block reads them in one round, several products' in rounds as well.
+    # Microseconds, cold weights, product after product / one launch: four of K x K and one of K / 16 x K, the last through tanh, at 1 / 4 / 8
+    # rows: K 1024 14.0 / 5.7, 16.4 / 6.1, 16.8 / 6.5; K 2304 25.2 / 11.6, 30.8 / 12.0, 33.8 / 13.0; K 2560 25.5 / 13.4, 47.2 / 14.2,
+    # 50.6 / 15.3; K 4096 39.9 / 29.6, 61.0 / 32.0, 63.1 / 36.1; K 9216 182 / 128, 153 / 124, 157 / 135.  One with a bias, 5/4 K x K: K 2304
+    # 7.0 / 6.1, 8.1 / 6.4, 8.7 / 7.0; K 4096 12.3 / 14.0, 18.1 / 15.2, 19.2 / 16.3; K 9216 47.4 / 41.4, 43.5 / 42.9, 44.0 / 46.8.  (At K 2304 a
+    # product of 36,864 rows of W is no slower either: 32.8 / 31.5, 34.0 / 32.5, 38.7 / 35.8.)
+    GROUP_K, GROUP_K_SINGLE = 9216, 2304
 
     def linear_group(self, parts, tanh=()):
         """Several products [x @ w^T (+ bias) for x, w, out_dtype, bias in parts] of inputs of one shape; bias: float32 [rows of w] or
-        None.  A few bf16 rows go in one launch, the bias added to the float32 sums; others one after the other (`linear`).
+        None.  A few bf16 rows go in one launch, the bias added to the float32 sums, which are rounded once; others one after the
+        other (`linear`, whose bias is added to the rounded product, which is rounded again).
         tanh: indices of the products that go through tanh, once rounded."""
         m, k = parts[0][0].shape
         if any(x.dim() != 2 or tuple(x.shape) != (m, k) or w.dim() != 2 or w.shape[1] != k for x, w, _, _ in parts):
             raise KernelError("linear_group: rows of one shape and matrices of as many columns")
-        one = (m <= self.GROUP_ROWS and k <= self.GROUP_K and k % 8 == 0 and len(parts) <= self.GROUP_PARTS and not self.force_linear and
+        one = (m <= self.GROUP_ROWS and k <= (self.GROUP_K if len(parts) > 1 else self.GROUP_K_SINGLE) and k % 8 == 0 and len(parts) <= self.GROUP_PARTS and not self.force_linear and
                all(x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0 for x, w, _, _ in parts))
         if not one:
             out = [self.linear(x, w, out_dtype, bias=bias) for x, w, out_dtype, bias in parts]
