@@ -252,11 +252,14 @@ def test_attention_of_uneven_portions_over_a_cache(ops, counts, held, H, KV, hd,
 
 # one long sequence first, last and between short ones, so that only the blocks that hold a query are launched: two sequences and as many
 # as are packed, more blocks of a sequence than lanes look at once (64, and a cache of many times that before them), a last block of
-# one row, a sequence without rows, windows; without a cache and over one
+# one row, a sequence without rows, windows; without a cache and over one; then several long ones, whose blocks come late positions first:
+# with as many positions in the cache and with very different ones, and one long one of more blocks than run at once
 @pytest.mark.parametrize("shape", [0, 1, 2, 3])
 @pytest.mark.parametrize("counts,held,H,KV,hd,window", [([1, 1, 1, 2113], (150, 611, 48, 700), 4, 2, 64, 0), ([2600, 3], (0, 0), 4, 2, 64, 0), ([1] * 11 + [641] + [1] * 12, (77,) * 24, 4, 2, 64, 0),
                                                         ([33, 0, 1500, 7, 64], (0, 0, 0, 0, 0), 2, 2, 256, 0), ([1, 700, 1, 1], (3000, 5000, 40, 3), 4, 1, 256, 400),
-                                                        ([5, 1025, 5, 5, 5], (4, 4000, 300, 20, 1), 8, 4, 128, 0)])
+                                                        ([5, 1025, 5, 5, 5], (4, 4000, 300, 20, 1), 8, 4, 128, 0),
+                                                        ([900, 3, 1100, 5, 1, 0, 4, 6, 33], (0,) * 9, 4, 2, 256, 0), ([700, 3, 650, 64, 1, 2, 4, 6], (5000, 1, 20, 333, 0, 64, 3, 900), 4, 1, 256, 0),
+                                                        ([600] + [1] * 21 + [577, 40], (0,) * 12 + (70,) * 12, 2, 1, 192, 100), ([3] * 9 + [2600], (0,) * 10, 32, 16, 256, 0)])
 def test_attention_launches_the_blocks_that_hold_queries(ops, counts, held, H, KV, hd, window, shape):
     """Every sequence's rows are what they are alone, bit for bit (a choice of the shape by size may give others: to rounding)."""
     n, page = len(counts), 64

@@ -118,20 +118,43 @@ __device__ __forceinline__ bf16_t bf16_bits(float f) {
 }
 union PFrag { uint4 u; pf_bf16x8 v; pf_s16x4 h[2]; };
 
-// The j-th block of positions in a launch of n sequences (up to 64), blocks of 1 << shift rows, those of late positions first (counted
-// with the cached ones before the step's rows, new_len or null: they see the most keys), of one position in the sequences'
-// order.  False: there is none.  A lane holds a sequence's first block and the one behind its last, in blocks of positions;
-// from(x), how many blocks stand at x or behind, is asked by 64 lanes for 64 places at once.
-__device__ __forceinline__ bool packed_block(const int* cu_rows, const int* new_len, int n, int shift, int j, int lane, int& seq, int& q0) {
-    const int at = min(lane, n - 1), rows = cu_rows[at + 1] - cu_rows[at];
-    const int count = lane < n ? (rows + (1 << shift) - 1) >> shift : 0, begin = new_len ? (new_len[at] - rows) >> shift : 0, end = begin + count;
+// The j-th block of positions in a launch of n sequences (up to 64, a lane each), blocks of 1 << shift rows.  False: there is none.  The lane
+// of a sequence holds its first row, its rows and its keys (new_len, or the rows), which are handed out as they are: asked for again they
+// would be a trip to memory more.
+struct PackedBlock { int seq, q0, row0, rows, keys; };
+// a sequence's blocks one after the other, late positions first
+__device__ __forceinline__ bool packed_block(const int* cu_rows, const int* new_len, int n, int shift, int j, int lane, PackedBlock& p) {
+    const int at = min(lane, n - 1), first = cu_rows[at], count = cu_rows[at + 1] - first, seen = new_len ? new_len[at] : count;
+    const int mine = lane < n ? (count + (1 << shift) - 1) >> shift : 0;
+    int up_to = mine;                                            // the blocks up to and with the lane's sequence
+    for (int o = 1; o < n; o <<= 1) {
+        const int x = __shfl_up(up_to, o, 64);
+        if (lane >= o) up_to += x;
+    }
+    const unsigned long long behind = __ballot(j < up_to);
+    if (!behind) return false;
+    const int s = __ffsll((long long)behind) - 1;
+    p = {s, (__builtin_amdgcn_readlane(up_to, s) - 1 - j) << shift, __builtin_amdgcn_readlane(first, s), __builtin_amdgcn_readlane(count, s), __builtin_amdgcn_readlane(seen, s)};
+    return true;
+}
+// Late positions first (counted with the cached ones before the step's rows: they see the most keys), of one position in the
+// sequences' order.  A lane holds a sequence's first block and the one behind its last, in blocks of positions (none: both 0);
+// from(x), how many blocks stand at x or behind, is asked by 64 lanes for 64 places at once, eight sequences a round.
+template <bool PAGED>
+__device__ __forceinline__ bool latest_block(const int* cu_rows, const int* new_len, int n, int shift, int j, int lane, PackedBlock& p) {
+    const int at = min(lane, n - 1), first = cu_rows[at], count = cu_rows[at + 1] - first, seen = PAGED ? new_len[at] : count;
+    const int begin = PAGED && lane < n ? (seen - count) >> shift : 0, end = lane < n ? begin + ((count + (1 << shift) - 1) >> shift) : 0;
     auto from = [&](int x) {
         int sum = 0;
-        for (int s = 0; s < n; s++) sum += max(__builtin_amdgcn_readlane(end, s) - max(__builtin_amdgcn_readlane(begin, s), x), 0);
+        for (int s0 = 0; s0 < n; s0 += 8)
+#pragma unroll
+            for (int s = 0; s < 8; s++) sum += max(__builtin_amdgcn_readlane(end, s0 + s) - (PAGED ? max(__builtin_amdgcn_readlane(begin, s0 + s), x) : x), 0);
         return sum;
     };
-    int b = 0, range = 0, behind = 0;                            // from(b) > j >= from(b + range), if there is such a block
-    for (int s = 0; s < n; s++) range = max(range, __builtin_amdgcn_readlane(end, s));
+    int b = 0, range = end, behind = 0;                          // from(b) > j >= from(b + range), if there is such a block
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) range = max(range, __shfl_xor(range, o, 64));
+    range = __builtin_amdgcn_readfirstlane(range);
     while (true) {
         const int step = (range + 63) >> 6, f = from(b + lane * step);
         const unsigned long long more = __ballot(f > j);
@@ -144,12 +167,11 @@ __device__ __forceinline__ bool packed_block(const int* cu_rows, const int* new_
             break;
         }
     }
-    const int r = j - behind;
     const bool mine = begin <= b && b < end;
-    const unsigned long long have = __ballot(mine), it = __ballot(mine && __popcll(have & ((1ull << lane) - 1)) == r);
-    seq = __ffsll((long long)it) - 1;
-    if (seq < 0) return false;
-    q0 = (b - __builtin_amdgcn_readlane(begin, seq)) << shift;
+    const unsigned long long have = __ballot(mine), it = __ballot(mine && __popcll(have & ((1ull << lane) - 1)) == j - behind);
+    if (!it) return false;
+    const int s = __ffsll((long long)it) - 1;
+    p = {s, (b - __builtin_amdgcn_readlane(begin, s)) << shift, __builtin_amdgcn_readlane(first, s), __builtin_amdgcn_readlane(count, s), __builtin_amdgcn_readlane(seen, s)};
     return true;
 }
 
@@ -164,7 +186,8 @@ template <int CG, int KG> struct PrefillShape {
 
 // Registers: up to 256 a lane at head size 256 (two waves a SIMD); smaller heads need fewer, and a block of four
 // waves then runs three to a SIMD (27B sizes, 2 x 7,900 tokens: 1.62 -> 1.42 ms; four to a SIMD spill and lose).
-template <int CG, int KG, bool PAGED>
+// LATEST: packed blocks in the order of latest_block (a kernel of its own: beside the other search in one it costs every block 0.4 us)
+template <int CG, int KG, bool PAGED, bool LATEST>
 __global__ void __launch_bounds__(64 * CG * KG, (HD <= 128 && CG * KG == 4 ? 3 : 2))
 attn_prefill_k(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char prefill_lds[];
@@ -176,22 +199,27 @@ attn_prefill_k(PrefillArgs a) {
 
     // ---- which part of the step this block owns ---------------------------------------------------------------
     const int G = a.H / a.KV, HG = G >> a.ghb_shift, PT = 1 << a.pt_shift, PB = 32 * PT;
-    int hg, kvh, seq, q0;                                        // late positions see the most keys: they start first
-    if (a.packed) {
-        const int sub = blockIdx.x % (HG * a.KV);
+    int hg, kvh, seq, q0, row0, Tq, L;                           // late positions see the most keys: they start first
+    if (LATEST || a.packed) {
+        const int sub = blockIdx.x % (HG * a.KV), j = blockIdx.x / (HG * a.KV), shift = 5 + a.pt_shift;
         hg = sub % HG;
         kvh = sub / HG;
-        if (!packed_block(a.cu_rows, PAGED ? a.new_len : nullptr, a.packed, 5 + a.pt_shift, blockIdx.x / (HG * a.KV), lane, seq, q0)) return;
+        PackedBlock p;
+        if (!(LATEST ? latest_block<PAGED>(a.cu_rows, a.new_len, a.packed, shift, j, lane, p)
+                     : packed_block(a.cu_rows, PAGED ? a.new_len : nullptr, a.packed, shift, j, lane, p))) return;
+        seq = p.seq; q0 = p.q0; row0 = p.row0; Tq = p.rows; L = p.keys;
     } else {
         const int rank = blockIdx.x / a.n_streams, stream = (blockIdx.x % a.n_streams + rank * a.turn) % a.n_streams;
         hg = stream % HG;
         kvh = (stream / HG) % a.KV;
         seq = stream / (HG * a.KV);
         q0 = (a.pos_blocks - 1 - rank) * PB;
+        row0 = a.cu_rows[seq];
+        Tq = a.cu_rows[seq + 1] - row0;
+        if (q0 >= Tq) return;
+        L = PAGED ? a.new_len[seq] : Tq;
     }
-    const int row0 = a.cu_rows[seq], Tq = a.cu_rows[seq + 1] - row0;
-    if (q0 >= Tq) return;
-    const int start = PAGED ? a.new_len[seq] - Tq : 0, L = start + Tq;
+    const int start = L - Tq;
     const int h = kvh * G + (hg << a.ghb_shift) + (cg >> a.pt_shift);
     const int qw0 = start + q0 + (cg & (PT - 1)) * 32;           // position of the wave's first query
     const int qpos = qw0 + col;
@@ -531,17 +559,22 @@ attn_prefill_k(PrefillArgs a) {
 }
 
 namespace {
-template <int CG, int KG, bool PAGED>
-int prefill_launch(const PrefillArgs& a, int blocks, hipStream_t stream) {
+template <int CG, int KG, bool PAGED, bool LATEST>
+int prefill_launch_as(const PrefillArgs& a, int blocks, hipStream_t stream) {
     using Shape = PrefillShape<CG, KG>;
     static bool configured = false;                                   // more LDS than a kernel gets without asking
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute((const void*)attn_prefill_k<CG, KG, PAGED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Shape::LDS);
+        hipError_t e = hipFuncSetAttribute((const void*)attn_prefill_k<CG, KG, PAGED, LATEST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Shape::LDS);
         if (e != hipSuccess) return tp_fail("attention prefill: cannot reserve %zu bytes of LDS: %s", (size_t)Shape::LDS, hipGetErrorString(e));
         configured = true;
     }
-    attn_prefill_k<CG, KG, PAGED><<<blocks, Shape::THREADS, Shape::LDS, stream>>>(a);
+    attn_prefill_k<CG, KG, PAGED, LATEST><<<blocks, Shape::THREADS, Shape::LDS, stream>>>(a);
     return 0;
+}
+template <int CG, int KG>
+int prefill_launch(const PrefillArgs& a, bool paged, bool latest, int blocks, hipStream_t stream) {
+    if constexpr (HD > 128) if (latest) return paged ? prefill_launch_as<CG, KG, true, true>(a, blocks, stream) : prefill_launch_as<CG, KG, false, true>(a, blocks, stream);
+    return paged ? prefill_launch_as<CG, KG, true, false>(a, blocks, stream) : prefill_launch_as<CG, KG, false, false>(a, blocks, stream);
 }
 }  // namespace
 
@@ -614,16 +647,24 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
     // is the choice from 512 tokens on, cached positions before them or not (2x2 / 2x4: 866 rows at 6,135 beside three tokens
     // 235 / 149 us, 600 at 4,096 137 / 103, 2 x 512 at 2,048 79 / 63, 8 prompts of up to 700 31 / 26; 257 tokens 15.5 / 16.8).
     // Where less than half of the launched blocks could hold a query, and the sequences are few, those that hold none are not launched:
-    // a block finds its sequence and its place by itself (packed_block), and the ones that see the most keys come first.  Launched
-    // between empty ones, the blocks of a long sequence met on some CUs and left others idle, and the last of them began when the
-    // first had ended.  Microseconds, 2B, every block launched / packed: 2,048 rows beside three tokens 71 / 54, at 2,048 cached
-    // 139 / 96, at 4,096 207 / 139 (alone: 50, 97, 139); 1,000 at 3,000 beside three 142 / 90; 3,000 beside two 93 / 72; prompts of
-    // 512, 77, 1,300 and 260 44 / 36; 9B, 2,048 at 2,048 beside three 172 / 148.  The search costs 0.3 to 0.5 us with 5 to 8
-    // sequences (prompts of 333, 97, 1,021, 5 and 260: 29.9 / 30.6), 1 with 16, 4 with 61; and where half of the blocks hold queries
-    // nothing is gained (9B, four of 1,000 rows at 2,000 beside four tokens: 203 / 212).
-    auto packs = [&](long held, long all) { return n_seq <= 24 && 2 * held < all; };
+    // a block finds its sequence and its place by itself.  Launched between empty ones, the blocks of a long sequence met on some CUs and
+    // left others idle, and the last of them began when the first had ended.  Microseconds, 2B, every block launched / packed: 2,048
+    // rows beside three tokens 66 / 48, at 2,000 cached 151 / 92, at 5,000 327 / 153; 1,000 at 2,000 beside three 105 / 70; prompts
+    // of 512, 77, 1,300 and 260 45 / 36.  Where half of the blocks hold queries nothing is gained (9B, four of 1,000 rows at
+    // 2,000 beside four tokens: 203 / 212).
+    // What is lost by it is the search.  One that puts late positions of all sequences first took 0.3 us with 4 sequences and 1.4 with 24
+    // (256 rows beside 23 tokens, heads of 64: 8.0 / 9.4 us), and of 718 steps with heads of 64, 128 and 256, 128 to 4,000 rows beside
+    // shorter ones, 2 to 24 sequences and 0 to 5,000 cached positions 261 were 2 to 15 % slower so than with every block launched.  Where one
+    // sequence has most of the rows (the others at most three quarters of its) its blocks lie in that order by themselves, and
+    // where the blocks run at once (up to three a CU) no order matters: there a sequence's blocks follow one another, which costs 0.2 to
+    // 0.4 us (8.2).  Others need the order (2B, prompts of 178, 786, 1,351, 1,293 and four short ones 50 / 52 without it, 46 with it), and
+    // have a faster search for it; with heads of up to 128 they gain nothing (2 % slower in the mean) and are launched whole.  So 11 of the 718 are
+    // 2 to 4 % slower, none more, and 421 faster, by up to 113 %.
+    const bool one_long = 4 * ((long)M - max_count) <= 3L * max_count;
+    auto in_sequence = [&](long held) { return one_long && held <= 3L * cus; };
+    auto packs = [&](long held, long all) { return n_seq <= 24 && 2 * held < all && (HD > 128 || in_sequence(held)); };
     int cg = 4, kg = 1;
-    bool uneven = false;
+    bool uneven = false, latest = false;
     {
         int gs, pts;
         auto longest = [&]() { return (long)tp_cdiv(max_count, 32 << pts) * n_seq * KV * (G >> gs); };
@@ -642,6 +683,7 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
         plan(cg, gs, pts);
         uneven = 4 * filled() < 3 * longest();                 // (of the shape that is chosen)
         a.packed = packs(filled(), longest()) ? n_seq : 0;
+        latest = a.packed && !in_sequence(filled());           // (with heads of more than 128 only)
     }
     plan(cg, a.ghb_shift, a.pt_shift);
     a.n_streams = n_seq * KV * (G >> a.ghb_shift);
@@ -662,9 +704,9 @@ extern "C" int tp_attn_prefill(const void* q, long q_stride, const void* k, long
     TP_REQUIRE(blocks < (1L << 31), "attention prefill: %ld blocks exceed one launch", blocks);
     hipStream_t s = (hipStream_t)stream;
     int rc;
-    if (cg == 4) rc = paged ? prefill_launch<4, 1, true>(a, (int)blocks, s) : prefill_launch<4, 1, false>(a, (int)blocks, s);
-    else if (kg == 4) rc = paged ? prefill_launch<2, 4, true>(a, (int)blocks, s) : prefill_launch<2, 4, false>(a, (int)blocks, s);
-    else rc = paged ? prefill_launch<2, 2, true>(a, (int)blocks, s) : prefill_launch<2, 2, false>(a, (int)blocks, s);
+    if (cg == 4) rc = prefill_launch<4, 1>(a, paged, latest, (int)blocks, s);
+    else if (kg == 4) rc = prefill_launch<2, 4>(a, paged, latest, (int)blocks, s);
+    else rc = prefill_launch<2, 2>(a, paged, latest, (int)blocks, s);
     if (rc) return rc;
     return tp_check_launch("attention prefill");
 }
