@@ -345,6 +345,7 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
         const float first = cand_val[(size_t)blockIdx.x * cand_cap + tid];
         const int first_id = cand_id[(size_t)blockIdx.x * cand_cap + tid];
         const unsigned listed = cand_count[blockIdx.x];
+        asm volatile("" :: "v"(first), "v"(first_id), "s"(listed));        // all three are here (else the compiler asks for the entries once it knows the length)
         if (listed <= (unsigned)cand_cap && listed >= (unsigned)k) {
             V = (int)listed;
             z = cand_val + (size_t)blockIdx.x * cand_cap;
@@ -545,8 +546,8 @@ sample_full_k(const float* __restrict__ logits, int V, float temperature, Draws 
 // Three launches: the histogram, the candidates (every block finds the bin from its row's histogram by itself), the sampler,
 // which also puts the histogram and the count back to zero.  A block asks for all of its logits together.
 // (8 rows of 256,000, top_k 256, microseconds: histogram 5.9, candidates 10.2; 8.7, 10.6 and 5.5 for the bin in a launch of its own while a thread
-// asked for its 32 logits one after the other.  Sampler 10.1; 12.8 with the exchanges of its sort as shuffles through LDS, the candidates
-// asked for once their number was known, and a barrier that waited for the zeros of the histogram.)
+// asked for its 32 logits one after the other.  Sampler 10.0; 12.8 with the exchanges of its sort as shuffles through LDS
+// and a barrier that waited for the zeros of the histogram; 10.1 with the candidates asked for once their number was known.)
 constexpr int FILTER_BINS = 4096;
 constexpr int FILTER_PER = 16, FILTER_PART = 256 * FILTER_PER;       // logits per thread and block
 constexpr int FILTER_FROM = 32768;                                   // smaller vocabularies: the sampler alone
