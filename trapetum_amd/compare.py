@@ -921,6 +921,7 @@ def time_besulix_kernels(engine, cfg, batch, context, prefill_tokens):
     by the cached rows it reads (decode) or its flops (prefill)."""
     import torch
     from .engine.batch import StepContext
+    from .parts.base import products
     model, ops, dev = engine.model, engine.model.rt.ops, engine.model.rt.device
     bf, f32 = torch.bfloat16, torch.float32
     blocks = [l.block for l in model.layers]
@@ -954,7 +955,7 @@ def time_besulix_kernels(engine, cfg, batch, context, prefill_tokens):
                 site = cache.site(e)
                 table = ctx.page_table(site.group_index)
                 kp, vp, cap = site.tensor("k"), site.tensor("v"), site.rows_cap or 0
-                prod("left_qkv_bias", [(lambda b=b: ops.linear(x, b.mixer.sides[0].w_qkv, bf, bias=b.mixer.sides[0].b_qkv)) for b in par], left.w_qkv)
+                prod("left_qkv_bias", [(lambda b=b: products(ops, [(x, b.mixer.sides[0].w_qkv, bf, b.mixer.sides[0].b_qkv)])) for b in par], left.w_qkv)
                 qkv = torch.randn((rows, (H + 2 * KV) * row), device=dev).to(bf)
                 q, k, v = qkv[:, :H * row], qkv[:, H * row:(H + KV) * row], qkv[:, (H + KV) * row:]
                 one([lambda: left._turn(ctx, v, KV, left.value_freq)] * 16, name="turn_values", bytes_each=rows * KV * row * 4.0)
@@ -980,14 +981,13 @@ def time_besulix_kernels(engine, cfg, batch, context, prefill_tokens):
                 shift, memory = cache.entry_state(e, "mixer.right.shift"), cache.entry_state(e, "mixer.right.memory")
                 one([lambda: ops.shift_mix(x, right.mu, shift, ctx.slot_ids, ctx.cu_rows, ctx.row_seq, one_row_each=decode)] * 16,
                     name="shift_mix", bytes_each=rows * D * 12.0)
-                for s in ("r", "g"):
-                    prod(f"right_{s}", [(lambda b=b, s=s: ops.linear(x, b.mixer.sides[1].w[s], bf)) for b in par], right.w[s])
-
-                def decay_rates(b):
-                    low = ops.unary_(ops.linear(x, b.mixer.sides[1].w["w1"], bf), "tanh")
-                    return ops.linear(low, b.mixer.sides[1].w["w2"], f32)
-                one([(lambda b=b: decay_rates(b)) for b in par], name="decay_w1_tanh_w2",
-                    bytes_each=2.0 * (elems(right.w["w1"]) + elems(right.w["w2"])) + rows * (D * 2.0 + inner * 4.0))
+                mixes = ("r", "k", "v", "g", "w1")           # five products of one launch in a step of a few rows, of five in a prefill
+                calls = [(lambda b=b: products(ops, [(x, b.mixer.sides[1].w[s], bf, None) for s in mixes], tanh=(4,))) for b in par]
+                of_all = sum(elems(right.w[s]) for s in mixes)
+                one(calls, name="right_r_k_v_g_w1", **({"bytes_each": 2.0 * of_all} if decode else {"flops_each": 2.0 * rows * of_all}))
+                low = torch.randn((rows, right.w["w2"].shape[1]), device=dev).to(bf)
+                one([(lambda b=b: ops.linear(low, b.mixer.sides[1].w["w2"], f32)) for b in par], name="decay_w2",
+                    bytes_each=2.0 * elems(right.w["w2"]) + rows * (low.shape[1] * 2.0 + inner * 4.0))
                 r_, k_, v_ = ((torch.randn((rows, inner), device=dev) * 0.3).to(bf) for _ in range(3))
                 rate = torch.randn((rows, inner), device=dev)
                 scan = lambda: ops.time_mix_scan(r_, k_, v_, rate, right.w0, right.bonus, memory, ctx.slot_ids, ctx.cu_rows,
@@ -1008,9 +1008,7 @@ def time_besulix_kernels(engine, cfg, batch, context, prefill_tokens):
                 ctx.entry = ctx.cache_owner = e
                 mm = mem[0].mixer
                 nh, dk, dv = mm.num_heads, mm.key_dim, mm.value_dim
-                prod("memory_in", [(lambda b=b: ops.linear(x, b.mixer.w_in, bf)) for b in mem], mm.w_in)
-                one([(lambda b=b: ops.linear(x, b.mixer.w_gates, f32, bias=b.mixer.b_gates)) for b in mem], name="memory_gates",
-                    bytes_each=2.0 * elems(mm.w_gates) + rows * D * 2.0)
+                prod("memory_in_gates", [(lambda b=b: products(ops, [(x, b.mixer.w_in, bf, None), (x, b.mixer.w_gates, f32, b.mixer.b_gates)])) for b in mem], mm.w_in)
                 u = (torch.randn((rows, mm.w_in.shape[0]), device=dev) * 0.3).to(bf)
                 gates = torch.randn((rows, 2 * nh), device=dev)
                 S, nrm, mx = (cache.entry_state(e, "mixer." + s) for s in ("memory", "normalizer", "maximum"))

@@ -78,6 +78,14 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     return block_sum_once<THREADS>(v, red);
 }
 
+// a barrier that waits for LDS alone: loads and stores on their way to and from memory hold nobody up
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // ---- device: functions of the model ---------------------------------------------------------------
 __device__ __forceinline__ float gelu_tanh_f(float g) {
     return 0.5f * g * (1.0f + tanhf(0.7978845608f * (g + 0.044715f * g * g * g)));

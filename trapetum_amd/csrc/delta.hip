@@ -195,9 +195,8 @@ __device__ __forceinline__ void mma_terms(const DFrag (&a)[3], const DFrag (&b)[
     c = mma(a[2], b[0], c); d = mma(a[0], b[1], d);
     c = mma(a[1], b[0], c); d = mma(a[0], b[0], d);
 }
-// A barrier for what the waves pass through LDS.  (__syncthreads() would also wait for every load from memory that is
+// (What the waves pass through LDS goes behind lds_barrier(): __syncthreads() would also wait for every load from memory that is
 // under way, and a chunk's loads are asked for a chunk ahead.)
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // where head h of (sequence, chunk) c keeps its two matrices' terms, its scalars, and the kv head's K transposed
 __device__ __forceinline__ bf16_t* ws_terms(const DeltaArgs& x, size_t c, int h, int which) { return x.ws_mat + ((c * x.H + h) * 2 + which) * 3 * DC * DC; }
 __device__ __forceinline__ float* ws_scalars(const DeltaArgs& x, size_t c, int h) { return x.ws_scal + (c * x.H + h) * 4 * DC; }

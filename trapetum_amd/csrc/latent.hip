@@ -122,7 +122,7 @@ extern "C" int tp_latent_prepare(const void* proj, long proj_stride, int dtype, 
     TP_REQUIRE(!table || (pool && page > 0 && table_w > 0), "latent_prepare: a page table without a cache pool");
     if (!table) { page = 1; rows_cap = 0; }
     TP_REQUIRE(rows_cap >= 0 && (rows_cap == 0 || rows_cap % page == 0), "latent_prepare: ring of %d rows is no multiple of the page size %d", rows_cap, page);
-    TP_REQUIRE(rot * sizeof(float) <= 32768, "latent_prepare: %d turning elements are more than a head may have", rot);
+    TP_REQUIRE(rot <= 8192, "latent_prepare: %d turning elements are more than a head may have (8192)", rot);
     hipStream_t s = (hipStream_t)stream;
     const int items = dr - rot / 2, per_head = items > 256 ? 256 : items > 0 ? items : 1, at_once = 256 / per_head, heads = items ? H + !!own : 0;
     // Four heads a thread once that many still fill the chip: one angle then serves four heads.  Below, more blocks with one

@@ -30,13 +30,6 @@ static inline int tp_step_threads(int rows, int cols) {
     if (cols < 4 || cols > 256 || (cols & (cols - 1)) || rows > 256) return 0;
     return (long)rows * cols > 4096 ? 1024 : 256;
 }
-// the barrier of a block whose loads from memory go on: it waits for LDS alone
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 // four columns' sums of a thread, added over the wave's lanes of the same columns (Q column groups in turn), into the wave's part
 __device__ __forceinline__ void step_parts(float4 o, int Q, int lane, float* part) {
     for (int x = Q; x < 64; x <<= 1) {

@@ -206,13 +206,6 @@ extern "C" int tp_recent_push(const int* tokens, int* recent, int* cursor, int B
 // r = u * kept mass; falls back to the first candidate.  One block per row: a radix select over the value
 // bits finds the k-th largest logit, an id select breaks ties at that value, the at most 1024 candidates are
 // sorted in LDS, and the first wave does the short scans (sums in candidate order within a lane, then over the lanes). ---
-// a barrier that waits for LDS alone: stores on their way to memory hold nobody up
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 __device__ __forceinline__ uint32_t value_key(float f) {           // larger float -> larger key; NaN lowest
     uint32_t u = __float_as_uint(f);
     if ((u & 0x7fffffffu) > 0x7f800000u) return 0u;
