@@ -594,8 +594,9 @@ mm_outputs_k(MatrixMemoryArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; u++) { sq[u] = sn[u]; qq[u] = qn[u]; }
     }
+    const float first = scales[wave][r];                 // of the first tile: goes into its one addition
 #pragma unroll
-    for (int tt = 0; tt < 4; tt++) {
+    for (int tt = 1; tt < 4; tt++) {
         const float f = scales[wave][16 * tt + r];
 #pragma unroll
         for (int x = 0; x < 4; x++) acc[x][tt] *= f;
@@ -614,35 +615,33 @@ mm_outputs_k(MatrixMemoryArgs a) {
 #pragma unroll
             for (int x = 0; x < 4; x++) none = __builtin_fmaf(v[u][x], 0.f, none);
         const bool finite = !__any(none != 0.f);
-        if (!finite) {
-            const int t = 16 * kb + r;
-            mm_f32x4 p[4] = {};
-            for (int s = 16 * kb; s < min(16 * kb + 16, n); s++) {
-                const float w = P[t][s];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const mm_f32x4 value = quad<VEC>(vh + (size_t)(begin + s) * a.v_stride, j0 + 16 * g + 4 * e, dv);
-#pragma unroll
-                    for (int x = 0; x < 4; x++) p[x][e] = s <= t ? __builtin_fmaf(value[x], w, p[x][e]) : p[x][e];
-                }
-            }
-#pragma unroll
-            for (int x = 0; x < 4; x++) acc[x][kb] += p[x];
-        }
 #pragma unroll
         for (int tt = kb; tt < 4; tt++) {
             if (tt >= tiles) break;
-            if (tt == kb && !finite) continue;
-            float w[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) w[u] = P[16 * tt + r][16 * kb + 4 * u + g];
             mm_f32x4 p[4] = {};
+            if (tt == kb && !finite) {
+                for (int s = 16 * kb; s < min(16 * kb + 16, n); s++) {
+                    const float w = P[16 * kb + r][s];
 #pragma unroll
-            for (int u = 0; u < 4; u++)
+                    for (int e = 0; e < 4; e++) {
+                        const mm_f32x4 value = quad<VEC>(vh + (size_t)(begin + s) * a.v_stride, j0 + 16 * g + 4 * e, dv);
 #pragma unroll
-                for (int x = 0; x < 4; x++) p[x] = mm_mfma(v[u][x], w[u], p[x]);
+                        for (int x = 0; x < 4; x++) p[x][e] = s <= 16 * kb + r ? __builtin_fmaf(value[x], w, p[x][e]) : p[x][e];
+                    }
+                }
+            } else {
+                float w[4];
 #pragma unroll
-            for (int x = 0; x < 4; x++) acc[x][tt] += p[x];
+                for (int u = 0; u < 4; u++) w[u] = P[16 * tt + r][16 * kb + 4 * u + g];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) p[x] = mm_mfma(v[u][x], w[u], p[x]);
+            }
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[x][tt][e] = tt == 0 ? __builtin_fmaf(acc[x][tt][e], first, p[x][e]) : acc[x][tt][e] + p[x][e];
         }
     }
 #pragma unroll
