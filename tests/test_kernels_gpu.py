@@ -1008,6 +1008,41 @@ def test_attention_decode_of_one_long_sequence_among_short_ones(ops, H, KV, hd, 
     assert rel_l2(got[:1], alone) < 8e-3
 
 
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("H,KV,hd", [(8, 4, 256), (3, 3, 64), (8, 2, 96), (16, 2, 240), (2, 2, 16)])
+def test_attention_decode_of_few_keys_in_one_launch(ops, H, KV, hd, fused):
+    """Up to WHOLE_KEYS keys a block has them all: at and beside a tile's, a page's, a round's and the launch's last key, behind a
+    window, in a ring; fused, the new token's row of the cache holds NaN until the launch writes it.  bfloat16 probabilities are not
+    rounded, so the result is off by the rounding of queries, keys and outputs: 2^-8 each at most, 2^-8 (1 + 1 / sqrt(hd)) in norm."""
+    lens, page = (1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 177, 191, 192), 64
+    n, width = len(lens), (H + 2 * KV) * hd
+    inv_freq = (10000.0 ** (-torch.arange(hd // 2).float() / (hd // 2))).contiguous()
+    for window, rows_cap in ((0, 0), (100, 0), (100, 128)):
+        per = 2 if rows_cap else 3
+        table = torch.randperm(n * per, generator=torch.Generator().manual_seed(7)).to(torch.int32).view(n, per)
+        pools = [randn(n * per, KV, page, hd, dtype=torch.bfloat16, seed=30 + i).cpu() for i in range(2)]
+        held = torch.tensor(lens, dtype=torch.int32)
+        rows = randn(n, width, dtype=torch.bfloat16, seed=33).cpu()
+        if fused:
+            ref = ref_ops.attention_decode_step(rows.float(), H, KV, hd, inv_freq, hd, held, table, pools[0].clone(), pools[1].clone(), rows_cap,
+                                                hd ** -0.5, 30.0, window, torch.float32)
+            for i, l in enumerate(lens):
+                r = (l - 1) % rows_cap if rows_cap else l - 1
+                for p in pools:
+                    p[int(table[i, r // page]), :, r % page] = math.nan
+        else:
+            ref = ref_ops.attention_decode(rows[:, :H * hd].contiguous(), H, KV, hd, held, table, pools[0], pools[1], rows_cap, hd ** -0.5, 30.0, window, torch.float32)
+        dev = [p.to(DEV) for p in pools]
+        common = (held.to(DEV), table.to(DEV), *dev, rows_cap, hd ** -0.5, 30.0, window, torch.bfloat16)
+        assert ops._decode_slices(None, n, KV, H, hd, max(lens)) == 0
+        if fused:
+            got = ops.attention_decode_step(rows.to(DEV), H, KV, hd, inv_freq.to(DEV), hd, *common, max_keys=max(lens))
+            assert all(bool(torch.isfinite(p.float()).all()) for p in dev)
+        else:
+            got = ops.attention_decode(rows[:, :H * hd].contiguous().to(DEV), H, KV, hd, *common, max_keys=max(lens))
+        assert rel_l2(got, ref) < 2 ** -8 * (1 + hd ** -0.5) + 2e-3, (window, rows_cap)
+
+
 def test_attention_far_key_stands_out(ops):
     """One key among hundreds carries the answer: its score is made to dominate, so a kernel that drops
     or misplaces it (a chunk boundary, a page boundary) returns another value row."""

@@ -515,8 +515,7 @@ def time_vogunex_kernels(engine, cfg, batch, context, prefill_tokens):
                     keys = min(context, mx.window)
                     per = next(g for g in (mx.DECODE_GROUP_LONG if keys >= mx.LONG_KEYS else mx.DECODE_GROUP, 4, 2, 1) if H % g == 0)
                     one([lambda: ops.attention_decode(q, H, 1, lrow, ctx.new_len, table, pool, pool, cap, mx.scale, 0.0, mx.window, bf,
-                                                      max_keys=ctx.max_rows_visible(site), head_groups=H // per,
-                                                      splits=ops.decode_splits(batch * (H // per), 1, lrow, keys))] * 8,
+                                                      max_keys=ctx.max_rows_visible(site), head_groups=H // per)] * 8,
                         name=f"latent_attention_{keys}_keys", bytes_each=2.0 * batch * keys * lrow)
                 else:
                     pairs = sum(min(p + 1, mx.window) for p in range(rows))
@@ -720,7 +719,7 @@ def time_golepel_kernels(engine, cfg, batch, context, prefill_tokens):
                 # as the mixer calls it: the heads in groups that each read the shared cached rows
                 per = next(g for g in (mx.DECODE_GROUP_LONG if context >= mx.LONG_KEYS else mx.DECODE_GROUP, 4, 2, 1) if H % g == 0)
                 one([lambda: ops.attention_decode(q, H, 1, row, ctx.new_len, table, pool, pool, 0, mx.scale, 0.0, 0, bf, max_keys=context,
-                                                  head_groups=H // per, splits=ops.decode_splits(batch * (H // per), 1, row, context))] * 8,
+                                                  head_groups=H // per)] * 8,
                     name=f"attention_ctx{context}", bytes_each=2.0 * batch * context * row)
             else:
                 pairs = rows * (rows + 1) / 2.0

@@ -70,6 +70,10 @@ __device__ __forceinline__ bf16_t bf16_bits(float f) {
 // chunks are fetched together with its key rows, before the scores are known, so the two latencies overlap.  Slices of the keys
 // (flash-decoding) write (max, sum, unnormalised output) to a workspace that a second kernel combines in
 // slice order.
+// Few keys (nsplit 0): a block of eight waves has all of them and writes the result itself.  What such a step waits for is
+// launches and trips to memory, not keys: the combination was a launch of 3 us for slices most of which were empty (chats of 1 / 64 up to
+// 60 keys: 9.8 / 11.8 us a layer in slices, 6.8 / 8.4 so; up to where: HipOps._decode_slices), and the new token's key and value, which the block
+// has just made, come from LDS instead of back from the cache.
 // =====================================================================================================
 struct DecodeArgs {
     const bf16_t* q; long q_stride; int H, KV; const int* new_len; const int* table; int table_w;
@@ -95,20 +99,23 @@ namespace {
 // of a key row fetch a whole 128-byte line per pair: step ks, lane group g -> head elements dofs .. dofs + 7.
 constexpr int DSTEPS = 2 * ((HD + 63) / 64);
 __device__ __forceinline__ int dofs(int ks, int g) { return (ks >> 1) * 64 + g * 16 + (ks & 1) * 8; }
-constexpr int DTH = 256;                         // 4 waves; each scores and sums its own 16 keys of a round
-constexpr int ROUND = 64;                        // keys a block takes per round
+constexpr int DWAVES = 4;                        // waves of a block that works on a slice; each scores and sums its own 16 keys of a round
+constexpr int WHOLE_WAVES = 8;                   // waves of a block that has all keys of its kv head (a launch without slices)
 constexpr int KGW = 64 / NCH > 16 ? 16 : 64 / NCH;   // key groups of a wave: lanes with one chunk index walk the keys KGW apart
 constexpr int VPT = (16 + KGW - 1) / KGW;        // value chunks a lane fetches per round
 }
 
-template <int QT>
-__global__ void __launch_bounds__(DTH)
+template <int QT, int WAVES = DWAVES>
+__global__ void __launch_bounds__(64 * WAVES)
 attn_decode_k(DecodeArgs a) {
-    __shared__ float p_lds[4][QT][16];               // a wave's probabilities of its 16 keys
-    __shared__ float alpha_lds[4][QT];
-    __shared__ float m_w[4][QT], l_w[4][QT];
-    __shared__ float red[4 * KGW * HD];
-    __shared__ __attribute__((aligned(16))) bf16_t q_lds[QT * HD];
+    constexpr int DTH = 64 * WAVES, ROUND = 16 * WAVES;        // threads; keys a block takes per round
+    constexpr bool WHOLE = WAVES > DWAVES;           // no slices: the block has all keys, one round of them or two
+    constexpr int RQ = WHOLE && QT > 1 ? 2 : 1;      // heads whose parts are added at a time
+    __shared__ float p_lds[WAVES][QT][16];           // a wave's probabilities of its 16 keys
+    __shared__ float alpha_lds[WAVES][QT];
+    __shared__ __attribute__((aligned(16))) float m_w[WHOLE ? QT : WAVES][WHOLE ? WAVES : QT], l_w[WHOLE ? QT : WAVES][WHOLE ? WAVES : QT];
+    __shared__ float red[RQ * WAVES * KGW * HD];
+    __shared__ __attribute__((aligned(16))) bf16_t q_lds[QT * HD], new_lds[WHOLE ? 2 * HD : 8];      // queries; the new key and value
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
     const int G = a.H / a.KV;
@@ -190,7 +197,7 @@ attn_decode_k(DecodeArgs a) {
     bf16x8 kf[DSTEPS];
     Frag vf[VPT];
     const int tb0 = t_begin + wave * 16;
-    const bool late = a.qkv && a.write_kv && tb0 < places && places - 1 < tb0 + 16;
+    const bool holds_new = a.qkv && a.write_kv && tb0 < places && places - 1 < tb0 + 16, late = !WHOLE && holds_new;
     if (tb0 < t_end && !late) load_round(tb0, kf, vf);
 
     // ---- the group's queries into LDS; in the fused form from the step's projections: K slices added, queries and
@@ -251,10 +258,11 @@ attn_decode_k(DecodeArgs a) {
             q_lds[qi * HD + f] = f32_to_bf16(x[0] * cs - x[1] * sn);
             q_lds[qi * HD + f + half] = f32_to_bf16(x[1] * cs + x[0] * sn);
             if (kv) {
-                kdst[f] = f32_to_bf16(x[2] * cs - x[3] * sn);
-                kdst[f + half] = f32_to_bf16(x[3] * cs + x[2] * sn);
-                vdst[f] = f32_to_bf16(x[4]);
-                vdst[f + half] = f32_to_bf16(x[5]);
+                const bf16_t k0 = f32_to_bf16(x[2] * cs - x[3] * sn), k1 = f32_to_bf16(x[3] * cs + x[2] * sn);
+                const bf16_t v0 = f32_to_bf16(x[4]), v1 = f32_to_bf16(x[5]);
+                kdst[f] = k0; kdst[f + half] = k1;
+                vdst[f] = v0; vdst[f + half] = v1;
+                if constexpr (WHOLE) { new_lds[f] = k0; new_lds[f + half] = k1; new_lds[HD + f] = v0; new_lds[HD + f + half] = v1; }
             }
         }
         for (int idx = tid; idx < G * rest; idx += DTH) {         // elements outside the rotation
@@ -266,8 +274,10 @@ attn_decode_k(DecodeArgs a) {
             else vals(std::integral_constant<int, 1>(), cols, x);
             q_lds[qi * HD + d] = f32_to_bf16(x[0]);
             if (kv) {
-                kdst[d] = f32_to_bf16(x[1]);
-                vdst[d] = f32_to_bf16(x[2]);
+                const bf16_t k0 = f32_to_bf16(x[1]), v0 = f32_to_bf16(x[2]);
+                kdst[d] = k0;
+                vdst[d] = v0;
+                if constexpr (WHOLE) { new_lds[d] = k0; new_lds[HD + d] = v0; }
             }
         }
         if (writer) __threadfence_block();
@@ -287,6 +297,25 @@ attn_decode_k(DecodeArgs a) {
         f.u.x &= keep; f.u.y &= keep; f.u.z &= keep; f.u.w &= keep;
         qf[ks] = f.v;
     }
+    // (WHOLE: the row that this block is writing comes from LDS; the one trip to memory was on the way meanwhile, and what lay in its
+    // place is not looked at: rows of the tile past it read the same row)
+    auto take_new = [&](int tb) {
+        if constexpr (WHOLE) {
+            const int t0 = tb < kept_al ? tb : tb + gap;
+            if (!(a.qkv && a.write_kv && tb < places && places - 1 < tb + 16)) return;
+            if (row_in_tile(t0, t0 + c) == p)
+#pragma unroll
+                for (int ks = 0; ks < DSTEPS; ks++) {
+                    const int d0 = dofs(ks, g);
+                    kf[ks] = ld_frag(new_lds + (d0 < HD ? d0 : 0), d0 < HD);
+                }
+#pragma unroll
+            for (int j = 0; j < VPT; j++) {
+                const int kk = kgw + j * KGW > 15 ? 15 : kgw + j * KGW;
+                if (row_in_tile(t0, t0 + kk) == p) vf[j].u = *reinterpret_cast<const uint4*>(new_lds + HD + ch * 8);
+            }
+        }
+    };
     float acc[QT][8];
 #pragma unroll
     for (int qi = 0; qi < QT; qi++)
@@ -299,6 +328,7 @@ attn_decode_k(DecodeArgs a) {
 
     for (int tb = tb0; tb < t_end; tb += ROUND) {
         if (tb != tb0 || late) load_round(tb, kf, vf);
+        take_new(tb);
         // ---- scores of 16 keys for the group's query heads: lane (c, g) gets keys g*4 .. g*4+3 of head c ----------
         f32x4 s = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -360,7 +390,59 @@ attn_decode_k(DecodeArgs a) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }
-    // ---- the four waves' results: rescale to a common maximum, add in wave and key-group order, write -------------
+    // ---- the waves' results: rescale to a common maximum, add in wave and key-group order, write -------------
+    if constexpr (WHOLE) {
+        const int used = min(WAVES, (t_end - t_begin + 15) >> 4);       // waves that had keys (the others leave -infinity and zeros)
+        if (c < QT && g == 0) { m_w[c][wave] = m_run; l_w[c][wave] = l_run; }
+#pragma unroll
+        for (int q0 = 0; q0 < QT; q0 += RQ) {
+            if (q0 >= G) continue;
+            if (q0 > 0) __syncthreads();
+            if (pv_lane)
+#pragma unroll
+                for (int u = 0; u < RQ; u++)
+#pragma unroll
+                    for (int e = 0; e < 8; e += 4)
+                        *reinterpret_cast<float4*>(red + ((u * WAVES + wave) * KGW + kgw) * HD + ch * 8 + e) = make_float4(acc[q0 + u][e], acc[q0 + u][e + 1], acc[q0 + u][e + 2], acc[q0 + u][e + 3]);
+            __syncthreads();
+            for (int idx = tid; idx < RQ * HD; idx += DTH) {
+                const int u = idx / HD, d = idx - u * HD, qi = q0 + u;
+                if (qi >= G) break;
+                float m[WAVES], l[WAVES], mx = -INFINITY, num = 0.f, den = 0.f;
+#pragma unroll
+                for (int w = 0; w < WAVES; w += 4) {
+                    *reinterpret_cast<float4*>(m + w) = *reinterpret_cast<const float4*>(&m_w[qi][w]);
+                    *reinterpret_cast<float4*>(l + w) = *reinterpret_cast<const float4*>(&l_w[qi][w]);
+                }
+#pragma unroll
+                for (int w = 0; w < WAVES; w++) mx = fmaxf(mx, m[w]);
+#pragma unroll
+                for (int w0 = 0; w0 < WAVES; w0 += 4) {
+                    if (w0 >= used) break;
+                    float part[4][KGW];
+#pragma unroll
+                    for (int w = 0; w < 4; w++)
+#pragma unroll
+                        for (int k2 = 0; k2 < KGW; k2++) part[w][k2] = red[((u * WAVES + w0 + w) * KGW + k2) * HD + d];
+#pragma unroll
+                    for (int w = 0; w < 4; w++) {
+                        const float f = __expf(m[w0 + w] - mx);
+                        float sum = 0.f;
+#pragma unroll
+                        for (int k2 = 0; k2 < KGW; k2++) sum += part[w][k2];
+                        num += f * sum;
+                        den += f * l[w0 + w];
+                    }
+                }
+                const int head = kvh * G + qi;
+                if (a.sink) den += __expf(a.sink[head] - mx);                 // (the query's own key is among them: mx is finite)
+                float o = num / den;
+                if constexpr (BY_POSITION) if (a.by_position.gate) o *= head_gate(a.by_position, seq, head);
+                a.out[((size_t)seq * a.H + head) * HD + d] = f32_to_bf16(o);
+            }
+        }
+        return;
+    } else {
     if (c < QT && g == 0) { m_w[wave][c] = m_run; l_w[wave][c] = l_run; }
 #pragma unroll
     for (int qi = 0; qi < QT; qi++) {
@@ -396,6 +478,7 @@ attn_decode_k(DecodeArgs a) {
             }
         }
         __syncthreads();
+    }
     }
 }
 
@@ -477,6 +560,9 @@ static int decode_launch(DecodeArgs a, int n_seq, void* workspace, hipStream_t s
     const int reach = a.window > 0 && a.chunk > 0 ? (a.window < a.chunk ? a.window : a.chunk) : (a.window > 0 ? a.window : a.chunk);
     TP_REQUIRE(a.rows_cap == 0 || (reach > 0 && reach <= a.rows_cap - a.pin), "attention decode: a reach of %d keys (window %d, chunk %d) does not fit a ring of %d rows", reach, a.window, a.chunk, a.rows_cap - a.pin);
     TP_REQUIRE(a.rows_cap >= 0 && a.rows_cap % a.page == 0, "attention decode: ring of %d rows is no multiple of the page size %d", a.rows_cap, a.page);
+    const bool whole = a.nsplit == 0;
+    if (whole) a.nsplit = 1;
+    TP_REQUIRE(!whole || G <= 8, "attention decode: %d query heads per kv head exceed the 8 of a block with all keys", G);
     TP_REQUIRE(a.nsplit >= 1 && a.nsplit <= 128 && (a.nsplit == 1 || workspace), "attention decode: %d slices (at most 128) need a workspace", a.nsplit);
     TP_REQUIRE(a.KV <= 65535 && n_seq <= 65535, "attention decode: grid too large");
     if (a.nsplit > 1) {
@@ -484,6 +570,14 @@ static int decode_launch(DecodeArgs a, int n_seq, void* workspace, hipStream_t s
         a.ws_ml = a.ws_o + (size_t)n_seq * a.H * a.nsplit * HD;
     }
     dim3 grid(a.KV, n_seq, a.nsplit);
+    if (whole) {
+        if (G <= 1) attn_decode_k<1, WHOLE_WAVES><<<grid, 64 * WHOLE_WAVES, 0, s>>>(a);
+        else if (G <= 2) attn_decode_k<2, WHOLE_WAVES><<<grid, 64 * WHOLE_WAVES, 0, s>>>(a);
+        else if (G <= 4) attn_decode_k<4, WHOLE_WAVES><<<grid, 64 * WHOLE_WAVES, 0, s>>>(a);
+        else attn_decode_k<8, WHOLE_WAVES><<<grid, 64 * WHOLE_WAVES, 0, s>>>(a);
+        return tp_check_launch("attention decode (whole)");
+    }
+    constexpr int DTH = 64 * DWAVES;
     if (G <= 1) attn_decode_k<1><<<grid, DTH, 0, s>>>(a);
     else if (G <= 2) attn_decode_k<2><<<grid, DTH, 0, s>>>(a);
     else if (G <= 4) attn_decode_k<4><<<grid, DTH, 0, s>>>(a);

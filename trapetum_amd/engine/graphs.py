@@ -3,8 +3,8 @@
 A decode step is some three hundred small launches; replaying them from a graph removes the host's share of
 the step (the reference reports the same lever for its own loop: runtime/README.md:49-58, and wraps capture
 and replay in `Graph`, runtime/src/lib.rs:1211-1236).  A graph is captured for a batch size out of a few (powers
-of two), for a bound on the lengths of its sequences (1024, 2048, ...: launch geometry that depends on lengths,
-the slices of the decode attention, is sized for the bound) and for one way of choosing the next tokens (none,
+of two), for a bound on the lengths of its sequences (192, 1024, 2048, ...: launch geometry that depends on lengths,
+the slices of the decode attention, is sized for the bound, and up to the first there are none) and for one way of choosing the next tokens (none,
 argmax, or sampling with given constants), which is part of the graph: it leaves the chosen ids where its next
 replay reads its tokens, so a generation loop needs neither a launch nor a copy between replays.  A batch of
 fewer sequences than the graph has rows fills the rest with rows that stand for no sequence: they read and write
@@ -20,6 +20,7 @@ import collections
 import numpy as np
 import torch
 
+from ..kernels.ops import WHOLE_KEYS
 from ..sampling.sampler import RECENT_WINDOW
 from .batch import StaticStep, StepContext, step_arrays
 
@@ -33,7 +34,7 @@ def graph_rows(n):
 
 
 def length_bound(longest, max_context):
-    bound = 1024
+    bound = WHOLE_KEYS if longest <= WHOLE_KEYS else 1024
     while bound < longest:
         bound *= 2
     return min(bound, max_context)
@@ -57,7 +58,7 @@ class _Captured:
 
 
 class GraphedDecode:
-    def __init__(self, model, cache, max_graphs=16):
+    def __init__(self, model, cache, max_graphs=24):
         if model.rt.device.type != "cuda":
             raise RuntimeError("HIP graphs need the GPU")
         self.model = model

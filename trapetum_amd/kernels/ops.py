@@ -93,6 +93,9 @@ BIAS_ACTIVATIONS = {None: 0, "gelu_erf": 1}          # what `bias_act` applies a
 GATE_GROUP = 16
 
 
+WHOLE_KEYS = 192               # keys up to which a decode step's attention is one launch without slices (HipOps._decode_slices)
+
+
 class KernelError(RuntimeError):
     """A kernel refused its operands, or the library could not be loaded."""
 
@@ -1321,6 +1324,20 @@ class HipOps:
             slices = whole
         return max(1, min(slices, -(-keys // (64 * rounds)), 128))
 
+    # Up to this many keys a block of eight waves has all keys of a pair of sequence and kv head, and nothing is left to combine
+    # (the kernel's 0 slices).  It walks 128 keys a round.  Microseconds of a layer, slices and their combination / whole, heads of 256,
+    # 2 heads a block, sequences x kv heads 1 x 4, 8 x 4, 64 x 4 and 64 x 8: 60 keys 9.8 / 6.8, 10.0 / 7.0, 11.8 / 8.4, 16.3 / 16.6; 128 keys 9.7 / 8.1, 10.7 / 8.8,
+    # 16.1 / 12.8, 24.2 / 23.7; 190 keys 9.8 / 9.9, 10.7 / 10.8, 18.6 / 15.7, 29.2 / 28.5; 256 keys 9.7 / 11.3, 10.7 / 12.1, 22.9 / 19.4, 36.6 / 35.7.  Eight heads a
+    # block, 1 x 2: 15.5 / 10.6, 15.4 / 13.2, 15.4 / 15.6, 15.4 / 16.9.  From WHOLE_PAIRS pairs on there is a slice of four waves each anyway.
+    WHOLE_KEYS, WHOLE_GROUP, WHOLE_PAIRS = WHOLE_KEYS, 8, 768
+
+    def _decode_slices(self, splits, n, KV, H, hd, keys):
+        if splits:
+            return int(splits)
+        if keys <= self.WHOLE_KEYS and H // KV <= self.WHOLE_GROUP and n * KV < self.WHOLE_PAIRS:
+            return 0
+        return self.decode_splits(n, KV, hd, keys)
+
     def _check_pools(self, what, dtype, n, KV, hd, new_len, table, k_pool, v_pool):
         if new_len.numel() != n or new_len.dtype != torch.int32:
             raise KernelError(f"{what}: one int32 length per sequence")
@@ -1355,7 +1372,7 @@ class HipOps:
         if self._fast_attention(q.dtype, H, groups, hd) and page >= 16 and page & (page - 1) == 0 and not (own_groups and groups != KV):
             lib = self.attn_lib(hd, by_position=pos is not None)
             keys = int(max_keys) if max_keys else k_pool.shape[0] * k_pool.shape[2]
-            nsplit = int(splits) if splits else self.decode_splits(n, groups, hd, keys)
+            nsplit = self._decode_slices(splits, n, groups, H, hd, keys)
             floats = lib.tp_attn_decode_workspace_floats(n, H, nsplit)
             ws = torch.empty(floats, dtype=torch.float32, device=self.device) if floats else None
             if groups != KV:
@@ -1416,7 +1433,7 @@ class HipOps:
         pos = self._positional("attention_decode_step", by_position, H, n, step=(rows.data_ptr(), rows.dtype, n_slices, slice_stride, row_stride))
         lib = self.attn_lib(hd, by_position=pos is not None)
         keys = int(max_keys) if max_keys else k_pool.shape[0] * k_pool.shape[2]
-        nsplit = int(splits) if splits else self.decode_splits(n, KV, hd, keys)
+        nsplit = self._decode_slices(splits, n, KV, H, hd, keys)
         floats = lib.tp_attn_decode_workspace_floats(n, H, nsplit)
         ws = torch.empty(floats, dtype=torch.float32, device=self.device) if floats else None
         out = torch.empty((n, H * hd), dtype=out_dtype, device=self.device)

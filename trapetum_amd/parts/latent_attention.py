@@ -173,8 +173,7 @@ class LatentAttention(Mixer):
             keys = ctx.max_rows_visible(site)
             per = next(g for g in (self.DECODE_GROUP_LONG if keys >= self.LONG_KEYS else self.DECODE_GROUP, 4, 2, 1) if H % g == 0)
             out = ops.attention_decode(q, H, 1, row, ctx.new_len, table, pool, pool, rows_cap, self.scale, 0.0, self.window,
-                                       ctx.dtype, max_keys=keys, head_groups=H // per,
-                                       splits=ops.decode_splits(m * (H // per), 1, row, keys), **more)
+                                       ctx.dtype, max_keys=keys, head_groups=H // per, **more)
         else:
             if owns:
                 ctx.offer_step_rows(latent=mine)
