@@ -1222,3 +1222,23 @@ def test_repetition_penalty(ops, vocab, window):
     untouched = z.cpu().clone()
     ops.apply_repetition_penalty(z, recent.to(DEV), 1.0)     # 1.0 switches it off
     assert torch.equal(z.cpu(), untouched)
+
+
+@pytest.mark.parametrize("kind", ["capped", "narrow", "levels", "nan", "masked", "sorted", "lowest"])
+def test_sample_by_groups_is_the_sampler_alone(ops, kind):
+    """Sampling over the groups' largest keys against the same call without a workspace, which reads whole rows by one block each: the
+    same tokens, at the smallest row that is cut into groups, groups of 2 to 128, either number of them, and lists that overflow."""
+    for rows, vocab in ((2, 8192), (3, 8195), (1, 20480), (3, 32000), (2, 100001), (2, 262144), (1, 262145), (1, 300001)):
+        z = torch.randn(rows, vocab, generator=torch.Generator().manual_seed(vocab)) * 2.0
+        if kind == "capped": z = 30.0 * torch.tanh(z / 30.0)
+        if kind == "narrow": z = z * 0.05 + 100.0
+        if kind == "levels": z = torch.round(z * 2.0) / 2.0
+        if kind == "nan": z[:, ::7], z[:, 5], z[-1, 11] = math.nan, -math.inf, math.inf
+        if kind == "masked": z[:, vocab // 3:] = -math.inf
+        if kind == "sorted": z = torch.sort(z, dim=1, descending=True).values.contiguous()
+        if kind == "lowest": z[:, 40:] = torch.finfo(torch.float32).min
+        z, u = z.to(DEV), torch.rand(rows, generator=torch.Generator().manual_seed(3)).to(DEV)
+        for top_k, top_p in ((0, 1.0), (1, 0.9), (256, 0.95), (512, 1.0), (513, 0.95), (1024, 1.0)):
+            alone = torch.empty(rows, dtype=torch.int32, device=DEV)
+            assert ops.lib.tp_sample(z.data_ptr(), rows, vocab, 0.8, top_k, top_p, u.data_ptr(), alone.data_ptr(), None, ops._stream()) == 0
+            assert torch.equal(ops.sample(z, 0.8, top_k, top_p, u), alone), (rows, vocab, top_k)

@@ -219,12 +219,14 @@ __device__ __forceinline__ float key_value(uint32_t k) {
 // ---- the sampler's short scans, done by the block's first wave (a single thread walking LDS pays its latency per
 // element: 45 us for 256 candidates) -----------------------------------------------------------------------------
 __device__ __forceinline__ unsigned wave_scan_incl(unsigned v, int lane) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const unsigned t = (unsigned)__shfl_up((int)v, o, 64);
-        if (lane >= o) v += t;
-    }
-    return v;
+    // within rows of 16 by moves (zeros come in from the left), then each row's last on to the rows behind it
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    const unsigned r0 = (unsigned)__builtin_amdgcn_readlane((int)v, 15), r1 = (unsigned)__builtin_amdgcn_readlane((int)v, 31), r2 = (unsigned)__builtin_amdgcn_readlane((int)v, 47);
+    const int row = lane >> 4;
+    return v + (row > 0 ? r0 : 0u) + (row > 1 ? r1 : 0u) + (row > 2 ? r2 : 0u);
 }
 __device__ __forceinline__ float wave_scan_incl(float v, int lane) {
 #pragma unroll
@@ -275,37 +277,71 @@ __device__ __forceinline__ uint32_t across(uint32_t v, int lane) {
         return lane & 32 ? r[0] : r[1];
     }
 }
-template <int STRIDE>
-__device__ __forceinline__ void sort_step(uint32_t& key, int& id, int tid, int size) {
-    const uint32_t ok = across<STRIDE>(key, tid), oi = across<STRIDE>((uint32_t)id, tid);
-    const bool before = key > ok || (key == ok && id < (int)oi);               // this thread's element belongs before the other
-    const bool wants_first = ((tid & STRIDE) == 0) == ((tid & size) == 0);
-    if (before != wants_first) { key = ok; id = (int)oi; }
+__device__ __forceinline__ int wave_least(int v, int lane) {
+    v = min(v, (int)across<32>((uint32_t)v, lane));
+    v = min(v, (int)across<16>((uint32_t)v, lane));
+    v = min(v, (int)across<8>((uint32_t)v, lane));
+    v = min(v, (int)across<4>((uint32_t)v, lane));
+    v = min(v, (int)across<2>((uint32_t)v, lane));
+    return min(v, (int)across<1>((uint32_t)v, lane));
 }
+// A candidate as one number, larger first: its value key, then the smaller id.
+__device__ __forceinline__ unsigned long long packed(uint32_t key, int id) { return (unsigned long long)key << 32 | (uint32_t)~id; }
 
-// Sorts the block's elements, one a thread (key, id), by (key descending, id ascending), over the first `n` threads (a power of
-// two from 64 to 1024): a bitonic network whose exchanges within a wave stay in registers, so that only the strides of 64 and more
-// meet in LDS (10 of 55 rounds at 1,024 elements, 6 of 45 at 512).  Waves beyond n keep their elements.
-__device__ __forceinline__ void block_sort(uint32_t& key, int& id, int n, uint32_t* lkey, int* lid) {
-    const int tid = threadIdx.x;
-    for (int size = 2; size <= n; size <<= 1) {
+// lanes whose bit STRIDE is clear
+__device__ constexpr unsigned long long lanes_below(int stride) {
+    unsigned long long m = 0;
+    for (int l = 0; l < 64; l++) if (!(l & stride)) m |= 1ull << l;
+    return m;
+}
+// One exchange: lanes of the mask `firsts` keep the larger of their element and that of lane ^ STRIDE, the others the smaller.
+template <int STRIDE>
+__device__ __forceinline__ void sort_step(unsigned long long& e, int lane, unsigned long long firsts) {
+    const unsigned long long o = (unsigned long long)across<STRIDE>((uint32_t)(e >> 32), lane) << 32 | across<STRIDE>((uint32_t)e, lane);
+    if (__builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_ballot_w64(e > o) ^ firsts)) e = o;
+}
+template <int SIZE, int STRIDE>
+__device__ __forceinline__ void sort_within(unsigned long long& e, int lane) {       // stage SIZE (up to 32) of a wave, from STRIDE down
+    constexpr unsigned long long firsts = ~(lanes_below(STRIDE) ^ lanes_below(SIZE));
+    sort_step<STRIDE>(e, lane, firsts);
+    if constexpr (STRIDE > 1) sort_within<SIZE, STRIDE / 2>(e, lane);
+}
+// the stages from `size` up to n of a bitonic network over the first n threads; those below 64 lie behind every wave already
+__device__ __forceinline__ void sort_stages(unsigned long long& e, int size, int n, unsigned long long* lds) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    int at = 0;                                                        // two places in turn: a round's reads are over before the next but one writes
+    lds_barrier();
+    for (; size <= n; size <<= 1) {
         for (int stride = size >> 1; stride >= 64; stride >>= 1) {
+            lds[at + tid] = e;
             lds_barrier();
-            lkey[tid] = key;
-            lid[tid] = id;
-            lds_barrier();
-            const uint32_t ok = lkey[tid ^ stride];
-            const int oi = lid[tid ^ stride];
-            const bool before = key > ok || (key == ok && id < oi), wants_first = ((tid & stride) == 0) == ((tid & size) == 0);
-            if (before != wants_first) { key = ok; id = oi; }
+            const unsigned long long o = lds[at + (tid ^ stride)];
+            at ^= 1024;
+            if ((e > o) != (((tid & stride) == 0) == ((tid & size) == 0))) e = o;
         }
-        if (size > 32) sort_step<32>(key, id, tid, size);
-        if (size > 16) sort_step<16>(key, id, tid, size);
-        if (size > 8) sort_step<8>(key, id, tid, size);
-        if (size > 4) sort_step<4>(key, id, tid, size);
-        if (size > 2) sort_step<2>(key, id, tid, size);
-        sort_step<1>(key, id, tid, size);
+        if (tid >= n) continue;                                        // (whole waves: they would take the others' issue slots)
+        const unsigned long long turn = __builtin_amdgcn_readfirstlane(tid & size) ? ~0ull : 0ull;
+        sort_step<32>(e, lane, lanes_below(32) ^ turn);
+        sort_step<16>(e, lane, lanes_below(16) ^ turn);
+        sort_step<8>(e, lane, lanes_below(8) ^ turn);
+        sort_step<4>(e, lane, lanes_below(4) ^ turn);
+        sort_step<2>(e, lane, lanes_below(2) ^ turn);
+        sort_step<1>(e, lane, lanes_below(1) ^ turn);
     }
+}
+// Sorts the block's elements, one a thread, larger first, over the first n threads (a power of two from 64 to 1024): exchanges
+// within a wave stay in registers, so that only strides of 64 and more meet in LDS (10 of 55 rounds at 1,024 elements, 6 of 45 at
+// 512).  Key and id compared as one number, and masks known when compiled: 45 rounds take 4.4 us less than compared one after the other.
+__device__ __forceinline__ void block_sort(unsigned long long& e, int n, unsigned long long* lds) {
+    const int lane = threadIdx.x & 63;
+    if ((int)threadIdx.x < n) {
+        sort_within<2, 1>(e, lane);
+        sort_within<4, 2>(e, lane);
+        sort_within<8, 4>(e, lane);
+        sort_within<16, 8>(e, lane);
+        sort_within<32, 16>(e, lane);
+    }
+    sort_stages(e, 64, n, lds);
 }
 
 // The rows' uniform numbers: an array on the device, or (null) up to TP_HOST_UNIFORMS of them that came with the launch, which saves a
@@ -314,46 +350,222 @@ __device__ __forceinline__ void block_sort(uint32_t& key, int& id, int n, uint32
 struct Draws { const float* at; float v[TP_HOST_UNIFORMS]; };
 __device__ __forceinline__ float draw_of(const Draws& d, int row) { return d.at ? d.at[row] : d.v[row]; }
 
-// With a candidate list (cand_count non-null): row b's candidates are cand_val/cand_id[b * cand_cap ..], a superset
-// of its top_k if their number fits cand_cap; the kernel then works on the list, else on the whole row.
+// ---- groups: a row of many logits is read once, by many blocks, which leave the largest key of every group of 2^shift neighbours (at
+// most GROUPS groups).  If t is the k-th largest of these, k logits are at least t, so the k largest all lie in groups whose
+// largest is at least t: the sampler looks at little more than k groups and has hardly more than k candidates, whatever the logits'
+// range.  (Before: a histogram of the top 12 key bits over many blocks, then everything from the bin of the k-th up copied to a list by many
+// blocks, then the sampler.  Microseconds, 8 rows of 256,000, k 256: 5.9 + 10.2 + 10.0 so, 4.0 + 13.3 here; the call
+// for 1 row of 32,000, which the sampler read by itself, 47.5 / 17.3.)
+constexpr int GROUPS = 4096, GROUPS_MANY = 8192;                     // groups of a row at most; for more than MANY candidates, whose
+constexpr int MANY = 512;                                            // groups are many to look at (k 1,024 of 256,000, 1 row: 29.1 / 25.8 us)
+constexpr int GROUP_PART = 4096;                                     // logits of a block (1,024 a wave)
+constexpr int GROUPS_FROM = 8192;                                    // rows of fewer logits: the sampler alone (1 row, k 256 / 1,024: 6,000 18.7 / 18.8 us against 15.0 / 20.0, 8,192 22.1 / 22.2 against 15.6 / 21.2)
+constexpr int LIST = 8192;                                           // candidates that the sampler's LDS holds
+
+static int group_shift(int V, int at_most) {
+    int s = 0;
+    while (((long)V + (1L << s) - 1) >> s > at_most) s++;
+    return s;
+}
+static int groups_of(int V, int shift) { return (int)(((long)V + (1L << shift) - 1) >> shift); }
+
+// the largest of a row of 16 lanes, in every lane (once lanes 8 apart agree, 4 on is as good as 4 across)
+__device__ __forceinline__ uint32_t row_largest(uint32_t m) {
+    m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x128, 0xf, 0xf, true));
+    m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x124, 0xf, 0xf, true));
+    m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4e, 0xf, 0xf, true));
+    return max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xb1, 0xf, 0xf, true));
+}
+
+__global__ void __launch_bounds__(256)
+group_max_k(const float* __restrict__ logits, int V, int shift, int groups, uint32_t* __restrict__ largest) {
+    const int lane = threadIdx.x & 63, begin = blockIdx.x * GROUP_PART + (threadIdx.x >> 6) * 1024 + lane, whole = shift > 6 ? (1 << (shift - 6)) - 1 : 0;
+    const float* z = logits + (size_t)blockIdx.y * V;
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = z[min(begin + u * 64, V - 1)];
+    uint32_t* const to = largest + (size_t)blockIdx.y * groups;
+    uint32_t m[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) m[u] = begin + u * 64 < V ? value_key(v[u]) : 0u;
+    if (shift == 6) {
+        // 64 neighbours are the lanes of one load: halves and rows of lanes are folded by swapping them between two loads' registers,
+        // which leaves four loads' largest in the four rows of 16 lanes
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const auto a = __builtin_amdgcn_permlane32_swap(m[4 * j], m[4 * j + 1], false, false), b = __builtin_amdgcn_permlane32_swap(m[4 * j + 2], m[4 * j + 3], false, false);
+            const auto c = __builtin_amdgcn_permlane16_swap(max(a[0], a[1]), max(b[0], b[1]), false, false);
+            const uint32_t largest_of = row_largest(max(c[0], c[1]));
+            const int u = 4 * j + ((lane >> 5) & 1) + ((lane >> 4) & 1) * 2, group = (begin - lane + u * 64) >> 6;
+            if ((lane & 15) == 0 && group < groups) to[group] = largest_of;
+        }
+        return;
+    }
+    if (shift == 5) {                                                // the same with rows of 16 lanes alone: two loads' in the four rows
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const auto c = __builtin_amdgcn_permlane16_swap(m[2 * j], m[2 * j + 1], false, false);
+            const uint32_t largest_of = row_largest(max(c[0], c[1]));
+            const int u = 2 * j + ((lane >> 4) & 1), group = (begin - lane + u * 64 + (lane & 32)) >> 5;
+            if ((lane & 15) == 0 && group < groups) to[group] = largest_of;
+        }
+        return;
+    }
+    uint32_t run = 0u;
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+        if (shift > 3) m[u] = row_largest(m[u]);
+        else {
+            if (shift > 0) m[u] = max(m[u], across<1>(m[u], lane));
+            if (shift > 1) m[u] = max(m[u], across<2>(m[u], lane));
+            if (shift > 2) m[u] = max(m[u], across<4>(m[u], lane));
+        }
+        if (shift > 5) m[u] = max(m[u], across<16>(m[u], lane));
+        if (shift > 5) m[u] = max(m[u], across<32>(m[u], lane));
+        run = (u & whole) == 0 ? m[u] : max(run, m[u]);
+        const int group = (begin + u * 64) >> shift;
+        if ((u & whole) == whole && (shift > 5 ? lane == 0 : (lane & ((1 << shift) - 1)) == 0) && group < groups) to[group] = run;
+    }
+}
+
+// One block per row.  largest (or null): the keys of the row's groups; the sampler then works on the candidates they lead to, else,
+// or where those are more than its list holds, on the whole row.
+template <int AT_MOST>                                               // groups
 __global__ void __launch_bounds__(1024)
-sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p,
-         Draws draws, int* __restrict__ out,
-         unsigned* __restrict__ cand_count, const float* __restrict__ cand_val, const int* __restrict__ cand_id,
-         int cand_cap, unsigned* __restrict__ row_hist, int row_bins) {
+sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, float top_p, Draws draws, int* __restrict__ out,
+         const uint32_t* __restrict__ largest, int groups, int shift) {
     __shared__ unsigned hist[256];
-    __shared__ uint32_t ckey[1024];
-    __shared__ int cid[1024];
-    __shared__ __attribute__((aligned(16))) float prob[1024];
+    constexpr int STAGE = 16384;                               // logits on their way into LDS at once; later the sort, keys, ids, weights
+    __shared__ __attribute__((aligned(16))) float stage[STAGE];
+    unsigned long long* const place = reinterpret_cast<unsigned long long*>(stage);
+    uint32_t* const ckey = reinterpret_cast<uint32_t*>(stage + 4096);
+    int* const cid = reinterpret_cast<int*>(stage + 5120);
+    float* const prob = stage + 6144;
     __shared__ unsigned s_prefix, s_remaining, s_count, s_eq_total;
     __shared__ int s_id_limit;
-    const float* z = logits + (size_t)blockIdx.x * V;
-    const int tid = threadIdx.x;
+    __shared__ __attribute__((aligned(16))) uint32_t list_val[LIST];      // (float bits; first the counters of the groups' keys)
+    __shared__ int list_id[LIST];
+    __shared__ unsigned short chosen[AT_MOST];
+    __shared__ __attribute__((aligned(16))) unsigned s_wave[16];
+    __shared__ unsigned s_above, s_inside, s_bucket, s_many;
+    const float* const z = logits + (size_t)blockIdx.x * V;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int k = top_k < V ? top_k : V;                       // of the whole row, whichever source is read
-    const int* ids = nullptr;                                  // candidate -> token id; null: the index is the id
-    uint32_t mkey = 0u;                                        // this thread's candidate; empty entries (key 0, id max) sink
-    int mid = 0x7fffffff, sorted = 1024;
-    if (cand_count) {
-        // (the list's first 1024 entries are asked for with its length: places that exist, used where the list reaches)
-        const float first = cand_val[(size_t)blockIdx.x * cand_cap + tid];
-        const int first_id = cand_id[(size_t)blockIdx.x * cand_cap + tid];
-        const unsigned listed = cand_count[blockIdx.x];
-        asm volatile("" :: "v"(first), "v"(first_id), "s"(listed));        // all three are here (else the compiler asks for the entries once it knows the length)
-        if (listed <= (unsigned)cand_cap && listed >= (unsigned)k) {
-            V = (int)listed;
-            z = cand_val + (size_t)blockIdx.x * cand_cap;
-            ids = cand_id + (size_t)blockIdx.x * cand_cap;
+    bool ids = false;                                          // the candidates are the list (else the row)
+    constexpr int IN_ORDER = 2048;                             // candidates that are put in order as they are
+    int sorted = 1024;
+    if (largest) {
+        constexpr int PER = AT_MOST / 1024;
+        uint32_t key[PER];
+#pragma unroll
+        for (int j = 0; j < PER; j++) key[j] = largest[(size_t)blockIdx.x * groups + min(j * 1024 + tid, groups - 1)];
+        // the k-th largest key of the groups: its top 12 bits, and 12 and 8 more while the groups from there up are many more than k
+        uint32_t from = 0u;                                    // keys from here up lead to candidates
+        unsigned need = (unsigned)k, counted = 0u;             // of the keys that share `from` above the level; groups beyond them
+        for (int level = 20; level >= 0; level = level == 20 ? 8 : level - 8) {
+            const int width = level == 0 ? 256 : 4096;
+            for (int i = tid; i < width; i += 1024) list_val[i] = 0u;
+            lds_barrier();
+#pragma unroll
+            for (int j = 0; j < PER; j++)
+                if (j * 1024 + tid < groups && (level == 20 || (level == 8 ? key[j] >> 20 == from >> 20 : key[j] >> 8 == from >> 8)))
+                    atomicAdd(&list_val[(key[j] >> level) & (unsigned)(width - 1)], 1u);
+            lds_barrier();
+            // four counters a thread, from the top
+            const int top = width - 1 - tid * 4;
+            const uint4 four = *reinterpret_cast<const uint4*>(list_val + max(top - 3, 0));
+            const unsigned c[4] = {top >= 0 ? four.w : 0u, top >= 0 ? four.z : 0u, top >= 0 ? four.y : 0u, top >= 0 ? four.x : 0u};
+            const unsigned mine = c[0] + c[1] + c[2] + c[3];
+            const unsigned incl = wave_scan_incl(mine, lane);
+            if (lane == 63) s_wave[wave] = incl;
+            if (tid == 0) { s_bucket = 0u; s_above = 0u; s_inside = 0u; }
+            lds_barrier();
+            unsigned above = incl - mine;
+#pragma unroll
+            for (int w = 0; w < 15; w++) above += w < wave ? s_wave[w] : 0u;
+            if (above < need && above + mine >= need) {        // exactly one thread
+                int j = 0;
+                for (; j < 3; j++) {
+                    if (above + c[j] >= need) break;
+                    above += c[j];
+                }
+                s_bucket = (unsigned)(top - j);
+                s_above = above;
+                s_inside = c[j];
+            }
+            lds_barrier();
+            from |= s_bucket << level;
+            counted += s_above;
+            need -= s_above;
+            if (counted + s_inside <= (unsigned)k + 64u) break;
+            lds_barrier();                                     // (the counters are cleared for the next level)
         }
-        if (ids && V <= 1024 && tid < V) { mkey = value_key(first); mid = first_id; }
-        lds_barrier();                                         // everyone has worked with the count
-        if (tid == 0) cand_count[blockIdx.x] = 0u;
-        for (int i = tid; i < row_bins; i += 1024) row_hist[(size_t)blockIdx.x * row_bins + i] = 0u;
+        // these groups, as pieces of at most 64 logits, and their logits from there up
+        if (tid == 0) { s_count = 0u; s_many = 0u; }
+        lds_barrier();
+        const int parts = shift > 6 ? 1 << (shift - 6) : 1;
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (j * 1024 + tid < groups && key[j] >= from) {
+                const unsigned to = atomicAdd(&s_many, (unsigned)parts);
+                for (int i = 0; i < parts; i++)
+                    if (to + i < (unsigned)AT_MOST) chosen[to + i] = (unsigned short)((j * 1024 + tid) * parts + i);
+            }
+        lds_barrier();
+        // The pieces come straight into LDS, 64 logits an instruction, all of up to 256 such on their way at once; then every thread
+        // looks at sixteen of them.  (Code that runs once waits for its instructions: with the loads in registers, unrolled eight or
+        // sixteen times, this part took two and a half times as long; 128 at a time, the next on their way, 1.4 times.)
+        const int many = (int)s_many, piece = min(shift, 6), per = 64 >> piece, units = many <= AT_MOST ? (many + per - 1) / per : 0;
+        const float least = from ? key_value(from) : -INFINITY;       // (NaN is not below it, and sinks)
+        const unsigned stage0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)stage, last = (unsigned)(V - 1) * 4u;
+        const unsigned within = (unsigned)(lane & ((1 << piece) - 1)) * 4u;
+        if (units > 0 && tid < 64 && many + tid < AT_MOST) chosen[many + tid] = 0;      // what stands past the last piece in its load
+        lds_barrier();
+        for (int u0 = 0; u0 < units; u0 += STAGE / 64) {
+            const int here = min(units - u0, STAGE / 64);
+            int p = (u0 + wave) * per + (lane >> piece);
+#pragma unroll 4
+            for (int u = wave; u < here; u += 16, p += 16 * per) {
+                const unsigned off = min(((unsigned)chosen[p & (AT_MOST - 1)] << (piece + 2)) + within, last);
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" :: "v"(off), "s"(z), "s"(stage0 + (unsigned)u * 256u) : "memory");
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            lds_barrier();
+            unsigned found = 0u;
+#pragma unroll
+            for (int j = 0; j < STAGE / 4096; j++) {
+                const int e = (j * 1024 + tid) * 4;
+                const float4 four = *reinterpret_cast<const float4*>(stage + e);
+                if (e < here * 64)
+                    found |= (!(four.x < least) ? 1u : 0u) << (4 * j) | (!(four.y < least) ? 2u : 0u) << (4 * j) | (!(four.z < least) ? 4u : 0u) << (4 * j) | (!(four.w < least) ? 8u : 0u) << (4 * j);
+            }
+            const unsigned own = (unsigned)__popc(found), incl = wave_scan_incl(own, lane);
+            unsigned to = 0u;
+            if (lane == 63) to = atomicAdd(&s_count, incl);            // one addition for all that a wave found
+            to = (unsigned)__builtin_amdgcn_readlane((int)to, 63) + incl - own;
+            for (; found; found &= found - 1u, to++) {
+                const int bit = __ffs(found) - 1, e = ((bit >> 2) * 1024 + tid) * 4 + (bit & 3), p = (u0 + (e >> 6)) * per + ((e & 63) >> piece);
+                const int id = ((int)chosen[min(p, many - 1)] << piece) + (e & ((1 << piece) - 1));
+                const bool real = p < many && id < V;                  // (what stands past a row's or the last piece's end sinks)
+                if (to < (unsigned)LIST) { list_val[to] = real ? __float_as_uint(stage[e]) : 0x7fffffffu; list_id[to] = real ? id : 0x7fffffff; }
+            }
+            lds_barrier();                                             // everyone has looked at them
+        }
+        if (many <= AT_MOST && s_count <= (unsigned)LIST) {     // (at least k: every group counted gave one)
+            V = (int)s_count;
+            ids = true;
+        }
     }
-    if (ids && V <= 1024) {
+    unsigned long long mine = packed(0u, 0x7fffffff);          // this thread's candidate; empty places sink
+    const bool few = ids && V <= IN_ORDER;
+    if (few) {
+        if (tid < V) mine = packed(value_key(__uint_as_float(list_val[tid])), list_id[tid]);
         sorted = 64;
-        while (sorted < V) sorted <<= 1;
+        while (sorted < V && sorted < 1024) sorted <<= 1;
     } else {
 
+    auto at = [&](int i) { return ids ? __uint_as_float(list_val[i]) : z[i]; };
     // 1. the k-th largest value key, 8 bits at a time from the top
     if (tid == 0) { s_prefix = 0u; s_remaining = (unsigned)k; }
     for (int shift = 24; shift >= 0; shift -= 8) {
@@ -361,7 +573,7 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
         __syncthreads();
         const unsigned prefix = s_prefix;
         for (int i = tid; i < V; i += blockDim.x) {
-            const uint32_t key = value_key(z[i]);
+            const uint32_t key = value_key(at(i));
             if (shift == 24 || (key >> (shift + 8)) == (prefix >> (shift + 8))) atomicAdd(&hist[(key >> shift) & 255u], 1u);
         }
         __syncthreads();
@@ -389,8 +601,8 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
             __syncthreads();
             const unsigned prefix = s_prefix;
             for (int i = tid; i < V; i += blockDim.x) {
-                if (value_key(z[i]) != tkey) continue;
-                const unsigned id = (unsigned)(ids ? ids[i] : i);
+                if (value_key(at(i)) != tkey) continue;
+                const unsigned id = (unsigned)(ids ? list_id[i] : i);
                 if (shift == 24 || (id >> (shift + 8)) == (prefix >> (shift + 8))) atomicAdd(&hist[(id >> shift) & 255u], 1u);
             }
             __syncthreads();
@@ -415,27 +627,40 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
     __syncthreads();
     const int id_limit = s_id_limit;
     for (int i = tid; i < V; i += blockDim.x) {
-        const uint32_t key = value_key(z[i]);
-        const int id = ids ? ids[i] : i;
+        const uint32_t key = value_key(at(i));
+        const int id = ids ? list_id[i] : i;
         if (key > tkey || (key == tkey && id <= id_limit)) {
             const unsigned at = atomicAdd(&s_count, 1u);
             if (at < 1024u) { ckey[at] = key; cid[at] = id; }
         }
     }
     __syncthreads();
-    mkey = ckey[tid];
-    mid = cid[tid];
+    mine = packed(ckey[tid], cid[tid]);
     }
-    // 4. in order; the first k are the candidates
-    block_sort(mkey, mid, sorted, ckey, cid);
+    // 4. in order; the first k are the candidates.  Of more than 1,024 the rest is put in order by itself, and of the two runs the
+    // larger of first and last, second and last but one, ... are the 1,024 largest, a sequence that the last stage puts in order.
+    block_sort(mine, sorted, place);
+    if (few && V > 1024) {
+        unsigned long long rest = packed(0u, 0x7fffffff);
+        if (1024 + tid < V) rest = packed(value_key(__uint_as_float(list_val[1024 + tid])), list_id[1024 + tid]);
+        int behind = 64;
+        while (1024 + behind < V) behind <<= 1;
+        block_sort(rest, behind, place);
+        lds_barrier();
+        place[1023 - tid] = rest;
+        lds_barrier();
+        rest = place[tid];
+        if (rest > mine) mine = rest;
+        sort_stages(mine, 1024, 1024, place);
+    }
     lds_barrier();
-    ckey[tid] = mkey;
-    cid[tid] = mid;
+    ckey[tid] = (uint32_t)(mine >> 32);
+    cid[tid] = (int)~(uint32_t)mine;
     lds_barrier();
     // 5. probabilities, the nucleus and the draw: the first wave, each lane 16 consecutive candidates; sums run over a
     // lane's candidates in order, then over the lanes in order
     const float mx = key_value(ckey[0]);
-    prob[tid] = tid < k ? expf((key_value(mkey) - mx) / temperature) : 0.f;
+    prob[tid] = tid < k ? expf((key_value((uint32_t)(mine >> 32)) - mx) / temperature) : 0.f;
     lds_barrier();
     if (tid < 64) {
         const int j0 = tid * 16;
@@ -457,8 +682,7 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
 #pragma unroll
         for (int j = 15; j >= 0; j--)
             if (j0 + j < k && c[j] >= top_p) first = j0 + j;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 64));
+        first = wave_least(first, tid);
         const int keep = first < k ? first + 1 : k;
         float last = 0.f;                                      // c of candidate keep - 1, in the lane that holds it
 #pragma unroll
@@ -471,8 +695,7 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
 #pragma unroll
         for (int j = 15; j >= 0; j--)
             if (j0 + j < keep && r < c[j]) hit = j0 + j;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) hit = min(hit, __shfl_xor(hit, o, 64));
+        hit = wave_least(hit, tid);
         if (tid == 0) out[blockIdx.x] = cid[hit < keep ? hit : 0];
     }
 }
@@ -481,6 +704,21 @@ sample_k(const float* __restrict__ logits, int V, float temperature, int top_k, 
 // exp((z_i - max) / T), r = u * sum, the token whose cumulative mass in id order first exceeds r.  One block per
 // row; thread t owns a contiguous range of ids, so sums run over ids in order within a thread, then over the threads
 // in order. ----------------------------------------------------------------------------------------------------
+// part: the sums of 1,024 threads' stretches -> what lies before each; returns the total
+__device__ __forceinline__ float full_scan(float* part, float& total, int tid) {
+    __syncthreads();
+    if (tid < 64) {                                  // the first wave: totals of 16 threads per lane, then over the lanes
+        float local = 0.f;
+        for (int j = 0; j < 16; j++) local += part[tid * 16 + j];
+        const float incl = wave_scan_incl(local, tid);
+        float run = incl - local;
+        for (int j = 0; j < 16; j++) { const float v = part[tid * 16 + j]; part[tid * 16 + j] = run; run += v; }   // exclusive sums
+        if (tid == 63) total = incl;
+    }
+    __syncthreads();
+    return total;
+}
+
 __global__ void __launch_bounds__(1024)
 sample_full_k(const float* __restrict__ logits, int V, float temperature, Draws draws,
               int* __restrict__ out) {
@@ -502,16 +740,7 @@ sample_full_k(const float* __restrict__ logits, int V, float temperature, Draws 
     float mine = 0.f;
     for (int i = begin; i < end; i++) { const float v = z[i]; mine += v == v ? expf((v - mx) / temperature) : 0.f; }
     part[tid] = mine;
-    __syncthreads();
-    if (tid < 64) {                                  // the first wave: totals of 16 threads per lane, then over the lanes
-        float local = 0.f;
-        for (int j = 0; j < 16; j++) local += part[tid * 16 + j];
-        const float incl = wave_scan_incl(local, tid);
-        float run = incl - local;
-        for (int j = 0; j < 16; j++) { const float v = part[tid * 16 + j]; part[tid * 16 + j] = run; run += v; }   // exclusive sums
-        if (tid == 63) s_total = incl;
-    }
-    __syncthreads();
+    full_scan(part, s_total, tid);
     const float r = draw_of(draws, blockIdx.x) * s_total;
     const float before = part[tid];
     // the first thread whose range reaches past r walks it; rounding may leave r past every range: the last one
@@ -531,108 +760,113 @@ sample_full_k(const float* __restrict__ logits, int V, float temperature, Draws 
     }
 }
 
-// ---- a coarse filter in front of the exact sampler, on many blocks: the sampler alone reads a row of 256,000
-// logits several times on one CU (0.4 ms).  A histogram of the top 12 bits of the value keys gives the bin that
-// holds the top_k-th largest logit; everything from that bin upwards (top_k plus that bin's other members, a few
-// hundred for logits of a language model) is copied to a candidate list, which the sampler then works on.  A list
-// that would not fit falls back to the whole row, so the result never depends on the filter. -------------------
-// Three launches: the histogram, the candidates (every block finds the bin from its row's histogram by itself), the sampler,
-// which also puts the histogram and the count back to zero.  A block asks for all of its logits together.
-// (8 rows of 256,000, top_k 256, microseconds: histogram 5.9, candidates 10.2; 8.7, 10.6 and 5.5 for the bin in a launch of its own while a thread
-// asked for its 32 logits one after the other.  Sampler 10.0; 12.8 with the exchanges of its sort as shuffles through LDS
-// and a barrier that waited for the zeros of the histogram; 10.1 with the candidates asked for once their number was known.)
-constexpr int FILTER_BINS = 4096;
-constexpr int FILTER_PER = 16, FILTER_PART = 256 * FILTER_PER;       // logits per thread and block
-constexpr int FILTER_FROM = 32768;                                   // smaller vocabularies: the sampler alone
+// ---- the same on many blocks, to the same bits: a thread's stretch of ids above is a chunk here.  One launch leaves the groups'
+// largest keys (above), one the chunks' sums (a block forms the exponentials of its chunks together, then a thread adds a chunk's in order),
+// one finds the chunk and walks it.  Microseconds, 1 / 8 / 64 rows of 256,000: one block a row 156 / 179 / 337, here 20 / 26 / 52.
+constexpr int FULL_CHUNKS = 1024;
+constexpr int FULL_LDS = 16000;                                      // floats of LDS that a block's chunks take at most
 
-__device__ __forceinline__ void part_of_row(const float* __restrict__ z, int begin, int V, float (&v)[FILTER_PER]) {
+template <int THREADS>
+__device__ __forceinline__ float row_max(const uint32_t* __restrict__ largest, int groups, uint32_t* red) {
+    uint32_t key[GROUPS / THREADS], m = 0u;
 #pragma unroll
-    for (int u = 0; u < FILTER_PER; u++) v[u] = z[min(begin + (int)threadIdx.x + u * 256, V - 1)];
+    for (int j = 0; j < GROUPS / THREADS; j++) key[j] = largest[min(j * THREADS + (int)threadIdx.x, groups - 1)];
+#pragma unroll
+    for (int j = 0; j < GROUPS / THREADS; j++) m = max(m, key[j]);
+    const int lane = threadIdx.x & 63;
+    m = max(m, across<32>(m, lane)); m = max(m, across<16>(m, lane)); m = max(m, across<8>(m, lane));
+    m = max(m, across<4>(m, lane)); m = max(m, across<2>(m, lane)); m = max(m, across<1>(m, lane));
+    if (lane == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / 64; w++) m = max(m, red[w]);
+    return m == 0u ? -INFINITY : key_value(m);                       // (NaN alone: as if there were nothing)
 }
 
 __global__ void __launch_bounds__(256)
-filter_hist_k(const float* __restrict__ logits, int V, unsigned* __restrict__ hist) {
-    __shared__ unsigned local[FILTER_BINS];
-    const int begin = blockIdx.x * FILTER_PART;
-    float v[FILTER_PER];
-    part_of_row(logits + (size_t)blockIdx.y * V, begin, V, v);
-    for (int i = threadIdx.x; i < FILTER_BINS; i += 256) local[i] = 0u;
-    __syncthreads();
+full_sums_k(const float* __restrict__ logits, int V, float temperature, const uint32_t* __restrict__ largest, int groups, int chunk, int chunks,
+            float* __restrict__ sums) {
+    extern __shared__ float e[];
+    __shared__ uint32_t red[4];
+    const int tid = threadIdx.x, first = blockIdx.x * chunks, stride = chunk | 1;
+    const float* z = logits + (size_t)blockIdx.y * V;
+    const float mx = row_max<256>(largest + (size_t)blockIdx.y * groups, groups, red);
+    const int begin = first * chunk, n = min(V - begin, chunks * chunk);           // (the last chunks may hold nothing)
+    // sixteen lanes a chunk, eight logits of a lane at once
+    const int mine = tid >> 4, own = min(chunk, n - mine * chunk);
+    if (mine < chunks)
+        for (int i0 = tid & 15; i0 < own; i0 += 128) {
+            float v[8];
 #pragma unroll
-    for (int u = 0; u < FILTER_PER; u++)
-        if (begin + (int)threadIdx.x + u * 256 < V) atomicAdd(&local[value_key(v[u]) >> 20], 1u);
-    __syncthreads();
-    unsigned* row = hist + (size_t)blockIdx.y * FILTER_BINS;
-    for (int i = threadIdx.x; i < FILTER_BINS; i += 256)
-        if (local[i]) atomicAdd(&row[i], local[i]);
-}
-
-// the bin of the row's k-th largest key; a block gathers its candidates in LDS and reserves their places with one addition
-// to the row's counter
-__global__ void __launch_bounds__(256)
-filter_collect_k(const float* __restrict__ logits, int V, const unsigned* __restrict__ hist, int k, unsigned* __restrict__ cand_count,
-                 float* __restrict__ cand_val, int* __restrict__ cand_id, int cand_cap) {
-    constexpr int LOCAL = 1024, PER = FILTER_BINS / 256;
-    __shared__ float lval[LOCAL];
-    __shared__ int lid[LOCAL];
-    __shared__ unsigned lcount, base, lowest_bin, above_wave[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int begin = blockIdx.x * FILTER_PART;
-    float v[FILTER_PER];
-    part_of_row(logits + (size_t)blockIdx.y * V, begin, V, v);
-    // thread t owns the PER bins from the top down to FILTER_BINS - (t + 1) PER; the one in which the count from the top reaches k
-    const unsigned* row = hist + (size_t)blockIdx.y * FILTER_BINS + FILTER_BINS - (tid + 1) * PER;
-    unsigned mine[PER], sum = 0u;
+            for (int j = 0; j < 8; j++) v[j] = z[begin + mine * chunk + min(i0 + 16 * j, own - 1)];
 #pragma unroll
-    for (int j = 0; j < PER; j += 4) *reinterpret_cast<uint4*>(mine + j) = *reinterpret_cast<const uint4*>(row + j);
-#pragma unroll
-    for (int j = 0; j < PER; j++) sum += mine[j];
-    const unsigned incl = wave_scan_incl(sum, lane);
-    if (lane == 63) above_wave[wave] = incl;
-    if (tid == 0) { lcount = 0u; lowest_bin = 0u; }
-    __syncthreads();
-    unsigned above = incl - sum;
-    for (int w = 0; w < wave; w++) above += above_wave[w];
-    if (above < (unsigned)k && above + sum >= (unsigned)k) {        // exactly one thread
-        int j = PER - 1;
-        for (; j > 0; j--) {
-            if (above + mine[j] >= (unsigned)k) break;
-            above += mine[j];
+            for (int j = 0; j < 8; j++)
+                if (i0 + 16 * j < own) e[mine * stride + i0 + 16 * j] = v[j] == v[j] ? expf((v[j] - mx) / temperature) : 0.f;
         }
-        lowest_bin = (unsigned)(FILTER_BINS - (tid + 1) * PER + j);
-    }
     __syncthreads();
-    const unsigned lowest = lowest_bin;
-#pragma unroll
-    for (int u = 0; u < FILTER_PER; u++) {
-        const int i = begin + tid + u * 256;
-        if (i < V && (value_key(v[u]) >> 20) >= lowest) {
-            const unsigned at = atomicAdd(&lcount, 1u);
-            if (at < (unsigned)LOCAL) { lval[at] = v[u]; lid[at] = i; }
-        }
-    }
-    __syncthreads();
-    const unsigned n = lcount;
-    if (n == 0u) return;
-    // more than the block can hold: the row's count is pushed past the capacity, and the sampler reads the whole row
-    if (tid == 0) base = atomicAdd(&cand_count[blockIdx.y], n <= (unsigned)LOCAL ? n : (unsigned)cand_cap + 1u);
-    __syncthreads();
-    if (n > (unsigned)LOCAL) return;
-    for (unsigned j = tid; j < n; j += 256) {
-        const unsigned at = base + j;
-        if (at < (unsigned)cand_cap) {
-            cand_val[(size_t)blockIdx.y * cand_cap + at] = lval[j];
-            cand_id[(size_t)blockIdx.y * cand_cap + at] = lid[j];
-        }
+    for (int c = tid; c < chunks && first + c < FULL_CHUNKS; c += 256) {
+        const int len = max(0, min(chunk, n - c * chunk));
+        float sum = 0.f;
+#pragma unroll 8
+        for (int i = 0; i < len; i++) sum += e[c * stride + i];
+        sums[(size_t)blockIdx.y * FULL_CHUNKS + first + c] = sum;
     }
 }
 
-constexpr int CAND_CAP = 8192;
+__global__ void __launch_bounds__(1024)
+full_pick_k(const float* __restrict__ logits, int V, float temperature, const uint32_t* __restrict__ largest, int groups, int chunk,
+            const float* __restrict__ sums, Draws draws, int* __restrict__ out) {
+    __shared__ float part[FULL_CHUNKS], e[FULL_LDS];
+    __shared__ uint32_t red[16];
+    __shared__ float s_total;
+    __shared__ int s_winner;
+    const int tid = threadIdx.x;
+    const float* z = logits + (size_t)blockIdx.x * V;
+    const float mine = sums[(size_t)blockIdx.x * FULL_CHUNKS + tid];
+    part[tid] = mine;
+    const float mx = row_max<1024>(largest + (size_t)blockIdx.x * groups, groups, red);
+    const float total = full_scan(part, s_total, tid);
+    const float r = draw_of(draws, blockIdx.x) * total, before = part[tid];
+    const int begin = tid * chunk, end = min(V, begin + chunk);
+    if (tid == 0) s_winner = (V - 1) / chunk;
+    __syncthreads();
+    if (begin < end && r < before + mine) atomicMin(&s_winner, tid);
+    __syncthreads();
+    const int winner = s_winner, from = winner * chunk, n = min(V, from + chunk) - from;
+    for (int i = tid; i < n; i += 1024) {
+        const float v = z[from + i];
+        e[i] = v == v ? expf((v - mx) / temperature) : 0.f;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float run = part[winner];
+        int pick = n - 1;
+        bool found = false;
+        for (int i0 = 0; i0 < n && !found; i0 += 8) {            // eight at a time out of LDS; past the last they add nothing that counts
+            float t[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) t[j] = e[min(i0 + j, n - 1)];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                run += t[j];
+                if (!found && i0 + j < n && r < run) { pick = i0 + j; found = true; }
+            }
+        }
+        out[blockIdx.x] = from + pick;
+    }
+}
 
-// bytes of the sampler's workspace for B rows; it must be zero before its first use and is left ready for the next
+static int full_chunk(int V) { return (V + FULL_CHUNKS - 1) / FULL_CHUNKS; }
+// (1 row: 16,384 15.5 us by one block, 16.9 here; 32,000 25.8 / 17.8)
+constexpr int FULL_FROM = 20480;
+static bool full_on_many_blocks(int V) { return V >= FULL_FROM && full_chunk(V) < FULL_LDS; }
+
+// bytes of the sampler's workspace for B rows (nothing has to lie in it)
 extern "C" long tp_sample_workspace_bytes(int B, int V) {
-    if (V < FILTER_FROM) return 0;
-    return (long)B * (FILTER_BINS * 4 + 4 + (long)CAND_CAP * 8);
+    if (V < GROUPS_FROM) return 0;
+    const long many = groups_of(V, group_shift(V, GROUPS_MANY)), full = groups_of(V, group_shift(V, GROUPS)) + (full_on_many_blocks(V) ? FULL_CHUNKS : 0);
+    return (long)B * (many > full ? many : full) * 4;
 }
 
 static int sample_launch(const float* logits, int B, int V, float temperature, int top_k, float top_p, const Draws& draws, int* out,
@@ -644,25 +878,31 @@ static int sample_launch(const float* logits, int B, int V, float temperature, i
     TP_REQUIRE(top_k > 0 || top_p >= 1.f, "sample: a nucleus (top_p %g) needs top_k between 1 and 1024", top_p);
     TP_REQUIRE(B <= 65535, "sample: %d rows exceed one launch", B);
     hipStream_t s = (hipStream_t)stream;
-    if (top_k == 0) {
+    const bool many = top_k > MANY;
+    const int shift = group_shift(V, many ? GROUPS_MANY : GROUPS), groups = groups_of(V, shift);
+    const bool in_groups = workspace && V >= GROUPS_FROM && shift <= 10 && (top_k > 0 || full_on_many_blocks(V));
+    uint32_t* const largest = in_groups ? (uint32_t*)workspace : nullptr;
+    if (in_groups) {
+        group_max_k<<<dim3(tp_cdiv(V, GROUP_PART), B), 256, 0, s>>>(logits, V, shift, groups, largest);
+        if (int rc = tp_check_launch("sample (groups)")) return rc;
+    }
+    if (top_k > 0) {
+        if (many) sample_k<GROUPS_MANY><<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, draws, out, largest, groups, shift);
+        else sample_k<GROUPS><<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, draws, out, largest, groups, shift);
+        return tp_check_launch("sample");
+    }
+    if (!in_groups) {
         sample_full_k<<<B, 1024, 0, s>>>(logits, V, temperature, draws, out);
         return tp_check_launch("sample (whole vocabulary)");
     }
-    if (!workspace || tp_sample_workspace_bytes(B, V) == 0) {
-        sample_k<<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, draws, out, nullptr, nullptr, nullptr, 0, nullptr, 0);
-        return tp_check_launch("sample");
-    }
-    unsigned* hist = (unsigned*)workspace;
-    unsigned* count = hist + (size_t)B * FILTER_BINS;
-    float* cand_val = (float*)(count + B);
-    int* cand_id = (int*)(cand_val + (size_t)B * CAND_CAP);
-    const dim3 grid(tp_cdiv(V, FILTER_PART), B);
-    filter_hist_k<<<grid, 256, 0, s>>>(logits, V, hist);
-    if (int rc = tp_check_launch("sample (histogram)")) return rc;
-    filter_collect_k<<<grid, 256, 0, s>>>(logits, V, hist, top_k < V ? top_k : V, count, cand_val, cand_id, CAND_CAP);
-    if (int rc = tp_check_launch("sample (candidates)")) return rc;
-    sample_k<<<B, 1024, 0, s>>>(logits, V, temperature, top_k, top_p, draws, out, count, cand_val, cand_id, CAND_CAP, hist, FILTER_BINS);
-    return tp_check_launch("sample");
+    float* const sums = (float*)(largest + (size_t)B * groups);
+    const int chunk = full_chunk(V);
+    int chunks = FULL_LDS / (chunk | 1);                             // of a block
+    if (chunks > 16) chunks = 16;
+    full_sums_k<<<dim3(tp_cdiv(FULL_CHUNKS, chunks), B), 256, (size_t)chunks * (chunk | 1) * 4, s>>>(logits, V, temperature, largest, groups, chunk, chunks, sums);
+    if (int rc = tp_check_launch("sample (sums)")) return rc;
+    full_pick_k<<<B, 1024, 0, s>>>(logits, V, temperature, largest, groups, chunk, sums, draws, out);
+    return tp_check_launch("sample (whole vocabulary)");
 }
 
 // uniforms: a float32 number per row, on the device

@@ -174,7 +174,6 @@ class HipOps:
             raise KernelError(f"the HIP kernel library could not be built or loaded: {e}") from None
         _bind(self.lib, _CORE_SIGS)
         self._attn = {}
-        self._sample_ws = {}
         from .. import flags
         plain = flags.force_plain()
         self.force_linear = 1 if plain else 0   # 1 plain, 2 skinny, 3 tiled (6: its wide tile, 7: its 128 x 96 tile, 8, 9: loads into LDS, 128 x 128 and 128 x 96; 10, 11: 64 x 32 and 64 x 64 tiles, two k steps ahead; 12 - 15: 256 x 256, 256 x 192, 192 x 256 and 256 x 128), 16 up to 64 rows through LDS, 4 multiply-adds (1-2 rows), 5 blocks of 8 rows of W
@@ -1508,12 +1507,9 @@ class HipOps:
             self._dev(out)
             if out.dtype != torch.int32 or out.shape != (logits.shape[0],) or not out.is_contiguous():
                 raise KernelError("sample: the output must be contiguous int32 [rows]")
-        # the candidate filter's workspace starts zeroed and every call leaves it zeroed again: kept between calls
         shape = tuple(logits.shape)
-        if shape not in self._sample_ws:
-            nbytes = self.lib.tp_sample_workspace_bytes(shape[0], shape[1])
-            self._sample_ws[shape] = torch.zeros(nbytes, dtype=torch.uint8, device=self.device) if nbytes else None
-        ws = self._sample_ws[shape]
+        nbytes = self.lib.tp_sample_workspace_bytes(shape[0], shape[1])
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device) if nbytes else None
         self._call(self.lib, entry, logits.data_ptr(), shape[0], shape[1], float(temperature),
                    int(top_k), float(top_p), draws, out.data_ptr(), ws.data_ptr() if ws is not None else None,
                    self._stream())
