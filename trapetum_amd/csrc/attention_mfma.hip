@@ -54,10 +54,9 @@ __device__ __forceinline__ float tanh_fast(float x) {
 __device__ __forceinline__ float score_of(float dot, float scale, float cap, float scale_over_cap) {
     return cap > 0.f ? cap * tanh_fast(dot * scale_over_cap) : dot * scale;
 }
-__device__ __forceinline__ bf16_t bf16_bits(float f) {
-    __bf16 b = (__bf16)f;                          // one conversion instruction on gfx950, round to nearest even
-    return __builtin_bit_cast(bf16_t, b);
-}
+// n / d of 0 <= n < 4096, 0 < d <= 256: (n + 1/2) / d lies 1/512 or more from every whole number, far more than the reciprocal's
+// error (an integer division is some thirty instructions)
+__device__ __forceinline__ int quotient(int n, int d) { return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d)); }
 }  // namespace
 
 // =====================================================================================================
@@ -92,6 +91,7 @@ struct DecodeArgs {
     // the first `keep` positions stay visible behind the window; in a ring they live in the `pin` rows in front of it
     int keep, pin;
     TpPositional by_position;
+    int G;                                           // query heads a kv head (set by the launch)
 };
 
 namespace {
@@ -118,8 +118,37 @@ attn_decode_k(DecodeArgs a) {
     __shared__ __attribute__((aligned(16))) bf16_t q_lds[QT * HD], new_lds[WHOLE ? 2 * HD : 8];      // queries; the new key and value
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
-    const int G = a.H / a.KV;
-    const int p = a.new_len[seq] - 1;
+    const int G = a.G;
+    const int held = a.new_len[seq];
+    // ---- the projections' columns of this thread's first pair are asked for before anything is known of the sequence: they wait for
+    // the kernel that has just written them, the keys for the sequence's length and page table, one after the other
+    constexpr int NE = 6;                            // the pair of a query head, and the new key's and value's
+    const int half = a.rot >> 1;
+    unsigned early[NE][4];                           // float32 of four slices, or bf16 in the first
+    float freq = 0.f;
+    auto ask = [&](int idx) {
+        const int qi = quotient(idx, half), f = idx - qi * half;
+        const unsigned q0 = (unsigned)(kvh * G + qi) * HD + f, k0 = a.write_kv ? (unsigned)(a.H + kvh) * HD + f : q0, v0 = a.write_kv ? k0 + (unsigned)a.KV * HD : q0;
+        const unsigned cols[6] = {q0, q0 + half, k0, k0 + half, v0, v0 + half};
+        if (a.qkv_f32) {
+            const char* slice = (const char*)a.qkv + (size_t)seq * a.row_stride * 4;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+#pragma unroll
+                for (int c = 0; c < NE; c++) early[c][u] = *reinterpret_cast<const unsigned*>(slice + cols[c] * 4u);
+                slice += u + 1 < a.n_slices ? a.slice_stride * 4 : 0;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < NE; c++) early[c][0] = *reinterpret_cast<const bf16_t*>((const char*)a.qkv + (size_t)seq * a.row_stride * 2 + cols[c] * 2u);
+        }
+        freq = a.inv_freq[f];
+    };
+    if constexpr (WHOLE) {
+        if (a.qkv && half > 0) ask(min(tid, G * half - 1));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int p = held - 1;
     int lo = a.window > 0 ? max(0, p - a.window + 1) : 0;
     if (a.chunk > 0) lo = max(lo, p / a.chunk * a.chunk);
     const int lo_al = lo & ~15;
@@ -129,7 +158,8 @@ attn_decode_k(DecodeArgs a) {
     const int kept_al = (a.keep + 15) & ~15;
     const int first = a.keep > 0 ? 0 : lo_al, gap = a.keep > 0 && lo_al > kept_al ? lo_al - kept_al : 0;
     const int places = p + 1 - gap;
-    int chunk = (places - first + a.nsplit - 1) / a.nsplit;
+    int chunk = places - first;
+    if constexpr (!WHOLE) chunk = (chunk + a.nsplit - 1) / a.nsplit;
     chunk = (chunk + ROUND - 1) / ROUND * ROUND;
     const int t_begin = first + split * chunk;           // in places
     const int t_end = min(places, t_begin + chunk);
@@ -164,7 +194,8 @@ attn_decode_k(DecodeArgs a) {
     // ---- loads of a round: the key row of lane c for the scores, value chunks for the sum.  Unconditional loads of
     // rows that exist: a hidden or surplus key gets probability 0 (or is skipped) in the sum ---------------------
     auto row_in_tile = [&](int tb, int t) {                        // a row of the tile that exists, for position t of it
-        return t > p ? p : (t < lo && t >= a.keep ? (lo < tb + 15 ? lo : tb + 15) : t);
+        const int m = min(t, p), low = min(max(lo, tb), tb + 15);
+        return m < a.keep ? m : max(m, low);
     };
     const float* bias = nullptr;                                   // of query head c of the group
     if constexpr (BY_POSITION)
@@ -174,7 +205,10 @@ attn_decode_k(DecodeArgs a) {
         const int tb = ub < kept_al ? ub : ub + gap;
         const size_t tile = tile_offset(__builtin_amdgcn_readfirstlane(tb));
         const int tk = row_in_tile(tb, tb + c);
-        const bf16_t* kp = a.k_pool + tile + (size_t)(tk - tb) * HD;
+        // (a row's address is the tile's plus 32 bits of the lane's: one instruction a load)
+        const char* const kt = reinterpret_cast<const char*>(a.k_pool + tile);
+        const char* const vt = reinterpret_cast<const char*>(a.v_pool + tile);
+        const unsigned kr = (unsigned)(tk - tb) * (HD * 2);
         if constexpr (BY_POSITION)
             if (bias)
 #pragma unroll
@@ -182,14 +216,14 @@ attn_decode_k(DecodeArgs a) {
 #pragma unroll
         for (int ks = 0; ks < DSTEPS; ks++) {
             const int d0 = dofs(ks, g);
-            kf[ks] = ld_frag(kp + (d0 < HD ? d0 : 0), d0 < HD);
+            kf[ks] = ld_frag(reinterpret_cast<const bf16_t*>(kt + (kr + (d0 < HD ? d0 : 0) * 2u)), d0 < HD);
         }
 #pragma unroll
         for (int j = 0; j < VPT; j++) {
             int kk = kgw + j * KGW;
             kk = kk > 15 ? 15 : kk;
             const int tv = row_in_tile(tb, tb + kk);
-            vf[j].u = *reinterpret_cast<const uint4*>(a.v_pool + tile + (size_t)(tv - tb) * HD + ch * 8);
+            vf[j].u = *reinterpret_cast<const uint4*>(vt + ((unsigned)(tv - tb) * (HD * 2) + ch * 16u));
         }
     };
     // The wave's first round is fetched while the queries are prepared, unless its tile holds the row that this
@@ -204,31 +238,34 @@ attn_decode_k(DecodeArgs a) {
     // the new key rotated (pair (f, f + rot/2), angle p * inv_freq[f], in float32), and the slice that holds position
     // p writes the key and the value into the cache before anyone in the block reads that row ---------------------
     if (a.qkv) {
-        const int half = a.rot >> 1, rest = HD - a.rot;
+        const int rest = HD - a.rot;
         // NC columns of the sequence's row at once: their loads are asked for together (of float32 slices four slices
         // at a time, added in slice order), so that a thread pays one trip to memory for all it needs, not one a column
-        auto vals = [&](auto ncol, const long* cols, float* out) {
+        // (a column's address is the block's row plus 32 bits of the lane's: one instruction a load)
+        auto vals = [&](auto ncol, const unsigned* cols, float* out) {
             constexpr int NC = decltype(ncol)::value;
             if (a.qkv_f32) {
-                const float* src = (const float*)a.qkv + (size_t)seq * a.row_stride;
+                const char* src = (const char*)a.qkv + (size_t)seq * a.row_stride * 4;
 #pragma unroll
                 for (int c = 0; c < NC; c++) out[c] = 0.f;
+#pragma unroll 1
                 for (int s0 = 0; s0 < a.n_slices; s0 += 4) {
                     float part[NC][4];
 #pragma unroll
-                    for (int c = 0; c < NC; c++)
+                    for (int u = 0; u < 4; u++) {
+                        const char* slice = src + (size_t)(s0 + u < a.n_slices ? s0 + u : a.n_slices - 1) * a.slice_stride * 4;
 #pragma unroll
-                        for (int u = 0; u < 4; u++)
-                            part[c][u] = src[(size_t)(s0 + u < a.n_slices ? s0 + u : a.n_slices - 1) * a.slice_stride + cols[c]];
+                        for (int c = 0; c < NC; c++) part[c][u] = *reinterpret_cast<const float*>(slice + cols[c] * 4u);
+                    }
 #pragma unroll
                     for (int c = 0; c < NC; c++)
 #pragma unroll
                         for (int u = 0; u < 4; u++) out[c] += s0 + u < a.n_slices ? part[c][u] : 0.f;
                 }
             } else {
-                const bf16_t* src = (const bf16_t*)a.qkv + (size_t)seq * a.row_stride;
+                const char* src = (const char*)a.qkv + (size_t)seq * a.row_stride * 2;
 #pragma unroll
-                for (int c = 0; c < NC; c++) out[c] = bf16_to_f32(src[cols[c]]);
+                for (int c = 0; c < NC; c++) out[c] = bf16_to_f32(*reinterpret_cast<const bf16_t*>(src + cols[c] * 2u));
             }
         };
         // the slice that holds position p (t_begin < places holds here) also rotates the new key and writes it and the value
@@ -243,16 +280,37 @@ attn_decode_k(DecodeArgs a) {
             kdst = a.k_pool + at;
             vdst = a.v_pool + at;
         }
-        const long kcol = (long)(a.H + kvh) * HD, vcol = (long)(a.H + a.KV + kvh) * HD;
+        const unsigned kcol = (unsigned)(a.H + kvh) * HD, vcol = (unsigned)(a.H + a.KV + kvh) * HD;
         for (int idx = tid; idx < G * half; idx += DTH) {
-            const int qi = idx / half, f = idx - qi * half;
-            const long col = (long)(kvh * G + qi) * HD;
+            const int qi = quotient(idx, half), f = idx - qi * half;
             const bool kv = writer && idx < half;                 // then qi == 0 and f == idx
-            const long cols[6] = {col + f, col + f + half, kcol + f, kcol + f + half, vcol + f, vcol + f + half};
+            const unsigned col = (unsigned)(kvh * G + qi) * HD;
+            const unsigned cols[6] = {col + f, col + f + half, kcol + f, kcol + f + half, vcol + f, vcol + f + half};
             float x[6];
-            if (writer) vals(std::integral_constant<int, 6>(), cols, x);     // (the whole block takes this branch or the other)
-            else vals(std::integral_constant<int, 2>(), cols, x);
-            const float ang = (float)p * a.inv_freq[f];
+            if constexpr (WHOLE) {
+                if (idx != tid) ask(idx);
+#pragma unroll
+                for (int c = 0; c < NE; c++) {
+                    x[c] = 0.f;
+                    if (a.qkv_f32) {
+#pragma unroll
+                        for (int u = 0; u < 4; u++) x[c] += u < a.n_slices ? __uint_as_float(early[c][u]) : 0.f;
+                    } else x[c] = __uint_as_float(early[c][0] << 16);
+                }
+                for (int sl = 4; sl < a.n_slices; sl++) {
+                    const char* slice = (const char*)a.qkv + ((size_t)seq * a.row_stride + (size_t)sl * a.slice_stride) * 4;
+                    float more[NE];
+#pragma unroll
+                    for (int c = 0; c < NE; c++) more[c] = *reinterpret_cast<const float*>(slice + (c < 2 || a.write_kv ? cols[c] : col) * 4u);
+#pragma unroll
+                    for (int c = 0; c < NE; c++) x[c] += more[c];
+                }
+            } else {
+                if (writer) vals(std::integral_constant<int, 6>(), cols, x);     // (the whole block takes this branch or the other)
+                else vals(std::integral_constant<int, 2>(), cols, x);
+                freq = a.inv_freq[f];
+            }
+            const float ang = (float)p * freq;
             float cs, sn;
             sincosf(ang, &sn, &cs);
             q_lds[qi * HD + f] = f32_to_bf16(x[0] * cs - x[1] * sn);
@@ -266,11 +324,11 @@ attn_decode_k(DecodeArgs a) {
             }
         }
         for (int idx = tid; idx < G * rest; idx += DTH) {         // elements outside the rotation
-            const int qi = idx / rest, d = a.rot + idx - qi * rest;
+            const int qi = quotient(idx, rest), d = a.rot + idx - qi * rest;
             const bool kv = writer && idx < rest;                 // then qi == 0
-            const long cols[3] = {(long)(kvh * G + qi) * HD + d, kcol + d, vcol + d};
+            const unsigned cols[3] = {(unsigned)(kvh * G + qi) * HD + d, kcol + d, vcol + d};
             float x[3];
-            if (writer) vals(std::integral_constant<int, 3>(), cols, x);
+            if (writer) vals(std::integral_constant<int, 3>(), cols, x);     // (the whole block takes this branch or the other)
             else vals(std::integral_constant<int, 1>(), cols, x);
             q_lds[qi * HD + d] = f32_to_bf16(x[0]);
             if (kv) {
@@ -550,6 +608,7 @@ static int decode_launch(DecodeArgs a, int n_seq, void* workspace, hipStream_t s
     TP_REQUIRE(a.H % a.KV == 0, "attention: %d query heads are no multiple of %d kv heads", a.H, a.KV);
     const int G = a.H / a.KV;
     TP_REQUIRE(G <= 16, "attention decode (matrix-core kernel): %d query heads per kv head exceed 16", G);
+    a.G = G;
     if (a.pool_kv == 0) a.pool_kv = a.KV;
     TP_REQUIRE(a.pool_kv > 0 && a.KV % a.pool_kv == 0 && (a.pool_kv == a.KV || !a.qkv),
                "attention decode: %d groups of heads cannot share %d kv heads of the cache", a.KV, a.pool_kv);
@@ -606,7 +665,7 @@ extern "C" int tp_attn_decode(const void* q, long q_stride, int n_seq, int H, in
     TP_REQUIRE(q_stride % 8 == 0 && (uintptr_t)q % 16 == 0, "attention decode: query rows must be 16-byte aligned");
     DecodeArgs a{(const bf16_t*)q, q_stride, H, KV, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool,
                  page, rows_cap, scale, cap, window, (bf16_t*)out, nullptr, nullptr, nsplit,
-                 nullptr, 0, 1, 0, 0, nullptr, 0, 0, 0, chunk, head_scale, sink, keep, pin, TpPositional{}};
+                 nullptr, 0, 1, 0, 0, nullptr, 0, 0, 0, chunk, head_scale, sink, keep, pin, TpPositional{}, 0};
     if (int rc = take_positional(a, by_position)) return rc;
     return decode_launch(a, n_seq, workspace, (hipStream_t)stream);
 }
@@ -621,7 +680,7 @@ extern "C" int tp_attn_decode_shared(const void* q, long q_stride, int n_seq, in
     TP_REQUIRE(q_stride % 8 == 0 && (uintptr_t)q % 16 == 0, "attention decode: query rows must be 16-byte aligned");
     DecodeArgs a{(const bf16_t*)q, q_stride, H, KV, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool,
                  page, rows_cap, scale, cap, window, (bf16_t*)out, nullptr, nullptr, nsplit,
-                 nullptr, 0, 1, 0, 0, nullptr, 0, 0, pool_kv, 0, nullptr, sink, 0, 0, TpPositional{}};
+                 nullptr, 0, 1, 0, 0, nullptr, 0, 0, pool_kv, 0, nullptr, sink, 0, 0, TpPositional{}, 0};
     return decode_launch(a, n_seq, workspace, (hipStream_t)stream);
 }
 
@@ -641,7 +700,7 @@ extern "C" int tp_attn_decode_fused(const void* qkv, int qkv_dtype, int n_slices
     TP_REQUIRE(row_stride >= (long)(H + (write_kv ? 2 * KV : 0)) * HD, "attention decode (fused): rows of %ld elements are too short", row_stride);
     DecodeArgs a{nullptr, 0, H, KV, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool,
                  page, rows_cap, scale, cap, window, (bf16_t*)out, nullptr, nullptr, nsplit,
-                 qkv, qkv_dtype == TP_F32 ? 1 : 0, n_slices, slice_stride, row_stride, inv_freq, rot, write_kv, 0, 0, nullptr, sink, keep, pin, TpPositional{}};
+                 qkv, qkv_dtype == TP_F32 ? 1 : 0, n_slices, slice_stride, row_stride, inv_freq, rot, write_kv, 0, 0, nullptr, sink, keep, pin, TpPositional{}, 0};
     if (int rc = take_positional(a, by_position)) return rc;
     return decode_launch(a, n_seq, workspace, (hipStream_t)stream);
 }

@@ -23,12 +23,9 @@ static inline int tp_cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 // ---- device: number formats ------------------------------------------------------------------
 __device__ __forceinline__ float bf16_to_f32(bf16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 
-__device__ __forceinline__ bf16_t f32_to_bf16(float f) {      // round to nearest even; NaN stays NaN
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)((u >> 16) | 0x40);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (bf16_t)(u >> 16);
-}
+// Round to nearest even; NaN stays NaN.  gfx950 has the instruction (v_cvt_pk_bf16_f32, two at once), which gives the bits of the eight
+// integer ones in its place for all 2^32 inputs.  Code that a launch runs once waits for its instructions to arrive.
+__device__ __forceinline__ bf16_t f32_to_bf16(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
 
 __device__ __forceinline__ float ld_f32(const float* p) { return *p; }
 __device__ __forceinline__ float ld_f32(const bf16_t* p) { return bf16_to_f32(*p); }

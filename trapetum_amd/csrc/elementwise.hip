@@ -223,43 +223,55 @@ __device__ __forceinline__ void st4(bf16_t* p, const float (&v)[4]) {
     *reinterpret_cast<uint2*>(p) = t;
 }
 
+// four elements at 32 bits of the lane's beyond a row that all lanes share: one instruction, no address arithmetic.  (A kernel of this kind
+// runs its code once, and waits for it: 64 bytes of instructions are some 50 cycles.)
+template <typename T>
+__device__ __forceinline__ void ld4(const T* row, unsigned i, float (&o)[4]) { ld4(reinterpret_cast<const T*>(reinterpret_cast<const char*>(row) + i * (unsigned)sizeof(T)), o); }
+template <typename T>
+__device__ __forceinline__ void st4(T* row, unsigned i, const float (&v)[4]) { st4(reinterpret_cast<T*>(reinterpret_cast<char*>(row) + i * (unsigned)sizeof(T)), v); }
+
 template <typename TR, typename T, int CPT, int NTH>
 __global__ void __launch_bounds__(NTH)
 add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int n_slices, long slice_stride,
                    const float* __restrict__ gain_post, float eps_post,
                    const float* __restrict__ gain_next, float eps_next, T* __restrict__ out, int D, int groups) {
     __shared__ float red[16], red_next[16];             // one for each of the two sums: no barrier between their uses
-    if (gain_post) gain_post += (size_t)part_of(groups) * D;
-    if (gain_next) gain_next += (size_t)part_of(groups) * D;
+    const unsigned part = groups > 1 ? (blockIdx.x % (unsigned)groups) * (unsigned)D : 0u;      // where the row's stretch of the gains begins
     float* sr = stream + (size_t)blockIdx.x * D;
     const TR* ar = rows + (size_t)blockIdx.x * D;
     float a[CPT][4], v[CPT][4], gp[CPT][4], gn[CPT][4];
 #pragma unroll
     for (int j = 0; j < CPT; j++) {
-        const int i = (threadIdx.x + j * NTH) * 4;
-        const bool ok = i < D;
-        const int ic = ok ? i : 0;                       // a chunk past the row reads the row's first and counts as zero
+        const unsigned i = (threadIdx.x + j * NTH) * 4u;
+        const bool ok = i < (unsigned)D;
+        const unsigned ic = ok ? i : 0u;                 // a chunk past the row reads the row's first and counts as zero
         // the stream, the gains and a group of slices are asked for together: a loop of load-then-add would pay one
         // trip to memory per slice.  Slices are added in slice order; past the last one the load repeats it and adds
-        // nothing.  Groups of four; a row of one chunk a lane takes twelve at a time while more than four are left
-        // (a product of few rows comes in up to sixteen slices).
-        ld4(sr + ic, v[j]);
-        if (gain_post) ld4(gain_post + ic, gp[j]);
-        if (gain_next) ld4(gain_next + ic, gn[j]);
-        ld4(ar + ic, a[j]);
+        // nothing.  Groups of four; a row of one chunk a lane takes twelve at a time while more than six are left, and six where
+        // more than four are (a product of few rows comes in up to sixteen slices; of seven 3.6 us, 3.5 so).
+        ld4(sr, ic, v[j]);
+        ld4(ar, ic, a[j]);
+        if (gain_post) ld4(gain_post, part + ic, gp[j]);
+        if (gain_next) ld4(gain_next, part + ic, gn[j]);
+        const TR* slice = ar;                            // the last one asked for
         auto add_group = [&](int s0, auto width) {
             constexpr int W = decltype(width)::value;
             float t[W][4];
 #pragma unroll
-            for (int u = 0; u < W; u++) ld4(ar + (size_t)(s0 + u < n_slices ? s0 + u : n_slices - 1) * slice_stride + ic, t[u]);
+            for (int u = 0; u < W; u++) {
+                slice += s0 + u < n_slices ? slice_stride : 0;
+                ld4(slice, ic, t[u]);
+            }
 #pragma unroll
             for (int u = 0; u < W; u++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) a[j][e] += s0 + u < n_slices ? t[u][e] : 0.f;
         };
         int s0 = 1;
-        if (CPT == 1)
-            for (; s0 + 4 < n_slices; s0 += 12) add_group(s0, std::integral_constant<int, 12>());
+        if (CPT == 1) {
+            for (; s0 + 6 < n_slices; s0 += 12) add_group(s0, std::integral_constant<int, 12>());
+            if (s0 + 4 < n_slices) { add_group(s0, std::integral_constant<int, 6>()); s0 += 6; }
+        }
         for (; s0 < n_slices; s0 += 4) add_group(s0, std::integral_constant<int, 4>());
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -280,7 +292,7 @@ add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
     float ss2 = 0.f;
 #pragma unroll
     for (int j = 0; j < CPT; j++) {
-        const int i = (threadIdx.x + j * NTH) * 4;
+        const unsigned i = (threadIdx.x + j * NTH) * 4u;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             float t = a[j][e];
@@ -288,7 +300,7 @@ add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
             v[j][e] += t;
             ss2 += v[j][e] * v[j][e];                    // chunks past the row hold zeros
         }
-        if (i < D) st4(sr + i, v[j]);
+        if (i < (unsigned)D) st4(sr, i, v[j]);
     }
     if (!gain_next) return;
     ss2 = block_sum_once<NTH>(ss2, red_next);
@@ -296,11 +308,11 @@ add_rms_norm_vec_k(float* __restrict__ stream, const TR* __restrict__ rows, int 
     T* orow = out + (size_t)blockIdx.x * D;
 #pragma unroll
     for (int j = 0; j < CPT; j++) {
-        const int i = (threadIdx.x + j * NTH) * 4;
+        const unsigned i = (threadIdx.x + j * NTH) * 4u;
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) o[e] = (v[j][e] * scale_s) * gn[j][e];
-        if (i < D) st4(orow + i, o);
+        if (i < (unsigned)D) st4(orow, i, o);
     }
 }
 
