@@ -3,7 +3,7 @@
 // The keys that the query sees are cut, from the first on, into groups of up to four; state w of eight takes the groups w, w + 8,
 // .. with a running softmax of its own, and the eight states are joined in order at the end.  What bounds it is latency: a
 // group's key and value rows are fetched while the group before is worked on, the dot products of its keys are summed over the
-// wave together (seven exchanges instead of six a key), and eight waves, one a state, have their chains in flight.  (One wave, a
+// wave together (seven exchanges instead of six a key, by lane moves), and eight waves, one a state, have their chains in flight.  (One wave, a
 // key after the other, took 0.63 us a key: 132 us of a float32 decode step's layer at 200 keys and heads of 256, 11 us so.)
 // Where a launch has many rows of few keys a wave takes a row and forms its eight states itself: the same bits (2,048 rows with a
 // window of 3 and heads of 64: 91 us by blocks, 14 by waves).
@@ -34,6 +34,7 @@ struct AttnSimpleArgs {
     int chunk; const float* head_scale; const float* sink;        // 0 and null: none
     TpPositional by_position;
     int keep, pin;                                       // positions seen beside the window; rows of the cache in front of its ring
+    int page_shift;                                      // the page size's power of two, -1 if it is none (set by the launch)
 };
 
 namespace {
@@ -81,9 +82,12 @@ struct Query {
             const int t = min(at(first + n), p);             // past the last key: a row that exists, without weight
             const T *kp, *vp;
             if (t < start) {
-                const int row = a.rows_cap > 0 && t >= a.pin ? a.pin + (t - a.pin) % (a.rows_cap - a.pin) : t;
-                const int pg = a.table[(size_t)seq * a.table_w + row / a.page];
-                const size_t off = (((size_t)pg * a.KV + g) * a.page + row % a.page) * a.hd;
+                // (a division is some thirty instructions, and a group has its keys' in a row before its loads)
+                const int ring = a.rows_cap - a.pin, u = t - a.pin;
+                const int row = a.rows_cap > 0 && u >= ring ? a.pin + u % ring : t;
+                const int page = a.page_shift >= 0 ? row >> a.page_shift : row / a.page;
+                const int pg = a.table[(size_t)seq * a.table_w + page];
+                const size_t off = (((size_t)pg * a.KV + g) * a.page + (row - page * a.page)) * a.hd;
                 kp = (const T*)a.k_pool + off;
                 vp = (const T*)a.v_pool + off;
             } else {
@@ -94,7 +98,7 @@ struct Query {
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
                 const int d = lane + 64 * j;
-                const int dc = d < a.hd ? d : 0;
+                const unsigned dc = d < a.hd ? d : 0;
                 const float kx = KEY ? ld_f32(kp + dc) : 0.f, vx = VALUE ? ld_f32(vp + dc) : 0.f;
                 if (KEY) kk[n][j] = d < a.hd ? kx : 0.f;
                 if (VALUE) vv[n][j] = d < a.hd ? vx : 0.f;
@@ -124,14 +128,22 @@ struct Query {
         const int mine = lane & (KEYS - 1);
         float s = part[0];
         if constexpr (KEYS == 4) {
-            const float s01 = ((lane & 1) ? part[1] : part[0]) + __shfl_xor((lane & 1) ? part[0] : part[1], 1, 64);
-            const float s23 = ((lane & 1) ? part[3] : part[2]) + __shfl_xor((lane & 1) ? part[2] : part[3], 1, 64);
-            s = ((lane & 2) ? s23 : s01) + __shfl_xor((lane & 2) ? s01 : s23, 2, 64);
+            const float s01 = ((lane & 1) ? part[1] : part[0]) + across_f<1>((lane & 1) ? part[0] : part[1], lane);
+            const float s23 = ((lane & 1) ? part[3] : part[2]) + across_f<1>((lane & 1) ? part[2] : part[3], lane);
+            s = ((lane & 2) ? s23 : s01) + across_f<2>((lane & 2) ? s01 : s23, lane);
         } else if constexpr (KEYS == 2) {
-            s = ((lane & 1) ? part[1] : part[0]) + __shfl_xor((lane & 1) ? part[0] : part[1], 1, 64);
+            s = ((lane & 1) ? part[1] : part[0]) + across_f<1>((lane & 1) ? part[0] : part[1], lane);
         }
+        if constexpr (KEYS == 1) {                           // (heads of more than 512: 11.0 us by shuffles, 13.2 by lane moves, 40 keys)
 #pragma unroll
-        for (int x = KEYS; x < 64; x <<= 1) s += __shfl_xor(s, x, 64);
+            for (int x = 1; x < 64; x <<= 1) s += __shfl_xor(s, x, 64);
+        } else {
+            if constexpr (KEYS == 2) s += across_f<2>(s, lane);
+            s += across_f<4>(s, lane);
+            s += across_f<8>(s, lane);
+            s += across_f<16>(s, lane);
+            s += across_f<32>(s, lane);
+        }
         s *= scale;
         if (a.cap > 0.f) s = softcap_f(s, a.cap);
         if (bias) s += bias[min(max(p - at(first + mine), 0), (int)a.by_position.reach)];
@@ -140,8 +152,8 @@ struct Query {
 
     // the largest score of a group, in every lane
     __device__ __forceinline__ float top_of(float s) const {
-#pragma unroll
-        for (int x = 1; x < KEYS; x <<= 1) s = fmaxf(s, __shfl_xor(s, x, 64));
+        if constexpr (KEYS > 1) s = fmaxf(s, across_f<1>(s, lane));
+        if constexpr (KEYS > 2) s = fmaxf(s, across_f<2>(s, lane));
         return s;
     }
 
@@ -149,8 +161,8 @@ struct Query {
     __device__ __forceinline__ void add(float s, const float (&vv)[KEYS][NJ], float& m, float& l, float (&o)[NJ]) const {
         const float m_new = fmaxf(m, top_of(s)), alpha = expf(m - m_new), pr = expf(s - m_new);
         float sum = pr;
-#pragma unroll
-        for (int x = 1; x < KEYS; x <<= 1) sum += __shfl_xor(sum, x, 64);
+        if constexpr (KEYS > 1) sum += across_f<1>(sum, lane);
+        if constexpr (KEYS > 2) sum += across_f<2>(sum, lane);
         l = fmaf(l, alpha, sum);
         float w[KEYS];
 #pragma unroll
@@ -310,7 +322,8 @@ attn_simple_rows_k(AttnSimpleArgs a, int M) {
         if (lane + 64 * j < a.hd) st_f32(out + lane + 64 * j, t[j] * inv);
 }
 
-static int launch(const AttnSimpleArgs& a, int dtype, int M, int most, hipStream_t s) {
+static int launch(AttnSimpleArgs a, int dtype, int M, int most, hipStream_t s) {
+    a.page_shift = a.page > 0 && (a.page & (a.page - 1)) == 0 ? __builtin_ctz((unsigned)a.page) : -1;
     TP_REQUIRE(a.keep >= 0 && a.pin >= 0 && (a.keep == 0 || (a.window > 0 && a.chunk == 0)), "attention: %d kept positions stand beside a window, without chunks", a.keep);
     TP_REQUIRE(a.rows_cap == 0 || (a.pin < a.rows_cap && a.keep <= a.pin), "attention: %d kept positions and %d rows before a ring do not fit a cache of %d rows", a.keep, a.pin, a.rows_cap);
     TP_REQUIRE(M > 0 && a.H > 0 && a.KV > 0 && a.hd > 0, "attention: empty shape rows=%d heads=%d kv=%d head_dim=%d", M, a.H, a.KV, a.hd);

@@ -52,6 +52,26 @@ __device__ __forceinline__ float wave_butterfly(float v, OP op) {
 __device__ __forceinline__ float wave_sum(float v) { return wave_butterfly(v, [](float a, float b) { return a + b; }); }
 __device__ __forceinline__ float wave_max(float v) { return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); }); }
 
+// The value of lane ^ STRIDE, by data-parallel moves (a shuffle through LDS takes three times as long).
+template <int STRIDE>
+__device__ __forceinline__ uint32_t across(uint32_t v, int lane) {
+    if constexpr (STRIDE == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);            // quads 1 0 3 2
+    else if constexpr (STRIDE == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);       // quads 2 3 0 1
+    else if constexpr (STRIDE == 4) {                                                                             // rows of 16 turned by 4 and by 12
+        const uint32_t back = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xf, 0xf, true), ahead = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x12c, 0xf, 0xf, true);
+        return lane & 4 ? back : ahead;
+    } else if constexpr (STRIDE == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);    // turned by 8
+    else if constexpr (STRIDE == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return lane & 16 ? r[0] : r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return lane & 32 ? r[0] : r[1];
+    }
+}
+template <int STRIDE>
+__device__ __forceinline__ float across_f(float v, int lane) { return __uint_as_float(across<STRIDE>(__float_as_uint(v), lane)); }
+
 // Sum over a block of up to 1024 threads (THREADS of them, where that is known); every thread gets the result.  `red` holds 16
 // floats of LDS.  The order of additions depends only on the block size, never on timing.
 template <int THREADS = 0>

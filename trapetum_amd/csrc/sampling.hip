@@ -260,23 +260,6 @@ __device__ __forceinline__ void pick_bucket(const unsigned* hist, bool from_top,
     rem_out = (unsigned)__shfl((int)r, L, 64);
 }
 
-// The value of lane ^ STRIDE, by data-parallel moves (a shuffle through LDS takes three times as long).
-template <int STRIDE>
-__device__ __forceinline__ uint32_t across(uint32_t v, int lane) {
-    if constexpr (STRIDE == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);            // quads 1 0 3 2
-    else if constexpr (STRIDE == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);       // quads 2 3 0 1
-    else if constexpr (STRIDE == 4) {                                                                             // rows of 16 turned by 4 and by 12
-        const uint32_t back = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xf, 0xf, true), ahead = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x12c, 0xf, 0xf, true);
-        return lane & 4 ? back : ahead;
-    } else if constexpr (STRIDE == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);    // turned by 8
-    else if constexpr (STRIDE == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-        return lane & 16 ? r[0] : r[1];
-    } else {
-        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-        return lane & 32 ? r[0] : r[1];
-    }
-}
 __device__ __forceinline__ int wave_least(int v, int lane) {
     v = min(v, (int)across<32>((uint32_t)v, lane));
     v = min(v, (int)across<16>((uint32_t)v, lane));
