@@ -1242,3 +1242,35 @@ def test_sample_by_groups_is_the_sampler_alone(ops, kind):
             alone = torch.empty(rows, dtype=torch.int32, device=DEV)
             assert ops.lib.tp_sample(z.data_ptr(), rows, vocab, 0.8, top_k, top_p, u.data_ptr(), alone.data_ptr(), None, ops._stream()) == 0
             assert torch.equal(ops.sample(z, 0.8, top_k, top_p, u), alone), (rows, vocab, top_k)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("M", [1, 5, 40, 300])
+@pytest.mark.parametrize("hd,rot,turn,rows_cap", [(128, 64, 128, 0), (64, 64, 32, 0), (96, 16, 48, 128), (24, 24, 6, 0)])
+def test_values_turned_with_queries_and_keys(ops, hd, rot, turn, rows_cap, M, dt):
+    """Values that turn in the launch that turns queries and keys: the bits of a launch of their own before it, in the step's rows and in
+    the cache, at few rows (a block a head), some (several heads a block) and many (a block a row), with and without the write."""
+    H, KV, page = 6, 2, 64
+    rows = randn(M, (H + 2 * KV) * hd, dtype=DT[dt], seed=11)
+    freq, v_freq = ((100.0 ** (-torch.arange(n // 2).float() / (n // 2))).contiguous().to(DEV) for n in (rot, turn))
+    cut = M // 3
+    row_seq = torch.tensor([0] * cut + [1] * (M - cut), dtype=torch.int32, device=DEV)
+    row_pos = torch.tensor(list(range(7, 7 + cut)) + list(range(M - cut)), dtype=torch.int32, device=DEV)
+    new_len = torch.tensor([7 + cut, M - cut], dtype=torch.int32, device=DEV)
+    pages = -(-(rows_cap or 310) // page)
+    table = torch.arange(2 * pages, dtype=torch.int32, device=DEV).view(2, pages)
+    for write in (True, False):
+        got = []
+        for together in (True, False):
+            t = rows.clone()
+            q, k, v = t[:, :H * hd], t[:, H * hd:(H + KV) * hd], t[:, (H + KV) * hd:]
+            pools = [torch.full((2 * pages, KV, page, hd), 7.0, dtype=DT[dt], device=DEV) for _ in range(2)]
+            if not together:
+                ops.rope_kv_write(v, None, None, KV, 0, hd, v_freq, turn, row_seq, row_pos, new_len, None, None, None, 0, write=False)
+            ops.rope_kv_write(q, k, v, H, KV, hd, freq, rot, row_seq, row_pos, new_len, table, *pools, rows_cap, write=write,
+                              **(dict(value_freq=v_freq) if together else {}))
+            got.append([t] + pools)
+        assert all(torch.equal(a, b) for a, b in zip(*got)), write
+        assert bool((got[0][2] != 7.0).any()) == write
+    with pytest.raises(Exception, match="values that turn"):
+        ops.rope_kv_write(q, None, None, H, 0, hd, freq, rot, row_seq, row_pos, new_len, None, None, None, 0, write=False, value_freq=v_freq)

@@ -585,17 +585,21 @@ extern "C" int tp_gather_rows(const float* x, const int* rows, float* out, int n
 // computes the cosine and sine of its pair once and applies them to all of them.  A key head goes into the
 // cache, with its value head, straight from registers; without a page table the keys are rotated and nothing is
 // cached (a step whose attention still has to read the cache as earlier steps left it caches its rows afterwards).
+// v_freq (or null): the values turn by their position as well, over their first v_rot elements, in place and before they are cached;
+// blocks from `groups` on turn and cache the value heads (a launch of their own took 3 us of a decode step's layer).
 template <typename T>
 __global__ void __launch_bounds__(128)
 rope_kv_write_k(T* __restrict__ q, long q_stride, T* __restrict__ k, long k_stride,
-                const T* __restrict__ v, long v_stride, int H, int KV, int hd,
-                const float* __restrict__ inv_freq, int rot,
+                T* __restrict__ v, long v_stride, int H, int KV, int hd,
+                const float* __restrict__ inv_freq, int rot, const float* __restrict__ v_freq, int v_rot, int groups,
                 const int* __restrict__ row_seq, const int* __restrict__ row_pos,
                 const int* __restrict__ new_len, const int* __restrict__ table, int table_w,
                 T* __restrict__ k_pool, T* __restrict__ v_pool, int page, int rows_cap, int pin, int hpb, int pairing) {
     const int r = blockIdx.x;
-    const int j_begin = blockIdx.y * hpb, j_end = min(j_begin + hpb, H + (k ? KV : 0));
+    const bool values = (int)blockIdx.y >= groups;
+    const int j_begin = values ? H + (blockIdx.y - groups) * hpb : blockIdx.y * hpb, j_end = min(j_begin + hpb, H + (k ? KV : 0));
     const int pos = row_pos[r];
+    if (values) { inv_freq = v_freq; rot = v_rot; }
     const int half = rot / 2;
     // where the row's keys and values go: the same page and row for every kv head
     size_t cache_at = 0;
@@ -618,7 +622,7 @@ rope_kv_write_k(T* __restrict__ q, long q_stride, T* __restrict__ k, long k_stri
         const int e0 = pairing == TP_ROPE_NEIGHBOURS ? 2 * f : f, e1 = pairing == TP_ROPE_NEIGHBOURS ? 2 * f + 1 : f + half;
         for (int j = j_begin; j < j_end; j++) {
             const bool is_q = j < H;
-            T* x = is_q ? q + (size_t)r * q_stride + (size_t)j * hd : k + (size_t)r * k_stride + (size_t)(j - H) * hd;
+            T* x = is_q ? q + (size_t)r * q_stride + (size_t)j * hd : values ? v + (size_t)r * v_stride + (size_t)(j - H) * hd : k + (size_t)r * k_stride + (size_t)(j - H) * hd;
             const float x0 = ld_f32(x + e0), x1 = ld_f32(x + e1);
             const float y0 = x0 * c - x1 * sn, y1 = x1 * c + x0 * sn;
             st_f32(x + e0, y0);
@@ -627,10 +631,13 @@ rope_kv_write_k(T* __restrict__ q, long q_stride, T* __restrict__ k, long k_stri
             const T* vsrc = v + (size_t)r * v_stride + (size_t)(j - H) * hd;
             if (cached) {
                 const size_t off = cache_at + (size_t)(j - H) * page * hd;
-                st_f32(k_pool + off + e0, y0);
-                st_f32(k_pool + off + e1, y1);
-                v_pool[off + e0] = vsrc[e0];
-                v_pool[off + e1] = vsrc[e1];
+                T* const pool = values ? v_pool : k_pool;
+                st_f32(pool + off + e0, y0);
+                st_f32(pool + off + e1, y1);
+                if (!v_freq) {
+                    v_pool[off + e0] = vsrc[e0];
+                    v_pool[off + e1] = vsrc[e1];
+                }
             }
         }
     }
@@ -639,7 +646,10 @@ rope_kv_write_k(T* __restrict__ q, long q_stride, T* __restrict__ k, long k_stri
             const size_t off = cache_at + (size_t)(j - H) * page * hd;
             const T* ksrc = k + (size_t)r * k_stride + (size_t)(j - H) * hd;
             const T* vsrc = v + (size_t)r * v_stride + (size_t)(j - H) * hd;
-            for (int d = rot + threadIdx.x; d < hd; d += blockDim.x) { k_pool[off + d] = ksrc[d]; v_pool[off + d] = vsrc[d]; }
+            for (int d = rot + threadIdx.x; d < hd; d += blockDim.x) {
+                if (!values) k_pool[off + d] = ksrc[d];
+                if (values || !v_freq) v_pool[off + d] = vsrc[d];
+            }
         }
 }
 
@@ -648,15 +658,20 @@ rope_kv_write_k(T* __restrict__ q, long q_stride, T* __restrict__ k, long k_stri
 // stores (the 2B prefills of the benchmark, 2,048 and 4,096 rows: 18.5 -> 12.9 us a layer on average).
 __global__ void __launch_bounds__(256)
 rope_kv_write_vec_k(bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ k, long k_stride,
-                    const bf16_t* __restrict__ v, long v_stride, int H, int KV, int hd,
-                    const float* __restrict__ inv_freq, int rot,
+                    bf16_t* __restrict__ v, long v_stride, int H, int KV, int hd,
+                    const float* __restrict__ inv_freq, int rot, const float* __restrict__ v_freq, int v_rot,
                     const int* __restrict__ row_seq, const int* __restrict__ row_pos,
                     const int* __restrict__ new_len, const int* __restrict__ table, int table_w,
                     bf16_t* __restrict__ k_pool, bf16_t* __restrict__ v_pool, int page, int rows_cap, int pin) {
     // cosine and sine of pair f at [f % 8][f / 8]: the threads of a wave, which turn neighbouring pieces of 8 pairs, then
     // read neighbouring words (pair by pair in the pairs' own order, a wave's reads fell on four banks)
-    __shared__ float cs[8 * 16], sn[8 * 16];
-    const int r = blockIdx.x, pos = row_pos[r], half = rot / 2;
+    __shared__ float cs[8 * 16], sn[8 * 16], v_cs[8 * 16], v_sn[8 * 16];
+    const int r = blockIdx.x, pos = row_pos[r], half = rot / 2, v_half = v_freq ? v_rot / 2 : 0;
+    for (int f = threadIdx.x; f < v_half; f += 256) {
+        const float ang = (float)pos * v_freq[f];
+        v_cs[(f & 7) * 16 + (f >> 3)] = cosf(ang);
+        v_sn[(f & 7) * 16 + (f >> 3)] = sinf(ang);
+    }
     for (int f = threadIdx.x; f < half; f += 256) {
         const float ang = (float)pos * inv_freq[f];
         cs[(f & 7) * 16 + (f >> 3)] = cosf(ang);
@@ -701,25 +716,50 @@ rope_kv_write_vec_k(bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ 
             const size_t off = cache_at + (size_t)(j - H) * page * hd;
             *reinterpret_cast<uint4*>(k_pool + off + f0) = lo.u;
             *reinterpret_cast<uint4*>(k_pool + off + f0 + half) = hi.u;
-            *reinterpret_cast<uint4*>(v_pool + off + f0) = v0;
-            *reinterpret_cast<uint4*>(v_pool + off + f0 + half) = v1;
+            if (!v_freq) {
+                *reinterpret_cast<uint4*>(v_pool + off + f0) = v0;
+                *reinterpret_cast<uint4*>(v_pool + off + f0 + half) = v1;
+            }
         }
     }
-    if (cached) {                                                 // elements outside the rotation
+    for (int item = threadIdx.x, v_pieces = v_half / 8; item < KV * v_pieces; item += 256) {      // values that turn
+        const int j = item / v_pieces, piece = item - j * v_pieces, f0 = piece * 8;
+        bf16_t* x = v + (size_t)r * v_stride + (size_t)j * hd;
+        Piece lo, hi;
+        lo.u = *reinterpret_cast<const uint4*>(x + f0);
+        hi.u = *reinterpret_cast<const uint4*>(x + f0 + v_half);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float x0 = bf16_to_f32(lo.h[e]), x1 = bf16_to_f32(hi.h[e]), c = v_cs[e * 16 + piece], sv = v_sn[e * 16 + piece];
+            lo.h[e] = f32_to_bf16(x0 * c - x1 * sv);
+            hi.h[e] = f32_to_bf16(x1 * c + x0 * sv);
+        }
+        *reinterpret_cast<uint4*>(x + f0) = lo.u;
+        *reinterpret_cast<uint4*>(x + f0 + v_half) = hi.u;
+        if (cached) {
+            bf16_t* const to = v_pool + cache_at + (size_t)j * page * hd;
+            *reinterpret_cast<uint4*>(to + f0) = lo.u;
+            *reinterpret_cast<uint4*>(to + f0 + v_half) = hi.u;
+        }
+    }
+    if (cached) {                                                 // elements outside the rotations
         const int rest = (hd - rot) / 8;
         for (int item = threadIdx.x; item < KV * rest; item += 256) {
             const int j = item / rest, d = rot + (item - j * rest) * 8;
-            const uint4 kk = *reinterpret_cast<const uint4*>(k + (size_t)r * k_stride + (size_t)j * hd + d);
-            const uint4 vv = *reinterpret_cast<const uint4*>(v + (size_t)r * v_stride + (size_t)j * hd + d);
             const size_t off = cache_at + (size_t)j * page * hd + d;
-            *reinterpret_cast<uint4*>(k_pool + off) = kk;
-            *reinterpret_cast<uint4*>(v_pool + off) = vv;
+            *reinterpret_cast<uint4*>(k_pool + off) = *reinterpret_cast<const uint4*>(k + (size_t)r * k_stride + (size_t)j * hd + d);
+            if (!v_freq) *reinterpret_cast<uint4*>(v_pool + off) = *reinterpret_cast<const uint4*>(v + (size_t)r * v_stride + (size_t)j * hd + d);
+        }
+        const int v_rest = v_freq ? (hd - v_rot) / 8 : 0;
+        for (int item = threadIdx.x; item < KV * v_rest; item += 256) {
+            const int j = item / v_rest, d = v_rot + (item - j * v_rest) * 8;
+            *reinterpret_cast<uint4*>(v_pool + cache_at + (size_t)j * page * hd + d) = *reinterpret_cast<const uint4*>(v + (size_t)r * v_stride + (size_t)j * hd + d);
         }
     }
 }
 
-extern "C" int tp_rope_kv_write(void* q, long q_stride, void* k, long k_stride, const void* v, long v_stride,
-                                int dtype, int M, int H, int KV, int hd, const float* inv_freq, int rot,
+extern "C" int tp_rope_kv_write(void* q, long q_stride, void* k, long k_stride, void* v, long v_stride,
+                                int dtype, int M, int H, int KV, int hd, const float* inv_freq, int rot, const float* v_freq, int v_rot,
                                 const int* row_seq, const int* row_pos, const int* new_len,
                                 const int* table, int table_w, void* k_pool, void* v_pool,
                                 int page, int rows_cap, int pin, int pairing, void* stream) {
@@ -730,6 +770,7 @@ extern "C" int tp_rope_kv_write(void* q, long q_stride, void* k, long k_stride, 
                pairing, TP_ROPE_HALVES, TP_ROPE_NEIGHBOURS);
     // table null: the keys are rotated and nothing is cached
     TP_REQUIRE(!k || (v && KV > 0), "rope_kv_write: keys without values");
+    TP_REQUIRE(!v_freq || (k && pairing == TP_ROPE_HALVES && v_rot > 0 && v_rot <= hd && v_rot % 2 == 0), "rope_kv_write: values turn over %d of %d elements, in halves, beside keys", v_rot, hd);
     TP_REQUIRE(!k || !table || (k_pool && v_pool && page > 0 && table_w > 0), "rope_kv_write: a page table without cache pools");
     if (!table) { page = 1; rows_cap = 0; pin = 0; }
     TP_REQUIRE(rows_cap >= 0 && (rows_cap == 0 || rows_cap % page == 0), "rope_kv_write: ring of %d rows is no multiple of the page size %d", rows_cap, page);
@@ -738,22 +779,23 @@ extern "C" int tp_rope_kv_write(void* q, long q_stride, void* k, long k_stride, 
     TP_REQUIRE(H + KV <= 65535, "rope_kv_write: %d heads exceed one launch", H + KV);
     const int heads = H + (k ? KV : 0);
     auto piecewise = [](const void* p, long stride) { return !p || ((uintptr_t)p % 16 == 0 && stride % 8 == 0); };
-    if (pairing == TP_ROPE_HALVES && dtype == TP_BF16 && M >= 256 && hd % 8 == 0 && rot % 16 == 0 && rot <= 256 && piecewise(q, q_stride) && piecewise(k, k_stride) &&
+    if (pairing == TP_ROPE_HALVES && dtype == TP_BF16 && M >= 256 && hd % 8 == 0 && rot % 16 == 0 && rot <= 256 && (!v_freq || (v_rot % 16 == 0 && v_rot <= 256)) && piecewise(q, q_stride) && piecewise(k, k_stride) &&
         piecewise(v, v_stride) && piecewise(k_pool, 8) && piecewise(v_pool, 8)) {
-        rope_kv_write_vec_k<<<M, 256, 0, s>>>((bf16_t*)q, q_stride, (bf16_t*)k, k_stride, (const bf16_t*)v, v_stride, H, KV, hd,
-            inv_freq, rot, row_seq, row_pos, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool, page, rows_cap, pin);
+        rope_kv_write_vec_k<<<M, 256, 0, s>>>((bf16_t*)q, q_stride, (bf16_t*)k, k_stride, (bf16_t*)v, v_stride, H, KV, hd,
+            inv_freq, rot, v_freq, v_rot, row_seq, row_pos, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool, page, rows_cap, pin);
         return tp_check_launch("rope_kv_write");
     }
     // many rows: one block per row shares each pair's cosine and sine over all heads; few rows: a block per head
     const int hpb = M >= 256 ? heads : (M >= 32 ? (heads + 3) / 4 : 1);
-    dim3 grid(M, (heads + hpb - 1) / hpb);
+    const int groups = (heads + hpb - 1) / hpb;
+    dim3 grid(M, groups + (v_freq ? (KV + hpb - 1) / hpb : 0));
     const int threads = hd <= 64 ? 64 : 128;
     if (dtype == TP_BF16)
-        rope_kv_write_k<bf16_t><<<grid, threads, 0, s>>>((bf16_t*)q, q_stride, (bf16_t*)k, k_stride, (const bf16_t*)v, v_stride, H, KV, hd,
-            inv_freq, rot, row_seq, row_pos, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool, page, rows_cap, pin, hpb, pairing);
+        rope_kv_write_k<bf16_t><<<grid, threads, 0, s>>>((bf16_t*)q, q_stride, (bf16_t*)k, k_stride, (bf16_t*)v, v_stride, H, KV, hd,
+            inv_freq, rot, v_freq, v_rot, groups, row_seq, row_pos, new_len, table, table_w, (bf16_t*)k_pool, (bf16_t*)v_pool, page, rows_cap, pin, hpb, pairing);
     else if (dtype == TP_F32)
-        rope_kv_write_k<float><<<grid, threads, 0, s>>>((float*)q, q_stride, (float*)k, k_stride, (const float*)v, v_stride, H, KV, hd,
-            inv_freq, rot, row_seq, row_pos, new_len, table, table_w, (float*)k_pool, (float*)v_pool, page, rows_cap, pin, hpb, pairing);
+        rope_kv_write_k<float><<<grid, threads, 0, s>>>((float*)q, q_stride, (float*)k, k_stride, (float*)v, v_stride, H, KV, hd,
+            inv_freq, rot, v_freq, v_rot, groups, row_seq, row_pos, new_len, table, table_w, (float*)k_pool, (float*)v_pool, page, rows_cap, pin, hpb, pairing);
     else return tp_fail("rope_kv_write: unknown dtype %d", dtype);
     return tp_check_launch("rope_kv_write");
 }

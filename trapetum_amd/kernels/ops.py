@@ -33,7 +33,7 @@ _CORE_SIGS = {
     "tp_mul_sigmoid": [_P, _L, _P, _L, _I, _I, _I, _P],
     "tp_gather_rows": [_P, _P, _P, _I, _I, _I, _P],
     "tp_sum_slices": [_P, _I, _L, _P, _I, _L, _P],
-    "tp_rope_kv_write": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _P],
+    "tp_rope_kv_write": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _I, _P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _P],
     "tp_kv_write": [_P, _L, _P, _L, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _P],
     "tp_gated_act": [_P, _P, _I, _I, _I, _I, _F, _F, _P],
     "tp_linear": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _F, _F, _P, _L, _I, _I, _P],
@@ -921,10 +921,13 @@ class HipOps:
                    x.shape[1], x.shape[0], self._stream())
         return out
 
+    turns_values = True                                  # `rope_kv_write` takes value_freq
+
     def rope_kv_write(self, q, k, v, H, KV, hd, inv_freq, rotary_dim, row_seq, row_pos, new_len, table,
-                      k_pool, v_pool, rows_cap, pairing="halves", write=True, pin=0):
+                      k_pool, v_pool, rows_cap, pairing="halves", write=True, pin=0, value_freq=None):
         """Rotate q and k in place and write k, v into the cache.  write=False: rotate only (a step whose attention
         reads the cache as earlier steps left it caches its rows afterwards, with `kv_write`).
+        value_freq: float32 [pairs], the values turn by their position too, over twice as many of their elements (None: they do not).
         pairing: one of ROPE_PAIRINGS, which elements of a head turn together."""
         if pairing not in ROPE_PAIRINGS:
             raise KernelError(f"rope_kv_write: pairing '{pairing}' has no kernel ({', '.join(ROPE_PAIRINGS)})")
@@ -936,6 +939,10 @@ class HipOps:
         if rotary_dim:
             if inv_freq is None or inv_freq.dtype != torch.float32 or inv_freq.numel() != rotary_dim // 2:
                 raise KernelError(f"rope_kv_write: a rotation over {rotary_dim} needs float32 inv_freq [{rotary_dim // 2}]")
+        if value_freq is not None:
+            self._dev(value_freq)
+            if k is None or pairing != "halves" or value_freq.dtype != torch.float32 or not value_freq.is_contiguous() or not 0 < 2 * value_freq.numel() <= hd:
+                raise KernelError(f"rope_kv_write: values that turn need keys beside them, pairs of halves and float32 frequencies of at most {hd // 2} pairs")
         for t, n in ((row_seq, m), (row_pos, m)):
             if t.dtype != torch.int32 or t.numel() != n:
                 raise KernelError("rope_kv_write: row_seq and row_pos must be int32, one entry per row")
@@ -951,7 +958,8 @@ class HipOps:
             self._check_pools("rope_kv_write", q.dtype, new_len.numel(), KV, hd, new_len, table, k_pool, v_pool)
             page, table_w = k_pool.shape[2], table.shape[1]
         self._call(self.lib, "tp_rope_kv_write", q.data_ptr(), qs, kp or None, ks, vp or None, vs, _code(q.dtype), m, H, KV, hd,
-                   inv_freq.data_ptr() if rotary_dim else None, rotary_dim, row_seq.data_ptr(), row_pos.data_ptr(),
+                   inv_freq.data_ptr() if rotary_dim else None, rotary_dim, value_freq.data_ptr() if value_freq is not None else None,
+                   2 * value_freq.numel() if value_freq is not None else 0, row_seq.data_ptr(), row_pos.data_ptr(),
                    new_len.data_ptr(), table.data_ptr() if write else None, table_w,
                    k_pool.data_ptr() if write else None, v_pool.data_ptr() if write else None,
                    page, rows_cap if write else 0, int(pin) if write else 0, ROPE_PAIRINGS[pairing], self._stream())

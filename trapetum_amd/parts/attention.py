@@ -376,8 +376,12 @@ class Attention(Mixer):
         else:
             q, k, v = qkv, None, None
         more.update(self._positional(ctx, qkv[:, self.gate_column:self.gate_column + H]))
+        turned = {}                                          # values that turn do so with the queries and keys where the kernel can
         if self.value_freq is not None:
-            self._turn(ctx, v, KV, self.value_freq)
+            if getattr(ops, "turns_values", False) and self.position.rotary_dim:
+                turned = dict(value_freq=self.value_freq)
+            else:
+                self._turn(ctx, v, KV, self.value_freq)
         # Sequences that go on by several tokens (or some start while others go on) see cached positions and the
         # step's own rows.  The attention reads the cached ones where they lie, as earlier steps left them, and the
         # step's rows from the step; only then are the step's rows cached: in a window's ring without a row to spare
@@ -386,7 +390,7 @@ class Attention(Mixer):
         if self.position.rotary_dim or not owns_cache:
             ops.rope_kv_write(q, k, v, H, KV, hd, self.inv_freq, self.position.rotary_dim,
                               ctx.row_seq, ctx.row_pos, ctx.new_len, table, k_pool, v_pool, rows_cap,
-                              write=not extend, **pin)
+                              write=not extend, **pin, **turned)
         elif not extend:                                     # nothing turns: the rows are cached as they are
             ops.kv_write(k, v, KV, hd, ctx.row_seq, ctx.row_pos, ctx.new_len, table, k_pool, v_pool, rows_cap, **pin)
         if ctx.mode == "decode":
