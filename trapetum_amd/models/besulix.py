@@ -34,7 +34,7 @@ def build_spec(c: BesulixConfig) -> ModelSpec:
                                   "head_temperature": "temp", "sink": "sink", "value_rotation": a.rot.base, "precise_weights": True})
             right = ("time_mix", {"hidden_size": D, "num_heads": r.heads, "head_dim": r.dim, "norm_eps": c.norm_eps})
             mixer = ("parallel", {"hidden_size": D, "left": left, "right": right, "combine": "weighted_sum",
-                                  "weights": (m.left_scale, m.right_scale)})
+                                  "weights": (m.left_scale, m.right_scale), "deferred": True, "whole": True})
         prefixes = {"mixer": p + "mix.", "pre_mixer_norm": p + "norm1"}
         ff = None
         if l.mlp is not None:

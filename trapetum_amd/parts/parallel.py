@@ -3,7 +3,7 @@
 combine "norm_mean": each output is divided by its root mean square over the model width and multiplied by a gain of
 its own (used as stored), in float32, before the two are averaged.  combine "weighted_sum": the outputs are added as
 they are, in float32, each times a constant of the model (`weights`); there are no gains.  With `deferred` that sum is left
-to the block's add (`ops.WeightedRows`), each side's last product in the form it has (K slices too).  The two mixers are any registered mixers; at most one of them may
+to the block's add (`ops.WeightedRows`), each side's last product in the form it has (K slices too), or in float32 (`whole`).  The two mixers are any registered mixers; at most one of them may
 keep tensors per token (it becomes this mixer's cache, so that another layer's run can read it), and the states they
 declare by name are kept under "left." and "right.".
 """
@@ -15,7 +15,7 @@ from .base import Mixer
 
 class ParallelMixers(Mixer):
     def __init__(self, hidden_size, left, right, eps=0.0, prefixes=("left.", "right."), tensors=("left.out", "right.out"),
-                 combine="norm_mean", weights=(1.0, 1.0), deferred=False):
+                 combine="norm_mean", weights=(1.0, 1.0), deferred=False, whole=False):
         if combine not in ("norm_mean", "weighted_sum"):
             raise ValueError(f"two mixers side by side are combined by norm_mean or weighted_sum, not '{combine}'")
         self.hidden_size, self.eps = int(hidden_size), float(eps)
@@ -26,7 +26,7 @@ class ParallelMixers(Mixer):
         self.deferred = bool(deferred)
         if self.deferred and combine != "weighted_sum":
             raise ValueError("only a weighted sum can be left to the block's add")
-        if combine == "weighted_sum" and not self.deferred:
+        if combine == "weighted_sum" and (whole or not self.deferred):
             import torch
             for m in self.sides:                     # the sum is formed in float32 from float32 products where a side can give them
                 if hasattr(m, "output_dtype"):
