@@ -1,10 +1,12 @@
 """The generation loop's decisions, on the CPU: batching, stops, early ends, slot reuse, limits."""
+import numpy as np
 import pytest
 import torch
 
 from trapetum_amd.cache import CacheError
 from trapetum_amd.engine.generate import generate, plan_batch
 from trapetum_amd.sampling import SamplingParams, initial_state, xorshift64
+from trapetum_amd.sampling.sampler import RequestSampling, draw
 
 from .cpu_engine import load_cpu_model
 from .plain import gemma2_plain as plain
@@ -89,6 +91,16 @@ def test_sampling_is_per_request(setup):
             seq.append(tok)
             recent.append(tok)
         assert together[i] == out, i
+
+
+@pytest.mark.parametrize("n,twice", [(1, False), (8, False), (64, False), (30, True)])
+def test_draws_of_several_requests_are_each_one_s_own(n, twice):
+    ours, alone = ([RequestSampling(7, 3 * i, [1]) for i in range(n)] for _ in range(2))
+    rows = [*range(n), *([0, 5] if twice else [])]
+    for _ in range(50):
+        got = np.asarray(draw([ours[i] for i in rows]), dtype=np.float32)
+        assert got.tolist() == [alone[i].next_uniform() for i in rows]
+    assert [r.state for r in ours] == [r.state for r in alone]
 
 
 def test_generator_matches_reference_xorshift():

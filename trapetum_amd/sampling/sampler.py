@@ -19,6 +19,7 @@ import torch
 MASK64 = (1 << 64) - 1
 RECENT_WINDOW = 128          # tokens the repetition penalty looks back over (serve.rs:327)
 MAX_TOP_K = 1024
+TO_UNIT = 1.0 / (1 << 53)    # a power of two: the product is the quotient
 
 
 @dataclasses.dataclass
@@ -69,6 +70,21 @@ class RequestSampling:
         self.recent.append(token)
 
 
+def draw(requests):
+    """`next_uniform` of each request, not yet rounded to float32 (what takes them does: an array of C floats or of numpy's).
+    The generator is written out: the calls were most of what the host did for a choice (64 requests 29 us, so 7.7; as the
+    steps of an array 6.8, and of 8 requests 3.5 against 1.4)."""
+    out = []
+    for r in requests:
+        s = r.state
+        s ^= (s << 13) & MASK64
+        s ^= s >> 7
+        s ^= (s << 17) & MASK64
+        r.state = s
+        out.append((s >> 11) * TO_UNIT)
+    return out
+
+
 class Sampler:
     def __init__(self, rt, params):
         params.validate()
@@ -114,7 +130,7 @@ class Sampler:
             ops.apply_repetition_penalty(logits, self.rt.upload_i32(recent), p.repetition_penalty)
         if p.temperature <= 0:
             return ops.argmax(logits)
-        uniforms = [r.next_uniform() for r in requests]
+        uniforms = draw(requests)
         if len(uniforms) > getattr(ops, "HOST_UNIFORMS", 0):              # more than go along with the launch (or kernels that take none)
             uniforms = self.rt.upload_i32(np.asarray(uniforms, dtype=np.float32).view(np.int32)).view(torch.float32)
         return ops.sample(logits, p.temperature, p.top_k, p.top_p, uniforms)
