@@ -957,9 +957,8 @@ def time_besulix_kernels(engine, cfg, batch, context, prefill_tokens):
                 prod("left_qkv_bias", [(lambda b=b: products(ops, [(x, b.mixer.sides[0].w_qkv, bf, b.mixer.sides[0].b_qkv)])) for b in par], left.w_qkv)
                 qkv = torch.randn((rows, (H + 2 * KV) * row), device=dev).to(bf)
                 q, k, v = qkv[:, :H * row], qkv[:, H * row:(H + KV) * row], qkv[:, (H + KV) * row:]
-                one([lambda: left._turn(ctx, v, KV, left.value_freq)] * 16, name="turn_values", bytes_each=rows * KV * row * 4.0)
                 one([lambda: ops.rope_kv_write(q, k, v, H, KV, row, left.inv_freq, left.position.rotary_dim, ctx.row_seq, ctx.row_pos,
-                                               ctx.new_len, table, kp, vp, cap)] * 16, name="rope_kv_write", bytes_each=rows * (H + 3 * KV) * row * 4.0)
+                                               ctx.new_len, table, kp, vp, cap, value_freq=left.value_freq)] * 16, name="rope_kv_write", bytes_each=rows * (H + 4 * KV) * row * 4.0)
                 more = dict(chunk=left.chunk, head_scale=left.temperature, sink=left.sink)
                 seen = min(context, (context - 1) % left.chunk + 1) if left.chunk else context
                 if decode:
@@ -1001,7 +1000,9 @@ def time_besulix_kernels(engine, cfg, batch, context, prefill_tokens):
                 yn = torch.randn((rows, inner), device=dev).to(bf)
                 prod("right_o", [(lambda b=b: ops.linear(yn, b.mixer.sides[1].w["o"], f32)) for b in par], right.w["o"])
                 oa, ob = torch.randn((rows, D), device=dev), torch.randn((rows, D), device=dev)
-                one([lambda: ops.weighted_sum(oa, 0.8, ob, 0.9)] * 16, name="weighted_sum", bytes_each=rows * D * 12.0)
+                stream, gain = torch.randn((rows, D), device=dev), torch.ones(D, device=dev)
+                one([lambda: ops.join_rms_norm(stream, oa, ob, gain, 1e-6, bf, wa=0.8, wb=0.9)] * 16, name="weighted_sum_add_norm",
+                    bytes_each=rows * D * 18.0)
             if mem:
                 e = entry(mem)
                 ctx.entry = ctx.cache_owner = e
