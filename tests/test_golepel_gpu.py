@@ -216,6 +216,28 @@ def test_head_linear(rt, m, h, n, k, lead):
     assert bool((wide[:, :, :lead] == 7.0).all())
 
 
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("m,h,n,k,lead", [(1, 2, 16, 32, 0), (16, 3, 40, 288, 8), (5, 2, 7, 96, 16), (15, 1, 17, 256, 8), (4, 16, 128, 192, 64), (17, 2, 24, 64, 0)])
+def test_head_linear_of_few_rows(rt, m, h, n, k, lead, gated):
+    """Up to 16 rows with K in whole steps of the matrix instruction (and one row more): every output within its own rounding
+    (bf16: 2^-8 of it) and 2^-20 of its terms' sum of absolute values (float32 sums of up to 288 products, 2^-24 each, in a tree
+    of the instruction's); the gate's sigmoid, a few units of 2^-23, lies inside that."""
+    x = rnd(m, h, lead + k, seed=72).to(rt.dtype).to(DEV)
+    w = rnd(h, n, k, seed=73, scale=0.3).to(rt.dtype).to(DEV)
+    gate = rnd(m, h * n + 3, seed=74).to(rt.dtype).to(DEV)[:, :h * n] if gated else None
+    xd, wd = x[:, :, lead:].double().cpu(), w.double().cpu()
+    want, size = torch.einsum("mhk,hnk->mhn", xd, wd), torch.einsum("mhk,hnk->mhn", xd.abs(), wd.abs())
+    if gated:
+        s = torch.sigmoid(gate.double().cpu()).view(m, h, n)
+        want, size = want * s, size * s
+    own = 2.0 ** -8 if rt.dtype == torch.bfloat16 else 2.0 ** -23
+    limit = own * want.abs() + (2.0 ** -20 if rt.dtype == torch.bfloat16 else 288 * 2.0 ** -24) * size
+    wide = torch.full((m, h, lead + n), 7.0, dtype=rt.dtype, device=DEV)
+    for got in (rt.ops.head_linear(x[:, :, lead:], w, gate=gate), rt.ops.head_linear(x[:, :, lead:], w, wide[:, :, lead:], gate=gate)):
+        assert bool(((got.double().cpu() - want).abs() <= limit).all())
+    assert bool((wide[:, :, :lead] == 7.0).all())
+
+
 @pytest.mark.parametrize("H", [4, 24])              # 24: more heads than a decode launch takes, run in groups
 @pytest.mark.parametrize("page,counts", [(16, (15, 1, 1, 1, 31, 2, 1, 40, 1, 1, 1, 1, 1, 2)), (64, (64, 1, 30, 1, 1, 1, 1, 1))])
 def test_latent_attention_sharp_scores(rt, page, counts, H):
