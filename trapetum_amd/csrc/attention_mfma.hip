@@ -552,7 +552,7 @@ attn_decode_combine_k(const float* __restrict__ ws_o, const float* __restrict__ 
     const int tid = threadIdx.x, lane = tid & 63, last = nsplit - 1;
     // the first 16 slices' sums are asked for before the weights are known: both come from memory at the same time
     constexpr int FIRST = 16, GROUP = 8;
-    const int d = tid < HD ? tid : HD - 1;                       // the block has max(HD, 64) threads
+    const int d = tid < HD ? tid : HD - 1;                       // the block has whole waves: every lane of each has a slice's weight
     const float2* ml = reinterpret_cast<const float2*>(ws_ml) + at;
     const float* sums = ws_o + (size_t)at * HD;
     const float2 ml0 = ml[lane < last ? lane : last];
@@ -644,7 +644,7 @@ static int decode_launch(DecodeArgs a, int n_seq, void* workspace, hipStream_t s
     else attn_decode_k<16><<<grid, DTH, 0, s>>>(a);
     if (int rc = tp_check_launch("attention decode")) return rc;
     if (a.nsplit > 1) {
-        attn_decode_combine_k<<<n_seq * a.H, HD < 64 ? 64 : HD, 0, s>>>(a.ws_o, a.ws_ml, a.nsplit, a.out, a.sink, a.H, a.by_position);
+        attn_decode_combine_k<<<n_seq * a.H, (HD + 63) / 64 * 64, 0, s>>>(a.ws_o, a.ws_ml, a.nsplit, a.out, a.sink, a.H, a.by_position);
         return tp_check_launch("attention decode (combine)");
     }
     return 0;
