@@ -542,17 +542,19 @@ attn_decode_k(DecodeArgs a) {
 
 // The slices of one (sequence, head): weights exp(m_s - max m) / sum, then every thread adds its head elements in slice
 // order.  Loads are unconditional (a slice without keys left its sum unwritten: its weight is zero and the value is
-// replaced by zero).  Few blocks, each of which runs its code once and waits for it: every wave forms the weights for
-// itself, slice s in lane s, and takes them lane by lane into scalar registers, without LDS or a barrier (8 sequences of
-// 700 keys with 8 heads of 256: 4.4 us with one wave's weights in LDS, 3.6 so; both launches 13.8 / 13.0, 11.0 / 9.9 of one sequence).
-__global__ void __launch_bounds__(256)
+// replaced by zero).  Little work, each part of which runs its code once and waits for it: a wave is a block and has 64 of
+// the head's elements; it forms the weights for itself, slice s in lane s, and takes them lane by lane into scalar registers,
+// without LDS or a barrier.  The attention's two launches, with 8 heads of 256 on 4 kv heads, by a block a head that forms its weights
+// once through LDS, by a block of such waves, by a wave a block: 8 sequences of 700 keys 13.8, 13.0, 12.8 us; one 11.0, 9.9, 9.7; two of
+// 7,000 in 128 slices 27.3, 26.2, 25.5.
+__global__ void __launch_bounds__(64)
 attn_decode_combine_k(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, int nsplit,
                       bf16_t* __restrict__ out, const float* __restrict__ sink, int H, TpPositional by_position) {
     const unsigned at = blockIdx.x * (unsigned)nsplit;           // blockIdx.x = sequence * heads + head
-    const int tid = threadIdx.x, lane = tid & 63, last = nsplit - 1;
+    const int lane = threadIdx.x, tid = blockIdx.y * 64 + lane, last = nsplit - 1;
     // the first 16 slices' sums are asked for before the weights are known: both come from memory at the same time
     constexpr int FIRST = 16, GROUP = 8;
-    const int d = tid < HD ? tid : HD - 1;                       // the block has whole waves: every lane of each has a slice's weight
+    const int d = tid < HD ? tid : HD - 1;                       // (a whole wave: every lane has a slice's weight)
     const float2* ml = reinterpret_cast<const float2*>(ws_ml) + at;
     const float* sums = ws_o + (size_t)at * HD;
     const float2 ml0 = ml[lane < last ? lane : last];
@@ -644,7 +646,7 @@ static int decode_launch(DecodeArgs a, int n_seq, void* workspace, hipStream_t s
     else attn_decode_k<16><<<grid, DTH, 0, s>>>(a);
     if (int rc = tp_check_launch("attention decode")) return rc;
     if (a.nsplit > 1) {
-        attn_decode_combine_k<<<n_seq * a.H, (HD + 63) / 64 * 64, 0, s>>>(a.ws_o, a.ws_ml, a.nsplit, a.out, a.sink, a.H, a.by_position);
+        attn_decode_combine_k<<<dim3(n_seq * a.H, (HD + 63) / 64), 64, 0, s>>>(a.ws_o, a.ws_ml, a.nsplit, a.out, a.sink, a.H, a.by_position);
         return tp_check_launch("attention decode (combine)");
     }
     return 0;
